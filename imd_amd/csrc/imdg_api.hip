@@ -42,6 +42,11 @@ hipError_t launch_copyrec(const StepArgs<R>&, int, hipStream_t);
 template <typename R>
 hipError_t launch_stress(const StepArgs<R>&, const TabDev<R>*, double*,
                          double*, int, hipStream_t);
+template <typename R>
+hipError_t launch_export(const StepArgs<R>&, int* const[2], long,
+                         const ExportDst&, int, hipStream_t);
+hipError_t launch_unsort(const RepDev*, Ctl*, const int*, int* const[2], long,
+                         const double*, int, double*, int, hipStream_t);
 void launch_build(const BuildArgs&, int, hipStream_t);
 const char* noalloc_message();
 void launch_check(const RepDev*, Ctl*, const int*, const double4*,
@@ -168,6 +173,10 @@ struct imdg_ctx {
   bool stress_valid = false;     // d_stress holds the last step's tensor
   double* d_stress = nullptr;    // 6 per slot: xx yy zz yz zx xy
   double* d_spart = nullptr;     // 6 per IMDG_BLOCK block
+  // results in input order on their way to the caller (imdg_get_atoms,
+  // imdg_get_stress); allocated at their first use, freed with the atoms
+  double* d_out = nullptr;
+  size_t out_len = 0;
   bool atoms_set = false;
   long target_steps = 0;
   // profiling
@@ -238,6 +247,8 @@ void free_all(imdg_ctx* c) {
   c->d_stress = nullptr;
   c->d_spart = nullptr;
   c->stress_valid = false;
+  c->d_out = nullptr;
+  c->out_len = 0;
 }
 
 void vec_prod(const double* u, const double* v, double* w) {
@@ -1103,25 +1114,37 @@ int build_until_fits(imdg_ctx* c) {
 // Device copies of the per-slot arrays needed to map results back.
 struct SlotView {
   Ctl ctl;
-  std::vector<double4> pos, mom;
-  std::vector<int> aid, acell, nnb;
+  std::vector<int> aid;
 };
 
-int read_slots(imdg_ctx* c, SlotView& v, bool state) {
+int read_slots(imdg_ctx* c, SlotView& v) {
   int rc = read_ctl(c, &v.ctl);
   if (rc) return rc;
   size_t ns = c->nslots;
   v.aid.resize(ns);
   HIPCHK(c, hipMemcpy(v.aid.data(), c->d_aid[v.ctl.rec_cur], sizeof(int) * ns,
                       hipMemcpyDeviceToHost));
-  if (state) {
-    v.pos.resize(ns);
-    v.mom.resize(ns);
-    HIPCHK(c, hipMemcpy(v.pos.data(), c->d_pos[v.ctl.pos_cur],
-                        sizeof(double4) * ns, hipMemcpyDeviceToHost));
-    HIPCHK(c, hipMemcpy(v.mom.data(), c->d_mom[v.ctl.pos_cur],
-                        sizeof(double4) * ns, hipMemcpyDeviceToHost));
-  }
+  return IMDG_OK;
+}
+
+// Room for len doubles of results in input order.
+int reserve_out(imdg_ctx* c, size_t len) {
+  if (c->d_out && len <= c->out_len) return IMDG_OK;
+  dfree(c, c->d_out);
+  c->d_out = nullptr;
+  c->out_len = 0;
+  int rc = dalloc(c, (void**)&c->d_out, sizeof(double) * len);
+  if (rc) return rc;
+  c->out_len = len;
+  return IMDG_OK;
+}
+
+// Waits for an export launch; an error if it met a slot without an atom.
+int export_check(imdg_ctx* c) {
+  Ctl h;
+  int rc = read_ctl(c, &h);
+  if (rc) return rc;
+  if (h.export_bad) return fail(c, IMDG_ERR_STATE, "a slot has no atom");
   return IMDG_OK;
 }
 
@@ -1803,7 +1826,7 @@ int imdg_get_eeam(imdg_ctx* c, double* P, double* dm) {
   hipSetDevice(c->dev);
   HIPCHK(c, hipStreamSynchronize(c->stream));
   SlotView v;
-  int rc = read_slots(c, v, false);
+  int rc = read_slots(c, v);
   if (rc) return rc;
   size_t ns = c->nslots;
   std::vector<double> hp(ns), hd(ns);
@@ -1846,10 +1869,10 @@ int imdg_get_stress(imdg_ctx* c, double* per_atom, double* total) {
     return fail(c, IMDG_ERR_STATE,
                 "no stress tensor of the last step (imdg_set_stress, then "
                 "imdg_run or imdg_move_atoms)");
-  SlotView v;
-  int rc = read_slots(c, v, false);
+  Ctl h;
+  int rc = read_ctl(c, &h);
   if (rc) return rc;
-  if (v.ctl.frozen)
+  if (h.frozen)
     return fail(c, IMDG_ERR_STATE, "list overflow pending (imdg_sync first)");
   if (total) {
     std::vector<double> sp((size_t)6 * c->nblk);
@@ -1865,20 +1888,14 @@ int imdg_get_stress(imdg_ctx* c, double* per_atom, double* total) {
     }
   }
   if (per_atom) {
-    std::vector<double> st((size_t)6 * c->nslots);
-    HIPCHK(c, hipMemcpy(st.data(), c->d_stress, sizeof(double) * st.size(),
-                        hipMemcpyDeviceToHost));
-    for (int r = 0; r < c->nrep; r++) {
-      const RepDev& R = c->rep[r];
-      for (int k = 0; k < R.natoms; k++) {
-        int s = R.atom_off + k;
-        long in = v.aid[s];
-        if (in < 0 || in >= c->natoms_tot)
-          return fail(c, IMDG_ERR_STATE, "slot %d has no atom", s);
-        for (int q = 0; q < 6; q++)
-          per_atom[(size_t)6 * in + q] = st[(size_t)6 * s + q];
-      }
-    }
+    const size_t n = c->natoms_tot;
+    if ((rc = reserve_out(c, 6 * n))) return rc;
+    HIPCHK(c, launch_unsort(c->d_rep, c->d_ctl, c->d_blk_rep, c->d_aid, n,
+                            c->d_stress, 6, c->d_out, c->nblk, c->stream));
+    if ((rc = export_check(c))) return rc;
+    if (n)
+      HIPCHK(c, hipMemcpy(per_atom, c->d_out, sizeof(double) * 6 * n,
+                          hipMemcpyDeviceToHost));
   }
   return IMDG_OK;
 }
@@ -1910,56 +1927,36 @@ int imdg_sync(imdg_ctx* c) {
 int imdg_get_atoms(imdg_ctx* c, double* x, double* p, double* f, double* epot,
                    double* rho, double* df) {
   if (!c || !c->atoms_set) return IMDG_ERR_ARG;
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  SlotView v;
-  int rc = read_slots(c, v, true);
+  // the wanted arrays one after the other in d_out
+  const struct {
+    double* host;
+    size_t comp;
+  } want[6] = {{x, 3}, {p, 3}, {f, 3}, {epot, 1}, {rho, 1}, {df, 1}};
+  const size_t n = c->natoms_tot;
+  size_t len = 0;
+  for (auto& w : want)
+    if (w.host) len += w.comp * n;
+  int rc = reserve_out(c, len);
   if (rc) return rc;
-  size_t ns = c->nslots;
-  std::vector<double> hf(4 * ns), he(ns), hr(ns), hb(4 * ns);
-  if (c->mixed) {
-    std::vector<float> t4(4 * ns), t(ns);
-    HIPCHK(c, hipMemcpy(t4.data(), c->d_frc, 4 * ns * 4, hipMemcpyDeviceToHost));
-    for (size_t k = 0; k < 4 * ns; k++) hf[k] = t4[k];
-    HIPCHK(c, hipMemcpy(t4.data(), c->d_recb, 4 * ns * 4, hipMemcpyDeviceToHost));
-    for (size_t k = 0; k < 4 * ns; k++) hb[k] = t4[k];
-    HIPCHK(c, hipMemcpy(t.data(), c->d_epot, ns * 4, hipMemcpyDeviceToHost));
-    for (size_t k = 0; k < ns; k++) he[k] = t[k];
-    HIPCHK(c, hipMemcpy(t.data(), c->d_rho, ns * 4, hipMemcpyDeviceToHost));
-    for (size_t k = 0; k < ns; k++) hr[k] = t[k];
-  } else {
-    HIPCHK(c, hipMemcpy(hf.data(), c->d_frc, 4 * ns * 8, hipMemcpyDeviceToHost));
-    HIPCHK(c, hipMemcpy(hb.data(), c->d_recb, 4 * ns * 8, hipMemcpyDeviceToHost));
-    HIPCHK(c, hipMemcpy(he.data(), c->d_epot, ns * 8, hipMemcpyDeviceToHost));
-    HIPCHK(c, hipMemcpy(hr.data(), c->d_rho, ns * 8, hipMemcpyDeviceToHost));
+  double* dev[6];
+  size_t at = 0;
+  for (int k = 0; k < 6; k++) {
+    dev[k] = want[k].host ? c->d_out + at : nullptr;
+    if (want[k].host) at += want[k].comp * n;
   }
-  bool eam = c->tab[1].present;
-  for (int r = 0; r < c->nrep; r++) {
-    const RepDev& R = c->rep[r];
-    for (int k = 0; k < R.natoms; k++) {
-      int s = R.atom_off + k;
-      long in = v.aid[s];
-      if (in < 0 || in >= c->natoms_tot)
-        return fail(c, IMDG_ERR_STATE, "slot %d has no atom", s);
-      if (x) {
-        x[3 * in] = v.pos[s].x;
-        x[3 * in + 1] = v.pos[s].y;
-        x[3 * in + 2] = v.pos[s].z;
-      }
-      if (p) {
-        p[3 * in] = v.mom[s].x;
-        p[3 * in + 1] = v.mom[s].y;
-        p[3 * in + 2] = v.mom[s].z;
-      }
-      if (f) {
-        f[3 * in] = hf[4 * s];
-        f[3 * in + 1] = hf[4 * s + 1];
-        f[3 * in + 2] = hf[4 * s + 2];
-      }
-      if (epot) epot[in] = he[s];
-      if (rho) rho[in] = eam ? hr[s] : 0.0;
-      if (df) df[in] = eam ? hb[4 * s + 3] : 0.0;
-    }
-  }
+  const ExportDst d = {dev[0], dev[1], dev[2], dev[3], dev[4], dev[5]};
+  if (c->mixed)
+    HIPCHK(c, launch_export<float>(step_args<float>(c), c->d_aid, n, d,
+                                   c->nblk, c->stream));
+  else
+    HIPCHK(c, launch_export<double>(step_args<double>(c), c->d_aid, n, d,
+                                    c->nblk, c->stream));
+  if ((rc = export_check(c))) return rc;
+  for (int k = 0; k < 6; k++)
+    if (dev[k] && n)
+      HIPCHK(c, hipMemcpy(want[k].host, dev[k],
+                          sizeof(double) * want[k].comp * n,
+                          hipMemcpyDeviceToHost));
   return IMDG_OK;
 }
 
@@ -2024,7 +2021,7 @@ int imdg_get_cells(imdg_ctx* c, int* cell3) {
   if (!c || !c->atoms_set || !cell3) return IMDG_ERR_ARG;
   HIPCHK(c, hipStreamSynchronize(c->stream));
   SlotView v;
-  int rc = read_slots(c, v, false);
+  int rc = read_slots(c, v);
   if (rc) return rc;
   size_t ns = c->nslots;
   std::vector<int> hc(ns);
@@ -2049,7 +2046,7 @@ int imdg_get_pairs(imdg_ctx* c, long* out, long cap, long* npairs) {
   HIPCHK(c, hipStreamSynchronize(c->stream));
   if (!c->d_nbr) return fail(c, IMDG_ERR_STATE, "no list");
   SlotView v;
-  int rc = read_slots(c, v, false);
+  int rc = read_slots(c, v);
   if (rc) return rc;
   size_t ns = c->nslots;
   std::vector<int> hn(ns), hc(ns);

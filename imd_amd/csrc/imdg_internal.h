@@ -150,6 +150,7 @@ struct Ctl {
   int is_short;
   int tiles_fallback;     // blocks whose tile exceeded the tile cap
   int exact_pairs;        // list candidates decided by the FP64 expression
+  int export_bad;         // a slot without an atom met by an export kernel
   unsigned int done[DC_N];
   long steps_done;
 };
@@ -284,6 +285,12 @@ struct StepArgs {
   const Tab64* tab64;     // EEAM energy term (tab64[1]); FP32 kernels only
   int lpa_den, lpa_frc;   // lanes per slot of the density / force loops
   int thr_den, thr_frc;   // threads per block of the density / force loops
+};
+
+// Destination of the export kernel: the caller's arrays on the device, in
+// input order (NULL: not wanted).
+struct ExportDst {
+  double *x, *p, *f, *epot, *rho, *df;
 };
 
 struct BuildArgs {
