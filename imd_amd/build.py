@@ -25,11 +25,18 @@ HOSTLIB = os.path.join(HOST, "libimdhost.so")
 HOSTEXE = os.path.join(HOST, "imd_gpu")
 
 # (source, extra flags, object): the step kernels are compiled once per
-# precision so that the two halves build in parallel
+# neighbour loop and precision so that the parts build in parallel
 HIP_UNITS = [
     ("imdg_build.hip", [], "imdg_build.o"),
-    ("imdg_step.hip", ["-DIMDG_STEP_FP32"], "imdg_step_f32.o"),
-    ("imdg_step.hip", ["-DIMDG_STEP_FP64"], "imdg_step_f64.o"),
+    ("imdg_step.hip", ["-DIMDG_STEP_PART=0"], "imdg_step.o"),
+    ("imdg_step.hip", ["-DIMDG_STEP_PART=1", "-DIMDG_STEP_REAL=float"],
+     "imdg_step_den32.o"),
+    ("imdg_step.hip", ["-DIMDG_STEP_PART=1", "-DIMDG_STEP_REAL=double"],
+     "imdg_step_den64.o"),
+    ("imdg_step.hip", ["-DIMDG_STEP_PART=2", "-DIMDG_STEP_REAL=float"],
+     "imdg_step_frc32.o"),
+    ("imdg_step.hip", ["-DIMDG_STEP_PART=2", "-DIMDG_STEP_REAL=double"],
+     "imdg_step_frc64.o"),
     ("imdg_api.hip", [], "imdg_api.o"),
     ("imdg_export.hip", [], "imdg_export.o"),
     ("imdg_noalloc.hip", [], "imdg_noalloc.o"),

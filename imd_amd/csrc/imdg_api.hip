@@ -150,11 +150,14 @@ struct imdg_ctx {
   int force_mode = 0;                  // 0 one species, 1 shared grid,
                                        // 2 several, 3 several on one grid
   int lpa_den = 0, lpa_frc = 0;        // lanes per slot of the two loops
+  bool lpa_auto_den = false;           // ... chosen by plan_steps for the
+  bool lpa_auto_frc = false;           // system's size, not by the user
   int thr_den = 0, thr_frc = 0;        // threads per block (0: default)
   int units_cap = 0;                   // wavefront partial slots allocated
   int lds_den_lo = 0, lds_den_n = 0;   // knots staged by the density loop
   int lds_frc_lo = 0, lds_frc_n = 0;   // knots staged by the force loop
   int grid_den = 0, grid_frc[2] = {0, 0}, grid_move = 0;
+  int split_den = 1, split_frc[2] = {1, 1};  // units a chunk is split into
   int units_max = 0;
   // one captured step (rebuild chain + density + force), replayed by
   // imdg_run when graphs are on (IMDG_GRAPH=1) and profiling is off
@@ -680,6 +683,33 @@ int upload_tables(imdg_ctx* c) {
   return IMDG_OK;
 }
 
+// Units a chunk of a neighbour loop is split into (1, 2 or 4, at most its
+// lanes per slot) for nchunk chunks on `waves` resident wavefronts: the
+// split with the shortest run of units per wavefront, a unit taking its
+// share of the chunk's neighbour work plus a fixed part (the per-atom work
+// runs with 1/split of the lanes).  The fixed part is EPI chunks' worth.
+int pick_split(int nchunk, int waves, int lanes) {
+  const double EPI = 0.15;
+  int best = 1;
+  double cost = 1e300;
+  for (int s = 1; s <= std::min(lanes, 4); s *= 2) {
+    const long rounds = ((long)nchunk * s + waves - 1) / std::max(1, waves);
+    const double t = rounds * (1.0 / s + EPI);
+    if (t < cost) {
+      cost = t;
+      best = s;
+    }
+  }
+  return best;
+}
+
+// Blocks of a loop of `units` units: no more than there are units (a block beyond that would only stage tables and add
+// a partial), a multiple of the 8 XCDs.
+int pick_grid(int resident, long units) {
+  if (units >= resident) return resident;
+  return std::min<long>(resident, (units + 7) / 8 * 8);
+}
+
 // Launch plan of the persistent step kernels: which knots each neighbour
 // loop stages in LDS (all knots of the tables it reads, when they fit next
 // to the kernel's static LDS) and the resident grid of each kernel.
@@ -697,12 +727,25 @@ int plan_steps(imdg_ctx* c) {
   c->force_mode = !nt1 ? (c->knots_jointn >= 0 ? 3 : 2)
                        : (c->knots_joint >= 0 ? 1 : 0);
   int mode = c->force_mode;
-  // default shapes (what imdg_autotune picks on the 2M-atom EAM crystal):
-  // four lanes per atom and full blocks, except the FP64 force loop, whose
-  // registers leave one lane per atom and 512 threads fastest
+  // Default lanes per slot.  Four lanes make the shortest pass: they win
+  // while every pass of the system can have a wavefront of its own (up to
+  // 65,000 atoms on 256 CUs: 32,000 atoms 47.1 us per step, 49.4 with two
+  // lanes).  Beyond that the FP32 one-grid loops are fastest with two, whose
+  // lists need less padding (256,000 atoms 86.7 us, 88.0 with four; 864,000
+  // atoms 215, 242).  FP64 and the other loops keep four (LJ crystal of
+  // 4,000 atoms in FP64: 39.3 us, 47.0 with one lane; 256,000 atoms 175,
+  // 179).
   const bool fp32 = sizeof(R) == 4;
-  if (c->lpa_den <= 0) c->lpa_den = 4;
-  if (c->lpa_frc <= 0) c->lpa_frc = fp32 ? 4 : 1;
+  const bool spread = (long)c->nchunk * 4 <= (long)c->ncu * IMDG_STEP_WAVES;
+  if (c->lpa_den <= 0) {
+    const bool onegrid = c->knots_dpoly >= 0 || c->knots_drho >= 0;
+    c->lpa_den = fp32 && onegrid && !spread ? 2 : 4;
+    c->lpa_auto_den = true;
+  }
+  if (c->lpa_frc <= 0) {
+    c->lpa_frc = fp32 && mode == 1 && !spread ? 2 : 4;
+    c->lpa_auto_frc = true;
+  }
   if (c->thr_den <= 0) c->thr_den = IMDG_STEP_THREADS;
   if (c->thr_frc <= 0) c->thr_frc = force_threads<R>(mode);
   int td = c->thr_den, tf = c->thr_frc;
@@ -733,6 +776,12 @@ int plan_steps(imdg_ctx* c) {
         step_grid_density<R>(nt1, false, 0, c->ncu, c->lpa_den, td, cub,
                              c->eeam);
   }
+  c->split_den = 1;
+  if (he) {
+    c->split_den =
+        pick_split(c->nchunk, c->grid_den * (td / IMDG_WAVE), c->lpa_den);
+    c->grid_den = pick_grid(c->grid_den, (long)c->nchunk * c->split_den);
+  }
   // force: pair and rho knots (or the interleaved table)
   if (mode == 1) {
     int len = c->tab[0].len[0];
@@ -762,7 +811,13 @@ int plan_steps(imdg_ctx* c) {
     }
     c->grid_frc[integ] = g;
   }
-  c->grid_move = step_grid_move<R>(c->ncu);
+  for (int integ = 0; integ < 2; integ++) {
+    c->split_frc[integ] = pick_split(
+        c->nchunk, c->grid_frc[integ] * (tf / IMDG_WAVE), c->lpa_frc);
+    c->grid_frc[integ] = pick_grid(c->grid_frc[integ],
+                                   (long)c->nchunk * c->split_frc[integ]);
+  }
+  c->grid_move = pick_grid(step_grid_move<R>(c->ncu), c->nchunk);
   if (c->grid_frc[0] == 0 || c->grid_frc[1] == 0 || c->grid_move == 0 ||
       (he && c->grid_den == 0))
     return fail(c, IMDG_ERR_HIP, "cannot size the persistent step kernels");
@@ -827,6 +882,8 @@ StepArgs<R> step_args(imdg_ctx* c) {
   a.final_inline = c->final_inline ? 1 : 0;
   a.lpa_den = c->lpa_den;
   a.lpa_frc = c->lpa_frc;
+  a.split_den = c->split_den;
+  a.split_frc = 1;  // set with the force launch
   a.rho = (R*)c->d_rho;
   a.epot = (R*)c->d_epot;
   a.frc = (R4*)c->d_frc;
@@ -976,6 +1033,7 @@ hipError_t enqueue_forces_t(imdg_ctx* c, bool integrate, bool store) {
   a.lds_lo = c->lds_frc_lo;
   a.lds_n = c->lds_frc_n;
   int grid = c->grid_frc[integrate ? 1 : 0];
+  a.split_frc = c->split_frc[integrate ? 1 : 0];
   a.unitsB = grid;
   {
     ProfScope ps(c, KC_FORCE);
@@ -1168,6 +1226,7 @@ int time_loop(imdg_ctx* c, bool density, int reps, double* ms,
     a.lds_lo = c->lds_frc_lo;
     a.lds_n = c->lds_frc_n;
     const int grid = c->grid_frc[integrate ? 1 : 0];
+    a.split_frc = c->split_frc[integrate ? 1 : 0];
     a.unitsB = grid;
     return launch_force<R>(a, t, c->force_mode, integrate, grid, c->stream);
   };
@@ -1200,6 +1259,7 @@ int autotune_t(imdg_ctx* c, int reps, imdg_tuning* out) {
   const int thr_f[4] = {256, 512, 768, 1024};
   int rc;
   double best_d = 0.0, best_f = 0.0;
+  c->lpa_auto_den = c->lpa_auto_frc = false;
   if (c->tab[1].present) {
     int bl = c->lpa_den, bt = c->thr_den;
     best_d = 1e300;
@@ -1554,6 +1614,8 @@ int imdg_set_atoms(imdg_ctx* c, int nrep, const imdg_replica* reps,
     return rc;
   c->nchunk = c->nslots / IMDG_CHUNK;
   c->part_chunk = nrep > 1 ? 1 : 0;
+  if (c->lpa_auto_den) c->lpa_den = 0;  // chosen anew for this system
+  if (c->lpa_auto_frc) c->lpa_frc = 0;
   c->units_cap = 0;  // partials are allocated below, for any plan
   if ((rc = c->mixed ? plan_steps<float>(c) : plan_steps<double>(c)))
     return rc;
@@ -1570,7 +1632,8 @@ int imdg_set_atoms(imdg_ctx* c, int nrep, const imdg_replica* reps,
   {
     // room for any launch plan: at most 32 resident wavefronts per CU
     c->units_cap = std::max(c->units_max, 32 * c->ncu);
-    size_t units = std::max(c->nchunk, c->units_cap);
+    size_t units = std::max((size_t)c->nchunk * (c->part_chunk ? 4 : 1),
+                            (size_t)c->units_cap);
     ALLOC(c->d_partA, sizeof(double) * units);
     ALLOC(c->d_partB, sizeof(double) * PB_N * units);
   }
@@ -2207,6 +2270,8 @@ int imdg_set_tuning(imdg_ctx* c, const imdg_tuning* t) {
     return fail(c, IMDG_ERR_ARG, "invalid tuning (lanes 1/2/4, threads a "
                 "multiple of 64 up to %d)", IMDG_STEP_THREADS);
   int old[4] = {c->lpa_den, c->thr_den, c->lpa_frc, c->thr_frc};
+  bool was_auto[2] = {c->lpa_auto_den, c->lpa_auto_frc};
+  c->lpa_auto_den = c->lpa_auto_frc = false;
   c->lpa_den = t->density_lanes;
   c->thr_den = t->density_threads;
   c->lpa_frc = t->force_lanes;
@@ -2218,6 +2283,8 @@ int imdg_set_tuning(imdg_ctx* c, const imdg_tuning* t) {
     c->lpa_den = old[0];
     c->thr_den = old[1];
     c->lpa_frc = old[2];
+    c->lpa_auto_den = was_auto[0];
+    c->lpa_auto_frc = was_auto[1];
     c->thr_frc = old[3];
     int rc = plan(c);
     if (rc) return rc;

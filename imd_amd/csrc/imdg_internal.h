@@ -283,6 +283,7 @@ struct StepArgs {
                           // its 2F' (rec_b.w), not a gather of atype
   const double2* knots64; // FP64 knots of the embedding (tab64[0]) and the
   const Tab64* tab64;     // EEAM energy term (tab64[1]); FP32 kernels only
+  int split_den, split_frc;  // units a chunk is split into (1, 2 or 4)
   int lpa_den, lpa_frc;   // lanes per slot of the density / force loops
   int thr_den, thr_frc;   // threads per block of the density / force loops
 };

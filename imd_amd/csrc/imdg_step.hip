@@ -69,31 +69,61 @@ __device__ __forceinline__ uint4 nt_load4(const void* p) {
   return make_uint4(v.x, v.y, v.z, v.w);
 }
 
-// Chunks of one wavefront: c, c + stride, ... below c1.  Blocks are
-// dispatched round-robin over the 8 XCDs; with xcd_remap the waves of XCD x
-// walk the x-th eighth of the chunks, so the neighbour records they gather
-// stay in that XCD's L2.  unit: the wavefront's partial slot.
+// Units of one wavefront: q, q + stride, ... below q1.  A unit is a 64-slot
+// chunk or, with split > 1, one of its split equal parts (whole passes over
+// 64 / L slots): systems with fewer chunks than the chip holds wavefronts
+// spread over more of them that way.  Blocks are dispatched round-robin over
+// the 8 XCDs; with xcd_remap the waves of XCD x walk the x-th eighth of the
+// units, so the neighbour records they gather stay in that XCD's L2.  Waves
+// of a block take consecutive units (their records share the CU's L1),
+// unless every wave has at most one: then consecutive blocks do, so that a
+// small system uses every CU before a second wave of any.
 struct Sched {
-  int c, c1, stride, unit;
+  int q, q1, stride;
 };
 
-__device__ __forceinline__ Sched make_sched(int nchunk, int xcd_remap) {
+__device__ __forceinline__ Sched make_sched(int nunit, int xcd_remap) {
   Sched s;
   int nwb = blockDim.x / IMDG_WAVE, w = threadIdx.x / IMDG_WAVE;
-  s.unit = blockIdx.x * nwb + w;
-  if (xcd_remap && (gridDim.x & 7) == 0) {
-    int x = blockIdx.x & 7, bx = blockIdx.x >> 3;
-    int per = (nchunk + 7) >> 3;
-    int c0 = min(x * per, nchunk);
-    s.c1 = min(c0 + per, nchunk);
-    s.stride = (gridDim.x >> 3) * nwb;
-    s.c = c0 + bx * nwb + w;
-  } else {
-    s.c1 = nchunk;
-    s.stride = gridDim.x * nwb;
-    s.c = s.unit;
+  int nb = gridDim.x, b = blockIdx.x, q0 = 0;
+  s.q1 = nunit;
+  if (xcd_remap && (nb & 7) == 0) {
+    int x = b & 7, per = (nunit + 7) >> 3;
+    q0 = min(x * per, nunit);
+    s.q1 = min(q0 + per, nunit);
+    nb >>= 3;
+    b >>= 3;
   }
+  s.stride = nb * nwb;
+  s.q = q0 + (s.q1 - q0 <= s.stride ? w * nb + b : b * nwb + w);
   return s;
+}
+
+// Passes [p0, p1) of unit q's chunk (L lanes per slot, L passes a chunk).
+struct Unit {
+  int c, p0, p1;
+};
+template <int L>
+__device__ __forceinline__ Unit unit_of(int q, int split) {
+  Unit u;
+  if (L == 1 || split == 1) {
+    u.c = q;
+    u.p0 = 0;
+    u.p1 = L;
+  } else {
+    const int sh = split == 2 ? 1 : 2, n = L >> sh;
+    u.c = q >> sh;
+    u.p0 = (q & (split - 1)) * n;
+    u.p1 = u.p0 + n;
+  }
+  return u;
+}
+
+// Whether the unit's passes cover chunk slot l.
+template <int L>
+__device__ __forceinline__ bool unit_has(const Unit& u, int l) {
+  const int p = l / (IMDG_WAVE / L);
+  return L == 1 || (p >= u.p0 && p < u.p1);
 }
 
 // Cell-offset vectors of a replica, in the force precision, into the
@@ -150,16 +180,16 @@ __device__ __forceinline__ void add_part(double (&acc)[PB_N],
     acc[q] = (q == PB_MAXD) ? fmax(acc[q], v[q]) : acc[q] + v[q];
 }
 
-// Partials of one chunk (part_chunk) or accumulation into the wavefront's
+// Partials of one unit (part_chunk) or accumulation into the wavefront's
 // running sums.
 __device__ __forceinline__ void put_part(double* partB, int part_chunk,
-                                         int c, double (&v)[PB_N],
+                                         int q0, double (&v)[PB_N],
                                          double (&acc)[PB_N]) {
   if (part_chunk) {
     wave_reduce_part(v);
     if ((threadIdx.x & (IMDG_WAVE - 1)) == 0) {
 #pragma unroll
-      for (int q = 0; q < PB_N; q++) partB[(size_t)c * PB_N + q] = v[q];
+      for (int q = 0; q < PB_N; q++) partB[(size_t)q0 * PB_N + q] = v[q];
     }
   } else {
     add_part(acc, v);
@@ -211,11 +241,22 @@ __device__ __forceinline__ void flag_short(Ctl* ctl, int is_short) {
     atomicOr(&ctl->is_short, 1);
 }
 
-// Knots of the launch's LDS range (block-wide, before any wave loop).
+// Knots of the launch's LDS range (block-wide, before any wave loop), eight
+// loads of a thread in flight together: every launch stages up to 120 KB per
+// CU, which at one load a trip is a tenth of a small system's step.
 template <typename R2>
 __device__ __forceinline__ void stage_knots(const R2* __restrict__ g, int lo,
                                             int n, R2* lds) {
-  for (int k = threadIdx.x; k < n; k += blockDim.x) lds[k] = g[lo + k];
+  const int T = blockDim.x;
+  for (int k0 = threadIdx.x; k0 < n; k0 += 8 * T) {
+    R2 v[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++)
+      if (k0 + u * T < n) v[u] = g[lo + k0 + u * T];
+#pragma unroll
+    for (int u = 0; u < 8; u++)
+      if (k0 + u * T < n) lds[k0 + u * T] = v[u];
+  }
 }
 
 template <typename R>
@@ -372,12 +413,13 @@ __device__ void finalize_step(StepArgs<R>& a, bool forces, bool moved,
     // several replicas: one wavefront per replica, chunk partials
     for (int r = fblk * nw + w; r < a.nrep; r += nfblk * nw) {
       const RepDev& Rp = a.rep[r];
-      int c0 = Rp.blk_off * (IMDG_BLOCK / IMDG_CHUNK);
-      int c1 = (Rp.blk_off + Rp.nblk) * (IMDG_BLOCK / IMDG_CHUNK);
+      const int c0 = Rp.blk_off * (IMDG_BLOCK / IMDG_CHUNK);
+      const int c1 = c0 + Rp.nblk * (IMDG_BLOCK / IMDG_CHUNK);
       double s[PB_N + 1], c[PB_N + 1];
 #pragma unroll
       for (int q = 0; q <= PB_N; q++) s[q] = c[q] = 0.0;
-      for (int u = c0 + l; u < c1; u += IMDG_WAVE) {
+      for (int u = c0 * a.split_frc + l; u < c1 * a.split_frc;
+           u += IMDG_WAVE) {
         const double* pb = a.partB + (size_t)u * PB_N;
 #pragma unroll
         for (int q = 0; q < PB_N; q++) {
@@ -386,8 +428,11 @@ __device__ void finalize_step(StepArgs<R>& a, bool forces, bool moved,
           else
             kahan_add(s[q], c[q], pb[q]);
         }
-        if (forces && a.has_eam) kahan_add(s[PB_N], c[PB_N], a.partA[u]);
       }
+      if (forces && a.has_eam)
+        for (int u = c0 * a.split_den + l; u < c1 * a.split_den;
+             u += IMDG_WAVE)
+          kahan_add(s[PB_N], c[PB_N], a.partA[u]);
       wave_combine(s, c);
       if (l == 0) {
         double tot[PB_N + 1];
@@ -1405,14 +1450,16 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS)
   const int kb0 = tr.off[0] - klo, len0 = tr.len[0];
   const R b0 = tr.begin[0], e0 = tr.end[0], is0 = tr.invstep[0];
 
-  Sched S = make_sched(a.nchunk, a.xcd_remap);
+  Sched S = make_sched(a.nchunk * a.split_den, a.xcd_remap);
   const int lane = threadIdx.x & (IMDG_WAVE - 1);
   const int ga = lane / L, gs = lane % L;
   R4* off = wofs[threadIdx.x / IMDG_WAVE][0];
   R4* olo = wofs[threadIdx.x / IMDG_WAVE][1];
   int cur = -1, is_short = 0;
   double acc = 0.0;
-  for (int c = S.c; c < S.c1; c += S.stride) {
+  for (int q = S.q; q < S.q1; q += S.stride) {
+    const Unit un = unit_of<L>(q, a.split_den);
+    const int c = un.c;
     int r = a.blk_rep[c / (IMDG_BLOCK / IMDG_CHUNK)];
     const RepDev& Rp = a.rep[r];
     if (r != cur) {
@@ -1424,7 +1471,7 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS)
       if (a.list16) w16 = chunk_bases(a.cmeta, c, lane, off);
     R rho_keep = (R)0, pee_keep = (R)0;
 #pragma unroll 1
-    for (int p = 0; p < L; p++) {
+    for (int p = un.p0; p < un.p1; p++) {
       int i = c * IMDG_CHUNK + p * (IMDG_WAVE / L) + ga;
       R rho = (R)0, pee = (R)0;
       if (i - Rp.atom_off < Rp.natoms) {
@@ -1500,7 +1547,7 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS)
     if (EE) pee_keep = to_slot_lane<L>(pee_keep, lane);
     int i = c * IMDG_CHUNK + lane;
     double emb = 0.0;
-    if (i - Rp.atom_off < Rp.natoms) {
+    if (i - Rp.atom_off < Rp.natoms && unit_has<L>(un, lane)) {
       R4 ui = rec[i];
       int it = NT1 ? 0 : (int)ui.w;
       R rho = rho_keep;
@@ -1572,7 +1619,7 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS)
     }
     if (a.part_chunk) {
       double s = wave_sum(emb);
-      if (lane == 0) a.partA[c] = s;
+      if (lane == 0) a.partA[q] = s;
     } else {
       acc += emb;
     }
@@ -1630,14 +1677,16 @@ __global__ void __launch_bounds__((ForceThreads<R, MODE>::value))
   const R rb = HE ? tr.begin[0] : (R)0, re = HE ? tr.end[0] : (R)0,
           ris = HE ? tr.invstep[0] : (R)0, r2is = HE ? tr.twoistep[0] : (R)0;
 
-  Sched S = make_sched(a.nchunk, a.xcd_remap);
+  Sched S = make_sched(a.nchunk * a.split_frc, a.xcd_remap);
   const int lane = threadIdx.x & (IMDG_WAVE - 1);
   const int ga = lane / L, gs = lane % L;
   R4* off = wofs[threadIdx.x / IMDG_WAVE][0];
   R4* olo = wofs[threadIdx.x / IMDG_WAVE][1];
   int cur = -1, is_short = 0;
   double acc[PB_N] = {0, 0, 0, 0, 0, 0};
-  for (int c = S.c; c < S.c1; c += S.stride) {
+  for (int q = S.q; q < S.q1; q += S.stride) {
+    const Unit un = unit_of<L>(q, a.split_frc);
+    const int c = un.c;
     int r = a.blk_rep[c / (IMDG_BLOCK / IMDG_CHUNK)];
     const RepDev& Rp = a.rep[r];
     if (r != cur) {
@@ -1651,7 +1700,7 @@ __global__ void __launch_bounds__((ForceThreads<R, MODE>::value))
     // of the pair gradients' FP32 remainders (FP32 one-grid loops)
     R kx = 0, ky = 0, kz = 0, kep = 0, kvir = 0, kvlo = 0;
 #pragma unroll 1
-    for (int p = 0; p < L; p++) {
+    for (int p = un.p0; p < un.p1; p++) {
       int i = c * IMDG_CHUNK + p * (IMDG_WAVE / L) + ga;
       R fx = 0, fy = 0, fz = 0, ep = 0, vir = 0, vlo = 0;
       if (i - Rp.atom_off < Rp.natoms) {
@@ -1762,7 +1811,7 @@ __global__ void __launch_bounds__((ForceThreads<R, MODE>::value))
     if (sizeof(R) == 4) kvlo = to_slot_lane<L>(kvlo, lane);
     int i = c * IMDG_CHUNK + lane;
     double v[PB_N] = {0, 0, 0, 0, 0, 0};
-    if (i - Rp.atom_off < Rp.natoms) {
+    if (i - Rp.atom_off < Rp.natoms && unit_has<L>(un, lane)) {
       if (a.store) {
         // per-atom energy: half of every pair term plus F(rho_i)
         R ei = (R)0.5 * kep + (HE ? a.epot[i] : (R)0);
@@ -1781,7 +1830,7 @@ __global__ void __launch_bounds__((ForceThreads<R, MODE>::value))
       if (INTEGRATE)
         integrate_slot(a, Rp, r, i, (double)kx, (double)ky, (double)kz, v);
     }
-    put_part(a.partB, a.part_chunk, c, v, acc);
+    put_part(a.partB, a.part_chunk, q, v, acc);
   }
   flush_part(a.partB, a.part_chunk, acc);
   flag_short(a.ctl, is_short);
@@ -1796,7 +1845,7 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS) k_move(StepArgs<R> a) {
   Sched S = make_sched(a.nchunk, a.xcd_remap);
   const int lane = threadIdx.x & (IMDG_WAVE - 1);
   double acc[PB_N] = {0, 0, 0, 0, 0, 0};
-  for (int c = S.c; c < S.c1; c += S.stride) {
+  for (int c = S.q; c < S.q1; c += S.stride) {
     int r = a.blk_rep[c / (IMDG_BLOCK / IMDG_CHUNK)];
     const RepDev& Rp = a.rep[r];
     int i = c * IMDG_CHUNK + lane;
@@ -2287,32 +2336,38 @@ hipError_t launch_stress(const StepArgs<R>& a, const TabDev<R>* tabs,
   return hipGetLastError();
 }
 
-#define IMDG_INSTANTIATE(R)                                                   \
-  template int step_grid_density<R>(bool, bool, size_t, int, int, int,     \
-                                    bool, bool);                              \
-  template int step_grid_force<R>(int, bool, bool, bool, bool, size_t, int,  \
-                                  int, int, bool, bool);                      \
-  template int force_threads<R>(int);                                         \
-  template int step_grid_move<R>(int);                                        \
-  template hipError_t launch_density<R>(const StepArgs<R>&,                   \
-                                        const TabDev<R>*, bool, int,          \
-                                        hipStream_t);                         \
-  template hipError_t launch_force<R>(const StepArgs<R>&, const TabDev<R>*,   \
-                                      int, bool, int, hipStream_t);           \
-  template hipError_t launch_move<R>(const StepArgs<R>&, int, hipStream_t);   \
-  template hipError_t launch_copyrec<R>(const StepArgs<R>&, int, hipStream_t); \
-  template hipError_t launch_stress<R>(const StepArgs<R>&, const TabDev<R>*,  \
-                                       double*, double*, int, hipStream_t);   \
-  template hipError_t launch_finalize<R>(const StepArgs<R>&, bool, bool,     \
+#define IMDG_INSTANTIATE_DEN(R)                                             \
+  template int step_grid_density<R>(bool, bool, size_t, int, int, int,      \
+                                    bool, bool);                            \
+  template hipError_t launch_density<R>(const StepArgs<R>&,                 \
+                                        const TabDev<R>*, bool, int,        \
+                                        hipStream_t);
+#define IMDG_INSTANTIATE_FRC(R)                                             \
+  template int step_grid_force<R>(int, bool, bool, bool, bool, size_t, int, \
+                                  int, int, bool, bool);                    \
+  template int force_threads<R>(int);                                       \
+  template hipError_t launch_force<R>(const StepArgs<R>&, const TabDev<R>*, \
+                                      int, bool, int, hipStream_t);
+#define IMDG_INSTANTIATE_REST(R)                                            \
+  template int step_grid_move<R>(int);                                      \
+  template hipError_t launch_move<R>(const StepArgs<R>&, int, hipStream_t); \
+  template hipError_t launch_copyrec<R>(const StepArgs<R>&, int,            \
+                                        hipStream_t);                       \
+  template hipError_t launch_stress<R>(const StepArgs<R>&,                  \
+                                       const TabDev<R>*, double*, double*,  \
+                                       int, hipStream_t);                   \
+  template hipError_t launch_finalize<R>(const StepArgs<R>&, bool, bool,    \
                                          hipStream_t);
 
-// One precision per object when IMDG_STEP_FP32 or IMDG_STEP_FP64 is
-// defined (the build compiles this file once per type, in parallel).
-#if defined(IMDG_STEP_FP32) || !defined(IMDG_STEP_FP64)
-IMDG_INSTANTIATE(float)
-#endif
-#if defined(IMDG_STEP_FP64) || !defined(IMDG_STEP_FP32)
-IMDG_INSTANTIATE(double)
+// One loop and precision per object: the build compiles this file once per
+// IMDG_STEP_PART and IMDG_STEP_REAL, in parallel.
+#if IMDG_STEP_PART == 1
+IMDG_INSTANTIATE_DEN(IMDG_STEP_REAL)
+#elif IMDG_STEP_PART == 2
+IMDG_INSTANTIATE_FRC(IMDG_STEP_REAL)
+#else
+IMDG_INSTANTIATE_REST(float)
+IMDG_INSTANTIATE_REST(double)
 #endif
 
 }  // namespace imdg

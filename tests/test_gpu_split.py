@@ -1,0 +1,54 @@
+"""Chunks of the neighbour loops split into units of some of their passes:
+systems of a few chunks (four units a chunk with four lanes), at sizes where
+four or two units a chunk are chosen and where the chunks fill the chip,
+against the oracle at the bars of the launch shapes; one wavefront's chunk
+that is not full; replicas, whose partial sums are per unit, over several
+steps and lanes."""
+import numpy as np
+import pytest
+
+from imd_amd import imdg as G
+from imd_amd import workloads as W
+
+from helpers import eam_tables, oracle_eam
+from test_gpu_tuning import TOL, _check_static
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("precision", [G.FP64, G.MIXED])
+@pytest.mark.parametrize("cells", [(5, 5, 5), (6, 5, 7), (23, 22, 21),
+                                   (28, 28, 28)])
+def test_units_match_oracle(cells, precision):
+    eam = eam_tables()
+    s = W.fcc_system(cells, 3.615, eam.masses, W.kT(600.0), 77, displace=0.03)
+    orc = oracle_eam(s, eam, nbl_margin=0.4, timestep=W.FS)
+    orc.calc_forces()
+    with G.eam_context(eam, [s], precision=precision) as gpu:
+        for lanes in (None, 4, 2, 1):
+            if lanes:
+                gpu.set_tuning(lanes, 1024, lanes, 512)
+            gpu.calc_forces()
+            _check_static(gpu, orc, *TOL[precision])
+
+
+@pytest.mark.parametrize("lanes", [1, 2, 4])
+def test_replica_units(lanes):
+    """The thermo records of a batch are those of each replica alone: FP64,
+    so the sums agree to rounding whatever their order (100 terms of 1e-16
+    each per atom, amplified over 10 steps by less than 10)."""
+    eam = eam_tables()
+    systems = [W.fcc_system(c, 3.615, eam.masses, W.kT(500.0), 5 + k,
+                            displace=0.02)
+               for k, c in enumerate(((5, 5, 5), (6, 6, 6), (9, 5, 7)))]
+    with G.eam_context(eam, systems, precision=G.FP64) as gpu:
+        gpu.set_tuning(lanes, 512, lanes, 512)
+        gpu.run(10)
+        th = gpu.thermo_history(0, 10)
+    for r, s in enumerate(systems):
+        with G.eam_context(eam, [s], precision=G.FP64) as one:
+            one.run(10)
+            t1 = one.thermo_history(0, 10)
+        scale = np.abs(t1[:, 0, 1:6]).max(axis=0) + 1e-300
+        scale[2] = np.abs(t1[:, 0, 1]).max()  # the virial's terms cancel
+        assert np.all(np.abs(th[:, r, 1:6] - t1[:, 0, 1:6]) <= 1e-12 * scale)
