@@ -139,6 +139,7 @@ struct imdg_ctx {
   int knots_pair = 0, knots_rho = 0;   // first knot of the rho / embed tables
   int knots_embed = 0;
   int knots_joint = -1;                // interleaved (pair, rho), one species
+  int knots_jval = -1;                 // FP64: interleaved table values
   int knots_dpoly = -1;                // FP32 rho segment polynomials
   int knots_jointn = -1;               // FP32, several species, one grid:
   int knots_dpolyn = -1;               // force and rho segment records
@@ -423,7 +424,8 @@ int upload_tables(imdg_ctx* c) {
   // for the force loop at an even knot index, for the len segments k, with
   // dv = p1 - p0 and d2v = p2 - 2 p1 + p0 as PAIR_INT2 forms them
   // (src/potaccess.h:347-349), in FP64 and then rounded once.
-  //   FP64: S[k] = (phi p0, phi dv, phi d2v, rho dv), then rho d2v[k].
+  //   FP64: S[k] = (phi p0, phi dv, phi d2v, rho dv), then rho d2v[k]; and
+  //         the rows (phi_k, rho_k), k = 0..len+1, for LDS.
   //   FP32: Q[k] = (phi p0, phi A, phi B, phi A_lo), then (rho A, rho D)[k],
   //         with A = dv - d2v/2, B = d2v/2, D = d2v: value p0 + chi (A +
   //         B chi) and gradient / (2 istep) A + D chi = A + B (2 chi)
@@ -432,7 +434,7 @@ int upload_tables(imdg_ctx* c) {
   //         zero: the reference evaluates it only at r^2 >= end, where the
   //         shifted radial tables vanish, so a clamp of the table argument
   //         replaces the cutoff tests.
-  c->knots_joint = -1;
+  c->knots_joint = c->knots_jval = -1;
   const HostTable &hp = c->tab[0], &hr = c->tab[1];
   bool same = !c->cubic && !c->eeam && c->cfg.ntypes == 1 && hp.present &&
               hr.present &&
@@ -465,6 +467,13 @@ int upload_tables(imdg_ctx* c) {
         R2 q;
         q.x = (R)d2v(hr, k);
         q.y = k + 1 < len ? (R)d2v(hr, k + 1) : (R)0;
+        kn.push_back(q);
+      }
+      c->knots_jval = (int)kn.size();
+      for (int k = 0; k < len + 2; k++) {
+        R2 q;
+        q.x = (R)at(hp, k);
+        q.y = (R)at(hr, k);
         kn.push_back(q);
       }
     } else {
@@ -727,15 +736,34 @@ int plan_steps(imdg_ctx* c) {
   c->force_mode = !nt1 ? (c->knots_jointn >= 0 ? 3 : 2)
                        : (c->knots_joint >= 0 ? 1 : 0);
   int mode = c->force_mode;
+  const bool fp32 = sizeof(R) == 4;
+  if (c->thr_den <= 0) c->thr_den = IMDG_STEP_THREADS;
+  if (c->thr_frc <= 0) c->thr_frc = force_threads<R>(mode);
+  int td = c->thr_den, tf = c->thr_frc;
+  // Staging the tables costs a launch 2 to 5 us, whatever the system's
+  // size: the loops of a small one read them from L2.  The lines (chunks
+  // per CU) lie where both are equally fast: FP32, 120 + 60 KB staged: 16,400
+  // atoms 45.5 us per step staged, 44.1 not, 32,000 atoms 44.0 and 46.2;
+  // the 32 KB of an LJ table in FP64 6,900 atoms 40.8 and 40.6, 32,000
+  // atoms 44.3 and 46.2; FP64 EAM, 80 + 80 KB and fewer wavefronts per CU:
+  // 55,000 atoms 69.9 and 69.1, 70,000 atoms 77.3 and 83.7.  The
+  // several-species loops always stage what fits: one more gather per
+  // neighbour each costs them as much (2,000 atoms 45.6 and 44.0, 32,000
+  // atoms 54.9 and 59.0).
+  const double stage_min = !nt1 ? 0.0 : !fp32 && he ? 3.5 : 1.5;
+  int no_lds = c->nchunk < stage_min * c->ncu;
+  if (const char* e = getenv("IMDG_TABLES_IN_LDS")) no_lds = (atoi(e) == 0);
+  // cubic segments, EEAM: the generic loops with the tables in HBM/L2
+  if (cub || c->eeam) no_lds = 1;
   // Default lanes per slot.  Four lanes make the shortest pass: they win
   // while every pass of the system can have a wavefront of its own (up to
   // 65,000 atoms on 256 CUs: 32,000 atoms 47.1 us per step, 49.4 with two
   // lanes).  Beyond that the FP32 one-grid loops are fastest with two, whose
   // lists need less padding (256,000 atoms 86.7 us, 88.0 with four; 864,000
-  // atoms 215, 242).  FP64 and the other loops keep four (LJ crystal of
-  // 4,000 atoms in FP64: 39.3 us, 47.0 with one lane; 256,000 atoms 175,
-  // 179).
-  const bool fp32 = sizeof(R) == 4;
+  // atoms 215, 242).  The FP64 one-grid force loop on staged tables has two
+  // wavefronts per SIMD and no latency to hide behind more lanes: one is
+  // fastest (256,000 atoms 124 us, 133 with four).  The other loops keep
+  // four (LJ crystal of 4,000 atoms in FP64: 39.3 us, 47.0 with one).
   const bool spread = (long)c->nchunk * 4 <= (long)c->ncu * IMDG_STEP_WAVES;
   if (c->lpa_den <= 0) {
     const bool onegrid = c->knots_dpoly >= 0 || c->knots_drho >= 0;
@@ -743,16 +771,11 @@ int plan_steps(imdg_ctx* c) {
     c->lpa_auto_den = true;
   }
   if (c->lpa_frc <= 0) {
-    c->lpa_frc = fp32 && mode == 1 && !spread ? 2 : 4;
+    c->lpa_frc = mode != 1 ? 4
+                 : fp32    ? (spread ? 4 : 2)
+                           : (no_lds ? 4 : 1);
     c->lpa_auto_frc = true;
   }
-  if (c->thr_den <= 0) c->thr_den = IMDG_STEP_THREADS;
-  if (c->thr_frc <= 0) c->thr_frc = force_threads<R>(mode);
-  int td = c->thr_den, tf = c->thr_frc;
-  int no_lds = 0;
-  if (const char* e = getenv("IMDG_TABLES_IN_LDS")) no_lds = (atoi(e) == 0);
-  // cubic segments, EEAM: the generic loops with the tables in HBM/L2
-  if (cub || c->eeam) no_lds = 1;
   // density: the rho knots (the several-species segment records stay in
   // HBM/L2: nt^2 columns)
   c->lds_den_lo = c->knots_rho;
@@ -785,8 +808,8 @@ int plan_steps(imdg_ctx* c) {
   // force: pair and rho knots (or the interleaved table)
   if (mode == 1) {
     int len = c->tab[0].len[0];
-    c->lds_frc_lo = c->knots_joint;
-    c->lds_frc_n = sizeof(R) == 8 ? 2 * len + (len + 1) / 2 : 3 * len;
+    c->lds_frc_lo = sizeof(R) == 8 ? c->knots_jval : c->knots_joint;
+    c->lds_frc_n = sizeof(R) == 8 ? len + 2 : 3 * len;
   } else if (mode == 3) {
     c->lds_frc_lo = c->knots_frho;
     c->lds_frc_n = nty * c->tab[1].len[0];
@@ -869,6 +892,7 @@ StepArgs<R> step_args(imdg_ctx* c) {
                    : 0;
   a.tab64 = (const Tab64*)c->d_tab64;
   a.joint = c->knots_joint;
+  a.jval = c->knots_jval;
   a.dpoly = c->knots_dpoly;
   a.jointn = c->knots_jointn;
   a.dpolyn = c->knots_dpolyn;

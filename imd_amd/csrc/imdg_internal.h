@@ -257,6 +257,8 @@ struct StepArgs {
   int lds_lo, lds_n;      // knots staged in LDS by this launch (n = 0: none)
   int joint;              // first knot of the interleaved single-species
                           // (pair, rho) table, -1 if there is none
+  int jval;               // FP64, with joint: first of the values (pair,
+                          // rho) the force loop stages in LDS
   int dpoly;              // first knot of the FP32 rho segment polynomials
                           // (one species), -1 if there are none
   int jointn, dpolyn;     // first knot of the FP32 several-species

@@ -1146,17 +1146,26 @@ __device__ __forceinline__ void force_group(
   }
 }
 
-// Four neighbours of the single-species force loop when the pair and rho
-// tables share their grid: one segment per neighbour, its record S[k] =
-// (phi p0, phi dv, phi d2v, rho dv) and Sr[k] = rho d2v.  The common factor
-// 2 istep of both gradients is applied once per atom by the caller (sums
-// s* are in units of 1 / (2 istep)); hFi = F'(rho_i) = 2F'/2.
-template <typename R, typename R4, typename PF>
+// Four neighbours of the FP64 single-species force loop when the pair and
+// rho tables share their grid: one segment per neighbour.  The common
+// factor 2 istep of both gradients is applied once per atom by the caller
+// (sums s* are in units of 1 / (2 istep)); hFi = F'(rho_i) = 2F'/2.
+//
+// LV: the table values themselves from LDS, V[k] = (phi_k, rho_k); p1 - p0
+// and p2 - 2 p1 + p0 are formed here, in the operations PAIR_INT2 forms them
+// with (the results are those of the records, bit for bit).  16 B per
+// segment, so 5,000 points take 80 KB of LDS; three 16 B reads per
+// neighbour and four more FP64 additions.  Otherwise the segment records
+// S[k] = (phi p0, phi dv, phi d2v, rho dv) and Sr[k] = rho d2v from L2: 40 B,
+// 200 KB for 5,000 points, which no LDS holds.  Those gathers bound the
+// loop: a step of 2,048,000 atoms takes 1590 us with the records, 908 with
+// the values (256,000 atoms 175, 124).
+template <bool LV, typename R, typename R4, typename R2, typename PF>
 __device__ __forceinline__ void force_group_sg(
     uint4 e4, PF pf, uint4& slot, const R4* __restrict__ rec,
     const R4* off, const R4& ui, R hFi, const R4* __restrict__ S,
-    const R* __restrict__ Sr, int len, R begin, R end, R invstep, R& sx,
-    R& sy, R& sz, R& ep, R& svir, R& r2min) {
+    const R* __restrict__ Sr, const R2* V, int len, R begin, R end, R invstep,
+    R& sx, R& sy, R& sz, R& ep, R& svir, R& r2min) {
   uint32_t en[4] = {e4.x, e4.y, e4.z, e4.w};
   R4 uj[4], o[4];
 #pragma unroll
@@ -1180,8 +1189,17 @@ __device__ __forceinline__ void force_group_sg(
   R d2r[4];
 #pragma unroll
   for (int u = 0; u < 4; u++) {
-    s4[u] = S[kk[u]];
-    d2r[u] = Sr[kk[u]];
+    if (LV) {
+      const R2 v0 = V[kk[u]], v1 = V[kk[u] + 1], v2 = V[kk[u] + 2];
+      s4[u].x = v0.x;
+      s4[u].y = v1.x - v0.x;
+      s4[u].z = v2.x - (R)2 * v1.x + v0.x;
+      s4[u].w = v1.y - v0.y;
+      d2r[u] = v2.y - (R)2 * v1.y + v0.y;
+    } else {
+      s4[u] = S[kk[u]];
+      d2r[u] = Sr[kk[u]];
+    }
   }
 #pragma unroll
   for (int u = 0; u < 4; u++) {
@@ -1753,16 +1771,19 @@ __global__ void __launch_bounds__((ForceThreads<R, MODE>::value))
                                              fz, ep, vir, vlo);
                            });
           } else {
+            // LT: the launch stages the table values, the records stay
+            // in L2
             const R4* __restrict__ S =
-                reinterpret_cast<const R4*>(K + (a.joint - klo));
+                reinterpret_cast<const R4*>(a.knots + a.joint);
             const R* __restrict__ Sr =
-                reinterpret_cast<const R*>(K + (a.joint - klo) + 2 * plen);
+                reinterpret_cast<const R*>(a.knots + a.joint + 2 * plen);
+            const R2* V = K + (a.jval - klo);
             list_walk<L>(nw, a.nnb[i],
                          [&](uint4 e4, ListRef<L> pf, uint4& slot) {
-                           force_group_sg<R>(e4, pf, slot, rec, off, ui,
-                                             (R)0.5 * dFi, S, Sr, plen, pb,
-                                             pe, pis, fx, fy, fz, ep, vir,
-                                             r2min);
+                           force_group_sg<LT>(e4, pf, slot, rec, off, ui,
+                                              (R)0.5 * dFi, S, Sr, V, plen,
+                                              pb, pe, pis, fx, fy, fz, ep,
+                                              vir, r2min);
                          });
           }
           is_short |= (r2min < pb);

@@ -1,7 +1,7 @@
 """Chunks of the neighbour loops split into units of some of their passes:
 systems of a few chunks (four units a chunk with four lanes), at sizes where
 four or two units a chunk are chosen and where the chunks fill the chip,
-against the oracle at the bars of the launch shapes; one wavefront's chunk
+with the tables staged or read from L2, against the oracle at the bars of the launch shapes; one wavefront's chunk
 that is not full; replicas, whose partial sums are per unit, over several
 steps and lanes."""
 import numpy as np
@@ -16,10 +16,14 @@ from test_gpu_tuning import TOL, _check_static
 pytestmark = pytest.mark.gpu
 
 
+@pytest.mark.parametrize("staged", ["default", "1"])
 @pytest.mark.parametrize("precision", [G.FP64, G.MIXED])
 @pytest.mark.parametrize("cells", [(5, 5, 5), (6, 5, 7), (23, 22, 21),
                                    (28, 28, 28)])
-def test_units_match_oracle(cells, precision):
+def test_units_match_oracle(cells, precision, staged, monkeypatch):
+    # tables from L2 (small systems) or staged in LDS
+    if staged != "default":
+        monkeypatch.setenv("IMDG_TABLES_IN_LDS", staged)
     eam = eam_tables()
     s = W.fcc_system(cells, 3.615, eam.masses, W.kT(600.0), 77, displace=0.03)
     orc = oracle_eam(s, eam, nbl_margin=0.4, timestep=W.FS)
@@ -30,6 +34,28 @@ def test_units_match_oracle(cells, precision):
                 gpu.set_tuning(lanes, 1024, lanes, 512)
             gpu.calc_forces()
             _check_static(gpu, orc, *TOL[precision])
+            if staged != "default":
+                assert gpu.info()["tables_in_lds"] == 3
+
+
+@pytest.mark.parametrize("npts", [5000, 5600, 700])
+def test_fp64_values_in_lds(npts, monkeypatch):
+    """The FP64 force loop on the staged table values gives the bits of the
+    records read from L2, over tables whose values fit in LDS and (5,600
+    points with the density loop's knots) nearly fill it."""
+    eam = W.johnson_eam(npts=npts)
+    s = W.fcc_system((7, 6, 6), 3.615, eam.masses, W.kT(900.0), 9,
+                     displace=0.08)
+    got = []
+    for lds in ("0", "1"):
+        monkeypatch.setenv("IMDG_TABLES_IN_LDS", lds)
+        with G.eam_context(eam, [s], precision=G.FP64) as gpu:
+            gpu.set_tuning(4, 512, 2, 512)
+            gpu.run(5)
+            got.append((gpu.atoms(), gpu.info()["tables_in_lds"]))
+    assert got[0][1] == 0 and got[1][1] == 3
+    for k, v in got[0][0].items():
+        assert np.array_equal(v, got[1][0][k]), k
 
 
 @pytest.mark.parametrize("lanes", [1, 2, 4])
