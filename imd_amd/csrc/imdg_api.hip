@@ -47,7 +47,7 @@ hipError_t launch_export(const StepArgs<R>&, int* const[2], long,
                          const ExportDst&, int, hipStream_t);
 hipError_t launch_unsort(const RepDev*, Ctl*, const int*, int* const[2], long,
                          const double*, int, double*, int, hipStream_t);
-void launch_build(const BuildArgs&, int, hipStream_t);
+void launch_build(const BuildArgs&, int, bool, hipStream_t);
 const char* noalloc_message();
 void launch_check(const RepDev*, Ctl*, const int*, const double4*,
                   const double4*, const double4*, double*, int, hipStream_t);
@@ -112,13 +112,13 @@ struct imdg_ctx {
   double4 *d_pos[2] = {nullptr, nullptr}, *d_mom[2] = {nullptr, nullptr};
   int* d_aid[2] = {nullptr, nullptr};
   double4* d_xnbl = nullptr;
-  int *d_cellid = nullptr, *d_cslot = nullptr, *d_acell = nullptr,
-      *d_perm = nullptr;
+  int *d_acell = nullptr, *d_bucket = nullptr;
+  int bucket_cap = 0;
+  Tile* d_tiles = nullptr;  // larger systems only (IMDG_TILE_FOLD)
   signed char* d_atype = nullptr;
   int *d_cell_cnt = nullptr, *d_cell_beg = nullptr, *d_cell_num = nullptr;
   int *d_cell_loc = nullptr, *d_tile_sum = nullptr, *d_tile_off = nullptr,
       *d_tile_rep = nullptr, *d_blkmax = nullptr;
-  Tile* d_tiles = nullptr;
   uint32_t* d_nbr = nullptr;
   size_t nbr_bytes = 0;
   int list_k = 0;  // longest list built so far, as last read by the host
@@ -930,6 +930,11 @@ StepArgs<R> step_args(imdg_ctx* c) {
   return a;
 }
 
+ListEnd list_end(imdg_ctx* c) {
+  return {c->d_ctl, c->d_rst, c->d_blk_rep, c->d_blkmax,
+          c->nblk,  c->nrep,  c->kmax};
+}
+
 BuildArgs build_args(imdg_ctx* c) {
   BuildArgs b;
   memset(&b, 0, sizeof b);
@@ -946,11 +951,11 @@ BuildArgs build_args(imdg_ctx* c) {
   b.xnbl = c->d_xnbl;
   b.rec_a = c->d_reca;
   b.mixed = c->mixed ? 1 : 0;
-  b.cellid = c->d_cellid;
-  b.cslot = c->d_cslot;
   b.acell = c->d_acell;
   b.atype = c->d_atype;
-  b.perm = c->d_perm;
+  b.bucket = c->d_bucket;
+  b.bucket_cap = c->bucket_cap;
+  b.scan_in_bin = c->ncells <= IMDG_SCAN_FOLD ? 1 : 0;
   b.cell_cnt = c->d_cell_cnt;
   b.cell_beg = c->d_cell_beg;
   b.cell_num = c->d_cell_num;
@@ -959,6 +964,7 @@ BuildArgs build_args(imdg_ctx* c) {
   b.tile_off = c->d_tile_off;
   b.tile_rep = c->d_tile_rep;
   b.blkmax = c->d_blkmax;
+  b.end = list_end(c);
   b.tiles = c->d_tiles;
   b.nbr = c->d_nbr;
   b.nnb = c->d_nnb;
@@ -1022,22 +1028,27 @@ void collect_profile(imdg_ctx* c) {
   c->pending.clear();
 }
 
+// Blocks of the cell sort: eight cells each, at most eight rounds of them.
 int grid_build(imdg_ctx* c) {
-  int g = (c->nslots + 255) / 256;
-  return std::max(1, std::min(g, 2048));
+  return std::max(1, std::min((c->ncells + 7) / 8, 2048));
 }
 
-int enqueue_build(imdg_ctx* c) {
+// The rebuild chain; done: end the rebuild in it (a step's density loop or
+// record copy does it otherwise).
+int enqueue_build(imdg_ctx* c, bool done) {
   ProfScope ps(c, KC_BUILD);
-  launch_build(build_args(c), grid_build(c), c->stream);
+  launch_build(build_args(c), grid_build(c), done, c->stream);
   HIPCHK(c, hipGetLastError());
   return IMDG_OK;
 }
 
 template <typename R>
-hipError_t enqueue_forces_t(imdg_ctx* c, bool integrate, bool store) {
+hipError_t enqueue_forces_t(imdg_ctx* c, bool integrate, bool store,
+                            bool end_rebuild) {
   StepArgs<R> a = step_args<R>(c);
   a.store = store ? 1 : 0;
+  a.end = list_end(c);
+  a.end_rebuild = end_rebuild ? 1 : 0;
   const TabDev<R>* t = (const TabDev<R>*)c->d_tabs;
   bool nt1 = c->cfg.ntypes == 1;
   hipError_t e;
@@ -1087,13 +1098,14 @@ hipError_t enqueue_move_t(imdg_ctx* c) {
 }
 
 // store: write rho, epot and frc (always without integration: the move
-// launch reads frc).
-int enqueue_forces(imdg_ctx* c, bool integrate, bool store = true) {
+// launch reads frc).  end_rebuild: the rebuild chain enqueued before ends
+// in this step's first loop.
+int enqueue_forces(imdg_ctx* c, bool integrate, bool store, bool end_rebuild) {
   store = store || !integrate;
   if (c->mixed)
-    HIPCHK(c, enqueue_forces_t<float>(c, integrate, store));
+    HIPCHK(c, enqueue_forces_t<float>(c, integrate, store, end_rebuild));
   else
-    HIPCHK(c, enqueue_forces_t<double>(c, integrate, store));
+    HIPCHK(c, enqueue_forces_t<double>(c, integrate, store, end_rebuild));
   HIPCHK(c, hipGetLastError());
   return IMDG_OK;
 }
@@ -1146,26 +1158,44 @@ size_t list_bytes(imdg_ctx* c, int kmax) {
   return (size_t)(c->nslots / IMDG_WAVE) * kmax * IMDG_WAVE * 4;
 }
 
-// Grow the list after an overflow and rebuild; *fixed = 1 if it had to.
+// Grow the list (or the cells' buckets) after an overflow and rebuild;
+// *fixed = 1 if it had to.
 int fix_overflow(imdg_ctx* c, int* fixed) {
   *fixed = 0;
   Ctl h;
   int rc = read_ctl(c, &h);
   if (rc) return rc;
   if (!h.frozen) return IMDG_OK;
-  int newk = std::max(c->kmax + IMDG_LIST_PAD, (int)ceil(h.kmax_seen * 1.2));
-  newk = (newk + IMDG_LIST_PAD - 1) / IMDG_LIST_PAD * IMDG_LIST_PAD;
   drop_graph(c);
-  dfree(c, c->d_nbr);
-  c->d_nbr = nullptr;
-  c->kmax = newk;
-  size_t bytes = list_bytes(c, newk);
-  if ((rc = dalloc(c, (void**)&c->d_nbr, bytes))) return rc;
-  c->nbr_bytes = bytes;
+  if (h.cell_over) {
+    // more atoms in a cell than its bucket has places: larger buckets, and
+    // the counters that the cell sort would have cleared
+    c->bucket_cap = (h.cell_over + h.cell_over / 4 + 15) / 8 * 8;
+    dfree(c, c->d_bucket);
+    c->d_bucket = nullptr;
+    if ((rc = dalloc(c, (void**)&c->d_bucket,
+                     sizeof(int) * c->bucket_cap * (size_t)c->ncells)))
+      return rc;
+    HIPCHK(c, hipMemsetAsync(c->d_cell_cnt, 0, sizeof(int) * c->ncells,
+                             c->stream));
+    int zero = 0;
+    HIPCHK(c, hipMemcpyAsync(&c->d_ctl->cell_over, &zero, sizeof(int),
+                             hipMemcpyHostToDevice, c->stream));
+  } else {
+    int newk =
+        std::max(c->kmax + IMDG_LIST_PAD, (int)ceil(h.kmax_seen * 1.2));
+    newk = (newk + IMDG_LIST_PAD - 1) / IMDG_LIST_PAD * IMDG_LIST_PAD;
+    dfree(c, c->d_nbr);
+    c->d_nbr = nullptr;
+    c->kmax = newk;
+    size_t bytes = list_bytes(c, newk);
+    if ((rc = dalloc(c, (void**)&c->d_nbr, bytes))) return rc;
+    c->nbr_bytes = bytes;
+  }
   int zero2[2] = {0, 0};  // frozen, overflow
   HIPCHK(c, hipMemcpyAsync(&c->d_ctl->frozen, zero2, 2 * sizeof(int),
                            hipMemcpyHostToDevice, c->stream));
-  if ((rc = enqueue_build(c))) return rc;
+  if ((rc = enqueue_build(c, true))) return rc;
   *fixed = 1;
   return IMDG_OK;
 }
@@ -1183,7 +1213,7 @@ int ensure_ready(imdg_ctx* c) {
 
 // Run the build chain until it fits (calc_forces / make_nblist path).
 int build_until_fits(imdg_ctx* c) {
-  int rc = enqueue_build(c);
+  int rc = enqueue_build(c, true);
   if (rc) return rc;
   for (int tries = 0; tries < 8; tries++) {
     int fixed = 0;
@@ -1512,7 +1542,7 @@ int imdg_set_atoms(imdg_ctx* c, int nrep, const imdg_replica* reps,
   c->in_off.assign(nrep, 0);
   long tot = 0;
   int slot = 0, cell = 0, stile = 0;
-  double kest = 0.0;
+  double kest = 0.0, percell = 0.0;
   for (int r = 0; r < nrep; r++) {
     RepDev& R = c->rep[r];
     memset(&R, 0, sizeof R);
@@ -1580,6 +1610,7 @@ int imdg_set_atoms(imdg_ctx* c, int nrep, const imdg_replica* reps,
     double dens = natoms[r] / fabs(vol);
     double rl = sqrt(R.cellsz);
     kest = std::max(kest, dens * 4.18879020478639 * rl * rl * rl);
+    percell = std::max(percell, (double)natoms[r] / R.ncells);
   }
   if (slot >= (1 << IMDG_IDX_BITS))
     return fail(c, IMDG_ERR_ARG, "too many atoms for 27-bit list indices");
@@ -1590,6 +1621,8 @@ int imdg_set_atoms(imdg_ctx* c, int nrep, const imdg_replica* reps,
   c->nstile = stile;
   c->kmax = std::max(16, (int)ceil(kest * c->cfg.nbl_size * 1.25));
   c->kmax = (c->kmax + IMDG_LIST_PAD - 1) / IMDG_LIST_PAD * IMDG_LIST_PAD;
+  // places of a cell's bucket: twice the mean (an overflow enlarges it)
+  c->bucket_cap = std::max(IMDG_BUCKET_MIN, (int)ceil(2 * percell) + 7) / 8 * 8;
 
   int rc;
 #define ALLOC(ptr, bytes)                                        \
@@ -1606,11 +1639,11 @@ int imdg_set_atoms(imdg_ctx* c, int nrep, const imdg_replica* reps,
     ALLOC(c->d_aid[k], sizeof(int) * ns);
   }
   ALLOC(c->d_xnbl, sizeof(double4) * ns);
-  ALLOC(c->d_cellid, sizeof(int) * ns);
-  ALLOC(c->d_cslot, sizeof(int) * ns);
   ALLOC(c->d_acell, sizeof(int) * ns);
   ALLOC(c->d_atype, ns);
-  ALLOC(c->d_perm, sizeof(int) * ns);
+  c->d_tiles = nullptr;
+  if (c->nblk > IMDG_TILE_FOLD) ALLOC(c->d_tiles, sizeof(Tile) * c->nblk);
+  ALLOC(c->d_bucket, sizeof(int) * c->bucket_cap * (size_t)c->ncells);
   ALLOC(c->d_cell_cnt, sizeof(int) * c->ncells);
   ALLOC(c->d_cell_beg, sizeof(int) * c->ncells);
   ALLOC(c->d_cell_num, sizeof(int) * c->ncells);
@@ -1619,7 +1652,6 @@ int imdg_set_atoms(imdg_ctx* c, int nrep, const imdg_replica* reps,
   ALLOC(c->d_tile_off, sizeof(int) * c->nstile);
   ALLOC(c->d_tile_rep, sizeof(int) * c->nstile);
   ALLOC(c->d_blkmax, sizeof(int) * c->nblk);
-  ALLOC(c->d_tiles, sizeof(Tile) * c->nblk);
   ALLOC(c->d_nnb, sizeof(int) * ns);
   ALLOC(c->d_reca, rs * 4 * ns);
   ALLOC(c->d_recb, rs * 4 * ns);
@@ -1734,11 +1766,9 @@ int imdg_set_atoms(imdg_ctx* c, int nrep, const imdg_replica* reps,
   HIPCHK(c, hipMemsetAsync(c->d_cell_cnt, 0, sizeof(int) * c->ncells, st));
   HIPCHK(c, hipMemsetAsync(c->d_cell_beg, 0, sizeof(int) * c->ncells, st));
   HIPCHK(c, hipMemsetAsync(c->d_cell_num, 0, sizeof(int) * c->ncells, st));
-  HIPCHK(c, hipMemsetAsync(c->d_tiles, 0, sizeof(Tile) * c->nblk, st));
   HIPCHK(c, hipMemsetAsync(c->d_acell, 0, sizeof(int) * ns, st));
   HIPCHK(c, hipMemsetAsync(c->d_atype, 0, ns, st));
   HIPCHK(c, hipMemsetAsync(c->d_nnb, 0, sizeof(int) * ns, st));
-  HIPCHK(c, hipMemsetAsync(c->d_perm, 0, sizeof(int) * ns, st));
   HIPCHK(c, hipMemsetAsync(c->d_reca, 0, rs * 4 * ns, st));
   HIPCHK(c, hipMemsetAsync(c->d_recb, 0, rs * 4 * ns, st));
   HIPCHK(c, hipMemsetAsync(c->d_rho, 0, rs * ns, st));
@@ -1776,7 +1806,7 @@ int imdg_calc_forces(imdg_ctx* c, int steps) {
   if (rc) return rc;
   c->stress_valid = false;
   if ((rc = build_until_fits(c))) return rc;
-  if ((rc = enqueue_forces(c, false))) return rc;
+  if ((rc = enqueue_forces(c, false, true, false))) return rc;
   HIPCHK(c, hipStreamSynchronize(c->stream));
   collect_profile(c);
   return IMDG_OK;
@@ -1868,8 +1898,8 @@ int imdg_deallocate_nblist(imdg_ctx* c) {
 static int capture_step(imdg_ctx* c) {
   hipGraph_t g = nullptr;
   HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-  int rc = enqueue_build(c);
-  if (!rc) rc = enqueue_forces(c, !c->split_move);
+  int rc = enqueue_build(c, false);
+  if (!rc) rc = enqueue_forces(c, !c->split_move, true, true);
   if (!rc && c->split_move) rc = enqueue_move(c);
   hipError_t e = hipStreamEndCapture(c->stream, &g);
   if (rc) {
@@ -1893,9 +1923,10 @@ int imdg_run(imdg_ctx* c, long nsteps) {
       HIPCHK(c, hipGraphLaunch(c->step_graph, c->stream));
   } else {
     for (long s = 0; s < nsteps; s++) {
-      if ((rc = enqueue_build(c))) return rc;
+      if ((rc = enqueue_build(c, false))) return rc;
       // per-atom outputs only on the last step: nothing reads them between
-      if ((rc = enqueue_forces(c, !c->split_move, s == nsteps - 1))) return rc;
+      if ((rc = enqueue_forces(c, !c->split_move, s == nsteps - 1, true)))
+        return rc;
       if (c->split_move && (rc = enqueue_move(c))) return rc;
     }
   }
@@ -2332,7 +2363,7 @@ int imdg_autotune(imdg_ctx* c, int reps, imdg_tuning* chosen) {
   if (rc) return rc;
   drop_graph(c);
   // leave forces and energies as calc_forces would
-  if ((rc = enqueue_forces(c, false))) return rc;
+  if ((rc = enqueue_forces(c, false, true, false))) return rc;
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return IMDG_OK;
 }

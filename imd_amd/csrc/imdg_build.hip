@@ -1,10 +1,14 @@
 // imdg_build.hip -- CDNA4 (gfx950) kernels of the list rebuild: wrap and
-// cell binning, per-replica scan, cell sort by input index, permutation of
-// the state into cell order, per-block neighbour tiles and the full
+// cell binning, per-replica scan, the sort of the state into cell order (by
+// input index within a cell), per-block neighbour tiles and the full
 // neighbour list.  Every kernel of the chain is launched every step and
 // returns at its first instructions unless the skin test of the previous
 // step (or the host) asked for a rebuild, so the fused loop never waits for
-// the host.
+// the host.  Each such idle launch costs the device about 1.7 us and the
+// host 2.7 us, which is what a small system's step consists of, so the chain
+// has as few as its data dependences allow: bin (with the scan of the cell
+// counts, for up to IMDG_SCAN_FOLD cells), sort, list; what ends it
+// (list_done) runs in the step's next kernel.
 //
 // Reference semantics (paths relative to the reference root):
 //   binning / wrap     src/imd_fix_cells_3d.c:36-201, src/imd_main_3d.c:1972-2065,
@@ -18,6 +22,8 @@
 //   skin test          check_nblist src/imd_forces_nbl.c:2007-2037
 #include "imdg_device.h"
 
+#include <algorithm>
+
 namespace imdg {
 
 // Blocks of the per-slot rebuild kernels cover IMDG_BLOCK slots of one
@@ -28,21 +34,72 @@ __device__ __forceinline__ int block_replica(const int* blk_rep) {
 
 // fix_cells/do_boundaries + cell_coord, for replicas that need a rebuild.
 // The atoms of a block are counted per cell in an LDS hash table first, so
-// the global counters see one atomic per distinct cell of the block (the
-// slot of an atom inside its cell is base + its rank in the block; the
-// order inside a cell is fixed later by k_cellsort).
+// the global counters see one atomic per distinct cell of the block.  An
+// atom's place in its cell is base + its rank in the block; its slot index
+// goes there in the cell's bucket (bucket_cap places; the order inside a
+// cell is fixed by k_sort).  A cell with more atoms than places is noted in
+// the control block: the chain then stops and the host enlarges the
+// buckets.
 #define BIN_HASH 256
 
-// Flag bit of a block's list-length maximum (blkmax): its tile exceeded the
-// tile cap and the list build read its candidates from HBM/L2.
-#define IMDG_BLK_FALLBACK (1 << 30)
+// Exclusive scan of the cell counts of every rebuilt replica by one block,
+// straight to first slots (cell_loc with tile_off = the replica's first
+// slot, as k_scan leaves them).
+__device__ void scan_cells(const BuildArgs& a, int* wsum) {
+  const int T = blockDim.x, nw = T / IMDG_WAVE;
+  const int lane = threadIdx.x % IMDG_WAVE, w = threadIdx.x / IMDG_WAVE;
+  for (int r = 0; r < a.nrep; r++) {
+    if (!a.rst[r].need_rebuild) continue;
+    const RepDev& R = a.rep[r];
+    for (int t = threadIdx.x; t < R.nstile; t += T)
+      a.tile_off[R.stile_off + t] = R.atom_off;
+    int run = 0;
+    for (int c0 = 0; c0 < R.ncells; c0 += 8 * T) {
+      // eight consecutive cells a thread, loaded past this CU's L1 (the
+      // counters are written by atomics)
+      const int lc = c0 + 8 * threadIdx.x;
+      int n[8], v = 0;
+#pragma unroll
+      for (int u = 0; u < 8; u++)
+        n[u] = lc + u < R.ncells
+                   ? __hip_atomic_load(&a.cell_cnt[R.cell_off + lc + u],
+                                       __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT)
+                   : 0;
+#pragma unroll
+      for (int u = 0; u < 8; u++) v += n[u];
+      int incl = v;
+#pragma unroll
+      for (int o = 1; o < IMDG_WAVE; o <<= 1) {
+        int y = __shfl_up(incl, o, IMDG_WAVE);
+        if (lane >= o) incl += y;
+      }
+      if (lane == IMDG_WAVE - 1) wsum[w] = incl;
+      __syncthreads();
+      int before = run + incl - v, tot = 0;
+      for (int k = 0; k < nw; k++) {
+        if (k < w) before += wsum[k];
+        tot += wsum[k];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+        if (lc + u < R.ncells) a.cell_loc[R.cell_off + lc + u] = before;
+        before += n[u];
+      }
+      run += tot;
+      __syncthreads();
+    }
+  }
+}
 
 __global__ void __launch_bounds__(IMDG_BLOCK) k_bin(BuildArgs a) {
 #pragma clang fp contract(off)
   __shared__ int hkey[BIN_HASH], hcnt[BIN_HASH], hbase[BIN_HASH];
+  __shared__ int wsum[IMDG_NWAVE], is_last;
   if (!a.ctl->any_rebuild || a.ctl->frozen) return;
   int r = block_replica(a.blk_rep);
-  if (!a.rst[r].need_rebuild) return;
+  const bool flagged = a.rst[r].need_rebuild != 0;
+  if (!flagged && !a.scan_in_bin) return;
   const RepDev& R = a.rep[r];
   for (int e = threadIdx.x; e < BIN_HASH; e += IMDG_BLOCK) {
     hkey[e] = -1;
@@ -50,8 +107,8 @@ __global__ void __launch_bounds__(IMDG_BLOCK) k_bin(BuildArgs a) {
   }
   __syncthreads();
   int i = blockIdx.x * IMDG_BLOCK + threadIdx.x;
-  bool active = i - R.atom_off < R.natoms;
-  int h = -1, rank = 0;
+  bool active = flagged && i - R.atom_off < R.natoms;
+  int h = -1, rank = 0, cell = 0;
   if (active) {
     double4* pos = a.pos[a.ctl->pos_cur];
     double4 p = pos[i];
@@ -74,8 +131,7 @@ __global__ void __launch_bounds__(IMDG_BLOCK) k_bin(BuildArgs a) {
       else if (c[d] < 0)
         c[d] = 0;
     }
-    int cell = R.cell_off + (c[0] * R.gdim[1] + c[1]) * R.gdim[2] + c[2];
-    a.cellid[i] = cell;
+    cell = R.cell_off + (c[0] * R.gdim[1] + c[1]) * R.gdim[2] + c[2];
     // at most IMDG_BLOCK distinct keys in BIN_HASH entries: probing ends
     h = (int)(((unsigned)cell * 2654435761u) >> 24) & (BIN_HASH - 1);
     for (;;) {
@@ -89,7 +145,25 @@ __global__ void __launch_bounds__(IMDG_BLOCK) k_bin(BuildArgs a) {
   for (int e = threadIdx.x; e < BIN_HASH; e += IMDG_BLOCK)
     if (hkey[e] >= 0) hbase[e] = atomicAdd(&a.cell_cnt[hkey[e]], hcnt[e]);
   __syncthreads();
-  if (active) a.cslot[i] = hbase[h] + rank;
+  if (active) {
+    const int m = hbase[h] + rank;
+    if (m < a.bucket_cap)
+      a.bucket[(size_t)cell * a.bucket_cap + m] = i;
+    else
+      atomicMax(&a.ctl->cell_over, m + 1);
+  }
+  if (!a.scan_in_bin) return;
+  // the last block to finish scans the cell counts
+  if (threadIdx.x == 0) {
+    __threadfence();
+    unsigned d = atomicAdd(&a.ctl->done[DC_SCAN], 1u);
+    is_last = (d == gridDim.x - 1);
+    if (is_last) a.ctl->done[DC_SCAN] = 0;
+  }
+  __syncthreads();
+  if (!is_last) return;
+  __threadfence();
+  scan_cells(a, wsum);
 }
 
 // Exclusive scan of the cell counts, two levels in one launch: every block
@@ -172,40 +246,60 @@ __device__ __forceinline__ int cell_first_slot(const BuildArgs& a,
   return a.tile_off[R.stile_off + lc / IMDG_SCAN_TILE] + a.cell_loc[cell];
 }
 
-__global__ void __launch_bounds__(IMDG_BLOCK) k_place(BuildArgs a) {
-  if (!a.ctl->any_rebuild || a.ctl->frozen) return;
-  int r = block_replica(a.blk_rep);
-  if (!a.rst[r].need_rebuild) return;
-  const RepDev& R = a.rep[r];
-  int i = blockIdx.x * IMDG_BLOCK + threadIdx.x;
-  if (i - R.atom_off >= R.natoms) return;
-  int cell = a.cellid[i];
-  a.perm[cell_first_slot(a, R, cell) + a.cslot[i]] = i;
-}
-
 // Per cell: first slot and count, counter reset, and the atoms of the cell
-// ordered by input index (deterministic list order).  32 lanes per cell:
-// each lane takes one atom and writes it at its rank among the cell's input
-// indices (unique); a cell with more atoms is sorted by its first lane.
+// moved to their new slots in the other buffers, ordered by input index
+// (deterministic list order), with the cell-relative records.  32 lanes per
+// cell: each lane takes one atom of the cell's bucket, finds its rank among
+// the cell's input indices (unique) and moves it: reads are scattered pieces
+// of 32 B, writes are the cell's run of slots.  A cell of a replica that is
+// not rebuilt is copied as it is.  The buffers are flipped by list_done once
+// the list fits (on an overflow the whole chain runs again from the old
+// buffers).  One launch for the former three (place, sort, permute).
 #define SORT_LANES 32
 
-__global__ void __launch_bounds__(256) k_cellsort(BuildArgs a) {
-  if (!a.ctl->any_rebuild || a.ctl->frozen) return;
-  const int* aid = a.aid[a.ctl->rec_cur];
+__device__ __forceinline__ void move_atom(const BuildArgs& a, const RepDev& R,
+                                          int pc, int rc, int from, int to,
+                                          int key, int cell) {
+  const double4 p = a.pos[pc][from];
+  const double4 m = a.mom[rc][from];
+  a.pos[pc ^ 1][to] = p;
+  a.mom[rc ^ 1][to] = m;
+  a.aid[rc ^ 1][to] = key;
+  a.acell[to] = cell;
+  a.atype[to] = (signed char)p.w;
+  a.xnbl[to] = p;
+  double c[3];
+  cell_centre(R, cell, c);
+  if (a.mixed)
+    reinterpret_cast<float4*>(a.rec_a)[to] =
+        make_float4((float)(p.x - c[0]), (float)(p.y - c[1]),
+                    (float)(p.z - c[2]), (float)p.w);
+  else
+    reinterpret_cast<double4*>(a.rec_a)[to] =
+        make_double4(p.x - c[0], p.y - c[1], p.z - c[2], p.w);
+}
+
+__global__ void __launch_bounds__(256) k_sort(BuildArgs a) {
+  if (!a.ctl->any_rebuild || a.ctl->frozen || a.ctl->cell_over) return;
+  const int pc = a.ctl->pos_cur, rc = a.ctl->rec_cur;
+  const int* aid = a.aid[rc];
   int seg = threadIdx.x / SORT_LANES, l = threadIdx.x % SORT_LANES;
   int base = (threadIdx.x % IMDG_WAVE) - l;  // first lane of the segment
   for (int c = blockIdx.x * (blockDim.x / SORT_LANES) + seg; c < a.ncells;
        c += gridDim.x * (blockDim.x / SORT_LANES)) {
     int r = a.cell_rep[c];
-    if (!a.rst[r].need_rebuild) continue;  // the whole segment skips
     const RepDev& R = a.rep[r];
-    int b = cell_first_slot(a, R, c), n = a.cell_cnt[c];
-    int* p = a.perm + b;
-    if (l == 0) {
-      a.cell_beg[c] = b;
-      a.cell_num[c] = n;
-      a.cell_cnt[c] = 0;
+    if (!a.rst[r].need_rebuild) {  // the whole segment
+      const int b = a.cell_beg[c], n = a.cell_num[c];
+      for (int s = b + l; s < b + n; s += SORT_LANES) {
+        a.pos[pc ^ 1][s] = a.pos[pc][s];
+        a.mom[rc ^ 1][s] = a.mom[rc][s];
+        a.aid[rc ^ 1][s] = aid[s];
+      }
+      continue;
     }
+    const int b = cell_first_slot(a, R, c), n = a.cell_cnt[c];
+    const int* p = a.bucket + (size_t)c * a.bucket_cap;
     if (n <= SORT_LANES) {
       int v = l < n ? p[l] : 0;
       int key = l < n ? aid[v] : 0x7fffffff;
@@ -214,90 +308,43 @@ __global__ void __launch_bounds__(256) k_cellsort(BuildArgs a) {
         int km = __shfl(key, base + m, IMDG_WAVE);
         rank += km < key;
       }
-      if (l < n) p[rank] = v;
-    } else if (l == 0) {
-      for (int k = 1; k < n; k++) {
-        int v = p[k], key = aid[v], m = k - 1;
-        while (m >= 0 && aid[p[m]] > key) {
-          p[m + 1] = p[m];
-          m--;
-        }
-        p[m + 1] = v;
+      if (l < n) move_atom(a, R, pc, rc, v, b + rank, key, c);
+    } else {
+      for (int e = l; e < n; e += SORT_LANES) {
+        const int v = p[e], key = aid[v];
+        int rank = 0;
+        for (int m = 0; m < n; m++) rank += aid[p[m]] < key;
+        move_atom(a, R, pc, rc, v, b + rank, key, c);
       }
+    }
+    if (l == 0) {
+      a.cell_beg[c] = b;
+      a.cell_num[c] = n;
+      a.cell_cnt[c] = 0;
     }
   }
 }
 
-// Tiles: for every block of a rebuilt replica, the slot runs of all cells
-// adjacent (27-stencil, periodic wrap, nothing beyond an open face) to the
-// cells of the block's atoms, sorted and merged.  One wavefront per block
-// (the first of the block's permutation launch): lane l handles neighbour
-// column l % 9 of the block's column l / 9 (at most 7 columns; more falls
-// back to a tile-less list), producing at most two slot ranges (a z range
-// split by the periodic wrap); the wavefront sorts and merges them.
+// Tile of a block of a rebuilt replica: the slot runs of all cells adjacent
+// (27-stencil, periodic wrap, nothing beyond an open face) to the cells of
+// the block's atoms, sorted and merged, in LDS.  One wavefront (the first of
+// the block's list launch): lane l handles neighbour column l % 9 of the
+// block's column l / 9 (at most 7 columns; more falls back to a tile-less
+// list), producing at most two slot ranges (a z range split by the periodic
+// wrap); the wavefront sorts and merges them.
 #define TILE_MAXRANGE 126
 #define TILE_MAXCOL 7
 
-// LDS rows of one wavefront's tile construction.
+// LDS rows of one wavefront's tile construction, and the tile.
 struct TileLds {
   int rb[TILE_MAXRANGE], re[TILE_MAXRANGE];
-  int4 run[IMDG_MAXRUN];
 };
 
-__device__ void build_tile(const BuildArgs& a, int b, TileLds& S);
-
-// Gather every slot into the other buffers (new cell-sorted order for the
-// rebuilt replicas, identity for the others) and write the cell-relative
-// records of the moved atoms.  The buffers are flipped by k_list_done once
-// the list fits (on an overflow the whole chain runs again from the old
-// buffers).
-__global__ void __launch_bounds__(IMDG_BLOCK) k_permute(BuildArgs a) {
-  __shared__ TileLds tl;
-  if (!a.ctl->any_rebuild || a.ctl->frozen) return;
-  int pc = a.ctl->pos_cur, rc = a.ctl->rec_cur;
-  const double4* pin = a.pos[pc];
-  double4* pout = a.pos[pc ^ 1];
-  const double4* min_ = a.mom[rc];
-  double4* mout = a.mom[rc ^ 1];
-  const int* ain = a.aid[rc];
-  int* aout = a.aid[rc ^ 1];
-  int r = block_replica(a.blk_rep);
-  const RepDev& R = a.rep[r];
-  int i = blockIdx.x * IMDG_BLOCK + threadIdx.x;
-  bool moved = a.rst[r].need_rebuild && (i - R.atom_off < R.natoms);
-  int old = moved ? a.perm[i] : i;
-  double4 p = pin[old];
-  pout[i] = p;
-  mout[i] = min_[old];
-  aout[i] = ain[old];
-  if (moved) {
-    int cell = a.cellid[old];
-    a.acell[i] = cell;
-    a.atype[i] = (signed char)p.w;
-    a.xnbl[i] = p;
-    double c[3];
-    cell_centre(R, cell, c);
-    if (a.mixed)
-      reinterpret_cast<float4*>(a.rec_a)[i] =
-          make_float4((float)(p.x - c[0]), (float)(p.y - c[1]),
-                      (float)(p.z - c[2]), (float)p.w);
-    else
-      reinterpret_cast<double4*>(a.rec_a)[i] =
-          make_double4(p.x - c[0], p.y - c[1], p.z - c[2], p.w);
-  }
-  // the block's tile for the list build (needs the cell ranges only)
-  if (a.rst[r].need_rebuild && threadIdx.x < IMDG_WAVE)
-    build_tile(a, blockIdx.x, tl);
-}
-
 // The tile of 128-slot block b of a rebuilt replica, built by one whole
-// wavefront (lane l); the cells of the block's first and last slots are
-// those the permutation gives them.
-__device__ void build_tile(const BuildArgs& a, int b, TileLds& S) {
+// wavefront (lane l).
+__device__ void build_tile(const BuildArgs& a, const RepDev& R, int b,
+                           TileLds& S, Tile& T) {
   int l = threadIdx.x % IMDG_WAVE;
-  int r = __builtin_amdgcn_readfirstlane(a.blk_rep[b]);
-  const RepDev& R = a.rep[r];
-  Tile& T = a.tiles[b];
   int s0 = b * IMDG_BLOCK;
   int s1 = min(s0 + IMDG_BLOCK, R.atom_off + R.natoms) - 1;
   if (s1 < s0) {
@@ -309,8 +356,8 @@ __device__ void build_tile(const BuildArgs& a, int b, TileLds& S) {
     return;
   }
   int g0 = R.gdim[0], g1 = R.gdim[1], g2 = R.gdim[2];
-  int lc0 = a.cellid[a.perm[s0]] - R.cell_off;
-  int lc1 = a.cellid[a.perm[s1]] - R.cell_off;
+  int lc0 = a.acell[s0] - R.cell_off;
+  int lc1 = a.acell[s1] - R.cell_off;
   int col0 = lc0 / g2, col1 = lc1 / g2, ncol = col1 - col0 + 1;
   bool ok = ncol <= TILE_MAXCOL;
   int nmine = 0, mb[2] = {0, 0}, me[2] = {0, 0};
@@ -422,7 +469,7 @@ __device__ void build_tile(const BuildArgs& a, int b, TileLds& S) {
       mine && (l == nr - 1 || (l < IMDG_WAVE - 1 && ((starts >> (l + 1)) & 1ull)));
   if (nrun > IMDG_MAXRUN) ok = false;
   // run begin (at its start lane) and end (the prefix max at its last lane)
-  int4* run = S.run;
+  int4* run = T.run;
   if (ok && start) run[runid].x = sb;
   if (ok && last_of_run) run[runid].z = pmax;
   wave_lds_sync();
@@ -438,19 +485,32 @@ __device__ void build_tile(const BuildArgs& a, int b, TileLds& S) {
   int tot = __shfl(pos, IMDG_WAVE - 1, IMDG_WAVE);
   pos -= len;
   ok = ok && tot <= a.tile_cap;
-  if (ok && l < nrun) T.run[l] = make_int4(run[l].x, len, pos, 0);
+  if (ok && l < nrun) run[l] = make_int4(run[l].x, len, pos, 0);
   if (l == 0) {
-    if (!ok) {
-      // counted by k_list_done (one counter word updated by every block
-      // would serialise the blocks)
-      T.ok = 0;
-      T.nrun = 0;
-      T.natoms = 0;
-    } else {
-      T.ok = 1;
-      T.nrun = nrun;
-      T.natoms = tot;
-    }
+    T.ok = ok ? 1 : 0;
+    T.nrun = ok ? nrun : 0;
+    T.natoms = ok ? tot : 0;
+  }
+}
+
+// Tiles of the rebuilt replicas, a wavefront each (larger systems).
+__global__ void __launch_bounds__(256) k_tile(BuildArgs a) {
+  __shared__ TileLds tl[256 / IMDG_WAVE];
+  __shared__ Tile tt[256 / IMDG_WAVE];
+  if (!a.ctl->any_rebuild || a.ctl->frozen || a.ctl->cell_over) return;
+  const int w = threadIdx.x / IMDG_WAVE, l = threadIdx.x % IMDG_WAVE;
+  const int b = blockIdx.x * (256 / IMDG_WAVE) + w;
+  if (b >= a.nblk) return;
+  const int r = __builtin_amdgcn_readfirstlane(a.blk_rep[b]);
+  if (!a.rst[r].need_rebuild) return;
+  build_tile(a, a.rep[r], b, tl[w], tt[w]);
+  wave_lds_sync();
+  Tile& T = a.tiles[b];
+  if (l < tt[w].nrun) T.run[l] = tt[w].run[l];
+  if (l == 0) {
+    T.nrun = tt[w].nrun;
+    T.natoms = tt[w].natoms;
+    T.ok = tt[w].ok;
   }
 }
 
@@ -756,12 +816,11 @@ template <bool MIXED>
 __global__ void __launch_bounds__(IMDG_BLOCK) k_list(BuildArgs a) {
   extern __shared__ __align__(16) unsigned char list_lds[];
   float3* trec = reinterpret_cast<float3*>(list_lds);
-  __shared__ int4 truns[IMDG_MAXRUN];
+  __shared__ Tile tile;
   __shared__ float off[3 * IMDG_NCODES];
-  __shared__ int tinfo[2];
   __shared__ int wmax[IMDG_NWAVE];
   __shared__ int cbase[IMDG_NWAVE][IMDG_META];
-  if (!a.ctl->any_rebuild || a.ctl->frozen) return;
+  if (!a.ctl->any_rebuild || a.ctl->frozen || a.ctl->cell_over) return;
   int b = blockIdx.x;
   int r = a.blk_rep[b];
   const RepDev& R = a.rep[r];
@@ -770,18 +829,27 @@ __global__ void __launch_bounds__(IMDG_BLOCK) k_list(BuildArgs a) {
   const double4* pos = a.pos[a.ctl->pos_cur ^ 1];
   int kmax = a.kmax, seen = 0;
   if (flagged) {
-    const Tile& T = a.tiles[b];
-    if (threadIdx.x == 0) {
-      tinfo[0] = T.nrun;
-      tinfo[1] = T.ok;
+    if (a.tiles) {
+      const Tile& T = a.tiles[b];
+      if (threadIdx.x == 0) {
+        tile.nrun = T.nrun;
+        tile.natoms = T.natoms;
+        tile.ok = T.ok;
+      }
+      for (int k = threadIdx.x; k < T.nrun; k += blockDim.x)
+        tile.run[k] = T.run[k];
+    } else if (threadIdx.x < IMDG_WAVE) {
+      // in the rows that will hold the tile's records (tile_cap + 4 of
+      // them: room for the ranges, see launch_build)
+      build_tile(a, R, b, *reinterpret_cast<TileLds*>(list_lds), tile);
     }
-    for (int k = threadIdx.x; k < T.nrun; k += blockDim.x) truns[k] = T.run[k];
     for (int k = threadIdx.x; k < 3 * IMDG_NCODES; k += blockDim.x)
       off[k] = (float)((&R.offs[0][0])[k]);
     __syncthreads();
-    const int nrun = tinfo[0], tok = tinfo[1];
+    const int4* truns = tile.run;
+    const int nrun = tile.nrun, tok = tile.ok;
     if (tok) {
-      int tot = T.natoms;
+      int tot = tile.natoms;
       // all of a thread's loads in flight together: 8 records per pass
       int k = 0;
       for (int t0 = threadIdx.x; t0 < tot; t0 += 8 * IMDG_BLOCK) {
@@ -888,56 +956,15 @@ __global__ void __launch_bounds__(IMDG_BLOCK) k_list(BuildArgs a) {
   if (threadIdx.x == 0) {
     int m = wmax[0];
     for (int k = 1; k < IMDG_NWAVE; k++) m = max(m, wmax[k]);
-    a.blkmax[b] = m | (flagged && !tinfo[1] ? IMDG_BLK_FALLBACK : 0);
+    a.blkmax[b] = m | (flagged && !tile.ok ? IMDG_BLK_FALLBACK : 0);
   }
 }
 
-// End of a rebuild (one block): the longest list; on an overflow freeze the
-// state (the host grows the list and runs the chain again from the old
-// buffers), otherwise clear the rebuild flags and flip the buffers that
-// k_permute filled.
-__global__ void __launch_bounds__(1024) k_list_done(BuildArgs a) {
-  __shared__ int wmax[1024 / IMDG_WAVE], wfb[1024 / IMDG_WAVE];
-  if (!a.ctl->any_rebuild || a.ctl->frozen) return;
-  int m = 0, fb = 0;
-  for (int b = threadIdx.x; b < a.nblk; b += blockDim.x)
-    if (a.rst[a.blk_rep[b]].need_rebuild) {
-      const int v = a.blkmax[b];
-      m = max(m, v & ~IMDG_BLK_FALLBACK);
-      fb += v & IMDG_BLK_FALLBACK ? 1 : 0;
-    }
-  for (int o = 32; o > 0; o >>= 1) {
-    m = max(m, __shfl_xor(m, o, IMDG_WAVE));
-    fb += __shfl_xor(fb, o, IMDG_WAVE);
-  }
-  if ((threadIdx.x % IMDG_WAVE) == 0) {
-    wmax[threadIdx.x / IMDG_WAVE] = m;
-    wfb[threadIdx.x / IMDG_WAVE] = fb;
-  }
-  __syncthreads();
-  if (threadIdx.x != 0) return;
-  for (int k = 1; k < (int)(blockDim.x / IMDG_WAVE); k++) {
-    m = max(m, wmax[k]);
-    fb += wfb[k];
-  }
-  m = max(m, wmax[0]);
-  a.ctl->tiles_fallback += fb;
-  if (m > a.ctl->kmax_seen) a.ctl->kmax_seen = m;
-  if (m > a.kmax) {
-    // keep the rebuild flags: the host grows the list and builds again
-    a.ctl->overflow = 1;
-    a.ctl->frozen = 1;
-  } else {
-    for (int q = 0; q < a.nrep; q++)
-      if (a.rst[q].need_rebuild) {
-        a.rst[q].rebuilt = 1;
-        a.rst[q].nbl_count += 1;
-        a.rst[q].need_rebuild = 0;
-      }
-    a.ctl->pos_cur ^= 1;
-    a.ctl->rec_cur ^= 1;
-    a.ctl->any_rebuild = 0;
-  }
+// The end of a rebuild as a launch of its own (one block), where no step
+// follows: make_nblist and the list of calc_forces.
+__global__ void __launch_bounds__(1024) k_list_done(ListEnd e) {
+  __shared__ int red[2 * (1024 / IMDG_WAVE)];
+  list_done(e, red);
 }
 
 // check_nblist alone: max displacement^2 per block of IMDG_BLOCK slots.
@@ -968,20 +995,24 @@ __global__ void __launch_bounds__(IMDG_BLOCK)
 // launchers
 // ---------------------------------------------------------------------------
 
-void launch_build(const BuildArgs& b, int grid, hipStream_t st) {
+// done: end the rebuild here (otherwise the step's next kernel does).
+void launch_build(const BuildArgs& b, int grid, bool done, hipStream_t st) {
   hipLaunchKernelGGL(k_bin, dim3(b.nblk), dim3(IMDG_BLOCK), 0, st, b);
-  hipLaunchKernelGGL(k_scan, dim3(b.nstile), dim3(IMDG_SCAN_TILE), 0, st, b);
-  hipLaunchKernelGGL(k_place, dim3(b.nblk), dim3(IMDG_BLOCK), 0, st, b);
-  hipLaunchKernelGGL(k_cellsort, dim3(grid), dim3(256), 0, st, b);
-  hipLaunchKernelGGL(k_permute, dim3(b.nblk), dim3(IMDG_BLOCK), 0, st, b);
-  const size_t tile_lds = (size_t)(b.tile_cap + 4) * sizeof(float3);
+  if (!b.scan_in_bin)
+    hipLaunchKernelGGL(k_scan, dim3(b.nstile), dim3(IMDG_SCAN_TILE), 0, st, b);
+  hipLaunchKernelGGL(k_sort, dim3(grid), dim3(256), 0, st, b);
+  if (b.tiles)
+    hipLaunchKernelGGL(k_tile, dim3((b.nblk + 3) / 4), dim3(256), 0, st, b);
+  const size_t tile_lds = std::max((size_t)(b.tile_cap + 4) * sizeof(float3),
+                                   sizeof(TileLds));
   if (b.mixed)
     hipLaunchKernelGGL((k_list<true>), dim3(b.nblk), dim3(IMDG_BLOCK),
                        tile_lds, st, b);
   else
     hipLaunchKernelGGL((k_list<false>), dim3(b.nblk), dim3(IMDG_BLOCK),
                        tile_lds, st, b);
-  hipLaunchKernelGGL(k_list_done, dim3(1), dim3(1024), 0, st, b);
+  if (done)
+    hipLaunchKernelGGL(k_list_done, dim3(1), dim3(1024), 0, st, b.end);
 }
 
 void launch_check(const RepDev* rep, Ctl* ctl, const int* blk_rep,

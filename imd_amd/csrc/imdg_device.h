@@ -11,10 +11,36 @@
 
 namespace imdg {
 
+// One DPP move of a double (both halves); rows outside the mask keep `old`.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_d(double old, double v) {
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(old),
+                                             __double2loint(v), CTRL, ROWS,
+                                             0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(old),
+                                             __double2hiint(v), CTRL, ROWS,
+                                             0xf, false);
+  return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double lane63_d(double v) {
+  return __hiloint2double(
+      __builtin_amdgcn_readlane(__double2hiint(v), 63),
+      __builtin_amdgcn_readlane(__double2loint(v), 63));
+}
+
+// Sum and maximum over the 64 lanes (every lane active), in every lane, by
+// DPP moves: quad permutes, row mirrors, and the broadcasts of lanes 15 and
+// 31 to the next rows (lane 63 ends with the total).  A cross-lane shuffle is
+// a trip through LDS (64 cycles and more, twice per double and level): the
+// reductions at the end of a small launch were 1 us of it.
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, IMDG_WAVE);
-  return v;
+  v += dpp_d<0xb1, 0xf>(0.0, v);
+  v += dpp_d<0x4e, 0xf>(0.0, v);
+  v += dpp_d<0x141, 0xf>(0.0, v);
+  v += dpp_d<0x140, 0xf>(0.0, v);
+  v += dpp_d<0x142, 0xa>(0.0, v);
+  v += dpp_d<0x143, 0xc>(0.0, v);
+  return lane63_d(v);
 }
 
 // Minimum over the 64 lanes (every lane active) through DPP
@@ -37,9 +63,13 @@ __device__ __forceinline__ int wave_min_i(int v) {
 
 
 __device__ __forceinline__ double wave_max(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, IMDG_WAVE));
-  return v;
+  v = fmax(v, dpp_d<0xb1, 0xf>(v, v));
+  v = fmax(v, dpp_d<0x4e, 0xf>(v, v));
+  v = fmax(v, dpp_d<0x141, 0xf>(v, v));
+  v = fmax(v, dpp_d<0x140, 0xf>(v, v));
+  v = fmax(v, dpp_d<0x142, 0xa>(v, v));
+  v = fmax(v, dpp_d<0x143, 0xc>(v, v));
+  return lane63_d(v);
 }
 
 // Error-free sum of two doubles (Knuth TwoSum).
@@ -60,6 +90,28 @@ __device__ __forceinline__ void kahan_add(double& s, double& c, double x) {
   else
     c += (x - t) + s;
   s = t;
+}
+
+// Compensated sum of (s, c) pairs over the 64 lanes in a fixed order
+// (TwoSum keeps every rounding error); the total, error added, in every lane.
+__device__ __forceinline__ double wave_sum_comp(double s, double c) {
+#define IMDG_COMB(CTRL, ROWS)                     \
+  do {                                            \
+    const double so = dpp_d<CTRL, ROWS>(0.0, s);  \
+    const double co = dpp_d<CTRL, ROWS>(0.0, c);  \
+    double t, e;                                  \
+    two_sum(s, so, t, e);                         \
+    s = t;                                        \
+    c = c + co + e;                               \
+  } while (0)
+  IMDG_COMB(0xb1, 0xf);
+  IMDG_COMB(0x4e, 0xf);
+  IMDG_COMB(0x141, 0xf);
+  IMDG_COMB(0x140, 0xf);
+  IMDG_COMB(0x142, 0xa);
+  IMDG_COMB(0x143, 0xc);
+#undef IMDG_COMB
+  return lane63_d(s + c);
 }
 
 __device__ __forceinline__ float rmin(float a, float b) { return fminf(a, b); }
@@ -187,6 +239,62 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// End of a rebuild, by one block: the longest list; on an overflow (of the
+// list or of a cell's bucket) freeze the state (the host enlarges what
+// overflowed and runs the chain again from the old buffers), otherwise clear
+// the rebuild flags and flip the buffers that k_sort filled.  red: two ints
+// per wavefront.  In a step it runs in block 0 of the density loop (or the
+// record copy): nothing else in that kernel reads what it writes, except
+// frozen, and the outputs of a density loop that goes on are computed again.
+__device__ inline void list_done(const ListEnd& e, int* red) {
+  if (!e.ctl->any_rebuild || e.ctl->frozen) return;
+  const int nw = blockDim.x / IMDG_WAVE, w = threadIdx.x / IMDG_WAVE;
+  const int over = e.ctl->cell_over;
+  int m = 0, fb = 0;
+  if (!over)
+    for (int b = threadIdx.x; b < e.nblk; b += blockDim.x)
+      if (e.rst[e.blk_rep[b]].need_rebuild) {
+        const int v = e.blkmax[b];
+        m = max(m, v & ~IMDG_BLK_FALLBACK);
+        fb += v & IMDG_BLK_FALLBACK ? 1 : 0;
+      }
+  for (int o = 32; o > 0; o >>= 1) {
+    m = max(m, __shfl_xor(m, o, IMDG_WAVE));
+    fb += __shfl_xor(fb, o, IMDG_WAVE);
+  }
+  if ((threadIdx.x % IMDG_WAVE) == 0) {
+    red[w] = m;
+    red[nw + w] = fb;
+  }
+  __syncthreads();
+  if (threadIdx.x >= IMDG_WAVE) return;
+  for (int k = 1; k < nw; k++) {
+    m = max(m, red[k]);
+    fb += red[nw + k];
+  }
+  m = max(m, red[0]);
+  const bool full = over || m > e.kmax;
+  if (!full)
+    for (int q = threadIdx.x; q < e.nrep; q += IMDG_WAVE)
+      if (e.rst[q].need_rebuild) {
+        e.rst[q].rebuilt = 1;
+        e.rst[q].nbl_count += 1;
+        e.rst[q].need_rebuild = 0;
+      }
+  if (threadIdx.x != 0) return;
+  e.ctl->tiles_fallback += fb;
+  if (m > e.ctl->kmax_seen) e.ctl->kmax_seen = m;
+  if (full) {
+    // keep the rebuild flags: the host grows the list and builds again
+    e.ctl->overflow = 1;
+    e.ctl->frozen = 1;
+  } else {
+    e.ctl->pos_cur ^= 1;
+    e.ctl->rec_cur ^= 1;
+    e.ctl->any_rebuild = 0;
+  }
 }
 
 }  // namespace imdg

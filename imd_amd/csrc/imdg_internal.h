@@ -33,8 +33,6 @@
 //    (a chunk across a plane of the grid, or very dense cells) keeps the
 //    32-bit format; cmeta[chunk * IMDG_META + code] holds the bases and
 //    cmeta[chunk * IMDG_META + IMDG_META_WIDE] marks such chunks;
-//  * tiles: for every block of IMDG_BLOCK slots, the slot runs of all
-//    cells adjacent to the block's cells, staged into LDS by the list build;
 //  * tables as knots (p0_k, dv_k = t[k+1] - t[k]), k = 0..len, of IMD's
 //    3-point interpolation, differences taken in FP64 and then rounded to
 //    the force precision; the per-step kernels copy the knots of the
@@ -50,6 +48,9 @@
 #define IMDG_CHUNK 64        // slots per wavefront step of the step kernels
 #define IMDG_STEP_THREADS 1024   // largest block of the step kernels
 #define IMDG_STEP_WAVES (IMDG_STEP_THREADS / IMDG_WAVE)
+#define IMDG_FIN_THREADS 512 // block of the finalize: a wavefront for each of
+                             // the seven sums of a replica
+#define IMDG_FIN_BLOCKS 1024
 #define IMDG_MAXTYPES 8
 #define IMDG_MAXCOLS (IMDG_MAXTYPES * IMDG_MAXTYPES)
 #define IMDG_RING 4096
@@ -91,14 +92,25 @@
 #define PB_N 6
 
 // done counters (last-block-done pattern) per kernel kind
-#define DC_PERMUTE 0
-#define DC_LIST 1
-#define DC_FINAL 2
-#define DC_SCAN 3
-#define DC_FINBLK 4   // finalising blocks of a step done (several replicas)
-#define DC_N 5
+#define DC_FINAL 0
+#define DC_SCAN 1
+#define DC_FINBLK 2   // finalising blocks of a step done (several replicas)
+#define DC_N 3
 
 #define IMDG_SCAN_TILE 1024  // cells per block of the cell-count scan
+// Up to this many cells the last block of the binning scans their counts
+// (about 1 us per 1024 cells and rebuild) and the scan's launch is left out
+// (1.7 us per step, one rebuild in 15 to 20 steps).
+#define IMDG_SCAN_FOLD 8192
+// Up to this many blocks the list's blocks build their own tiles (about 5 us
+// of latency in the list's launch); a larger system has a launch for them
+// (2,048,000 atoms, 16,000 blocks: list 694 us instead of 792).
+#define IMDG_TILE_FOLD 1024
+#define IMDG_BUCKET_MIN 32   // smallest bucket (atoms of a cell)
+
+// Flag bit of a block's list-length maximum (blkmax): its tile exceeded the
+// tile cap and the list build read its candidates from HBM/L2.
+#define IMDG_BLK_FALLBACK (1 << 30)
 
 struct RepDev {
   double box[3][3];       // rows: box_x, box_y, box_z
@@ -144,24 +156,28 @@ struct Ctl {
   int any_rebuild;        // some replica needs a list rebuild
   int frozen;             // list overflow: every kernel is a no-op until
                           // the host grows the list and re-runs the build
-  int overflow;           // set by the list build, turned into frozen by
-                          // its last block (frozen never changes mid-kernel)
+                          // (set by list_done: a density block that began
+                          // before that only recomputes its outputs)
+  int overflow;
   int kmax_seen;
   int is_short;
   int tiles_fallback;     // blocks whose tile exceeded the tile cap
   int exact_pairs;        // list candidates decided by the FP64 expression
+  int cell_over;          // atoms of a cell that has more than its bucket's
+                          // places (0: none): the chain stops there
   int export_bad;         // a slot without an atom met by an export kernel
   unsigned int done[DC_N];
   long steps_done;
 };
 
-// One block's tile: slot runs copied to consecutive LDS records.
-struct Tile {
-  int nrun;
-  int natoms;             // records in the tile
-  int ok;                 // 0: did not fit, list holds global slots
-  int pad;
-  int4 run[IMDG_MAXRUN];  // (first slot, length, first LDS record, 0)
+// What the end of a rebuild works on (list_done): run by block 0 of the
+// step's first loop, or by a launch of its own.
+struct ListEnd {
+  Ctl* ctl;
+  RepState* rst;
+  const int* blk_rep;
+  const int* blkmax;      // longest list of every block (k_list)
+  int nblk, nrep, kmax;
 };
 
 // Table of one interpolated function set on the device.
@@ -285,6 +301,8 @@ struct StepArgs {
                           // its 2F' (rec_b.w), not a gather of atype
   const double2* knots64; // FP64 knots of the embedding (tab64[0]) and the
   const Tab64* tab64;     // EEAM energy term (tab64[1]); FP32 kernels only
+  ListEnd end;            // the end of the step's rebuild, by block 0 of the
+  int end_rebuild;        // first loop (end_rebuild = 1)
   int split_den, split_frc;  // units a chunk is split into (1, 2 or 4)
   int lpa_den, lpa_frc;   // lanes per slot of the density / force loops
   int thr_den, thr_frc;   // threads per block of the density / force loops
@@ -294,6 +312,15 @@ struct StepArgs {
 // input order (NULL: not wanted).
 struct ExportDst {
   double *x, *p, *f, *epot, *rho, *df;
+};
+
+// Tile of a block of IMDG_BLOCK slots (list build).
+struct Tile {
+  int4 run[IMDG_MAXRUN];  // (first slot, length, first LDS record, 0)
+  int nrun;
+  int natoms;             // records in the tile
+  int ok;                 // 0: did not fit, the list reads from HBM/L2
+  int pad;
 };
 
 struct BuildArgs {
@@ -308,11 +335,11 @@ struct BuildArgs {
   double4* xnbl;
   void* rec_a;            // float4 or double4 per slot (see mixed)
   int mixed;
-  int* cellid;            // cell of slot (binning order)
-  int* cslot;             // slot inside the cell from the atomic counter
-  int* acell;             // cell of slot after the permutation
-  signed char* atype;     // type of slot after the permutation
-  int* perm;              // new slot -> old slot
+  int* acell;             // cell of slot (new order)
+  signed char* atype;     // type of slot (new order)
+  int* bucket;            // slots (old order) of each cell's atoms,
+  int bucket_cap;         // bucket_cap places per cell
+  int scan_in_bin;        // the last block of k_bin scans the cell counts
   int* cell_cnt;          // atomic counters (zero outside a rebuild)
   int* cell_loc;          // first slot of a cell relative to its scan tile
   int* tile_sum;          // atoms per scan tile
@@ -320,10 +347,12 @@ struct BuildArgs {
   const int* tile_rep;    // scan tile -> replica
   int* cell_beg;
   int* cell_num;
-  Tile* tiles;
   uint32_t* nbr;
   int* nnb;
   int* blkmax;            // longest list of every block (k_list)
+  ListEnd end;
+  Tile* tiles;            // tiles built by a launch of their own (NULL: by
+                          // the list's blocks)
   int tile_cap;           // records a tile may hold (<= IMDG_TILE_CAP)
   int* cmeta;             // chunk metadata of the 16-bit list format
   int list16;             // build the 16-bit format where a chunk allows

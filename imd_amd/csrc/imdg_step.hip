@@ -22,6 +22,8 @@
 //   skin test          check_nblist src/imd_forces_nbl.c:2007-2037
 #include "imdg_device.h"
 
+#include <algorithm>
+
 namespace imdg {
 
 // Largest block of the force loop (its launch bound).  FP32: 1024 threads
@@ -317,142 +319,83 @@ __device__ bool replica_step_end(StepArgs<R>& a, int r, const double* tot,
   return need != 0;
 }
 
-// Wavefront-wide compensated combine of per-lane (sum, compensation)
-// pairs in a fixed shuffle order (TwoSum keeps the error); max for
-// PB_MAXD.  Result valid in every lane.
-__device__ __forceinline__ void wave_combine(double (&s)[PB_N + 1],
-                                             double (&c)[PB_N + 1]) {
+// Compensated sums of a replica's partials in a fixed order (the result
+// does not depend on which block finishes last), thermostat, skin decision,
+// thermo record; called by a whole block.  One wavefront per quantity (the
+// six of partB, then partA's embedding energy), so the 7 reductions of a
+// small launch run side by side: one chain of loads, additions and lane
+// moves each.  Returns (thread 0) whether the replica needs a rebuild.
+// One replica: partials per block of the finalising kernel and of the
+// density loop; several: per unit, the replica's own range.
+template <typename R>
+__device__ bool finalize_replica(StepArgs<R>& a, int r, bool forces,
+                                 bool moved, double* ltot) {
+  const int nw = blockDim.x / IMDG_WAVE;
+  const int w = threadIdx.x / IMDG_WAVE, l = threadIdx.x % IMDG_WAVE;
+  int b0 = 0, b1 = a.unitsB, e0 = 0, e1 = a.unitsA;
+  if (a.part_chunk) {
+    const RepDev& Rp = a.rep[r];
+    const int c0 = Rp.blk_off * (IMDG_BLOCK / IMDG_CHUNK);
+    const int c1 = c0 + Rp.nblk * (IMDG_BLOCK / IMDG_CHUNK);
+    b0 = c0 * a.split_frc;
+    b1 = c1 * a.split_frc;
+    e0 = c0 * a.split_den;
+    e1 = c1 * a.split_den;
+  }
+  if (!forces || !a.has_eam) e1 = e0;
+  for (int q = w; q <= PB_N; q += nw) {
+    const double* p = q < PB_N ? a.partB + q : a.partA;
+    const int st = q < PB_N ? PB_N : 1;
+    const int u0 = q < PB_N ? b0 : e0, u1 = q < PB_N ? b1 : e1;
+    double s = 0.0, c = 0.0;
+    for (int k = u0; k < u1; k += 4 * IMDG_WAVE) {
+      double v[4];  // four loads of a lane in flight
 #pragma unroll
-  for (int q = 0; q <= PB_N; q++) {
+      for (int j = 0; j < 4; j++) {
+        const int u = k + j * IMDG_WAVE + l;
+        v[j] = u < u1 ? p[(size_t)u * st] : 0.0;
+      }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      double so = __shfl_xor(s[q], o, IMDG_WAVE);
-      double co = __shfl_xor(c[q], o, IMDG_WAVE);
-      if (q == PB_MAXD) {
-        s[q] = fmax(s[q], so);
-      } else {
-        double t, e;
-        two_sum(s[q], so, t, e);
-        s[q] = t;
-        c[q] = c[q] + co + e;
+      for (int j = 0; j < 4; j++) {
+        if (q == PB_MAXD)
+          s = fmax(s, v[j]);
+        else
+          kahan_add(s, c, v[j]);
       }
     }
+    const double t = q == PB_MAXD ? wave_max(s) : wave_sum_comp(s, c);
+    if (l == 0) ltot[q] = t;
   }
+  __syncthreads();
+  bool need = false;
+  if (threadIdx.x == 0) {
+    double tot[PB_N + 1];
+#pragma unroll
+    for (int k = 0; k <= PB_N; k++) tot[k] = ltot[k];
+    need = replica_step_end(a, r, tot, forces, moved);
+  }
+  __syncthreads();
+  return need;
 }
 
-// Compensated sums of the partials of every replica (fixed order, so the
-// result does not depend on which block finishes last), thermostat, skin
-// decision, thermo record.  One replica: the whole block sums the block
-// partials (fblk = 0, nfblk = 1).  Several replicas: one wavefront per
-// replica sums that replica's chunk partials, with no block barrier per
-// replica; the replicas are spread over the nfblk finalising blocks (this
-// is block fblk), which OR their rebuild decisions into the control block.
+// The end of a step by block fblk of nfblk: the replicas fblk, fblk + nfblk,
+// ...  Several blocks OR their rebuild decisions into the control block.
 template <typename R>
 __device__ void finalize_step(StepArgs<R>& a, bool forces, bool moved,
                               int fblk, int nfblk) {
-  __shared__ double lred[IMDG_STEP_WAVES][PB_N + 1][2];
-  __shared__ int any_s;
-  int nw = blockDim.x / IMDG_WAVE;
-  int w = threadIdx.x / IMDG_WAVE, l = threadIdx.x % IMDG_WAVE;
-  if (threadIdx.x == 0) any_s = 0;
-  __syncthreads();
-  if (!a.part_chunk) {
-    // one replica: partials per wavefront of the finalising kernel (B) and
-    // of the density kernel (A)
-    int unitsB = a.unitsB;
-    double s[PB_N + 1], c[PB_N + 1];
-#pragma unroll
-    for (int q = 0; q <= PB_N; q++) s[q] = c[q] = 0.0;
-    for (int u = threadIdx.x; u < unitsB; u += blockDim.x) {
-      const double* pb = a.partB + (size_t)u * PB_N;
-#pragma unroll
-      for (int q = 0; q < PB_N; q++) {
-        if (q == PB_MAXD)
-          s[q] = fmax(s[q], pb[q]);
-        else
-          kahan_add(s[q], c[q], pb[q]);
-      }
-    }
-    if (forces && a.has_eam)
-      for (int u = threadIdx.x; u < a.unitsA; u += blockDim.x)
-        kahan_add(s[PB_N], c[PB_N], a.partA[u]);
-    wave_combine(s, c);
-    if (l == 0) {
-#pragma unroll
-      for (int q = 0; q <= PB_N; q++) {
-        lred[w][q][0] = s[q];
-        lred[w][q][1] = c[q];
-      }
-    }
-    __syncthreads();
-    // the wavefront results in wavefront order, one quantity per thread
-    __shared__ double ltot[PB_N + 1];
-    int q = threadIdx.x;
-    if (q <= PB_N) {
-      double ss = lred[0][q][0], cc = lred[0][q][1];
-      for (int k = 1; k < nw; k++) {
-        if (q == PB_MAXD) {
-          ss = fmax(ss, lred[k][q][0]);
-        } else {
-          double t, e;
-          two_sum(ss, lred[k][q][0], t, e);
-          ss = t;
-          cc = cc + lred[k][q][1] + e;
-        }
-      }
-      ltot[q] = (q == PB_MAXD) ? ss : ss + cc;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      double tot[PB_N + 1];
-#pragma unroll
-      for (int k = 0; k <= PB_N; k++) tot[k] = ltot[k];
-      if (replica_step_end(a, 0, tot, forces, moved)) any_s = 1;
-    }
-  } else {
-    // several replicas: one wavefront per replica, chunk partials
-    for (int r = fblk * nw + w; r < a.nrep; r += nfblk * nw) {
-      const RepDev& Rp = a.rep[r];
-      const int c0 = Rp.blk_off * (IMDG_BLOCK / IMDG_CHUNK);
-      const int c1 = c0 + Rp.nblk * (IMDG_BLOCK / IMDG_CHUNK);
-      double s[PB_N + 1], c[PB_N + 1];
-#pragma unroll
-      for (int q = 0; q <= PB_N; q++) s[q] = c[q] = 0.0;
-      for (int u = c0 * a.split_frc + l; u < c1 * a.split_frc;
-           u += IMDG_WAVE) {
-        const double* pb = a.partB + (size_t)u * PB_N;
-#pragma unroll
-        for (int q = 0; q < PB_N; q++) {
-          if (q == PB_MAXD)
-            s[q] = fmax(s[q], pb[q]);
-          else
-            kahan_add(s[q], c[q], pb[q]);
-        }
-      }
-      if (forces && a.has_eam)
-        for (int u = c0 * a.split_den + l; u < c1 * a.split_den;
-             u += IMDG_WAVE)
-          kahan_add(s[PB_N], c[PB_N], a.partA[u]);
-      wave_combine(s, c);
-      if (l == 0) {
-        double tot[PB_N + 1];
-#pragma unroll
-        for (int q = 0; q <= PB_N; q++)
-          tot[q] = (q == PB_MAXD) ? s[q] : s[q] + c[q];
-        if (replica_step_end(a, r, tot, forces, moved)) atomicOr(&any_s, 1);
-      }
-    }
-  }
-  __syncthreads();
+  __shared__ double ltot[PB_N + 1];
+  bool any = false;
+  for (int r = fblk; r < a.nrep; r += nfblk)
+    any |= finalize_replica(a, r, forces, moved, ltot);
   if (threadIdx.x == 0) {
     if (moved && nfblk == 1) {
-      a.ctl->any_rebuild = any_s ? 1 : 0;
+      a.ctl->any_rebuild = any ? 1 : 0;
       a.ctl->steps_done += 1;
     } else if (moved) {
       // every block has read steps_done (its thermo records) before it
       // counts itself done; the last one advances the step.  The flag is
       // clear at this point (the last rebuild cleared it).
-      if (any_s) atomicOr(&a.ctl->any_rebuild, 1);
+      if (any) atomicOr(&a.ctl->any_rebuild, 1);
       unsigned t = atomicAdd(&a.ctl->done[DC_FINBLK], 1u);
       if (t == (unsigned)nfblk - 1) {
         a.ctl->done[DC_FINBLK] = 0;
@@ -1454,7 +1397,9 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS)
   // register serves both: the remainder is at a constant distance)
   __shared__ R4 wofs[IMDG_STEP_WAVES][2][IMDG_NCODES];
   __shared__ ColPar<R> cpr[IMDG_MAXCOLS];
+  __shared__ int done_red[2 * IMDG_STEP_WAVES];
   if (a.ctl->frozen) return;
+  if (a.end_rebuild && blockIdx.x == 0) list_done(a.end, done_red);
   const TabDev<R>& tr = tabs[1];
   const TabDev<R>& te = tabs[2];
   const int klo = LT ? a.lds_lo : 0;
@@ -1881,10 +1826,10 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS) k_move(StepArgs<R> a) {
   if (a.final_inline) last_block_finalize(a, false, true);
 }
 
-// The end of a step as a launch of its own (one block), when the step
-// kernels leave it out (final_inline = 0).
+// The end of a step as a launch of its own (one block per replica, up to
+// IMDG_FIN_BLOCKS), when the step kernels leave it out (final_inline = 0).
 template <typename R>
-__global__ void __launch_bounds__(IMDG_STEP_THREADS)
+__global__ void __launch_bounds__(IMDG_FIN_THREADS)
     k_finalize(StepArgs<R> a, int forces, int moved) {
   if (a.ctl->frozen) return;
   finalize_step(a, forces != 0, moved != 0, blockIdx.x, gridDim.x);
@@ -1894,7 +1839,9 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS)
 // (u, type) records (rec_a is rewritten by the integration in that loop).
 template <typename R>
 __global__ void __launch_bounds__(256) k_copyrec(StepArgs<R> a, int nslots) {
+  __shared__ int done_red[2 * (256 / IMDG_WAVE)];
   if (a.ctl->frozen) return;
+  if (a.end_rebuild && blockIdx.x == 0) list_done(a.end, done_red);
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < nslots) a.rec_b[i] = a.rec_a[i];
 }
@@ -2327,13 +2274,7 @@ hipError_t launch_move(const StepArgs<R>& a, int grid, hipStream_t st) {
 template <typename R>
 hipError_t launch_finalize(const StepArgs<R>& a, bool forces, bool moved,
                            hipStream_t st) {
-  // several replicas: one block per IMDG_STEP_WAVES replicas (one wavefront
-  // each); one replica: one wavefront (its lanes sum the block partials, and
-  // no combine over wavefronts follows: the end of the step is a chain of
-  // dependent operations, and a shorter chain ends it sooner)
-  int nblk =
-      a.part_chunk ? (a.nrep + IMDG_STEP_WAVES - 1) / IMDG_STEP_WAVES : 1;
-  int threads = a.part_chunk ? IMDG_STEP_THREADS : IMDG_WAVE;
+  const int nblk = std::min(a.nrep, IMDG_FIN_BLOCKS), threads = IMDG_FIN_THREADS;
   hipLaunchKernelGGL((k_finalize<R>), dim3(nblk), dim3(threads), 0, st, a,
                      forces ? 1 : 0, moved ? 1 : 0);
   return hipGetLastError();

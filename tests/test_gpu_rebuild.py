@@ -1,0 +1,95 @@
+"""The rebuild chain: cells with more atoms than their bucket has places (a
+dense cluster in an empty box: the buckets are sized from the mean and have
+to grow, in calc_forces and in the middle of fused steps), the scan of the
+cell counts in the binning's last block or in its own launch, and replicas
+of which only some rebuild."""
+import numpy as np
+import pytest
+
+from imd_amd import imdg as G
+from imd_amd import workloads as W
+
+from helpers import (canon_pairs_gpu, canon_pairs_oracle, eam_tables,
+                     oracle_eam)
+from test_gpu_tuning import TOL, _check_static
+
+pytestmark = pytest.mark.gpu
+
+
+def _cluster(temp=0.0):
+    """A 6^3-cell block in a box 12 times as wide: 64 times fewer atoms per
+    cell on average than in the block."""
+    s = W.eam_crystal(n_cells=6, temp_k=temp, seed=8, displace=0.02)
+    s.x = s.x + 100.0
+    s.box = s.box * 12.0
+    return s
+
+
+@pytest.mark.parametrize("precision", [G.FP64, G.MIXED])
+def test_bucket_overflow_static(precision):
+    eam, s = eam_tables(), _cluster()
+    # list radius 8 A: about 43 atoms in a full cell, 32 places in a bucket
+    orc = oracle_eam(s, eam, nbl_margin=3.0, timestep=W.FS)
+    orc.calc_forces()
+    with G.eam_context(eam, [s], precision=precision, nbl_margin=3.0) as gpu:
+        gpu.calc_forces()
+        _check_static(gpu, orc, *TOL[precision])
+        assert canon_pairs_gpu(gpu.pairs()) == canon_pairs_oracle(orc.pairs())
+
+
+def test_bucket_overflow_in_run():
+    """The overflow met by fused steps: the missing steps are run again and
+    the trajectory is that of a context whose buckets already fit."""
+    eam, s = eam_tables(), _cluster(temp=300.0)
+    got = []
+    for first in (False, True):
+        with G.eam_context(eam, [s], precision=G.FP64, nbl_margin=3.0) as gpu:
+            if first:
+                gpu.make_nblist()
+            gpu.run(12)
+            got.append((gpu.atoms(), gpu.thermo_history(0, 12)))
+    for k, v in got[0][0].items():
+        assert np.array_equal(v, got[1][0][k]), k
+    assert np.array_equal(got[0][1][..., :6], got[1][1][..., :6])
+
+
+# 27, 8,000 and 8,820 cells: the scan in the binning's last block up to 8,192
+# cells, in its own launch beyond
+@pytest.mark.parametrize("box", [(3, 3, 3), (20, 20, 20), (21, 21, 20)])
+def test_scan_paths_match_oracle(box):
+    eam = eam_tables()
+    s = W.eam_crystal(n_cells=5, temp_k=300.0, seed=21, displace=0.05)
+    edge = 5.4 + 1e-6
+    if box != (3, 3, 3):
+        s.x = s.x + np.array(box) * edge * 0.9   # across the faces
+        s.box = np.diag(np.array(box) * edge)
+    orc = oracle_eam(s, eam, nbl_margin=0.4, timestep=W.FS)
+    orc.calc_forces()
+    with G.eam_context(eam, [s], precision=G.FP64) as gpu:
+        assert gpu.grid() == box
+        gpu.calc_forces()
+        _check_static(gpu, orc, *TOL[G.FP64])
+        assert canon_pairs_gpu(gpu.pairs()) == canon_pairs_oracle(orc.pairs())
+
+
+def test_some_replicas_rebuild():
+    """A hot and two cold replicas: the hot one rebuilds while the others are
+    copied; each follows the trajectory it has alone, bit for bit."""
+    eam = eam_tables()
+    systems = [W.eam_crystal(n_cells=n, temp_k=t, seed=50 + n, displace=0.02)
+               for n, t in ((5, 1.0), (6, 1500.0), (7, 1.0))]
+    with G.eam_context(eam, systems, precision=G.MIXED) as gpu:
+        gpu.set_tuning(4, 512, 4, 512)
+        gpu.run(60)
+        both, th = gpu.atoms(), gpu.thermo_history(0, 60)
+    at = 0
+    for r, s in enumerate(systems):
+        with G.eam_context(eam, [s], precision=G.MIXED) as one:
+            one.set_tuning(4, 512, 4, 512)
+            one.run(60)
+            alone, t1 = one.atoms(), one.thermo_history(0, 60)
+        for k in ("x", "p", "f", "rho"):
+            assert np.array_equal(both[k][at:at + s.n], alone[k]), (r, k)
+        assert np.array_equal(th[:, r, 6], t1[:, 0, 6])
+        at += s.n
+    assert th[1:, 1, 6].sum() > 0 and th[1:, 0, 6].sum() == 0
