@@ -47,7 +47,12 @@ hipError_t launch_export(const StepArgs<R>&, int* const[2], long,
                          const ExportDst&, int, hipStream_t);
 hipError_t launch_unsort(const RepDev*, Ctl*, const int*, int* const[2], long,
                          const double*, int, double*, int, hipStream_t);
-void launch_build(const BuildArgs&, int, bool, hipStream_t);
+template <typename R>
+bool head_fits(int);
+template <typename R>
+hipError_t launch_head(const StepArgs<R>&, const BuildArgs&, bool, hipStream_t);
+void launch_sort(const BuildArgs&, int, hipStream_t);
+void launch_list(const BuildArgs&, bool, hipStream_t);
 const char* noalloc_message();
 void launch_check(const RepDev*, Ctl*, const int*, const double4*,
                   const double4*, const double4*, double*, int, hipStream_t);
@@ -138,6 +143,8 @@ struct imdg_ctx {
   int part_chunk = 0;
   int knots_pair = 0, knots_rho = 0;   // first knot of the rho / embed tables
   int knots_embed = 0;
+  int off0[4] = {0, 0, 0, 0};          // first knot of column 0 of each
+  int off64[2] = {0, 0};               // table, of the FP64 ones
   int knots_joint = -1;                // interleaved (pair, rho), one species
   int knots_jval = -1;                 // FP64: interleaved table values
   int knots_dpoly = -1;                // FP32 rho segment polynomials
@@ -160,6 +167,9 @@ struct imdg_ctx {
   int grid_den = 0, grid_frc[2] = {0, 0}, grid_move = 0;
   int split_den = 1, split_frc[2] = {1, 1};  // units a chunk is split into
   int units_max = 0;
+  // small system: a step begins with one block that ends the step before it
+  // and sorts (k_head)
+  bool head = false;
   // one captured step (rebuild chain + density + force), replayed by
   // imdg_run when graphs are on (IMDG_GRAPH=1) and profiling is off
   bool use_graph = false;
@@ -380,17 +390,12 @@ int upload_tables(imdg_ctx* c) {
     if (!h.present) continue;
     for (int col = 0; col < h.ncols; col++) {
       td[t].off[col] = (int)kn.size();
+      if (col == 0) c->off0[t] = td[t].off[0];
       td[t].len[col] = h.len[col];
       td[t].begin[col] = (R)h.begin[col];
       td[t].end[col] = (R)h.end[col];
       td[t].invstep[col] = (R)h.invstep[col];
       td[t].twoistep[col] = (R)(2 * h.invstep[col]);
-      {
-        const double is = h.invstep[col], c0 = -h.begin[col] * is;
-        td[t].ilo[col] = (R)(is - (double)(R)is);
-        td[t].t0[col] = (R)c0;
-        td[t].t0lo[col] = (R)(c0 - (double)(R)c0);
-      }
       if (c->cubic) {
         std::vector<double> seg;
         if (!cubic_segments(h, col, t < 2, c->cfg.interpolation, seg))
@@ -650,6 +655,7 @@ int upload_tables(imdg_ctx* c) {
       if (!h.present) continue;
       for (int col = 0; col < h.ncols && col < IMDG_MAXTYPES; col++) {
         t64[q].off[col] = (int)k64.size();
+        if (col == 0) c->off64[q] = t64[q].off[0];
         t64[q].len[col] = h.len[col];
         t64[q].begin[col] = h.begin[col];
         t64[q].end[col] = h.end[col];
@@ -915,6 +921,20 @@ StepArgs<R> step_args(imdg_ctx* c) {
   a.partB = c->d_partB;
   a.ring = c->d_ring;
   a.nrep = c->nrep;
+  a.natoms0 = c->natoms[0];
+  for (int t = 0; t < 4; t++) {
+    const HostTable& h = c->tab[t];
+    if (!h.present) continue;
+    a.col0[t] = {c->off0[t], h.len[0], (R)h.begin[0], (R)h.end[0],
+                 (R)h.invstep[0], (R)(2 * h.invstep[0]), (R)0, (R)0, (R)0};
+    const double is = h.invstep[0], c0 = -h.begin[0] * is;
+    a.col0[t].ilo = (R)(is - (double)(R)is);
+    a.col0[t].t0 = (R)c0;
+    a.col0[t].t0lo = (R)(c0 - (double)(R)c0);
+    if (t >= 2)
+      a.col64[t - 2] = {c->off64[t - 2], h.len[0], h.begin[0], h.end[0], is,
+                        2 * is, 0.0, 0.0, 0.0};
+  }
   a.nchunk = c->nchunk;
   a.part_chunk = c->part_chunk;
   a.unitsA = c->grid_den;  // one partial per block
@@ -1034,17 +1054,34 @@ int grid_build(imdg_ctx* c) {
 }
 
 // The rebuild chain; done: end the rebuild in it (a step's density loop or
-// record copy does it otherwise).
-int enqueue_build(imdg_ctx* c, bool done) {
+// record copy does it otherwise); fin: the step before ends in its head
+// (small systems).
+int enqueue_build(imdg_ctx* c, bool done, bool fin) {
   ProfScope ps(c, KC_BUILD);
-  launch_build(build_args(c), grid_build(c), done, c->stream);
+  const BuildArgs b = build_args(c);
+  if (c->head) {
+    // the partials of the step before are those of its integrating force
+    // launch
+    if (c->mixed) {
+      StepArgs<float> a = step_args<float>(c);
+      a.unitsB = c->grid_frc[1];
+      HIPCHK(c, launch_head<float>(a, b, fin, c->stream));
+    } else {
+      StepArgs<double> a = step_args<double>(c);
+      a.unitsB = c->grid_frc[1];
+      HIPCHK(c, launch_head<double>(a, b, fin, c->stream));
+    }
+  } else {
+    launch_sort(b, grid_build(c), c->stream);
+  }
+  launch_list(b, done, c->stream);
   HIPCHK(c, hipGetLastError());
   return IMDG_OK;
 }
 
 template <typename R>
 hipError_t enqueue_forces_t(imdg_ctx* c, bool integrate, bool store,
-                            bool end_rebuild) {
+                            bool end_rebuild, bool fin) {
   StepArgs<R> a = step_args<R>(c);
   a.store = store ? 1 : 0;
   a.end = list_end(c);
@@ -1074,7 +1111,7 @@ hipError_t enqueue_forces_t(imdg_ctx* c, bool integrate, bool store,
     ProfScope ps(c, KC_FORCE);
     e = launch_force<R>(a, t, c->force_mode, integrate, grid, c->stream);
   }
-  if (e == hipSuccess && !c->final_inline) {
+  if (e == hipSuccess && !c->final_inline && fin) {
     ProfScope ps(c, KC_FINAL);
     e = launch_finalize<R>(a, true, integrate, c->stream);
   }
@@ -1099,13 +1136,15 @@ hipError_t enqueue_move_t(imdg_ctx* c) {
 
 // store: write rho, epot and frc (always without integration: the move
 // launch reads frc).  end_rebuild: the rebuild chain enqueued before ends
-// in this step's first loop.
-int enqueue_forces(imdg_ctx* c, bool integrate, bool store, bool end_rebuild) {
+// in this step's first loop.  fin: end the step (false: the head of the
+// next one does).
+int enqueue_forces(imdg_ctx* c, bool integrate, bool store, bool end_rebuild,
+                   bool fin) {
   store = store || !integrate;
   if (c->mixed)
-    HIPCHK(c, enqueue_forces_t<float>(c, integrate, store, end_rebuild));
+    HIPCHK(c, enqueue_forces_t<float>(c, integrate, store, end_rebuild, fin));
   else
-    HIPCHK(c, enqueue_forces_t<double>(c, integrate, store, end_rebuild));
+    HIPCHK(c, enqueue_forces_t<double>(c, integrate, store, end_rebuild, fin));
   HIPCHK(c, hipGetLastError());
   return IMDG_OK;
 }
@@ -1195,7 +1234,7 @@ int fix_overflow(imdg_ctx* c, int* fixed) {
   int zero2[2] = {0, 0};  // frozen, overflow
   HIPCHK(c, hipMemcpyAsync(&c->d_ctl->frozen, zero2, 2 * sizeof(int),
                            hipMemcpyHostToDevice, c->stream));
-  if ((rc = enqueue_build(c, true))) return rc;
+  if ((rc = enqueue_build(c, true, false))) return rc;
   *fixed = 1;
   return IMDG_OK;
 }
@@ -1213,7 +1252,7 @@ int ensure_ready(imdg_ctx* c) {
 
 // Run the build chain until it fits (calc_forces / make_nblist path).
 int build_until_fits(imdg_ctx* c) {
-  int rc = enqueue_build(c, true);
+  int rc = enqueue_build(c, true, false);
   if (rc) return rc;
   for (int tries = 0; tries < 8; tries++) {
     int fixed = 0;
@@ -1668,6 +1707,11 @@ int imdg_set_atoms(imdg_ctx* c, int nrep, const imdg_replica* reps,
   ALLOC(c->d_ring, sizeof(ThermoRec) * IMDG_RING * nrep);
   if ((rc = c->mixed ? upload_tables<float>(c) : upload_tables<double>(c)))
     return rc;
+  c->head = nrep == 1 && c->nslots <= IMDG_HEAD_SLOTS &&
+            c->ncells <= IMDG_HEAD_CELLS && !c->split_move &&
+            !c->final_inline &&
+            (c->mixed ? head_fits<float>(c->nslots)
+                      : head_fits<double>(c->nslots));
   c->nchunk = c->nslots / IMDG_CHUNK;
   c->part_chunk = nrep > 1 ? 1 : 0;
   if (c->lpa_auto_den) c->lpa_den = 0;  // chosen anew for this system
@@ -1806,7 +1850,7 @@ int imdg_calc_forces(imdg_ctx* c, int steps) {
   if (rc) return rc;
   c->stress_valid = false;
   if ((rc = build_until_fits(c))) return rc;
-  if ((rc = enqueue_forces(c, false, true, false))) return rc;
+  if ((rc = enqueue_forces(c, false, true, false, true))) return rc;
   HIPCHK(c, hipStreamSynchronize(c->stream));
   collect_profile(c);
   return IMDG_OK;
@@ -1898,8 +1942,8 @@ int imdg_deallocate_nblist(imdg_ctx* c) {
 static int capture_step(imdg_ctx* c) {
   hipGraph_t g = nullptr;
   HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-  int rc = enqueue_build(c, false);
-  if (!rc) rc = enqueue_forces(c, !c->split_move, true, true);
+  int rc = enqueue_build(c, false, false);
+  if (!rc) rc = enqueue_forces(c, !c->split_move, true, true, true);
   if (!rc && c->split_move) rc = enqueue_move(c);
   hipError_t e = hipStreamEndCapture(c->stream, &g);
   if (rc) {
@@ -1923,9 +1967,11 @@ int imdg_run(imdg_ctx* c, long nsteps) {
       HIPCHK(c, hipGraphLaunch(c->step_graph, c->stream));
   } else {
     for (long s = 0; s < nsteps; s++) {
-      if ((rc = enqueue_build(c, false))) return rc;
+      const bool last = s == nsteps - 1;
+      if ((rc = enqueue_build(c, false, c->head && s > 0))) return rc;
       // per-atom outputs only on the last step: nothing reads them between
-      if ((rc = enqueue_forces(c, !c->split_move, s == nsteps - 1, true)))
+      if ((rc = enqueue_forces(c, !c->split_move, last, true,
+                               last || !c->head)))
         return rc;
       if (c->split_move && (rc = enqueue_move(c))) return rc;
     }
@@ -2363,7 +2409,7 @@ int imdg_autotune(imdg_ctx* c, int reps, imdg_tuning* chosen) {
   if (rc) return rc;
   drop_graph(c);
   // leave forces and energies as calc_forces would
-  if ((rc = enqueue_forces(c, false, true, false))) return rc;
+  if ((rc = enqueue_forces(c, false, true, false, true))) return rc;
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return IMDG_OK;
 }

@@ -20,7 +20,7 @@
 //                      same direction and operation order as the reference, so
 //                      the pair set is identical
 //   skin test          check_nblist src/imd_forces_nbl.c:2007-2037
-#include "imdg_device.h"
+#include "imdg_sort.h"
 
 #include <algorithm>
 
@@ -93,7 +93,6 @@ __device__ void scan_cells(const BuildArgs& a, int* wsum) {
 }
 
 __global__ void __launch_bounds__(IMDG_BLOCK) k_bin(BuildArgs a) {
-#pragma clang fp contract(off)
   __shared__ int hkey[BIN_HASH], hcnt[BIN_HASH], hbase[BIN_HASH];
   __shared__ int wsum[IMDG_NWAVE], is_last;
   if (!a.ctl->any_rebuild || a.ctl->frozen) return;
@@ -110,28 +109,7 @@ __global__ void __launch_bounds__(IMDG_BLOCK) k_bin(BuildArgs a) {
   bool active = flagged && i - R.atom_off < R.natoms;
   int h = -1, rank = 0, cell = 0;
   if (active) {
-    double4* pos = a.pos[a.ctl->pos_cur];
-    double4 p = pos[i];
-    double x[3] = {p.x, p.y, p.z};
-    for (int d = 0; d < 3; d++) {
-      if (R.pbc[d] != 1) continue;
-      double f = -floor(x[0] * R.tbox[d][0] + x[1] * R.tbox[d][1] +
-                        x[2] * R.tbox[d][2]);
-      x[0] += f * R.box[d][0];
-      x[1] += f * R.box[d][1];
-      x[2] += f * R.box[d][2];
-    }
-    pos[i] = make_double4(x[0], x[1], x[2], p.w);
-    int c[3];
-    for (int d = 0; d < 3; d++) {
-      c[d] = (int)(R.gdim[d] * (x[0] * R.tbox[d][0] + x[1] * R.tbox[d][1] +
-                                x[2] * R.tbox[d][2]));
-      if (c[d] >= R.gdim[d])
-        c[d] = R.gdim[d] - 1;
-      else if (c[d] < 0)
-        c[d] = 0;
-    }
-    cell = R.cell_off + (c[0] * R.gdim[1] + c[1]) * R.gdim[2] + c[2];
+    cell = wrap_and_bin(R, a.pos[a.ctl->pos_cur], i);
     // at most IMDG_BLOCK distinct keys in BIN_HASH entries: probing ends
     h = (int)(((unsigned)cell * 2654435761u) >> 24) & (BIN_HASH - 1);
     for (;;) {
@@ -255,30 +233,6 @@ __device__ __forceinline__ int cell_first_slot(const BuildArgs& a,
 // not rebuilt is copied as it is.  The buffers are flipped by list_done once
 // the list fits (on an overflow the whole chain runs again from the old
 // buffers).  One launch for the former three (place, sort, permute).
-#define SORT_LANES 32
-
-__device__ __forceinline__ void move_atom(const BuildArgs& a, const RepDev& R,
-                                          int pc, int rc, int from, int to,
-                                          int key, int cell) {
-  const double4 p = a.pos[pc][from];
-  const double4 m = a.mom[rc][from];
-  a.pos[pc ^ 1][to] = p;
-  a.mom[rc ^ 1][to] = m;
-  a.aid[rc ^ 1][to] = key;
-  a.acell[to] = cell;
-  a.atype[to] = (signed char)p.w;
-  a.xnbl[to] = p;
-  double c[3];
-  cell_centre(R, cell, c);
-  if (a.mixed)
-    reinterpret_cast<float4*>(a.rec_a)[to] =
-        make_float4((float)(p.x - c[0]), (float)(p.y - c[1]),
-                    (float)(p.z - c[2]), (float)p.w);
-  else
-    reinterpret_cast<double4*>(a.rec_a)[to] =
-        make_double4(p.x - c[0], p.y - c[1], p.z - c[2], p.w);
-}
-
 __global__ void __launch_bounds__(256) k_sort(BuildArgs a) {
   if (!a.ctl->any_rebuild || a.ctl->frozen || a.ctl->cell_over) return;
   const int pc = a.ctl->pos_cur, rc = a.ctl->rec_cur;
@@ -995,12 +949,17 @@ __global__ void __launch_bounds__(IMDG_BLOCK)
 // launchers
 // ---------------------------------------------------------------------------
 
-// done: end the rebuild here (otherwise the step's next kernel does).
-void launch_build(const BuildArgs& b, int grid, bool done, hipStream_t st) {
+// The sort into cell order; grid: blocks of the cell sort.
+void launch_sort(const BuildArgs& b, int grid, hipStream_t st) {
   hipLaunchKernelGGL(k_bin, dim3(b.nblk), dim3(IMDG_BLOCK), 0, st, b);
   if (!b.scan_in_bin)
     hipLaunchKernelGGL(k_scan, dim3(b.nstile), dim3(IMDG_SCAN_TILE), 0, st, b);
   hipLaunchKernelGGL(k_sort, dim3(grid), dim3(256), 0, st, b);
+}
+
+// The list, after the sort.  done: end the rebuild here (otherwise the
+// step's next kernel does).
+void launch_list(const BuildArgs& b, bool done, hipStream_t st) {
   if (b.tiles)
     hipLaunchKernelGGL(k_tile, dim3((b.nblk + 3) / 4), dim3(256), 0, st, b);
   const size_t tile_lds = std::max((size_t)(b.tile_cap + 4) * sizeof(float3),

@@ -106,6 +106,10 @@
 // of latency in the list's launch); a larger system has a launch for them
 // (2,048,000 atoms, 16,000 blocks: list 694 us instead of 792).
 #define IMDG_TILE_FOLD 1024
+// Up to this many slots and cells (one replica) a step begins with a single
+// block that ends the step before and sorts, instead of three launches.
+#define IMDG_HEAD_SLOTS 7168
+#define IMDG_HEAD_CELLS 4096
 #define IMDG_BUCKET_MIN 32   // smallest bucket (atoms of a cell)
 
 // Flag bit of a block's list-length maximum (blkmax): its tile exceeded the
@@ -188,13 +192,6 @@ struct TabDev {
   int len[IMDG_MAXCOLS];  // usable segments (rows of the IMD column)
   R begin[IMDG_MAXCOLS], end[IMDG_MAXCOLS], invstep[IMDG_MAXCOLS];
   R twoistep[IMDG_MAXCOLS];
-  // the table argument t = (x - begin) istep as t0 + x istep with the
-  // constants split into R parts, istep = invstep + ilo and -begin istep =
-  // t0 + t0lo (ilo = t0lo = 0 in FP64): the FP32 loops take the segment
-  // from fma(x, invstep, t0) and add fma(x, ilo, t0lo) to its fraction, so
-  // the rounding of the two constants shifts no fraction (a shift common
-  // to every pair of a shell does not average out in the virial)
-  R ilo[IMDG_MAXCOLS], t0[IMDG_MAXCOLS], t0lo[IMDG_MAXCOLS];
 };
 
 // The embedding function (and the EEAM energy term) in FP64 for the FP32
@@ -208,6 +205,22 @@ struct Tab64 {
   int len[IMDG_MAXTYPES];
   double begin[IMDG_MAXTYPES], end[IMDG_MAXTYPES], invstep[IMDG_MAXTYPES];
   double twoistep[IMDG_MAXTYPES];
+};
+
+// Column 0 of a table, in the kernel arguments: the single-species loops
+// read their column's parameters from there (no trip to memory before the
+// first list word).
+template <typename R>
+struct Col0 {
+  int off, len;
+  R begin, end, invstep, twoistep;
+  // the table argument t = (x - begin) istep as t0 + x istep with the
+  // constants split into R parts, istep = invstep + ilo and -begin istep =
+  // t0 + t0lo (ilo = t0lo = 0 in FP64): the FP32 loops take the segment
+  // from fma(x, invstep, t0) and add fma(x, ilo, t0lo) to its fraction, so
+  // the rounding of the two constants shifts no fraction (a shift common
+  // to every pair of a shell does not average out in the virial)
+  R ilo, t0, t0lo;
 };
 
 // Column parameters as the NT > 1 neighbour loops read them from LDS.
@@ -256,6 +269,9 @@ struct StepArgs {
   double* partB;          // [unit * PB_N]
   ThermoRec* ring;        // [IMDG_RING * nrep]
   int nrep;
+  int natoms0;            // atoms of replica 0 (slots from 0)
+  Col0<R> col0[4];        // column 0 of pair, rho, embed, EEAM term
+  Col0<double> col64[2];  // ... of the FP64 embedding and EEAM term
   int nchunk;             // 64-slot chunks of all replicas
   int part_chunk;         // partials per chunk (1) or per wavefront (0)
   int unitsA;             // wavefront partials written by the density loop

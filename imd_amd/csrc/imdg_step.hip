@@ -20,9 +20,10 @@
 //   integrators        move_atoms_nve src/imd_integrate.c:122-358,
 //                      move_atoms_nvt src/imd_integrate.c:949-1141
 //   skin test          check_nblist src/imd_forces_nbl.c:2007-2037
-#include "imdg_device.h"
+#include "imdg_sort.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace imdg {
 
@@ -755,16 +756,56 @@ __device__ __forceinline__ int entry_slot(uint32_t e, const float4* off,
              : (int)(e & IMDG_IDX_MASK);
 }
 
-// The chunk's base slots into the w of the wavefront's offset row and its
-// format (true: 16-bit entries).  Called by every lane of the wavefront.
-__device__ __forceinline__ bool chunk_bases(const int* __restrict__ cmeta,
-                                            int c, int lane, float4* off) {
-  const int v = cmeta[(size_t)c * IMDG_META + min(lane, IMDG_META_WIDE)];
+// This lane's part of the chunk's metadata (16-bit lists).
+__device__ __forceinline__ int chunk_meta(const int* __restrict__ cmeta, int c,
+                                          int lane) {
+  return cmeta[(size_t)c * IMDG_META + min(lane, IMDG_META_WIDE)];
+}
+
+// The chunk's base slots (chunk_meta) into the w of the wavefront's offset
+// row and its format (true: 16-bit entries).  Called by every lane of the
+// wavefront.
+__device__ __forceinline__ bool chunk_bases(int v, int lane, float4* off) {
   if (lane < IMDG_NCODES) off[lane].w = __int_as_float(v);
   const int wide = __shfl(v, IMDG_META_WIDE, IMDG_WAVE);
   wave_lds_sync();
   return wide == 0;
 }
+
+// Replica of chunk c and its slots.  With one replica they come from the
+// kernel arguments: no chain of loads before the chunk's own.
+struct ChunkRep {
+  int r, off, n;
+};
+template <typename R>
+__device__ __forceinline__ ChunkRep chunk_rep(const StepArgs<R>& a, int c) {
+  if (a.nrep == 1) return {0, 0, a.natoms0};
+  const int r = a.blk_rep[c / (IMDG_BLOCK / IMDG_CHUNK)];
+  return {r, a.rep[r].atom_off, a.rep[r].natoms};
+}
+
+// Record and list length of the slot of a lane's next pass, loaded while
+// the pass before it (or the chunk's metadata) is on its way: the list words
+// of a pass then wait for one load less.
+template <typename R>
+struct NextSlot {
+  typedef typename V4<R>::T R4;
+  int i, nn;
+  bool mine;
+  R4 u;
+  __device__ __forceinline__ void load(const R4* __restrict__ rec,
+                                       const int* __restrict__ nnb, int i_,
+                                       const ChunkRep& cr) {
+    i = i_;
+    mine = i - cr.off < cr.n;
+    nn = 0;
+    u.x = u.y = u.z = u.w = (R)0;
+    if (mine) {
+      u = rec[i];
+      nn = nnb[i];
+    }
+  }
+};
 
 // One walk over a slot's list in the chunk's format; NT: the list words'
 // loads are non-temporal (the list_nt policy, chosen per launch).
@@ -794,10 +835,26 @@ struct ForceCols {
   R rb, re, ris, r2is;
 };
 
+// Column `it` of a table, for an interpolation (its split constants are
+// column 0's affair).
+template <typename T>
+__device__ __forceinline__ auto col_of(const T& t, int it) {
+  typedef std::remove_cv_t<std::remove_reference_t<decltype(t.begin[0])>> R;
+  Col0<R> c;
+  c.off = t.off[it];
+  c.len = t.len[it];
+  c.begin = t.begin[it];
+  c.end = t.end[it];
+  c.invstep = t.invstep[it];
+  c.twoistep = t.twoistep[it];
+  c.ilo = c.t0 = c.t0lo = (R)0;
+  return c;
+}
+
 // Table argument of the FP32 segment tables (one grid): t = (r^2 - begin)
 // istep as fma(r^2, istep, t0) clamped to [0, len - 1/2] (med3), segment
 // k = (int)t, fraction chi = fract(t) + fma(r^2, ilo, t0lo): the low parts
-// of the split constants (TabDev::ilo, t0lo) go into the fraction, where
+// of the split constants (Col0::ilo, t0lo) go into the fraction, where
 // FP32 still resolves them, instead of shifting every pair of a shell the
 // same way.
 struct TArg {
@@ -805,13 +862,13 @@ struct TArg {
 };
 
 template <typename R>
-__device__ __forceinline__ TArg targ(const TabDev<R>& t) {
+__device__ __forceinline__ TArg targ(const Col0<R>& t) {
   TArg a;
-  a.istep = (float)t.invstep[0];
-  a.ilo = (float)t.ilo[0];
-  a.t0 = (float)t.t0[0];
-  a.t0lo = (float)t.t0lo[0];
-  a.tz = (float)t.len[0] - 0.5f;
+  a.istep = (float)t.invstep;
+  a.ilo = (float)t.ilo;
+  a.t0 = (float)t.t0;
+  a.t0lo = (float)t.t0lo;
+  a.tz = (float)t.len - 0.5f;
   return a;
 }
 
@@ -1400,18 +1457,17 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS)
   __shared__ int done_red[2 * IMDG_STEP_WAVES];
   if (a.ctl->frozen) return;
   if (a.end_rebuild && blockIdx.x == 0) list_done(a.end, done_red);
-  const TabDev<R>& tr = tabs[1];
-  const TabDev<R>& te = tabs[2];
+  const Col0<R>& tr = a.col0[1];
   const int klo = LT ? a.lds_lo : 0;
   if (LT) stage_knots(a.knots, a.lds_lo, a.lds_n, (R2*)dyn_lds);
-  if (!NT1) stage_colpar(tr, klo, cpr);
+  if (!NT1) stage_colpar(tabs[1], klo, cpr);
   __syncthreads();
   const R2* __restrict__ K = LT ? (const R2*)dyn_lds : a.knots;
   const R4* __restrict__ rec = a.rec_a;
   const int nt = a.ntypes;
   // single-species column
-  const int kb0 = tr.off[0] - klo, len0 = tr.len[0];
-  const R b0 = tr.begin[0], e0 = tr.end[0], is0 = tr.invstep[0];
+  const int kb0 = tr.off - klo, len0 = tr.len;
+  const R b0 = tr.begin, e0 = tr.end, is0 = tr.invstep;
 
   Sched S = make_sched(a.nchunk * a.split_den, a.xcd_remap);
   const int lane = threadIdx.x & (IMDG_WAVE - 1);
@@ -1423,22 +1479,28 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS)
   for (int q = S.q; q < S.q1; q += S.stride) {
     const Unit un = unit_of<L>(q, a.split_den);
     const int c = un.c;
-    int r = a.blk_rep[c / (IMDG_BLOCK / IMDG_CHUNK)];
-    const RepDev& Rp = a.rep[r];
-    if (r != cur) {
-      wave_offsets(Rp, off, olo);
-      cur = r;
+    const ChunkRep cr = chunk_rep(a, c);
+    NextSlot<R> next;
+    next.load(rec, a.nnb, c * IMDG_CHUNK + un.p0 * (IMDG_WAVE / L) + ga, cr);
+    int meta = 0;
+    if constexpr (sizeof(R) == 4)
+      if (a.list16) meta = chunk_meta(a.cmeta, c, lane);
+    if (cr.r != cur) {
+      wave_offsets(a.rep[cr.r], off, olo);
+      cur = cr.r;
     }
     bool w16 = false;
     if constexpr (sizeof(R) == 4)
-      if (a.list16) w16 = chunk_bases(a.cmeta, c, lane, off);
+      if (a.list16) w16 = chunk_bases(meta, lane, off);
     R rho_keep = (R)0, pee_keep = (R)0;
 #pragma unroll 1
     for (int p = un.p0; p < un.p1; p++) {
-      int i = c * IMDG_CHUNK + p * (IMDG_WAVE / L) + ga;
+      const NextSlot<R> cs = next;
+      const int i = cs.i;
       R rho = (R)0, pee = (R)0;
-      if (i - Rp.atom_off < Rp.natoms) {
-        R4 ui = rec[i];
+      if (p + 1 < un.p1) next.load(rec, a.nnb, i + IMDG_WAVE / L, cr);
+      if (cs.mine) {
+        const R4 ui = cs.u;
         int it = NT1 ? 0 : (int)ui.w;
         DensityCol<R> col0 = {kb0, len0, b0, e0, is0};
         R r2min = (R)3.0e38;
@@ -1447,14 +1509,14 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS)
           const float* __restrict__ DQ =
               reinterpret_cast<const float*>(K + (a.dpoly - klo));
           const TArg ta = targ(tr);
-          walk_either<L, NTL>(w16, a.nbr, i, a.kmax, gs, a.nnb[i],
+          walk_either<L, NTL>(w16, a.nbr, i, a.kmax, gs, cs.nn,
                          [&](uint4 e4, auto pf, uint4& slot) {
                            density_group_poly(e4, pf, slot, rec, off, olo,
                                               ui, DQ, ta, rho, r2min);
                          });
         } else {
           auto generic = [&]() {
-            list_walk<L>(nw, a.nnb[i],
+            list_walk<L>(nw, cs.nn,
                          [&](uint4 e4, ListRef<L> pf, uint4& slot) {
                            density_group<R, NT1, CUB, EE>(
                                e4, pf, slot, rec, off, ui, it, nt, K, cpr,
@@ -1467,7 +1529,7 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS)
               const float* DR =
                   reinterpret_cast<const float*>(K + (a.drho - klo));
               const TArg ta = targ(tr);
-              walk_either<L, NTL>(w16, a.nbr, i, a.kmax, gs, a.nnb[i],
+              walk_either<L, NTL>(w16, a.nbr, i, a.kmax, gs, cs.nn,
                              [&](uint4 e4, auto pf, uint4& slot) {
                                density_group_polyl(e4, pf, slot, rec, off,
                                                    olo, ui, DR, len0, ta, rho,
@@ -1483,7 +1545,7 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS)
               const float4* __restrict__ DQ =
                   reinterpret_cast<const float4*>(a.knots + a.dpolyn);
               const TArg ta = targ(tr);
-              walk_either<L, NTL>(w16, a.nbr, i, a.kmax, gs, a.nnb[i],
+              walk_either<L, NTL>(w16, a.nbr, i, a.kmax, gs, cs.nn,
                              [&](uint4 e4, auto pf, uint4& slot) {
                                density_group_polyn(e4, pf, slot, rec, off,
                                                    olo, ui, DQ, it * nt, len0,
@@ -1510,7 +1572,7 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS)
     if (EE) pee_keep = to_slot_lane<L>(pee_keep, lane);
     int i = c * IMDG_CHUNK + lane;
     double emb = 0.0;
-    if (i - Rp.atom_off < Rp.natoms && unit_has<L>(un, lane)) {
+    if (i - cr.off < cr.n && unit_has<L>(un, lane)) {
       R4 ui = rec[i];
       int it = NT1 ? 0 : (int)ui.w;
       R rho = rho_keep;
@@ -1519,22 +1581,23 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS)
       // read FP64 knots of their own)
       double Fd, dFd;
       if constexpr (sizeof(R) == 4) {
-        const Tab64& E = a.tab64[0];
-        const double2* __restrict__ ke = a.knots64 + E.off[it];
+        const Col0<double> E = NT1 ? a.col64[0] : col_of(a.tab64[0], it);
+        const double2* __restrict__ ke = a.knots64 + E.off;
         double chi;
-        int k = tab_knot<CUB>(seg_locate((double)rho, E.begin[it], E.end[it],
-                                         E.invstep[it], E.len[it], chi));
+        int k = tab_knot<CUB>(seg_locate((double)rho, E.begin, E.end,
+                                         E.invstep, E.len, chi));
         double2 p = ke[k], q = ke[k + 1];
         Fd = tab_val<CUB, double>(p, q, chi);
-        dFd = tab_grad<CUB, double>(p, q, chi, E.twoistep[it]);
+        dFd = tab_grad<CUB, double>(p, q, chi, E.twoistep);
       } else {
-        const R2* __restrict__ ke = a.knots + te.off[it];
+        const Col0<R> te = NT1 ? a.col0[2] : col_of(tabs[2], it);
+        const R2* __restrict__ ke = a.knots + te.off;
         R chi;
-        int k = tab_knot<CUB>(seg_locate(rho, te.begin[it], te.end[it],
-                                         te.invstep[it], te.len[it], chi));
+        int k = tab_knot<CUB>(seg_locate(rho, te.begin, te.end, te.invstep,
+                                         te.len, chi));
         R2 p = ke[k], q = ke[k + 1];
         Fd = tab_val<CUB, R>(p, q, chi);
-        dFd = tab_grad<CUB, R>(p, q, chi, te.twoistep[it]);
+        dFd = tab_grad<CUB, R>(p, q, chi, te.twoistep);
       }
       if (EE) {
         // EEAM energy term E(P) and EAM_DM = 2E'(P)
@@ -1617,13 +1680,12 @@ __global__ void __launch_bounds__((ForceThreads<R, MODE>::value))
   __shared__ R4 wofs[IMDG_STEP_WAVES][2][IMDG_NCODES];
   __shared__ ColPar<R> cpp[IMDG_MAXCOLS], cpr[IMDG_MAXCOLS];
   if (a.ctl->frozen) return;
-  const TabDev<R>& tp = tabs[0];
-  const TabDev<R>& tr = tabs[1];
+  const Col0<R>&tp = a.col0[0], &tr = a.col0[1];
   const int klo = LT ? a.lds_lo : 0;
   if (LT) stage_knots(a.knots, a.lds_lo, a.lds_n, (R2*)dyn_lds);
   if (!NT1) {
-    if (HP) stage_colpar(tp, klo, cpp);
-    if (HE) stage_colpar(tr, klo, cpr);
+    if (HP) stage_colpar(tabs[0], klo, cpp);
+    if (HE) stage_colpar(tabs[1], klo, cpr);
   }
   __syncthreads();
   const R2* __restrict__ K = LT ? (const R2*)dyn_lds : a.knots;
@@ -1633,12 +1695,12 @@ __global__ void __launch_bounds__((ForceThreads<R, MODE>::value))
   const signed char* __restrict__ atype = a.atype;
   const int nt = a.ntypes;
   // single-species columns
-  const int pk0 = HP ? tp.off[0] - klo : 0, plen = HP ? tp.len[0] : 0;
-  const R pb = HP ? tp.begin[0] : (R)0, pe = HP ? tp.end[0] : (R)0,
-          pis = HP ? tp.invstep[0] : (R)0, p2is = HP ? tp.twoistep[0] : (R)0;
-  const int rk0 = HE ? tr.off[0] - klo : 0, rlen = HE ? tr.len[0] : 0;
-  const R rb = HE ? tr.begin[0] : (R)0, re = HE ? tr.end[0] : (R)0,
-          ris = HE ? tr.invstep[0] : (R)0, r2is = HE ? tr.twoistep[0] : (R)0;
+  const int pk0 = HP ? tp.off - klo : 0, plen = HP ? tp.len : 0;
+  const R pb = HP ? tp.begin : (R)0, pe = HP ? tp.end : (R)0,
+          pis = HP ? tp.invstep : (R)0, p2is = HP ? tp.twoistep : (R)0;
+  const int rk0 = HE ? tr.off - klo : 0, rlen = HE ? tr.len : 0;
+  const R rb = HE ? tr.begin : (R)0, re = HE ? tr.end : (R)0,
+          ris = HE ? tr.invstep : (R)0, r2is = HE ? tr.twoistep : (R)0;
 
   Sched S = make_sched(a.nchunk * a.split_frc, a.xcd_remap);
   const int lane = threadIdx.x & (IMDG_WAVE - 1);
@@ -1650,24 +1712,30 @@ __global__ void __launch_bounds__((ForceThreads<R, MODE>::value))
   for (int q = S.q; q < S.q1; q += S.stride) {
     const Unit un = unit_of<L>(q, a.split_frc);
     const int c = un.c;
-    int r = a.blk_rep[c / (IMDG_BLOCK / IMDG_CHUNK)];
-    const RepDev& Rp = a.rep[r];
-    if (r != cur) {
-      wave_offsets(Rp, off, olo);
-      cur = r;
+    const ChunkRep cr = chunk_rep(a, c);
+    NextSlot<R> next;
+    next.load(rec, a.nnb, c * IMDG_CHUNK + un.p0 * (IMDG_WAVE / L) + ga, cr);
+    int meta = 0;
+    if constexpr (sizeof(R) == 4)
+      if (a.list16) meta = chunk_meta(a.cmeta, c, lane);
+    if (cr.r != cur) {
+      wave_offsets(a.rep[cr.r], off, olo);
+      cur = cr.r;
     }
     bool w16 = false;
     if constexpr (sizeof(R) == 4)
-      if (a.list16) w16 = chunk_bases(a.cmeta, c, lane, off);
+      if (a.list16) w16 = chunk_bases(meta, lane, off);
     // the slot's sums kept by this lane (pass gs); vlo: the virial's sum
     // of the pair gradients' FP32 remainders (FP32 one-grid loops)
     R kx = 0, ky = 0, kz = 0, kep = 0, kvir = 0, kvlo = 0;
 #pragma unroll 1
     for (int p = un.p0; p < un.p1; p++) {
-      int i = c * IMDG_CHUNK + p * (IMDG_WAVE / L) + ga;
+      const NextSlot<R> cs = next;
+      const int i = cs.i;
       R fx = 0, fy = 0, fz = 0, ep = 0, vir = 0, vlo = 0;
-      if (i - Rp.atom_off < Rp.natoms) {
-        R4 ui = rec[i];
+      if (p + 1 < un.p1) next.load(rec, a.nnb, i + IMDG_WAVE / L, cr);
+      if (cs.mine) {
+        const R4 ui = cs.u;
         int it = NT1 ? 0 : (int)atype[i];
         R dFi = HE ? ui.w : (R)0;
         const uint32_t* nw = list_words<L>(a.nbr, i, a.kmax, gs);
@@ -1684,7 +1752,7 @@ __global__ void __launch_bounds__((ForceThreads<R, MODE>::value))
                  : nullptr;
           const TArg ta = targ(tp);
           if (a.type_bit)
-            walk_either<L, NTL>(w16, a.nbr, i, a.kmax, gs, a.nnb[i],
+            walk_either<L, NTL>(w16, a.nbr, i, a.kmax, gs, cs.nn,
                            [&](uint4 e4, auto pf, uint4& slot) {
                              force_group_sgn<true, LT>(
                                  e4, pf, slot, rec, atype, off, olo, ui,
@@ -1692,7 +1760,7 @@ __global__ void __launch_bounds__((ForceThreads<R, MODE>::value))
                                  fx, fy, fz, ep, vir, vlo, r2min);
                            });
           else
-            walk_either<L, NTL>(w16, a.nbr, i, a.kmax, gs, a.nnb[i],
+            walk_either<L, NTL>(w16, a.nbr, i, a.kmax, gs, cs.nn,
                            [&](uint4 e4, auto pf, uint4& slot) {
                              force_group_sgn<false, LT>(
                                  e4, pf, slot, rec, atype, off, olo, ui,
@@ -1709,7 +1777,7 @@ __global__ void __launch_bounds__((ForceThreads<R, MODE>::value))
             const float2* __restrict__ Rr =
                 reinterpret_cast<const float2*>(K + (a.joint - klo) + 2 * plen);
             const TArg ta = targ(tp);
-            walk_either<L, NTL>(w16, a.nbr, i, a.kmax, gs, a.nnb[i],
+            walk_either<L, NTL>(w16, a.nbr, i, a.kmax, gs, cs.nn,
                            [&](uint4 e4, auto pf, uint4& slot) {
                              force_group_sgf(e4, pf, slot, rec, off, olo, ui,
                                              0.5f * dFi, Q, Rr, ta, fx, fy,
@@ -1723,7 +1791,7 @@ __global__ void __launch_bounds__((ForceThreads<R, MODE>::value))
             const R* __restrict__ Sr =
                 reinterpret_cast<const R*>(a.knots + a.joint + 2 * plen);
             const R2* V = K + (a.jval - klo);
-            list_walk<L>(nw, a.nnb[i],
+            list_walk<L>(nw, cs.nn,
                          [&](uint4 e4, ListRef<L> pf, uint4& slot) {
                            force_group_sg<LT>(e4, pf, slot, rec, off, ui,
                                               (R)0.5 * dFi, S, Sr, V, plen,
@@ -1736,7 +1804,7 @@ __global__ void __launch_bounds__((ForceThreads<R, MODE>::value))
           ForceCols<R> fc = {pk0, plen, pb, pe, pis, p2is,
                              rk0, rlen, rb, re, ris, r2is};
           const R dmi = EE ? a.eedm[i] : (R)0;
-          list_walk<L>(nw, a.nnb[i],
+          list_walk<L>(nw, cs.nn,
                        [&](uint4 e4, ListRef<L> pf, uint4& slot) {
                          force_group<R, NT1, HP, HE, CUB, EE>(
                              e4, pf, slot, rec, atype, off, ui, dFi, it, nt,
@@ -1777,7 +1845,7 @@ __global__ void __launch_bounds__((ForceThreads<R, MODE>::value))
     if (sizeof(R) == 4) kvlo = to_slot_lane<L>(kvlo, lane);
     int i = c * IMDG_CHUNK + lane;
     double v[PB_N] = {0, 0, 0, 0, 0, 0};
-    if (i - Rp.atom_off < Rp.natoms && unit_has<L>(un, lane)) {
+    if (i - cr.off < cr.n && unit_has<L>(un, lane)) {
       if (a.store) {
         // per-atom energy: half of every pair term plus F(rho_i)
         R ei = (R)0.5 * kep + (HE ? a.epot[i] : (R)0);
@@ -1794,7 +1862,8 @@ __global__ void __launch_bounds__((ForceThreads<R, MODE>::value))
                                    (double)p2is
                              : -0.5 * (double)kvir;
       if (INTEGRATE)
-        integrate_slot(a, Rp, r, i, (double)kx, (double)ky, (double)kz, v);
+        integrate_slot(a, a.rep[cr.r], cr.r, i, (double)kx, (double)ky,
+                       (double)kz, v);
     }
     put_part(a.partB, a.part_chunk, q, v, acc);
   }
@@ -1833,6 +1902,110 @@ __global__ void __launch_bounds__(IMDG_FIN_THREADS)
     k_finalize(StepArgs<R> a, int forces, int moved) {
   if (a.ctl->frozen) return;
   finalize_step(a, forces != 0, moved != 0, blockIdx.x, gridDim.x);
+}
+
+// Sort of one replica into cell order by one block of IMDG_STEP_THREADS
+// threads: binning with the cell counters in LDS, scan, and per cell (32
+// lanes) the rank of each atom among the cell's input indices, as k_sort
+// does.  lds: 2 IMDG_HEAD_CELLS + nslots ints.
+__device__ void sort_block(const BuildArgs& a, int* lds) {
+  __shared__ int wsum[IMDG_STEP_WAVES];
+  const RepDev& R = a.rep[0];
+  const int n = R.natoms, T = blockDim.x;
+  const int lane = threadIdx.x % IMDG_WAVE, w = threadIdx.x / IMDG_WAVE;
+  int* cnt = lds;
+  int* first = cnt + IMDG_HEAD_CELLS;
+  int* perm = first + IMDG_HEAD_CELLS;
+  const int pc = a.ctl->pos_cur, rc = a.ctl->rec_cur;
+  const int* aid = a.aid[rc];
+  // an atom's cell and its place there (the buckets hold at least two ints
+  // per atom: they have twice the mean occupation, IMDG_BUCKET_MIN at least)
+  int* icell = a.bucket;
+  int* iplace = a.bucket + n;
+  for (int c = threadIdx.x; c < R.ncells; c += T) cnt[c] = 0;
+  __syncthreads();
+  for (int i = threadIdx.x; i < n; i += T) {
+    const int c = wrap_and_bin(R, a.pos[pc], i);
+    icell[i] = c;
+    iplace[i] = atomicAdd(&cnt[c], 1);
+  }
+  __syncthreads();
+  int run = 0;
+  for (int c0 = 0; c0 < R.ncells; c0 += T) {
+    const int c = c0 + threadIdx.x, v = c < R.ncells ? cnt[c] : 0;
+    int incl = v;
+#pragma unroll
+    for (int o = 1; o < IMDG_WAVE; o <<= 1) {
+      int y = __shfl_up(incl, o, IMDG_WAVE);
+      if (lane >= o) incl += y;
+    }
+    if (lane == IMDG_WAVE - 1) wsum[w] = incl;
+    __syncthreads();
+    int before = run + incl - v;
+    for (int k = 0; k < T / IMDG_WAVE; k++) {
+      if (k < w) before += wsum[k];
+      run += wsum[k];
+    }
+    if (c < R.ncells) first[c] = before;
+    __syncthreads();
+  }
+  for (int i = threadIdx.x; i < n; i += T)
+    perm[first[icell[i]] + iplace[i]] = i;
+  __syncthreads();
+  const int seg = threadIdx.x / SORT_LANES, l = threadIdx.x % SORT_LANES;
+  const int base = lane - l;
+  for (int c = seg; c < R.ncells; c += T / SORT_LANES) {
+    const int b = first[c], m = cnt[c];
+    const int* p = perm + b;
+    if (m <= SORT_LANES) {
+      const int v = l < m ? p[l] : 0;
+      const int key = l < m ? aid[v] : 0x7fffffff;
+      int rank = 0;
+      for (int k = 0; k < m; k++)
+        rank += __shfl(key, base + k, IMDG_WAVE) < key;
+      if (l < m) move_atom(a, R, pc, rc, v, b + rank, key, c);
+    } else {
+      for (int e = l; e < m; e += SORT_LANES) {
+        const int v = p[e], key = aid[v];
+        int rank = 0;
+        for (int k = 0; k < m; k++) rank += aid[p[k]] < key;
+        move_atom(a, R, pc, rc, v, b + rank, key, c);
+      }
+    }
+    if (l == 0) {
+      a.cell_beg[c] = b;
+      a.cell_num[c] = m;
+    }
+  }
+}
+
+// The head of a small system's step (one replica, one block): the end of the
+// step before (fin; a run's last step ends in k_finalize) and, when its skin
+// test or the host asks for it, the sort into cell order.  The finalize, the
+// binning and the sort as launches of their own are 8 us of an 864-atom
+// step's 29, with this one it takes 25.  One block sorts 864 atoms in about
+// 14 us and 4,000 in 45 (the launches 20 to 25 whatever the size), so the
+// line (IMDG_HEAD_SLOTS) is where a rebuild every 15 steps or so makes both
+// equal: 6,900 atoms 28.8 us per step and 29.6, 11,000 atoms 32.1 and 30.5.
+template <typename R>
+__global__ void __launch_bounds__(IMDG_STEP_THREADS)
+    k_head(StepArgs<R> a, BuildArgs b, int fin) {
+  extern __shared__ __align__(16) unsigned char dyn_lds[];
+  __shared__ double ltot[PB_N + 1];
+  __shared__ int rebuild;
+  if (a.ctl->frozen) return;
+  if (fin) {
+    const bool need = finalize_replica(a, 0, true, true, ltot);
+    if (threadIdx.x == 0) {
+      a.ctl->any_rebuild = need ? 1 : 0;
+      a.ctl->steps_done += 1;
+      rebuild = need ? 1 : 0;
+    }
+  } else if (threadIdx.x == 0) {
+    rebuild = a.ctl->any_rebuild;
+  }
+  __syncthreads();
+  if (rebuild) sort_block(b, reinterpret_cast<int*>(dyn_lds));
 }
 
 // Pair-only systems: the force loop gathers rec_b, which holds a copy of the
@@ -2280,6 +2453,26 @@ hipError_t launch_finalize(const StepArgs<R>& a, bool forces, bool moved,
   return hipGetLastError();
 }
 
+// LDS of the head of a step.
+static size_t head_lds(int nslots) {
+  return sizeof(int) * (2 * (size_t)IMDG_HEAD_CELLS + nslots);
+}
+
+// Whether a system of nslots slots can have its sort in the head of a step.
+template <typename R>
+bool head_fits(int nslots) {
+  return persistent_grid(reinterpret_cast<const void*>(&k_head<R>),
+                         IMDG_STEP_THREADS, head_lds(nslots), 1) > 0;
+}
+
+template <typename R>
+hipError_t launch_head(const StepArgs<R>& a, const BuildArgs& b, bool fin,
+                       hipStream_t st) {
+  hipLaunchKernelGGL((k_head<R>), dim3(1), dim3(IMDG_STEP_THREADS),
+                     head_lds(b.nslots), st, a, b, fin ? 1 : 0);
+  return hipGetLastError();
+}
+
 template <typename R>
 hipError_t launch_copyrec(const StepArgs<R>& a, int nslots, hipStream_t st) {
   hipLaunchKernelGGL((k_copyrec<R>), dim3((nslots + 255) / 256), dim3(256), 0,
@@ -2311,6 +2504,9 @@ hipError_t launch_stress(const StepArgs<R>& a, const TabDev<R>* tabs,
   template hipError_t launch_force<R>(const StepArgs<R>&, const TabDev<R>*, \
                                       int, bool, int, hipStream_t);
 #define IMDG_INSTANTIATE_REST(R)                                            \
+  template bool head_fits<R>(int);                                          \
+  template hipError_t launch_head<R>(const StepArgs<R>&, const BuildArgs&,  \
+                                     bool, hipStream_t);                    \
   template int step_grid_move<R>(int);                                      \
   template hipError_t launch_move<R>(const StepArgs<R>&, int, hipStream_t); \
   template hipError_t launch_copyrec<R>(const StepArgs<R>&, int,            \

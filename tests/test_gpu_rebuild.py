@@ -37,6 +37,38 @@ def test_bucket_overflow_static(precision):
         assert canon_pairs_gpu(gpu.pairs()) == canon_pairs_oracle(orc.pairs())
 
 
+@pytest.mark.parametrize("precision", [G.FP64, G.MIXED])
+@pytest.mark.parametrize("margin,kept", [(3.0, 1372), (0.4, 1372), (0.4, 1)])
+def test_one_block_sort(margin, kept, precision):
+    """A small system, whose steps begin with one block that finalizes the
+    step before and sorts: 51 atoms a cell (more than the lanes that sort
+    one), 13, and a single atom; static and over steps with rebuilds, whose
+    records end with the last step's."""
+    eam = eam_tables()
+    s = W.eam_crystal(n_cells=7, temp_k=900.0, seed=31, displace=0.05)
+    s.x, s.p, s.type, s.mass = (v[:kept] for v in (s.x, s.p, s.type, s.mass))
+    orc = oracle_eam(s, eam, nbl_margin=margin, timestep=W.FS)
+    orc.calc_forces()
+    with G.eam_context(eam, [s], precision=precision,
+                       nbl_margin=margin) as gpu:
+        gpu.calc_forces()
+        _check_static(gpu, orc, *TOL[precision])
+        assert canon_pairs_gpu(gpu.pairs()) == canon_pairs_oracle(orc.pairs())
+    runs = []
+    for parts in ((40,), (1, 13, 26)):
+        with G.eam_context(eam, [s], precision=precision,
+                           nbl_margin=margin) as gpu:
+            for n in parts:
+                gpu.run(n)
+            runs.append((gpu.atoms(), gpu.thermo_history(0, 40)))
+    assert np.array_equal(runs[0][1], runs[1][1])
+    assert np.array_equal(runs[0][1][:, 0, 0], np.arange(40))
+    for k, v in runs[0][0].items():
+        assert np.array_equal(v, runs[1][0][k]), k
+    if margin == 0.4 and kept > 1:
+        assert runs[0][1][1:, 0, 6].sum() > 0
+
+
 def test_bucket_overflow_in_run():
     """The overflow met by fused steps: the missing steps are run again and
     the trajectory is that of a context whose buckets already fit."""
