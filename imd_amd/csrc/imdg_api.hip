@@ -38,8 +38,6 @@ hipError_t launch_move(const StepArgs<R>&, int, hipStream_t);
 template <typename R>
 hipError_t launch_finalize(const StepArgs<R>&, bool, bool, hipStream_t);
 template <typename R>
-hipError_t launch_copyrec(const StepArgs<R>&, int, hipStream_t);
-template <typename R>
 hipError_t launch_stress(const StepArgs<R>&, const TabDev<R>*, double*,
                          double*, int, hipStream_t);
 template <typename R>
@@ -54,8 +52,9 @@ hipError_t launch_head(const StepArgs<R>&, const BuildArgs&, bool, hipStream_t);
 void launch_sort(const BuildArgs&, int, hipStream_t);
 void launch_list(const BuildArgs&, bool, hipStream_t);
 const char* noalloc_message();
-void launch_check(const RepDev*, Ctl*, const int*, const double4*,
-                  const double4*, const double4*, double*, int, hipStream_t);
+void launch_check(const RepDev*, RepState*, Ctl*, const int*, const double4*,
+                  const double4*, const double4*, double*, int, int, int*,
+                  hipStream_t);
 }  // namespace imdg
 
 using namespace imdg;
@@ -80,6 +79,13 @@ struct DevBuf {
   size_t bytes = 0;
 };
 
+// Pinned host memory of a context: where small results land without a
+// staging copy.
+struct Pinned {
+  Ctl ctl;
+  int invalid;
+};
+
 }  // namespace
 
 struct imdg_ctx {
@@ -87,6 +93,7 @@ struct imdg_ctx {
   std::string err;
   int dev = 0;
   hipStream_t stream = nullptr;
+  Pinned* h_pin = nullptr;
   bool mixed = false;
   bool cubic = false;   // 4-point or spline tables (cubic segments)
   bool eeam = false;    // EEAM energy term present (tab[3])
@@ -970,6 +977,9 @@ BuildArgs build_args(imdg_ctx* c) {
   }
   b.xnbl = c->d_xnbl;
   b.rec_a = c->d_reca;
+  b.rec_b = c->d_recb;
+  b.pair_only = c->tab[1].present ? 0 : 1;
+  b.list_ends = b.pair_only && c->nblk <= IMDG_LIST_ENDS ? 1 : 0;
   b.mixed = c->mixed ? 1 : 0;
   b.acell = c->d_acell;
   b.atype = c->d_atype;
@@ -1053,8 +1063,8 @@ int grid_build(imdg_ctx* c) {
   return std::max(1, std::min((c->ncells + 7) / 8, 2048));
 }
 
-// The rebuild chain; done: end the rebuild in it (a step's density loop or
-// record copy does it otherwise); fin: the step before ends in its head
+// The rebuild chain; done: end the rebuild in it (a step's density loop does
+// it otherwise, if there is one); fin: the step before ends in its head
 // (small systems).
 int enqueue_build(imdg_ctx* c, bool done, bool fin) {
   ProfScope ps(c, KC_BUILD);
@@ -1074,7 +1084,7 @@ int enqueue_build(imdg_ctx* c, bool done, bool fin) {
   } else {
     launch_sort(b, grid_build(c), c->stream);
   }
-  launch_list(b, done, c->stream);
+  launch_list(b, done || b.pair_only, c->stream);
   HIPCHK(c, hipGetLastError());
   return IMDG_OK;
 }
@@ -1089,17 +1099,11 @@ hipError_t enqueue_forces_t(imdg_ctx* c, bool integrate, bool store,
   const TabDev<R>* t = (const TabDev<R>*)c->d_tabs;
   bool nt1 = c->cfg.ntypes == 1;
   hipError_t e;
-  {
-    // the force loop gathers (u, 2F') records: from the density loop with
-    // EAM, a copy of the (u, type) records without
+  if (a.has_eam) {
     ProfScope ps(c, KC_DENSITY);
-    if (a.has_eam) {
-      a.lds_lo = c->lds_den_lo;
-      a.lds_n = c->lds_den_n;
-      e = launch_density<R>(a, t, nt1, c->grid_den, c->stream);
-    } else {
-      e = launch_copyrec<R>(a, c->nslots, c->stream);
-    }
+    a.lds_lo = c->lds_den_lo;
+    a.lds_n = c->lds_den_n;
+    e = launch_density<R>(a, t, nt1, c->grid_den, c->stream);
     if (e != hipSuccess) return e;
   }
   a.lds_lo = c->lds_frc_lo;
@@ -1186,9 +1190,10 @@ int enqueue_stress(imdg_ctx* c) {
 }
 
 int read_ctl(imdg_ctx* c, Ctl* h) {
-  HIPCHK(c, hipMemcpyAsync(h, c->d_ctl, sizeof(Ctl), hipMemcpyDeviceToHost,
-                           c->stream));
+  HIPCHK(c, hipMemcpyAsync(&c->h_pin->ctl, c->d_ctl, sizeof(Ctl),
+                           hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
+  *h = c->h_pin->ctl;
   c->list_k = h->kmax_seen;  // the list policy's size estimate
   return IMDG_OK;
 }
@@ -1518,6 +1523,12 @@ int imdg_ctx_create(const imdg_config* cfg, imdg_ctx** out) {
     delete c;
     return IMDG_ERR_HIP;
   }
+  if (hipHostMalloc((void**)&c->h_pin, sizeof(Pinned), hipHostMallocDefault) !=
+      hipSuccess) {
+    hipStreamDestroy(c->stream);
+    delete c;
+    return IMDG_ERR_NOMEM;
+  }
   *out = c;
   return IMDG_OK;
 }
@@ -1530,6 +1541,7 @@ int imdg_ctx_destroy(imdg_ctx* c) {
   drop_graph(c);
   for (auto e : c->event_pool) hipEventDestroy(e);
   free_all(c);
+  hipHostFree(c->h_pin);
   if (c->stream) hipStreamDestroy(c->stream);
   delete c;
   return IMDG_OK;
@@ -1849,9 +1861,19 @@ int imdg_calc_forces(imdg_ctx* c, int steps) {
   int rc = ensure_ready(c);
   if (rc) return rc;
   c->stress_valid = false;
-  if ((rc = build_until_fits(c))) return rc;
-  if ((rc = enqueue_forces(c, false, true, false, true))) return rc;
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  // list and forces without a look at the list in between: on an overflow
+  // the forces are no-ops, and are evaluated again on the enlarged list
+  if ((rc = enqueue_build(c, false, false))) return rc;
+  if ((rc = enqueue_forces(c, false, true, true, true))) return rc;
+  Ctl h;
+  if ((rc = read_ctl(c, &h))) return rc;
+  if (h.frozen) {
+    int fixed = 0;
+    if ((rc = fix_overflow(c, &fixed))) return rc;
+    if ((rc = build_until_fits(c))) return rc;
+    if ((rc = enqueue_forces(c, false, true, false, true))) return rc;
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+  }
   collect_profile(c);
   return IMDG_OK;
 }
@@ -1872,30 +1894,12 @@ int imdg_check_nblist(imdg_ctx* c, int* invalid) {
   if (!c) return IMDG_ERR_ARG;
   int rc = ensure_ready(c);
   if (rc) return rc;
-  launch_check(c->d_rep, c->d_ctl, c->d_blk_rep, c->d_pos[0], c->d_pos[1],
-               c->d_xnbl, c->d_maxd, c->nblk, c->stream);
+  launch_check(c->d_rep, c->d_rst, c->d_ctl, c->d_blk_rep, c->d_pos[0],
+               c->d_pos[1], c->d_xnbl, c->d_maxd, c->nrep, c->nblk,
+               &c->h_pin->invalid, c->stream);
   HIPCHK(c, hipGetLastError());
-  std::vector<double> maxd(c->nblk);
-  std::vector<RepState> st(c->nrep);
-  HIPCHK(c, hipMemcpyAsync(maxd.data(), c->d_maxd, sizeof(double) * c->nblk,
-                           hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipMemcpyAsync(st.data(), c->d_rst, sizeof(RepState) * c->nrep,
-                           hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  int any = 0;
-  for (int r = 0; r < c->nrep; r++) {
-    double m = 0.0;
-    for (int b = 0; b < c->rep[r].nblk; b++)
-      m = std::max(m, maxd[c->rep[r].blk_off + b]);
-    st[r].need_rebuild = (m > c->rep[r].skin2) ? 1 : st[r].need_rebuild;
-    any |= st[r].need_rebuild;
-  }
-  HIPCHK(c, hipMemcpyAsync(c->d_rst, st.data(), sizeof(RepState) * c->nrep,
-                           hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipMemcpyAsync(&c->d_ctl->any_rebuild, &any, sizeof(int),
-                           hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  if (invalid) *invalid = any;
+  if (invalid) *invalid = c->h_pin->invalid;
   return IMDG_OK;
 }
 

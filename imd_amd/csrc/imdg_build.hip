@@ -549,18 +549,19 @@ __device__ __noinline__ bool exact_pair(const RepDev& R,
 
 // Cell-relative position of slot j in FP32.
 template <bool MIXED>
-__device__ __forceinline__ float3 rec_xyz(const BuildArgs& a, int j) {
+__device__ __forceinline__ float3 rec_xyz(const void* rec, int j) {
   if (MIXED) {
-    const float* p = reinterpret_cast<const float*>(a.rec_a) + 4 * (size_t)j;
+    const float* p = reinterpret_cast<const float*>(rec) + 4 * (size_t)j;
     return make_float3(p[0], p[1], p[2]);
   }
-  const double* p = reinterpret_cast<const double*>(a.rec_a) + 4 * (size_t)j;
+  const double* p = reinterpret_cast<const double*>(rec) + 4 * (size_t)j;
   return make_float3((float)p[0], (float)p[1], (float)p[2]);
 }
 
 // What one lane carries through the candidate loops of its atom.
 struct ListLane {
   int i;
+  const void* rec;  // the (u, type) records
   float3 ui;
   float lo, hi;
   char* lst;  // the lane's first entry (group 0) in the chunk's format
@@ -638,7 +639,7 @@ __device__ __forceinline__ void list_cell(
       if (TOK) {
         uj[u] = make_float3(q[3 * u], q[3 * u + 1], q[3 * u + 2]);
       } else {
-        uj[u] = rec_xyz<MIXED>(a, jb + min(t0 + u, jn - 1));
+        uj[u] = rec_xyz<MIXED>(L.rec, jb + min(t0 + u, jn - 1));
       }
     }
     bool in[4], band[4];
@@ -781,6 +782,7 @@ __global__ void __launch_bounds__(IMDG_BLOCK) k_list(BuildArgs a) {
   bool flagged = a.rst[r].need_rebuild != 0;
   // the permuted positions (k_list_done flips the buffers afterwards)
   const double4* pos = a.pos[a.ctl->pos_cur ^ 1];
+  const void* rec = build_records(a);
   int kmax = a.kmax, seen = 0;
   if (flagged) {
     if (a.tiles) {
@@ -814,7 +816,7 @@ __global__ void __launch_bounds__(IMDG_BLOCK) k_list(BuildArgs a) {
           t[u] = t0 + u * IMDG_BLOCK;
           if (t[u] < tot) {
             while (t[u] >= truns[k].z + truns[k].y) k++;
-            v[u] = rec_xyz<MIXED>(a, truns[k].x + (t[u] - truns[k].z));
+            v[u] = rec_xyz<MIXED>(rec, truns[k].x + (t[u] - truns[k].z));
           }
         }
 #pragma unroll
@@ -866,7 +868,8 @@ __global__ void __launch_bounds__(IMDG_BLOCK) k_list(BuildArgs a) {
     if (mine) {
       ListLane L;
       L.i = i;
-      L.ui = rec_xyz<MIXED>(a, i);
+      L.rec = rec;
+      L.ui = rec_xyz<MIXED>(rec, i);
       const float cs = (float)R.cellsz;
       L.lo = cs * (float)(1.0 - IMDG_SCREEN_BAND);
       L.hi = cs * (float)(1.0 + IMDG_SCREEN_BAND);
@@ -912,6 +915,18 @@ __global__ void __launch_bounds__(IMDG_BLOCK) k_list(BuildArgs a) {
     for (int k = 1; k < IMDG_NWAVE; k++) m = max(m, wmax[k]);
     a.blkmax[b] = m | (flagged && !tile.ok ? IMDG_BLK_FALLBACK : 0);
   }
+  if (!a.list_ends) return;
+  __shared__ int red[2 * IMDG_NWAVE], is_last;
+  if (threadIdx.x == 0) {
+    __threadfence();
+    unsigned d = atomicAdd(&a.ctl->done[DC_LIST], 1u);
+    is_last = (d == gridDim.x - 1);
+    if (is_last) a.ctl->done[DC_LIST] = 0;
+  }
+  __syncthreads();
+  if (!is_last) return;
+  __threadfence();
+  list_done(a.end, red);
 }
 
 // The end of a rebuild as a launch of its own (one block), where no step
@@ -921,27 +936,61 @@ __global__ void __launch_bounds__(1024) k_list_done(ListEnd e) {
   list_done(e, red);
 }
 
-// check_nblist alone: max displacement^2 per block of IMDG_BLOCK slots.
+// check_nblist alone: max displacement^2 per block of IMDG_BLOCK slots; the
+// last block to finish takes each replica's maximum, marks the replicas
+// beyond half the skin and tells the host (*invalid, host memory) whether
+// any replica is marked.
 __global__ void __launch_bounds__(IMDG_BLOCK)
-    k_check(const RepDev* rep, Ctl* ctl, const int* blk_rep,
+    k_check(const RepDev* rep, RepState* rst, Ctl* ctl, const int* blk_rep,
             const double4* pos0, const double4* pos1, const double4* xnbl,
-            double* maxd) {
+            double* maxd, int nrep, int* invalid) {
   __shared__ double red[IMDG_NWAVE];
-  if (ctl->frozen) return;
+  __shared__ int is_last, any;
   int lb = blockIdx.x;
-  int r = blk_rep[lb];
-  const RepDev& Rp = rep[r];
-  int i = lb * IMDG_BLOCK + threadIdx.x;
-  const double4* pos = ctl->pos_cur ? pos1 : pos0;
-  double v = 0.0;
-  if ((i - Rp.atom_off) < Rp.natoms) v = disp2(pos[i], xnbl[i]);
-  v = wave_max(v);
-  if ((threadIdx.x % IMDG_WAVE) == 0) red[threadIdx.x / IMDG_WAVE] = v;
+  if (!ctl->frozen) {
+    int r = blk_rep[lb];
+    const RepDev& Rp = rep[r];
+    int i = lb * IMDG_BLOCK + threadIdx.x;
+    const double4* pos = ctl->pos_cur ? pos1 : pos0;
+    double v = 0.0;
+    if ((i - Rp.atom_off) < Rp.natoms) v = disp2(pos[i], xnbl[i]);
+    v = wave_max(v);
+    if ((threadIdx.x % IMDG_WAVE) == 0) red[threadIdx.x / IMDG_WAVE] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      double m = red[0];
+      for (int k = 1; k < IMDG_NWAVE; k++) m = fmax(m, red[k]);
+      maxd[lb] = m;
+    }
+  }
+  if (threadIdx.x == 0) {
+    __threadfence();
+    unsigned d = atomicAdd(&ctl->done[DC_CHECK], 1u);
+    is_last = (d == gridDim.x - 1);
+    if (is_last) ctl->done[DC_CHECK] = 0;
+    any = 0;
+  }
+  __syncthreads();
+  if (!is_last) return;
+  __threadfence();
+  // one wavefront per replica
+  const int lane = threadIdx.x % IMDG_WAVE;
+  for (int r = threadIdx.x / IMDG_WAVE; r < nrep; r += IMDG_NWAVE) {
+    const RepDev& Rp = rep[r];
+    double m = 0.0;
+    for (int b = lane; b < Rp.nblk; b += IMDG_WAVE)
+      m = fmax(m, __hip_atomic_load(&maxd[Rp.blk_off + b], __ATOMIC_RELAXED,
+                                    __HIP_MEMORY_SCOPE_AGENT));
+    m = wave_max(m);
+    if (lane == 0) {
+      if (m > Rp.skin2) rst[r].need_rebuild = 1;
+      if (rst[r].need_rebuild) atomicOr(&any, 1);
+    }
+  }
   __syncthreads();
   if (threadIdx.x == 0) {
-    double m = red[0];
-    for (int k = 1; k < IMDG_NWAVE; k++) m = fmax(m, red[k]);
-    maxd[lb] = m;
+    ctl->any_rebuild = any;
+    *invalid = any;
   }
 }
 
@@ -958,7 +1007,7 @@ void launch_sort(const BuildArgs& b, int grid, hipStream_t st) {
 }
 
 // The list, after the sort.  done: end the rebuild here (otherwise the
-// step's next kernel does).
+// density loop of the step does).
 void launch_list(const BuildArgs& b, bool done, hipStream_t st) {
   if (b.tiles)
     hipLaunchKernelGGL(k_tile, dim3((b.nblk + 3) / 4), dim3(256), 0, st, b);
@@ -970,16 +1019,16 @@ void launch_list(const BuildArgs& b, bool done, hipStream_t st) {
   else
     hipLaunchKernelGGL((k_list<false>), dim3(b.nblk), dim3(IMDG_BLOCK),
                        tile_lds, st, b);
-  if (done)
+  if (done && !b.list_ends)
     hipLaunchKernelGGL(k_list_done, dim3(1), dim3(1024), 0, st, b.end);
 }
 
-void launch_check(const RepDev* rep, Ctl* ctl, const int* blk_rep,
-                  const double4* pos0, const double4* pos1,
-                  const double4* xnbl, double* maxd, int nblk,
-                  hipStream_t st) {
-  hipLaunchKernelGGL(k_check, dim3(nblk), dim3(IMDG_BLOCK), 0, st, rep, ctl,
-                     blk_rep, pos0, pos1, xnbl, maxd);
+void launch_check(const RepDev* rep, RepState* rst, Ctl* ctl,
+                  const int* blk_rep, const double4* pos0,
+                  const double4* pos1, const double4* xnbl, double* maxd,
+                  int nrep, int nblk, int* invalid, hipStream_t st) {
+  hipLaunchKernelGGL(k_check, dim3(nblk), dim3(IMDG_BLOCK), 0, st, rep, rst,
+                     ctl, blk_rep, pos0, pos1, xnbl, maxd, nrep, invalid);
 }
 
 }  // namespace imdg

@@ -233,6 +233,13 @@ __device__ __forceinline__ double disp2(double4 a, double4 b) {
   return d0 * d0 + d1 * d1 + d2 * d2;
 }
 
+// Pair-only systems: the records the step number `step` gathers, rec_a in
+// even steps and rec_b in odd ones (the step's integration writes the other).
+template <typename P>
+__device__ __forceinline__ P* pair_records(P* rec_a, P* rec_b, long step) {
+  return (step & 1) ? rec_b : rec_a;
+}
+
 // Make the LDS stores of this wavefront visible to its own later loads
 // (no block barrier: the waves of a block run independent schedules).
 __device__ __forceinline__ void wave_lds_sync() {
@@ -245,9 +252,10 @@ __device__ __forceinline__ void wave_lds_sync() {
 // list or of a cell's bucket) freeze the state (the host enlarges what
 // overflowed and runs the chain again from the old buffers), otherwise clear
 // the rebuild flags and flip the buffers that k_sort filled.  red: two ints
-// per wavefront.  In a step it runs in block 0 of the density loop (or the
-// record copy): nothing else in that kernel reads what it writes, except
-// frozen, and the outputs of a density loop that goes on are computed again.
+// per wavefront.  In a step with EAM it runs in block 0 of the density loop:
+// nothing else in that kernel reads what it writes, except frozen, and the
+// outputs of a density loop that goes on are computed again.  (The force
+// loop reads the flip, so a pair-only step ends its rebuild before it.)
 __device__ inline void list_done(const ListEnd& e, int* red) {
   if (!e.ctl->any_rebuild || e.ctl->frozen) return;
   const int nw = blockDim.x / IMDG_WAVE, w = threadIdx.x / IMDG_WAVE;

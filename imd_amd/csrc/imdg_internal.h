@@ -18,6 +18,9 @@
 //    the coordinates are small, so FP32 keeps ~1e-7 A; the separation of a
 //    listed pair is (u_j - u_i) + offset(cell offset), offset being
 //    o . (box / grid) for o in {-1,0,1}^3 (periodic images included);
+//    Without EAM there is no 2F': the force loop gathers (u, type) from one
+//    of the two and its integration writes the other, in turn with the
+//    parity of the step counter;
 //  * nbr: uint32 full neighbour list, entry = slot | code << 27 where code
 //    is the cell offset (ox+1)*9+(oy+1)*3+(oz+1); padded per atom to a
 //    multiple of 8 with entries pointing at the atom itself through the
@@ -95,7 +98,9 @@
 #define DC_FINAL 0
 #define DC_SCAN 1
 #define DC_FINBLK 2   // finalising blocks of a step done (several replicas)
-#define DC_N 3
+#define DC_LIST 3
+#define DC_CHECK 4
+#define DC_N 5
 
 #define IMDG_SCAN_TILE 1024  // cells per block of the cell-count scan
 // Up to this many cells the last block of the binning scans their counts
@@ -110,6 +115,9 @@
 // block that ends the step before and sorts, instead of three launches.
 #define IMDG_HEAD_SLOTS 7168
 #define IMDG_HEAD_CELLS 4096
+// Pair-only systems of up to this many blocks end a rebuild in the list's
+// last block (a release fence in each); larger ones in a launch of its own.
+#define IMDG_LIST_ENDS 128
 #define IMDG_BUCKET_MIN 32   // smallest bucket (atoms of a cell)
 
 // Flag bit of a block's list-length maximum (blkmax): its tile exceeded the
@@ -258,7 +266,7 @@ struct StepArgs {
   const int* acell;       // cell of every slot (current order)
   const signed char* atype;  // type of every slot (current order)
   R4* rec_a;              // (u, type)
-  R4* rec_b;              // (u, 2F')
+  R4* rec_b;              // (u, 2F'); pair-only systems: see pair_records
   const uint32_t* nbr;
   const int* nnb;
   const R2* knots;        // knots of all tables
@@ -350,6 +358,9 @@ struct BuildArgs {
   int* aid[2];
   double4* xnbl;
   void* rec_a;            // float4 or double4 per slot (see mixed)
+  void* rec_b;            // pair_only: the records of odd steps
+  int pair_only;
+  int list_ends;          // the last block of k_list ends the rebuild
   int mixed;
   int* acell;             // cell of slot (new order)
   signed char* atype;     // type of slot (new order)

@@ -38,6 +38,12 @@ __device__ __forceinline__ int wrap_and_bin(const RepDev& R, double4* pos,
 // Lanes of one cell in the sorts.
 #define SORT_LANES 32
 
+// The (u, type) records of the step being built for.
+__device__ __forceinline__ void* build_records(const BuildArgs& a) {
+  return a.pair_only ? pair_records(a.rec_a, a.rec_b, a.ctl->steps_done)
+                     : a.rec_a;
+}
+
 __device__ __forceinline__ void move_atom(const BuildArgs& a, const RepDev& R,
                                           int pc, int rc, int from, int to,
                                           int key, int cell) {
@@ -51,12 +57,13 @@ __device__ __forceinline__ void move_atom(const BuildArgs& a, const RepDev& R,
   a.xnbl[to] = p;
   double c[3];
   cell_centre(R, cell, c);
+  void* rec = build_records(a);
   if (a.mixed)
-    reinterpret_cast<float4*>(a.rec_a)[to] =
+    reinterpret_cast<float4*>(rec)[to] =
         make_float4((float)(p.x - c[0]), (float)(p.y - c[1]),
                     (float)(p.z - c[2]), (float)p.w);
   else
-    reinterpret_cast<double4*>(a.rec_a)[to] =
+    reinterpret_cast<double4*>(rec)[to] =
         make_double4(p.x - c[0], p.y - c[1], p.z - c[2], p.w);
 }
 

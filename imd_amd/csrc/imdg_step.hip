@@ -484,6 +484,7 @@ template <typename R>
 __device__ __forceinline__ void integrate_slot(StepArgs<R>& a,
                                                const RepDev& Rp, int r, int i,
                                                double fx, double fy, double fz,
+                                               typename V4<R>::T* rec_out,
                                                double (&v)[PB_N]) {
   typedef typename V4<R>::T R4;
   int pc = a.ctl->pos_cur;
@@ -506,7 +507,7 @@ __device__ __forceinline__ void integrate_slot(StepArgs<R>& a,
   ra.y = (R)(x1 - c[1]);
   ra.z = (R)(x2 - c[2]);
   ra.w = (R)xi.w;
-  a.rec_a[i] = ra;
+  rec_out[i] = ra;
   v[PB_KE] = kt.ke;
   v[PB_E1] = kt.e1;
   v[PB_E2] = kt.e2;
@@ -1689,9 +1690,12 @@ __global__ void __launch_bounds__((ForceThreads<R, MODE>::value))
   }
   __syncthreads();
   const R2* __restrict__ K = LT ? (const R2*)dyn_lds : a.knots;
-  // the gathered records (rec_b): (u, 2F') from the density loop with EAM,
-  // a copy of (u, type) without; the integration below rewrites rec_a
-  const R4* __restrict__ rec = a.rec_b;
+  // the gathered records and those the integration writes: with EAM rec_b,
+  // (u, 2F') from the density loop, and rec_a; without, in turn
+  const long step = HE ? 0 : a.ctl->steps_done;
+  const R4* __restrict__ rec =
+      HE ? a.rec_b : pair_records(a.rec_a, a.rec_b, step);
+  R4* rec_out = HE ? a.rec_a : pair_records(a.rec_a, a.rec_b, step + 1);
   const signed char* __restrict__ atype = a.atype;
   const int nt = a.ntypes;
   // single-species columns
@@ -1863,7 +1867,7 @@ __global__ void __launch_bounds__((ForceThreads<R, MODE>::value))
                              : -0.5 * (double)kvir;
       if (INTEGRATE)
         integrate_slot(a, a.rep[cr.r], cr.r, i, (double)kx, (double)ky,
-                       (double)kz, v);
+                       (double)kz, rec_out, v);
     }
     put_part(a.partB, a.part_chunk, q, v, acc);
   }
@@ -1879,6 +1883,9 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS) k_move(StepArgs<R> a) {
   if (a.ctl->frozen) return;
   Sched S = make_sched(a.nchunk, a.xcd_remap);
   const int lane = threadIdx.x & (IMDG_WAVE - 1);
+  R4* rec_out = a.has_eam ? a.rec_a
+                          : pair_records(a.rec_a, a.rec_b,
+                                         a.ctl->steps_done + 1);
   double acc[PB_N] = {0, 0, 0, 0, 0, 0};
   for (int c = S.q; c < S.q1; c += S.stride) {
     int r = a.blk_rep[c / (IMDG_BLOCK / IMDG_CHUNK)];
@@ -1887,7 +1894,8 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS) k_move(StepArgs<R> a) {
     double v[PB_N] = {0, 0, 0, 0, 0, 0};
     if (i - Rp.atom_off < Rp.natoms) {
       R4 f = a.frc[i];
-      integrate_slot(a, Rp, r, i, (double)f.x, (double)f.y, (double)f.z, v);
+      integrate_slot(a, Rp, r, i, (double)f.x, (double)f.y, (double)f.z,
+                     rec_out, v);
     }
     put_part(a.partB, a.part_chunk, c, v, acc);
   }
@@ -2008,17 +2016,6 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS)
   if (rebuild) sort_block(b, reinterpret_cast<int*>(dyn_lds));
 }
 
-// Pair-only systems: the force loop gathers rec_b, which holds a copy of the
-// (u, type) records (rec_a is rewritten by the integration in that loop).
-template <typename R>
-__global__ void __launch_bounds__(256) k_copyrec(StepArgs<R> a, int nslots) {
-  __shared__ int done_red[2 * (256 / IMDG_WAVE)];
-  if (a.ctl->frozen) return;
-  if (a.end_rebuild && blockIdx.x == 0) list_done(a.end, done_red);
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < nslots) a.rec_b[i] = a.rec_a[i];
-}
-
 // Per-atom stress tensor of the step just done (STRESS_TENS:
 // src/imd_forces_nbl.c:558-581, 1283-1318, src/imd_integrate.c:411-431,
 // 1085-1094): S_i = -1/2 sum_j g_ij d d^T over the full list, with d = x_j -
@@ -2026,7 +2023,8 @@ __global__ void __launch_bounds__(256) k_copyrec(StepArgs<R> a, int nslots) {
 // 1/2 (2F'_i rho'_j + 2F'_j rho'_i)), plus p_i p_i^T / m_i with the
 // momenta after the step; components xx yy zz yz zx xy.  It gathers rec_b,
 // which still holds the (u, 2F') records the step's force loop read (the
-// integration rewrites rec_a only), on the generic knot tables.  Launched
+// integration rewrites rec_a only; without EAM, the records of the step
+// before the counter's), on the generic knot tables.  Launched
 // only on steps whose stress is read.  One thread per slot in
 // IMDG_BLOCK-thread blocks (one replica each); each block also writes the
 // sums of its atoms' six components to spart (FP64).
@@ -2062,7 +2060,8 @@ __global__ void __launch_bounds__(IMDG_BLOCK)
   const bool hp = a.has_pair != 0, he = a.has_eam != 0;
   const int nt = a.ntypes;
   const R2* __restrict__ K = a.knots;
-  const R4* __restrict__ rec = a.rec_b;
+  const R4* __restrict__ rec =
+      he ? a.rec_b : pair_records(a.rec_a, a.rec_b, a.ctl->steps_done - 1);
   const bool cub = a.cubic != 0;
   // twice the derivative of a table at segment knot k0 (3-point knots or
   // cubic segments)
@@ -2473,13 +2472,6 @@ hipError_t launch_head(const StepArgs<R>& a, const BuildArgs& b, bool fin,
   return hipGetLastError();
 }
 
-template <typename R>
-hipError_t launch_copyrec(const StepArgs<R>& a, int nslots, hipStream_t st) {
-  hipLaunchKernelGGL((k_copyrec<R>), dim3((nslots + 255) / 256), dim3(256), 0,
-                     st, a, nslots);
-  return hipGetLastError();
-}
-
 // nblk: IMDG_BLOCK-slot blocks of all replicas; stress holds 6 doubles per
 // slot, spart 6 per block.
 template <typename R>
@@ -2509,8 +2501,6 @@ hipError_t launch_stress(const StepArgs<R>& a, const TabDev<R>* tabs,
                                      bool, hipStream_t);                    \
   template int step_grid_move<R>(int);                                      \
   template hipError_t launch_move<R>(const StepArgs<R>&, int, hipStream_t); \
-  template hipError_t launch_copyrec<R>(const StepArgs<R>&, int,            \
-                                        hipStream_t);                       \
   template hipError_t launch_stress<R>(const StepArgs<R>&,                  \
                                        const TabDev<R>*, double*, double*,  \
                                        int, hipStream_t);                   \

@@ -9,8 +9,8 @@ import pytest
 from imd_amd import imdg as G
 from imd_amd import workloads as W
 
-from helpers import (canon_pairs_gpu, canon_pairs_oracle, eam_tables,
-                     oracle_eam)
+from helpers import (canon_pairs_gpu, canon_pairs_oracle, eam_tables, lj,
+                     oracle_eam, oracle_lj)
 from test_gpu_tuning import TOL, _check_static
 
 pytestmark = pytest.mark.gpu
@@ -125,3 +125,42 @@ def test_some_replicas_rebuild():
         assert np.array_equal(th[:, r, 6], t1[:, 0, 6])
         at += s.n
     assert th[1:, 1, 6].sum() > 0 and th[1:, 0, 6].sum() == 0
+
+
+@pytest.mark.parametrize("precision", [G.FP64, G.MIXED])
+@pytest.mark.parametrize("nrep,cells", [(1, 7), (1, 17), (3, 7)])
+def test_pair_only_record_turns(nrep, cells, precision):
+    """Without EAM the records alternate with the step counter: one run, runs
+    of odd lengths and the separate entry points give the same trajectory
+    through its rebuilds, and a static evaluation at its end the oracle's
+    forces."""
+    systems = [W.fcc_system((cells, cells + r, cells), 1.5496, [1.0], 0.7,
+                            60 + r) for r in range(nrep)]
+    end = []
+    for parts in ((30,), (1, 2, 7, 20), None):
+        with G.pair_context(lj(), systems, precision=precision,
+                            nbl_margin=0.15) as gpu:
+            if parts:
+                for n in parts:
+                    gpu.run(n)
+            else:
+                for _ in range(30):
+                    gpu.calc_forces()
+                    gpu.move_atoms()
+                    gpu.check_nblist()
+            th = gpu.thermo_history(0, 30)
+            end.append((gpu.atoms(), th[..., 6]))
+            rebuilt = np.nonzero(th[1:, 0, 6])[0] + 1
+    for a, t in end[1:]:
+        assert np.array_equal(t, end[0][1])
+        for k in ("x", "p", "f", "epot"):
+            assert np.array_equal(a[k], end[0][0][k]), k
+    assert rebuilt.size
+    a = end[0][0]
+    systems[0].x, systems[0].p = (a[k][:systems[0].n] for k in ("x", "p"))
+    orc = oracle_lj(systems[0], nbl_margin=0.15, timestep=0.002)
+    orc.calc_forces()
+    with G.pair_context(lj(), [systems[0]], precision=precision,
+                        nbl_margin=0.15) as gpu:
+        gpu.calc_forces()
+        _check_static(gpu, orc, *TOL[precision], has_eam=False)
