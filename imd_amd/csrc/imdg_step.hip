@@ -608,15 +608,15 @@ __device__ __forceinline__ void ready(const uint4& e) {
 // before the next body's gathers need it.  The initial values are selects
 // rather than plain loads: a phi of loads would be folded into one load
 // next to its use, which undoes the prefetch.  Lists are padded with
-// far-away entries to a multiple of 16, so with 1 or 2 lanes per slot the
-// body count is rounded up to even inside the padding and B always runs;
-// with 4 lanes a body is 16 entries and B past the last body is skipped.
+// far-away entries to a multiple of 16, so every body is whole; B past the
+// last body is skipped (running it inside the padding instead, without the
+// branch, evaluated 64 entries of a 54-neighbour list with 2 lanes where 56
+// do: 508 us per step of 2,048,000 atoms, 482 with the branch).
 template <int L, bool NT = false, typename F>
 __device__ __forceinline__ void list_walk(const uint32_t* w, int nnb, F body) {
   constexpr int E = IMDG_GROUP * L;                    // entries per body
   constexpr size_t BW = (size_t)L * IMDG_WAVE * IMDG_GROUP;  // words per body
-  int nbody = (nnb + E - 1) / E;
-  if (L <= 2) nbody = (nbody + 1) & ~1;
+  const int nbody = (nnb + E - 1) / E;
   const int blast = nbody > 0 ? nbody - 1 : 0;
   uint4 A = ListRef<L, NT>{w}.load();
   uint4 B = ListRef<L, NT>{w + (size_t)min(1, blast) * BW}.load();
@@ -627,7 +627,7 @@ __device__ __forceinline__ void list_walk(const uint32_t* w, int nnb, F body) {
   ready(A);  // both ways into the loop head then have A's words in hand
   for (int h = 0; 2 * h < nbody; h++) {
     body(A, ListRef<L, NT>{w + (size_t)min(2 * h + 2, blast) * BW}, A);
-    if (L <= 2 || 2 * h + 1 < nbody) {
+    if (2 * h + 1 < nbody) {
       body(B, ListRef<L, NT>{w + (size_t)min(2 * h + 3, blast) * BW}, B);
       // take the wait for the next A here, where only B's prefetch is newer
       // than it (at the loop head the wait counter is merged over the loop
@@ -697,8 +697,7 @@ __device__ __forceinline__ void list_walk16(const uint16_t* w, int nnb,
                                             F body) {
   constexpr int E = IMDG_GROUP * L;
   constexpr size_t BW = (size_t)L * IMDG_WAVE * IMDG_GROUP;  // halfwords
-  int nbody = (nnb + E - 1) / E;
-  if (L <= 2) nbody = (nbody + 1) & ~1;
+  const int nbody = (nnb + E - 1) / E;
   const int blast = nbody > 0 ? nbody - 1 : 0;
   uint4 A = ListRef16<L, NT>{w}.load();
   uint4 B = ListRef16<L, NT>{w + (size_t)min(1, blast) * BW}.load();
@@ -710,7 +709,7 @@ __device__ __forceinline__ void list_walk16(const uint16_t* w, int nnb,
   for (int h = 0; 2 * h < nbody; h++) {
     body(unpack16<L>(A),
          ListRef16<L, NT>{w + (size_t)min(2 * h + 2, blast) * BW}, A);
-    if (L <= 2 || 2 * h + 1 < nbody) {
+    if (2 * h + 1 < nbody) {
       body(unpack16<L>(B),
            ListRef16<L, NT>{w + (size_t)min(2 * h + 3, blast) * BW}, B);
       ready(A);
