@@ -167,11 +167,13 @@ struct imdg_ctx {
   int lpa_den = 0, lpa_frc = 0;        // lanes per slot of the two loops
   bool lpa_auto_den = false;           // ... chosen by plan_steps for the
   bool lpa_auto_frc = false;           // system's size, not by the user
+  bool thr_auto_den = false, thr_auto_frc = false;  // the block sizes too
   int thr_den = 0, thr_frc = 0;        // threads per block (0: default)
   int units_cap = 0;                   // wavefront partial slots allocated
   int lds_den_lo = 0, lds_den_n = 0;   // knots staged by the density loop
   int lds_frc_lo = 0, lds_frc_n = 0;   // knots staged by the force loop
   int grid_den = 0, grid_frc[2] = {0, 0}, grid_move = 0;
+  int wide_den = 1, wide_frc = 1;  // lanes per slot beyond lpa_*: 1, 2, 4
   int split_den = 1, split_frc[2] = {1, 1};  // units a chunk is split into
   int units_max = 0;
   // small system: a step begins with one block that ends the step before it
@@ -705,8 +707,8 @@ int upload_tables(imdg_ctx* c) {
   return IMDG_OK;
 }
 
-// Units a chunk of a neighbour loop is split into (1, 2 or 4, at most its
-// lanes per slot) for nchunk chunks on `waves` resident wavefronts: the
+// Units a chunk of a neighbour loop is split into (a power of two, at most
+// its lanes per slot) for nchunk chunks on `waves` resident wavefronts: the
 // split with the shortest run of units per wavefront, a unit taking its
 // share of the chunk's neighbour work plus a fixed part (the per-atom work
 // runs with 1/split of the lanes).  The fixed part is EPI chunks' worth.
@@ -714,7 +716,7 @@ int pick_split(int nchunk, int waves, int lanes) {
   const double EPI = 0.15;
   int best = 1;
   double cost = 1e300;
-  for (int s = 1; s <= std::min(lanes, 4); s *= 2) {
+  for (int s = 1; s <= lanes; s *= 2) {
     const long rounds = ((long)nchunk * s + waves - 1) / std::max(1, waves);
     const double t = rounds * (1.0 / s + EPI);
     if (t < cost) {
@@ -723,6 +725,18 @@ int pick_split(int nchunk, int waves, int lanes) {
     }
   }
   return best;
+}
+
+// With four lanes per slot and wavefronts to spare, each of them becomes 2
+// or 4: a pass is then one or two bodies instead of four to six in a row.
+// The line is a quarter of the resident wavefronts (864 atoms 24.2 us per
+// step with 4 lanes, 21.3 with 16; 4,000 atoms 27.1 and 24.8; 11,000 atoms in
+// FP64 30.6 and 30.9, 16,000 of two species 38.1 and 41.8).
+int pick_wide(int nchunk, int waves, int lanes) {
+  int w = 1;
+  if (lanes == 4)
+    while (w < 4 && (long)nchunk * lanes * w * 2 <= waves / 4) w *= 2;
+  return w;
 }
 
 // Blocks of a loop of `units` units: no more than there are units (a block beyond that would only stage tables and add
@@ -750,9 +764,6 @@ int plan_steps(imdg_ctx* c) {
                        : (c->knots_joint >= 0 ? 1 : 0);
   int mode = c->force_mode;
   const bool fp32 = sizeof(R) == 4;
-  if (c->thr_den <= 0) c->thr_den = IMDG_STEP_THREADS;
-  if (c->thr_frc <= 0) c->thr_frc = force_threads<R>(mode);
-  int td = c->thr_den, tf = c->thr_frc;
   // Staging the tables costs a launch 2 to 5 us, whatever the system's
   // size: the loops of a small one read them from L2.  The lines (chunks
   // per CU) lie where both are equally fast: FP32, 120 + 60 KB staged: 16,400
@@ -768,6 +779,20 @@ int plan_steps(imdg_ctx* c) {
   if (const char* e = getenv("IMDG_TABLES_IN_LDS")) no_lds = (atoi(e) == 0);
   // cubic segments, EEAM: the generic loops with the tables in HBM/L2
   if (cub || c->eeam) no_lds = 1;
+  // Default block: full, so that one staging serves 16 (FP64 forces 8)
+  // wavefronts; the smallest systems stage nothing and have at most one unit
+  // per CU, in a block of one wavefront (864 atoms 19.5 us per step, 21.3 in
+  // full blocks).
+  const bool tiny = no_lds && nt1 && c->nchunk * 16 <= c->ncu;
+  if (c->thr_den <= 0) {
+    c->thr_den = tiny ? IMDG_WAVE : IMDG_STEP_THREADS;
+    c->thr_auto_den = true;
+  }
+  if (c->thr_frc <= 0) {
+    c->thr_frc = tiny ? IMDG_WAVE : force_threads<R>(mode);
+    c->thr_auto_frc = true;
+  }
+  const int td = c->thr_den, tf = c->thr_frc;
   // Default lanes per slot.  Four lanes make the shortest pass: they win
   // while every pass of the system can have a wavefront of its own (up to
   // 65,000 atoms on 256 CUs: 32,000 atoms 47.1 us per step, 49.4 with two
@@ -812,10 +837,17 @@ int plan_steps(imdg_ctx* c) {
         step_grid_density<R>(nt1, false, 0, c->ncu, c->lpa_den, td, cub,
                              c->eeam);
   }
-  c->split_den = 1;
+  c->split_den = c->wide_den = 1;
   if (he) {
-    c->split_den =
-        pick_split(c->nchunk, c->grid_den * (td / IMDG_WAVE), c->lpa_den);
+    const bool lt = c->lds_den_n > 0;
+    c->wide_den =
+        pick_wide(c->nchunk, c->grid_den * (td / IMDG_WAVE), c->lpa_den);
+    if (c->wide_den > 1)
+      c->grid_den = step_grid_density<R>(
+          nt1, lt, c->lds_den_n * sizeof(R2), c->ncu,
+          c->lpa_den * c->wide_den, td, cub, c->eeam);
+    c->split_den = pick_split(c->nchunk, c->grid_den * (td / IMDG_WAVE),
+                              c->lpa_den * c->wide_den);
     c->grid_den = pick_grid(c->grid_den, (long)c->nchunk * c->split_den);
   }
   // force: pair and rho knots (or the interleaved table)
@@ -847,9 +879,17 @@ int plan_steps(imdg_ctx* c) {
     }
     c->grid_frc[integ] = g;
   }
+  c->wide_frc = pick_wide(
+      c->nchunk, std::min(c->grid_frc[0], c->grid_frc[1]) * (tf / IMDG_WAVE),
+      c->lpa_frc);
   for (int integ = 0; integ < 2; integ++) {
-    c->split_frc[integ] = pick_split(
-        c->nchunk, c->grid_frc[integ] * (tf / IMDG_WAVE), c->lpa_frc);
+    if (c->wide_frc > 1)
+      c->grid_frc[integ] = step_grid_force<R>(
+          mode, integ, c->lds_frc_n > 0, hp, he, c->lds_frc_n * sizeof(R2),
+          c->ncu, c->lpa_frc * c->wide_frc, tf, cub, c->eeam);
+    c->split_frc[integ] =
+        pick_split(c->nchunk, c->grid_frc[integ] * (tf / IMDG_WAVE),
+                   c->lpa_frc * c->wide_frc);
     c->grid_frc[integ] = pick_grid(c->grid_frc[integ],
                                    (long)c->nchunk * c->split_frc[integ]);
   }
@@ -917,8 +957,8 @@ StepArgs<R> step_args(imdg_ctx* c) {
   a.eeP = (R*)c->d_eeP;
   a.eedm = (R*)c->d_eedm;
   a.final_inline = c->final_inline ? 1 : 0;
-  a.lpa_den = c->lpa_den;
-  a.lpa_frc = c->lpa_frc;
+  a.lpa_den = c->lpa_den * c->wide_den;
+  a.lpa_frc = c->lpa_frc * c->wide_frc;
   a.split_den = c->split_den;
   a.split_frc = 1;  // set with the force launch
   a.rho = (R*)c->d_rho;
@@ -1358,6 +1398,7 @@ int autotune_t(imdg_ctx* c, int reps, imdg_tuning* out) {
   int rc;
   double best_d = 0.0, best_f = 0.0;
   c->lpa_auto_den = c->lpa_auto_frc = false;
+  c->thr_auto_den = c->thr_auto_frc = false;
   if (c->tab[1].present) {
     int bl = c->lpa_den, bt = c->thr_den;
     best_d = 1e300;
@@ -1728,6 +1769,8 @@ int imdg_set_atoms(imdg_ctx* c, int nrep, const imdg_replica* reps,
   c->part_chunk = nrep > 1 ? 1 : 0;
   if (c->lpa_auto_den) c->lpa_den = 0;  // chosen anew for this system
   if (c->lpa_auto_frc) c->lpa_frc = 0;
+  if (c->thr_auto_den) c->thr_den = 0;
+  if (c->thr_auto_frc) c->thr_frc = 0;
   c->units_cap = 0;  // partials are allocated below, for any plan
   if ((rc = c->mixed ? plan_steps<float>(c) : plan_steps<double>(c)))
     return rc;
@@ -2375,8 +2418,10 @@ int imdg_set_tuning(imdg_ctx* c, const imdg_tuning* t) {
     return fail(c, IMDG_ERR_ARG, "invalid tuning (lanes 1/2/4, threads a "
                 "multiple of 64 up to %d)", IMDG_STEP_THREADS);
   int old[4] = {c->lpa_den, c->thr_den, c->lpa_frc, c->thr_frc};
-  bool was_auto[2] = {c->lpa_auto_den, c->lpa_auto_frc};
+  const bool was_auto[4] = {c->lpa_auto_den, c->lpa_auto_frc,
+                            c->thr_auto_den, c->thr_auto_frc};
   c->lpa_auto_den = c->lpa_auto_frc = false;
+  c->thr_auto_den = c->thr_auto_frc = false;
   c->lpa_den = t->density_lanes;
   c->thr_den = t->density_threads;
   c->lpa_frc = t->force_lanes;
@@ -2390,6 +2435,8 @@ int imdg_set_tuning(imdg_ctx* c, const imdg_tuning* t) {
     c->lpa_frc = old[2];
     c->lpa_auto_den = was_auto[0];
     c->lpa_auto_frc = was_auto[1];
+    c->thr_auto_den = was_auto[2];
+    c->thr_auto_frc = was_auto[3];
     c->thr_frc = old[3];
     int rc = plan(c);
     if (rc) return rc;

@@ -327,7 +327,7 @@ struct StepArgs {
   const Tab64* tab64;     // EEAM energy term (tab64[1]); FP32 kernels only
   ListEnd end;            // the end of the step's rebuild, by block 0 of the
   int end_rebuild;        // first loop (end_rebuild = 1)
-  int split_den, split_frc;  // units a chunk is split into (1, 2 or 4)
+  int split_den, split_frc;  // units a chunk is split into (1 .. lanes)
   int lpa_den, lpa_frc;   // lanes per slot of the density / force loops
   int thr_den, thr_frc;   // threads per block of the density / force loops
 };

@@ -114,7 +114,7 @@ __device__ __forceinline__ Unit unit_of(int q, int split) {
     u.p0 = 0;
     u.p1 = L;
   } else {
-    const int sh = split == 2 ? 1 : 2, n = L >> sh;
+    const int sh = 31 - __clz(split), n = L >> sh;
     u.c = q >> sh;
     u.p0 = (q & (split - 1)) * n;
     u.p1 = u.p0 + n;
@@ -546,15 +546,10 @@ template <int L, typename R>
 __device__ __forceinline__ R lane_group_sum(R v) {
   if (L >= 2) v += __shfl_xor(v, 1, IMDG_WAVE);
   if (L >= 4) v += __shfl_xor(v, 2, IMDG_WAVE);
+  if (L >= 8) v += __shfl_xor(v, 4, IMDG_WAVE);
+  if (L >= 16) v += __shfl_xor(v, 8, IMDG_WAVE);
   return v;
 }
-template <int L, typename R>
-__device__ __forceinline__ R lane_group_min(R v) {
-  if (L >= 2) v = rmin(v, __shfl_xor(v, 1, IMDG_WAVE));
-  if (L >= 4) v = rmin(v, __shfl_xor(v, 2, IMDG_WAVE));
-  return v;
-}
-
 // Four list entries of one lane: with L lanes per slot, one body covers L
 // groups of the grouped layout (4L entries of the slot); lane s of the slot
 // reads words s*(4/L) .. s*(4/L) + 4/L - 1 of each of them.
@@ -807,16 +802,72 @@ struct NextSlot {
   }
 };
 
+// Walk with 8 or 16 lanes per slot (small systems): a body is 32 or 64
+// entries, mostly the whole list, so there is nothing to prefetch.  Latency
+// bounds these launches: each body in a row is half a microsecond.  Lane s
+// takes word s % 4 of every (L/4)-th group, from group s / 4; groups beyond
+// the padded list are padding entries.
+template <bool F16>
+struct NoPrefetch {
+  static constexpr bool W16 = F16;
+  __device__ __forceinline__ uint4 load() const {
+    return make_uint4(0u, 0u, 0u, 0u);
+  }
+};
+template <int L, bool W16, typename F>
+__device__ __forceinline__ void list_walk_wide(const uint32_t* nbr, int i,
+                                               int kmax, int s, int nnb,
+                                               F body) {
+  constexpr int G = IMDG_WAVE * IMDG_GROUP;  // entries per group of a chunk
+  const int ng = (nnb + IMDG_LIST_PAD - 1) / IMDG_LIST_PAD *
+                 (IMDG_LIST_PAD / IMDG_GROUP);
+  const uint32_t pad =
+      W16 ? ((uint32_t)IMDG_CODE_PAD << IMDG_K16_BITS) |
+                (uint32_t)(i & (IMDG_CHUNK - 1))
+          : (uint32_t)i | ((uint32_t)IMDG_CODE_PAD << IMDG_IDX_BITS);
+  const uint16_t* w16 =
+      reinterpret_cast<const uint16_t*>(list16_of(nbr, i, kmax)) + (s & 3);
+  const uint32_t* w32 =
+      reinterpret_cast<const uint32_t*>(list_of(nbr, i, kmax)) + (s & 3);
+  for (int g0 = s >> 2; g0 - (s >> 2) < ng; g0 += L) {
+    uint32_t e[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int g = g0 + u * (L / 4);
+      e[u] = pad;
+      if (g < ng) e[u] = W16 ? (uint32_t)w16[(size_t)g * G]
+                             : w32[(size_t)g * G];
+    }
+    uint4 none;
+    body(make_uint4(e[0], e[1], e[2], e[3]), NoPrefetch<W16>{}, none);
+  }
+}
+
 // One walk over a slot's list in the chunk's format; NT: the list words'
 // loads are non-temporal (the list_nt policy, chosen per launch).
 template <int L, bool NT, typename F>
 __device__ __forceinline__ void walk_either(bool w16, const uint32_t* nbr,
                                             int i, int kmax, int s, int nnb,
                                             F body) {
-  if (w16)
+  if constexpr (L > 4) {
+    if (w16)
+      list_walk_wide<L, true>(nbr, i, kmax, s, nnb, body);
+    else
+      list_walk_wide<L, false>(nbr, i, kmax, s, nnb, body);
+  } else if (w16)
     list_walk16<L, NT>(list_words16<L>(nbr, i, kmax, s), nnb, body);
   else
     list_walk<L, NT>(list_words<L>(nbr, i, kmax, s), nnb, body);
+}
+
+// The same for the loops that read 32-bit lists only.
+template <int L, typename F>
+__device__ __forceinline__ void walk32(const uint32_t* nbr, int i, int kmax,
+                                       int s, int nnb, F body) {
+  if constexpr (L > 4)
+    list_walk_wide<L, false>(nbr, i, kmax, s, nnb, body);
+  else
+    list_walk<L>(list_words<L>(nbr, i, kmax, s), nnb, body);
 }
 
 // Single-species column of the density loop.
@@ -1504,7 +1555,6 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS)
         int it = NT1 ? 0 : (int)ui.w;
         DensityCol<R> col0 = {kb0, len0, b0, e0, is0};
         R r2min = (R)3.0e38;
-        const uint32_t* nw = list_words<L>(a.nbr, i, a.kmax, gs);
         if constexpr (sizeof(R) == 4 && NT1 && !CUB && !EE) {
           const float* __restrict__ DQ =
               reinterpret_cast<const float*>(K + (a.dpoly - klo));
@@ -1516,8 +1566,8 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS)
                          });
         } else {
           auto generic = [&]() {
-            list_walk<L>(nw, cs.nn,
-                         [&](uint4 e4, ListRef<L> pf, uint4& slot) {
+            walk32<L>(a.nbr, i, a.kmax, gs, cs.nn,
+                         [&](uint4 e4, auto pf, uint4& slot) {
                            density_group<R, NT1, CUB, EE>(
                                e4, pf, slot, rec, off, ui, it, nt, K, cpr,
                                col0, rho, pee, is_short, r2min);
@@ -1741,7 +1791,6 @@ __global__ void __launch_bounds__((ForceThreads<R, MODE>::value))
         const R4 ui = cs.u;
         int it = NT1 ? 0 : (int)atype[i];
         R dFi = HE ? ui.w : (R)0;
-        const uint32_t* nw = list_words<L>(a.nbr, i, a.kmax, gs);
         if constexpr (MODE == FM_SGN && sizeof(R) == 4 && !CUB && !EE) {
           // several species on one grid: sums in units of 1/(2 istep)
           R r2min = (R)3.0e38;
@@ -1794,8 +1843,8 @@ __global__ void __launch_bounds__((ForceThreads<R, MODE>::value))
             const R* __restrict__ Sr =
                 reinterpret_cast<const R*>(a.knots + a.joint + 2 * plen);
             const R2* V = K + (a.jval - klo);
-            list_walk<L>(nw, cs.nn,
-                         [&](uint4 e4, ListRef<L> pf, uint4& slot) {
+            walk32<L>(a.nbr, i, a.kmax, gs, cs.nn,
+                         [&](uint4 e4, auto pf, uint4& slot) {
                            force_group_sg<LT>(e4, pf, slot, rec, off, ui,
                                               (R)0.5 * dFi, S, Sr, V, plen,
                                               pb, pe, pis, fx, fy, fz, ep,
@@ -1807,8 +1856,8 @@ __global__ void __launch_bounds__((ForceThreads<R, MODE>::value))
           ForceCols<R> fc = {pk0, plen, pb, pe, pis, p2is,
                              rk0, rlen, rb, re, ris, r2is};
           const R dmi = EE ? a.eedm[i] : (R)0;
-          list_walk<L>(nw, cs.nn,
-                       [&](uint4 e4, ListRef<L> pf, uint4& slot) {
+          walk32<L>(a.nbr, i, a.kmax, gs, cs.nn,
+                       [&](uint4 e4, auto pf, uint4& slot) {
                          force_group<R, NT1, HP, HE, CUB, EE>(
                              e4, pf, slot, rec, atype, off, ui, dFi, it, nt,
                              K, cpp, cpr, fc, a.eedm, dmi, fx, fy, fz, ep,
@@ -2172,8 +2221,17 @@ __global__ void __launch_bounds__(IMDG_BLOCK)
 // launch plans and launchers
 // ---------------------------------------------------------------------------
 
+// lpa: lanes per slot (8 and 16: the default policy's instances only).
 template <typename R, bool NT1, bool LT, bool CUB, bool EE, bool NTL>
 const void* density_fn_l(int lpa) {
+  if constexpr (!NTL) {
+    if (lpa == 16)
+      return reinterpret_cast<const void*>(
+          &k_density<R, NT1, LT, 16, CUB, EE, NTL>);
+    if (lpa == 8)
+      return reinterpret_cast<const void*>(
+          &k_density<R, NT1, LT, 8, CUB, EE, NTL>);
+  }
   if (lpa == 4)
     return reinterpret_cast<const void*>(
         &k_density<R, NT1, LT, 4, CUB, EE, NTL>);
@@ -2190,13 +2248,21 @@ template <typename R, bool NT1, bool LT, bool CUB, bool EE>
 const void* density_fn(int lpa, bool ntl) {
   constexpr bool ONEGRID = sizeof(R) == 4 && !CUB && !EE;
   if constexpr (ONEGRID)
-    if (ntl) return density_fn_l<R, NT1, LT, CUB, EE, true>(lpa);
+    if (ntl && lpa <= 4) return density_fn_l<R, NT1, LT, CUB, EE, true>(lpa);
   return density_fn_l<R, NT1, LT, CUB, EE, false>(lpa);
 }
 
 template <typename R, int MODE, bool INTEGRATE, bool HP, bool HE, bool LT,
           bool CUB, bool EE, bool NTL>
 const void* force_fn4(int lpa) {
+  if constexpr (!NTL) {
+    if (lpa == 16)
+      return reinterpret_cast<const void*>(
+          &k_force<R, MODE, INTEGRATE, HP, HE, LT, 16, CUB, EE, NTL>);
+    if (lpa == 8)
+      return reinterpret_cast<const void*>(
+          &k_force<R, MODE, INTEGRATE, HP, HE, LT, 8, CUB, EE, NTL>);
+  }
   if (lpa == 4)
     return reinterpret_cast<const void*>(
         &k_force<R, MODE, INTEGRATE, HP, HE, LT, 4, CUB, EE, NTL>);
@@ -2215,7 +2281,7 @@ const void* force_fn3(int lpa, bool ntl) {
   constexpr bool ONEGRID = sizeof(R) == 4 && INTEGRATE && !CUB && !EE &&
                            (MODE == FM_SG || MODE == FM_SGN);
   if constexpr (ONEGRID)
-    if (ntl)
+    if (ntl && lpa <= 4)
       return force_fn4<R, MODE, INTEGRATE, HP, HE, LT, CUB, EE, true>(lpa);
   return force_fn4<R, MODE, INTEGRATE, HP, HE, LT, CUB, EE, false>(lpa);
 }
@@ -2268,7 +2334,7 @@ const void* force_fn_var(bool integrate, bool hp, bool he, int lpa, bool ntl,
 }
 
 // mode: 0 one species, 1 one species on a shared grid (needs hp and he),
-// 2 several species; lpa: lanes per slot (1, 2 or 4); cub: cubic-segment
+// 2 several species; lpa: lanes per slot (1, 2, 4, 8 or 16); cub: cubic-segment
 // tables, ee: EEAM (both: modes 0 and 2 only, lt false)
 template <typename R>
 const void* force_fn(int mode, bool integrate, bool lt, bool hp, bool he,

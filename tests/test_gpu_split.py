@@ -10,7 +10,7 @@ import pytest
 from imd_amd import imdg as G
 from imd_amd import workloads as W
 
-from helpers import eam_tables, oracle_eam
+from helpers import eam_tables, lj, oracle_eam, oracle_lj
 from test_gpu_tuning import TOL, _check_static
 
 pytestmark = pytest.mark.gpu
@@ -36,6 +36,39 @@ def test_units_match_oracle(cells, precision, staged, monkeypatch):
             _check_static(gpu, orc, *TOL[precision])
             if staged != "default":
                 assert gpu.info()["tables_in_lds"] == 3
+
+
+@pytest.mark.parametrize("precision", [G.FP64, G.MIXED])
+@pytest.mark.parametrize("case", ["eam", "alloy", "lj", "spline", "vacancies"])
+def test_wide_lanes_match_oracle(case, precision):
+    """Systems small enough for 8 or 16 lanes per slot with four asked for:
+    every loop variant, lists longer and shorter than one body (64 entries),
+    and unequal ones, against the oracle."""
+    interp = G.INTERP_3POINT
+    if case == "lj":
+        s = W.fcc_system((7, 6, 8), 1.5496, [1.0], 0.7, 12, displace=0.02)
+        orc = oracle_lj(s, nbl_margin=0.3, timestep=0.002)
+        make = lambda: G.pair_context(lj(), [s], precision=precision)
+    else:
+        nsp = 2 if case == "alloy" else 1
+        eam = eam_tables(nspecies=nsp, rc=5.5 if nsp == 2 else 5.0)
+        if case == "spline":
+            interp = G.INTERP_SPLINE
+        s = W.fcc_system((6, 7, 6), 3.615, eam.masses, W.kT(700.0), 13,
+                         displace=0.04,
+                         type_fractions=(0.6, 0.4) if nsp == 2 else None,
+                         vacancy_fraction=0.4 if case == "vacancies" else 0.0)
+        orc = oracle_eam(s, eam, interp=interp, nbl_margin=0.4,
+                         timestep=W.FS)
+        make = lambda: G.eam_context(eam, [s], precision=precision,
+                                     interpolation=interp)
+    orc.calc_forces()
+    with make() as gpu:
+        gpu.calc_forces()
+        _check_static(gpu, orc, *TOL[precision], has_eam=case != "lj")
+        gpu.set_tuning(4, 256, 4, 256)
+        gpu.calc_forces()
+        _check_static(gpu, orc, *TOL[precision], has_eam=case != "lj")
 
 
 @pytest.mark.parametrize("npts", [5000, 5600, 700])
