@@ -173,7 +173,9 @@ struct imdg_ctx {
   int lds_den_lo = 0, lds_den_n = 0;   // knots staged by the density loop
   int lds_frc_lo = 0, lds_frc_n = 0;   // knots staged by the force loop
   int grid_den = 0, grid_frc[2] = {0, 0}, grid_move = 0;
-  int wide_den = 1, wide_frc = 1;  // lanes per slot beyond lpa_*: 1, 2, 4
+  int wide_den = 1;  // lanes per slot of the loops as launched: lpa_* times
+  int lanes_frc[2] = {1, 1};  // 1, 2 or 4; the force loop without and with
+                              // integration
   int split_den = 1, split_frc[2] = {1, 1};  // units a chunk is split into
   int units_max = 0;
   // small system: a step begins with one block that ends the step before it
@@ -879,17 +881,23 @@ int plan_steps(imdg_ctx* c) {
     }
     c->grid_frc[integ] = g;
   }
-  c->wide_frc = pick_wide(
+  const int wide = pick_wide(
       c->nchunk, std::min(c->grid_frc[0], c->grid_frc[1]) * (tf / IMDG_WAVE),
       c->lpa_frc);
+  c->lanes_frc[0] = c->lanes_frc[1] = c->lpa_frc * wide;
+  // A static evaluation of a pair-only system keeps its order of summation
+  // (4 lanes, FP64 one) whatever the size, unless the user chose the lanes:
+  // in a perfect crystal the forces are what that order leaves of terms that
+  // cancel, and stay the same bits.
+  if (!he && c->lpa_auto_frc) c->lanes_frc[0] = fp32 ? 4 : 1;
   for (int integ = 0; integ < 2; integ++) {
-    if (c->wide_frc > 1)
+    if (c->lanes_frc[integ] != c->lpa_frc)
       c->grid_frc[integ] = step_grid_force<R>(
           mode, integ, c->lds_frc_n > 0, hp, he, c->lds_frc_n * sizeof(R2),
-          c->ncu, c->lpa_frc * c->wide_frc, tf, cub, c->eeam);
+          c->ncu, c->lanes_frc[integ], tf, cub, c->eeam);
     c->split_frc[integ] =
         pick_split(c->nchunk, c->grid_frc[integ] * (tf / IMDG_WAVE),
-                   c->lpa_frc * c->wide_frc);
+                   c->lanes_frc[integ]);
     c->grid_frc[integ] = pick_grid(c->grid_frc[integ],
                                    (long)c->nchunk * c->split_frc[integ]);
   }
@@ -958,7 +966,6 @@ StepArgs<R> step_args(imdg_ctx* c) {
   a.eedm = (R*)c->d_eedm;
   a.final_inline = c->final_inline ? 1 : 0;
   a.lpa_den = c->lpa_den * c->wide_den;
-  a.lpa_frc = c->lpa_frc * c->wide_frc;
   a.split_den = c->split_den;
   a.split_frc = 1;  // set with the force launch
   a.rho = (R*)c->d_rho;
@@ -1150,6 +1157,7 @@ hipError_t enqueue_forces_t(imdg_ctx* c, bool integrate, bool store,
   a.lds_n = c->lds_frc_n;
   int grid = c->grid_frc[integrate ? 1 : 0];
   a.split_frc = c->split_frc[integrate ? 1 : 0];
+  a.lpa_frc = c->lanes_frc[integrate ? 1 : 0];
   a.unitsB = grid;
   {
     ProfScope ps(c, KC_FORCE);
@@ -1365,6 +1373,7 @@ int time_loop(imdg_ctx* c, bool density, int reps, double* ms,
     a.lds_n = c->lds_frc_n;
     const int grid = c->grid_frc[integrate ? 1 : 0];
     a.split_frc = c->split_frc[integrate ? 1 : 0];
+    a.lpa_frc = c->lanes_frc[integrate ? 1 : 0];
     a.unitsB = grid;
     return launch_force<R>(a, t, c->force_mode, integrate, grid, c->stream);
   };

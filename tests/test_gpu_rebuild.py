@@ -140,6 +140,7 @@ def test_pair_only_record_turns(nrep, cells, precision):
     for parts in ((30,), (1, 2, 7, 20), None):
         with G.pair_context(lj(), systems, precision=precision,
                             nbl_margin=0.15) as gpu:
+            gpu.set_tuning(4, 512, 4, 512)   # one order of summation
             if parts:
                 for n in parts:
                     gpu.run(n)
