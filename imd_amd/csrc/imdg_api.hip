@@ -126,7 +126,8 @@ struct imdg_ctx {
   double4* d_xnbl = nullptr;
   int *d_acell = nullptr, *d_bucket = nullptr;
   int bucket_cap = 0;
-  Tile* d_tiles = nullptr;  // larger systems only (IMDG_TILE_FOLD)
+  bool list_shared = false;  // several lanes per atom build its list
+  Tile* d_tiles = nullptr;   // (then without tiles in memory)
   signed char* d_atype = nullptr;
   int *d_cell_cnt = nullptr, *d_cell_beg = nullptr, *d_cell_num = nullptr;
   int *d_cell_loc = nullptr, *d_tile_sum = nullptr, *d_tile_off = nullptr,
@@ -1005,8 +1006,9 @@ StepArgs<R> step_args(imdg_ctx* c) {
 }
 
 ListEnd list_end(imdg_ctx* c) {
-  return {c->d_ctl, c->d_rst, c->d_blk_rep, c->d_blkmax,
-          c->nblk,  c->nrep,  c->kmax};
+  const int sh = c->list_shared ? 1 : 0;  // a block per chunk: two per block
+  return {c->d_ctl, c->d_rst, c->d_blk_rep, c->d_blkmax, c->nblk << sh,
+          sh,       c->nrep,  c->kmax};
 }
 
 BuildArgs build_args(imdg_ctx* c) {
@@ -1042,6 +1044,7 @@ BuildArgs build_args(imdg_ctx* c) {
   b.tile_rep = c->d_tile_rep;
   b.blkmax = c->d_blkmax;
   b.end = list_end(c);
+  b.list_shared = c->list_shared ? 1 : 0;
   b.tiles = c->d_tiles;
   b.nbr = c->d_nbr;
   b.nnb = c->d_nnb;
@@ -1742,8 +1745,12 @@ int imdg_set_atoms(imdg_ctx* c, int nrep, const imdg_replica* reps,
   ALLOC(c->d_xnbl, sizeof(double4) * ns);
   ALLOC(c->d_acell, sizeof(int) * ns);
   ALLOC(c->d_atype, ns);
+  // by the largest replica: of several, few rebuild in one step
+  c->list_shared = true;
+  for (const RepDev& R : c->rep)
+    if (R.nblk > IMDG_SHARE_BLOCKS) c->list_shared = false;
   c->d_tiles = nullptr;
-  if (c->nblk > IMDG_TILE_FOLD) ALLOC(c->d_tiles, sizeof(Tile) * c->nblk);
+  if (!c->list_shared) ALLOC(c->d_tiles, sizeof(Tile) * c->nblk);
   ALLOC(c->d_bucket, sizeof(int) * c->bucket_cap * (size_t)c->ncells);
   ALLOC(c->d_cell_cnt, sizeof(int) * c->ncells);
   ALLOC(c->d_cell_beg, sizeof(int) * c->ncells);
@@ -1752,7 +1759,7 @@ int imdg_set_atoms(imdg_ctx* c, int nrep, const imdg_replica* reps,
   ALLOC(c->d_tile_sum, sizeof(int) * c->nstile);
   ALLOC(c->d_tile_off, sizeof(int) * c->nstile);
   ALLOC(c->d_tile_rep, sizeof(int) * c->nstile);
-  ALLOC(c->d_blkmax, sizeof(int) * c->nblk);
+  ALLOC(c->d_blkmax, sizeof(int) * 2 * c->nblk);
   ALLOC(c->d_nnb, sizeof(int) * ns);
   ALLOC(c->d_reca, rs * 4 * ns);
   ALLOC(c->d_recb, rs * 4 * ns);

@@ -7,7 +7,8 @@
 // the host.  Each such idle launch costs the device about 1.7 us and the
 // host 2.7 us, which is what a small system's step consists of, so the chain
 // has as few as its data dependences allow: bin (with the scan of the cell
-// counts, for up to IMDG_SCAN_FOLD cells), sort, list; what ends it
+// counts, for up to IMDG_SCAN_FOLD cells), sort, list (with its blocks' tiles,
+// for up to IMDG_SHARE_BLOCKS blocks); what ends it
 // (list_done) runs in the step's next kernel.
 //
 // Reference semantics (paths relative to the reference root):
@@ -294,13 +295,12 @@ struct TileLds {
   int rb[TILE_MAXRANGE], re[TILE_MAXRANGE];
 };
 
-// The tile of 128-slot block b of a rebuilt replica, built by one whole
+// The tile of ns slots from s0 of a rebuilt replica, built by one whole
 // wavefront (lane l).
-__device__ void build_tile(const BuildArgs& a, const RepDev& R, int b,
+__device__ void build_tile(const BuildArgs& a, const RepDev& R, int s0, int ns,
                            TileLds& S, Tile& T) {
   int l = threadIdx.x % IMDG_WAVE;
-  int s0 = b * IMDG_BLOCK;
-  int s1 = min(s0 + IMDG_BLOCK, R.atom_off + R.natoms) - 1;
+  int s1 = min(s0 + ns, R.atom_off + R.natoms) - 1;
   if (s1 < s0) {
     if (l == 0) {
       T.nrun = 0;
@@ -447,7 +447,8 @@ __device__ void build_tile(const BuildArgs& a, const RepDev& R, int b,
   }
 }
 
-// Tiles of the rebuilt replicas, a wavefront each (larger systems).
+// Tiles of the rebuilt replicas, a wavefront each, for k_list (built by its
+// own blocks they cost it 100 us at 2,048,000 atoms, 20 here).
 __global__ void __launch_bounds__(256) k_tile(BuildArgs a) {
   __shared__ TileLds tl[256 / IMDG_WAVE];
   __shared__ Tile tt[256 / IMDG_WAVE];
@@ -457,7 +458,7 @@ __global__ void __launch_bounds__(256) k_tile(BuildArgs a) {
   if (b >= a.nblk) return;
   const int r = __builtin_amdgcn_readfirstlane(a.blk_rep[b]);
   if (!a.rst[r].need_rebuild) return;
-  build_tile(a, a.rep[r], b, tl[w], tt[w]);
+  build_tile(a, a.rep[r], b * IMDG_BLOCK, IMDG_BLOCK, tl[w], tt[w]);
   wave_lds_sync();
   Tile& T = a.tiles[b];
   if (l < tt[w].nrun) T.run[l] = tt[w].run[l];
@@ -518,6 +519,7 @@ __device__ __forceinline__ int tile_index(const int4* runs, int nrun, int j) {
 // |u| below a cell diagonal), so everything outside the band is decided
 // exactly as the FP64 expression would decide it.
 #define IMDG_SCREEN_BAND 1.0e-4
+#define LIST_MAXWAVE 4  // wavefronts of a block of the list
 
 // The reference's decision for one candidate: r^2 of (image of the partner)
 // - (owner) in FP64 with separate roundings, owner being the atom whose
@@ -614,13 +616,48 @@ typedef __attribute__((address_space(3))) const float3 lds_float3;
 typedef __attribute__((address_space(3))) const char lds_char;
 typedef __attribute__((address_space(3))) const float lds_float;
 
+// Which of four candidates t0 .. t0+3 (of jn, slots jb + t) of one neighbour
+// cell are neighbours of the lane's atom: FP32 screen, FP64 decision inside
+// the band (one branch per four candidates; the band is rarely hit).  The
+// separation is u_j + w with w = o - u_i formed once per cell: two roundings
+// of a few Angstrom, far inside the screening band.  SELF: the atom may be a
+// candidate of itself.
+template <bool SELF>
+__device__ __forceinline__ void screen4(const BuildArgs& a, const RepDev& R,
+                                        const double4* __restrict__ pos,
+                                        const ListLane& L,
+                                        const float3 (&uj)[4], int jb, int jn,
+                                        int t0, float w0, float w1, float w2,
+                                        bool owner, int code, bool (&in)[4]) {
+  bool band[4];
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    int j = jb + t0 + u;
+    bool valid = (t0 + u < jn) && !(SELF && j == L.i);
+    float d0 = uj[u].x + w0;
+    float d1 = uj[u].y + w1;
+    float d2 = uj[u].z + w2;
+    float r2 = d0 * d0 + d1 * d1 + d2 * d2;
+    const bool inside = r2 < L.lo, near = r2 < L.hi;
+    in[u] = valid & inside;
+    band[u] = (valid & near) ^ in[u];  // near but not inside
+  }
+  if (band[0] || band[1] || band[2] || band[3]) {
+    atomicAdd(&a.ctl->exact_pairs,
+              (int)band[0] + (int)band[1] + (int)band[2] + (int)band[3]);
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      if (band[u])
+        in[u] = exact_pair(R, pos, L.i, jb + t0 + u,
+                           wrap_shift(L.cx, code / 9 - 1, R.gdim[0]),
+                           wrap_shift(L.cy, (code / 3) % 3 - 1, R.gdim[1]),
+                           wrap_shift(L.cz, code % 3 - 1, R.gdim[2]), owner);
+  }
+}
+
 // Candidates of one neighbour cell, four at a time (their records in
-// flight together): FP32 screen, FP64 decision inside the band (one branch
-// per four candidates; the band is rarely hit), append.  The separation is
-// u_j + (o - u_i), with o - u_i formed once per cell: two roundings of a
-// few Angstrom, far inside the screening band.  Candidate t of the cell is
-// entry ebase + t.  SELF: the atom's own cell (code 13), where the atom is
-// a candidate of itself.
+// flight together), each appended when it is a neighbour.  Candidate t of
+// the cell is entry ebase + t.  SELF: the atom's own cell (code 13).
 template <bool MIXED, bool TOK, bool W16, bool SELF>
 __device__ __forceinline__ void list_cell(
     const BuildArgs& a, const RepDev& R, const double4* __restrict__ pos,
@@ -642,35 +679,42 @@ __device__ __forceinline__ void list_cell(
         uj[u] = rec_xyz<MIXED>(L.rec, jb + min(t0 + u, jn - 1));
       }
     }
-    bool in[4], band[4];
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      int j = jb + t0 + u;
-      bool valid = (t0 + u < jn) && !(SELF && j == L.i);
-      float d0 = uj[u].x + w0;
-      float d1 = uj[u].y + w1;
-      float d2 = uj[u].z + w2;
-      float r2 = d0 * d0 + d1 * d1 + d2 * d2;
-      const bool inside = r2 < L.lo, near = r2 < L.hi;
-      in[u] = valid & inside;
-      band[u] = (valid & near) ^ in[u];  // near but not inside
-    }
-    if (band[0] || band[1] || band[2] || band[3]) {
-      atomicAdd(&a.ctl->exact_pairs,
-                (int)band[0] + (int)band[1] + (int)band[2] + (int)band[3]);
-#pragma unroll
-      for (int u = 0; u < 4; u++)
-        if (band[u])
-          in[u] = exact_pair(R, pos, L.i, jb + t0 + u,
-                             wrap_shift(L.cx, code / 9 - 1, R.gdim[0]),
-                             wrap_shift(L.cy, (code / 3) % 3 - 1, R.gdim[1]),
-                             wrap_shift(L.cz, code % 3 - 1, R.gdim[2]),
-                             owner);
-    }
+    bool in[4];
+    screen4<SELF>(a, R, pos, L, uj, jb, jn, t0, w0, w1, w2, owner, code, in);
 #pragma unroll
     for (int u = 0; u < 4; u++)
       if (in[u]) list_put<W16>(L, ebase + (uint32_t)(t0 + u));
   }
+}
+
+// The hits among candidates tb0 .. tb0+31 of one neighbour cell, as bits.
+template <bool MIXED, bool TOK>
+__device__ __forceinline__ uint32_t cell_hits(
+    const BuildArgs& a, const RepDev& R, const double4* __restrict__ pos,
+    lds_float3* trec, const ListLane& L, int jb, int jn, int tb, int tb0,
+    float o0, float o1, float o2, int code) {
+  const float w0 = o0 - L.ui.x, w1 = o1 - L.ui.y, w2 = o2 - L.ui.z;
+  lds_char* run = (lds_char*)trec + __umul24((unsigned)tb, 12u);
+  const int te = min(jn, tb0 + 32);
+  uint32_t hits = 0u;
+  for (int t0 = tb0; t0 < te; t0 += 4) {
+    float3 uj[4];
+    lds_float* q = (lds_float*)(run + __umul24((unsigned)t0, 12u));
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      if (TOK)
+        uj[u] = make_float3(q[3 * u], q[3 * u + 1], q[3 * u + 2]);
+      else
+        uj[u] = rec_xyz<MIXED>(L.rec, jb + min(t0 + u, jn - 1));
+    }
+    bool in[4];
+    screen4<true>(a, R, pos, L, uj, jb, jn, t0, w0, w1, w2, code >= 13, code,
+                  in);
+    hits |= ((in[0] ? 1u : 0u) | (in[1] ? 2u : 0u) | (in[2] ? 4u : 0u) |
+             (in[3] ? 8u : 0u))
+            << (t0 - tb0);
+  }
+  return hits;
 }
 
 // The candidate loops of one atom: the 9 neighbour columns (ox, oy) in a
@@ -754,6 +798,104 @@ __device__ __forceinline__ void list_atom(const BuildArgs& a, const RepDev& R,
   }
 }
 
+// The tile's FP32 positions into LDS, all of a thread's loads in flight
+// together: 8 records per pass.
+template <bool MIXED>
+__device__ __forceinline__ void stage_tile(const Tile& tile,
+                                           const void* __restrict__ rec,
+                                           float3* trec) {
+  const int4* truns = tile.run;
+  const int tot = tile.natoms, T = blockDim.x;
+  int k = 0;
+  for (int t0 = threadIdx.x; t0 < tot; t0 += 8 * T) {
+    float3 v[8];
+    int t[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      t[u] = t0 + u * T;
+      if (t[u] < tot) {
+        while (t[u] >= truns[k].z + truns[k].y) k++;
+        v[u] = rec_xyz<MIXED>(rec, truns[k].x + (t[u] - truns[k].z));
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 8; u++)
+      if (t[u] < tot) trec[t[u]] = v[u];
+  }
+}
+
+// 16-bit format of a chunk, by a whole wavefront whose lanes are the chunk's
+// slots (mine: the slot has an atom, in cell cx, cy, cz): the chunk's base
+// slot per code, and whether every neighbour cell run lies within
+// IMDG_K16_SPAN slots of it (a lane without an atom has no runs).  cb: the
+// wavefront's LDS row; also written to the chunk's metadata.  Returns whether
+// the format fits.
+__device__ __forceinline__ bool chunk_format(const BuildArgs& a,
+                                             const RepDev& R, int chunk,
+                                             bool mine, int cx, int cy, int cz,
+                                             int* cb) {
+  const int lane = threadIdx.x & (IMDG_WAVE - 1);
+  const int g0 = R.gdim[0], g1 = R.gdim[1], g2 = R.gdim[2];
+  const bool p0 = R.pbc[0] == 1, p1 = R.pbc[1] == 1, p2 = R.pbc[2] == 1;
+  bool bad = false;
+#pragma unroll
+  for (int k = 0; k < 27; k++) {
+    int n0 = cx + k / 9 - 1, n1 = cy + (k / 3) % 3 - 1, n2 = cz + k % 3 - 1;
+    int sx = n0 < 0 ? -1 : (n0 >= g0 ? 1 : 0);
+    int sy = n1 < 0 ? -1 : (n1 >= g1 ? 1 : 0);
+    int sz = n2 < 0 ? -1 : (n2 >= g2 ? 1 : 0);
+    bool valid = mine & ((sx == 0) | p0) & ((sy == 0) | p1) & ((sz == 0) | p2);
+    int nc = valid ? R.cell_off + ((n0 - sx * g0) * g1 + n1 - sy * g1) * g2 +
+                         n2 - sz * g2
+                   : R.cell_off;
+    int jb = a.cell_beg[nc], jn = valid ? a.cell_num[nc] : 0;
+    int lo = wave_min_i(jn > 0 ? jb : 0x7fffffff);
+    if (lo == 0x7fffffff) lo = 0;
+    bad |= jn > 0 && (jb < lo || jb + jn - lo > IMDG_K16_SPAN);
+    if (lane == 0) cb[k] = lo;
+  }
+  const int wide = __ballot(bad) != 0ull ? 1 : 0;
+  if (lane == 0) {
+    cb[IMDG_CODE_PAD] = chunk * IMDG_CHUNK;
+    cb[IMDG_META_WIDE] = wide;
+  }
+  wave_lds_sync();
+  if (lane <= IMDG_META_WIDE)
+    a.cmeta[(size_t)chunk * IMDG_META + lane] = cb[lane];
+  return __builtin_amdgcn_readfirstlane(wide) == 0;
+}
+
+// The end of a block of the list (unit b): its longest list (list_done
+// reduces the blocks: one atomic word updated by every block would serialise
+// them), with bit 30 when its tile fell back to HBM/L2 loads; then the end
+// of the rebuild by the last block, where the list does that.
+__device__ __forceinline__ void list_block_end(const BuildArgs& a, int b,
+                                               int seen, bool fallback,
+                                               int* wmax) {
+  __shared__ int red[2 * LIST_MAXWAVE], is_last;
+  const int nw = blockDim.x / IMDG_WAVE;
+  for (int o = 32; o > 0; o >>= 1)
+    seen = max(seen, __shfl_xor(seen, o, IMDG_WAVE));
+  if ((threadIdx.x % IMDG_WAVE) == 0) wmax[threadIdx.x / IMDG_WAVE] = seen;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int m = wmax[0];
+    for (int k = 1; k < nw; k++) m = max(m, wmax[k]);
+    a.blkmax[b] = m | (fallback ? IMDG_BLK_FALLBACK : 0);
+  }
+  if (!a.list_ends) return;
+  if (threadIdx.x == 0) {
+    __threadfence();
+    unsigned d = atomicAdd(&a.ctl->done[DC_LIST], 1u);
+    is_last = (d == gridDim.x - 1);
+    if (is_last) a.ctl->done[DC_LIST] = 0;
+  }
+  __syncthreads();
+  if (!is_last) return;
+  __threadfence();
+  list_done(a.end, red);
+}
+
 // Full neighbour list.  For each cell offset o of the 27, the reference
 // evaluates a pair from the atom whose cell has the other in its half
 // stencil (o lexicographically positive: the stencil of
@@ -785,86 +927,28 @@ __global__ void __launch_bounds__(IMDG_BLOCK) k_list(BuildArgs a) {
   const void* rec = build_records(a);
   int kmax = a.kmax, seen = 0;
   if (flagged) {
-    if (a.tiles) {
-      const Tile& T = a.tiles[b];
-      if (threadIdx.x == 0) {
-        tile.nrun = T.nrun;
-        tile.natoms = T.natoms;
-        tile.ok = T.ok;
-      }
-      for (int k = threadIdx.x; k < T.nrun; k += blockDim.x)
-        tile.run[k] = T.run[k];
-    } else if (threadIdx.x < IMDG_WAVE) {
-      // in the rows that will hold the tile's records (tile_cap + 4 of
-      // them: room for the ranges, see launch_build)
-      build_tile(a, R, b, *reinterpret_cast<TileLds*>(list_lds), tile);
+    const Tile& T = a.tiles[b];
+    if (threadIdx.x == 0) {
+      tile.nrun = T.nrun;
+      tile.natoms = T.natoms;
+      tile.ok = T.ok;
     }
+    for (int k = threadIdx.x; k < T.nrun; k += blockDim.x)
+      tile.run[k] = T.run[k];
     for (int k = threadIdx.x; k < 3 * IMDG_NCODES; k += blockDim.x)
       off[k] = (float)((&R.offs[0][0])[k]);
     __syncthreads();
     const int4* truns = tile.run;
     const int nrun = tile.nrun, tok = tile.ok;
-    if (tok) {
-      int tot = tile.natoms;
-      // all of a thread's loads in flight together: 8 records per pass
-      int k = 0;
-      for (int t0 = threadIdx.x; t0 < tot; t0 += 8 * IMDG_BLOCK) {
-        float3 v[8];
-        int t[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-          t[u] = t0 + u * IMDG_BLOCK;
-          if (t[u] < tot) {
-            while (t[u] >= truns[k].z + truns[k].y) k++;
-            v[u] = rec_xyz<MIXED>(rec, truns[k].x + (t[u] - truns[k].z));
-          }
-        }
-#pragma unroll
-        for (int u = 0; u < 8; u++)
-          if (t[u] < tot) trec[t[u]] = v[u];
-      }
-    }
+    if (tok) stage_tile<MIXED>(tile, rec, trec);
     __syncthreads();
     const int i = b * IMDG_BLOCK + threadIdx.x;
     const bool mine = i - R.atom_off < R.natoms;
     int cx = 0, cy = 0, cz = 0;
     if (mine) cell_coords(R, a.acell[i], cx, cy, cz);
-    // 16-bit format: the chunk's (wavefront's) base slot per code, and
-    // whether every neighbour cell run lies within IMDG_K16_SPAN slots of
-    // it (a lane without an atom has no runs)
     bool w16 = false;
-    const int w = threadIdx.x / IMDG_WAVE, lane = threadIdx.x & 63;
-    if (a.list16) {
-      const int g0 = R.gdim[0], g1 = R.gdim[1], g2 = R.gdim[2];
-      const bool p0 = R.pbc[0] == 1, p1 = R.pbc[1] == 1, p2 = R.pbc[2] == 1;
-      const int chunk = i >> 6;
-      bool bad = false;
-#pragma unroll
-      for (int k = 0; k < 27; k++) {
-        int n0 = cx + k / 9 - 1, n1 = cy + (k / 3) % 3 - 1, n2 = cz + k % 3 - 1;
-        int sx = n0 < 0 ? -1 : (n0 >= g0 ? 1 : 0);
-        int sy = n1 < 0 ? -1 : (n1 >= g1 ? 1 : 0);
-        int sz = n2 < 0 ? -1 : (n2 >= g2 ? 1 : 0);
-        bool valid = mine & ((sx == 0) | p0) & ((sy == 0) | p1) & ((sz == 0) | p2);
-        int nc = valid ? R.cell_off + ((n0 - sx * g0) * g1 + n1 - sy * g1) * g2 +
-                             n2 - sz * g2
-                       : R.cell_off;
-        int jb = a.cell_beg[nc], jn = valid ? a.cell_num[nc] : 0;
-        int lo = wave_min_i(jn > 0 ? jb : 0x7fffffff);
-        if (lo == 0x7fffffff) lo = 0;
-        bad |= jn > 0 && (jb < lo || jb + jn - lo > IMDG_K16_SPAN);
-        if (lane == 0) cbase[w][k] = lo;
-      }
-      const int wide = __ballot(bad) != 0ull ? 1 : 0;
-      if (lane == 0) {
-        cbase[w][IMDG_CODE_PAD] = chunk * IMDG_CHUNK;
-        cbase[w][IMDG_META_WIDE] = wide;
-      }
-      wave_lds_sync();
-      if (lane <= IMDG_META_WIDE)
-        a.cmeta[(size_t)chunk * IMDG_META + lane] = cbase[w][lane];
-      w16 = __builtin_amdgcn_readfirstlane(wide) == 0;
-    }
+    const int w = threadIdx.x / IMDG_WAVE;
+    if (a.list16) w16 = chunk_format(a, R, i >> 6, mine, cx, cy, cz, cbase[w]);
     if (mine) {
       ListLane L;
       L.i = i;
@@ -903,30 +987,187 @@ __global__ void __launch_bounds__(IMDG_BLOCK) k_list(BuildArgs a) {
       seen = L.cnt;
     }
   }
-    // block max of the list length (k_list_done reduces the blocks: one
-  // atomic word updated by every block would serialise them)
-  for (int o = 32; o > 0; o >>= 1)
-    seen = max(seen, __shfl_xor(seen, o, IMDG_WAVE));
-  if ((threadIdx.x % IMDG_WAVE) == 0) wmax[threadIdx.x / IMDG_WAVE] = seen;
-  __syncthreads();
-  // with bit 30: the block's tile fell back to HBM/L2 loads
-  if (threadIdx.x == 0) {
-    int m = wmax[0];
-    for (int k = 1; k < IMDG_NWAVE; k++) m = max(m, wmax[k]);
-    a.blkmax[b] = m | (flagged && !tile.ok ? IMDG_BLK_FALLBACK : 0);
+  list_block_end(a, b, seen, flagged && !tile.ok, wmax);
+}
+
+// Entry e at place m of slot i's list.
+template <bool W16>
+__device__ __forceinline__ void list_at(char* lst, int m, uint32_t e) {
+  if (W16)
+    *reinterpret_cast<uint16_t*>(lst + ((size_t)(m >> 2) << 9) +
+                                 2 * (m & 3)) = (uint16_t)e;
+  else
+    *reinterpret_cast<uint32_t*>(lst + ((size_t)(m >> 2) << 10) +
+                                 4 * (m & 3)) = e;
+}
+
+// One atom's list by the LIST_LANES lanes that share it: lane s takes the
+// neighbour cells s, s + LIST_LANES, ...; the hits of each cell stay as bits
+// of a mask (a cell of more than 32 atoms is screened again when its entries
+// are written); a prefix over the lanes gives every cell's place in the
+// list, in the order of the codes: the same list as list_atom's.
+#define LIST_LANES 4
+#define LIST_ROUNDS ((27 + LIST_LANES - 1) / LIST_LANES)
+
+template <bool MIXED, bool TOK, bool W16>
+__device__ __forceinline__ int list_shared(
+    const BuildArgs& a, const RepDev& R, const double4* __restrict__ pos,
+    lds_float3* trec, const int4* truns, int nrun, const float* off,
+    const int* cb, const ListLane& L, int s) {
+  const int g0 = R.gdim[0], g1 = R.gdim[1], g2 = R.gdim[2];
+  const bool p0 = R.pbc[0] == 1, p1 = R.pbc[1] == 1, p2 = R.pbc[2] == 1;
+  // first slot and count of the lane's cell of round q (count 0: none)
+  auto cell_of = [&](int q, int& jb, int& jn) {
+    const int k = s + q * LIST_LANES;
+    int n0 = L.cx + k / 9 - 1, n1 = L.cy + (k / 3) % 3 - 1,
+        n2 = L.cz + k % 3 - 1;
+    const int sx = n0 < 0 ? -1 : (n0 >= g0 ? 1 : 0);
+    const int sy = n1 < 0 ? -1 : (n1 >= g1 ? 1 : 0);
+    const int sz = n2 < 0 ? -1 : (n2 >= g2 ? 1 : 0);
+    const bool valid = (k < 27) & ((sx == 0) | p0) & ((sy == 0) | p1) &
+                       ((sz == 0) | p2);
+    n0 -= sx * g0;
+    n1 -= sy * g1;
+    n2 -= sz * g2;
+    const int nc = valid ? R.cell_off + (n0 * g1 + n1) * g2 + n2 : R.cell_off;
+    jb = a.cell_beg[nc];
+    jn = valid ? a.cell_num[nc] : 0;
+  };
+  int run = 0, jb, jn, jb2, jn2;
+  cell_of(0, jb2, jn2);
+#pragma unroll 1
+  for (int q = 0; q < LIST_ROUNDS; q++) {
+    jb = jb2;
+    jn = jn2;
+    if (q + 1 < LIST_ROUNDS) cell_of(q + 1, jb2, jn2);
+    const int k = min(s + q * LIST_LANES, 26);
+    const int tb = TOK && jn > 0 ? tile_index(truns, nrun, jb) : 0;
+    const float o0 = off[3 * k], o1 = off[3 * k + 1], o2 = off[3 * k + 2];
+    const uint32_t first = cell_hits<MIXED, TOK>(a, R, pos, trec, L, jb, jn,
+                                                 tb, 0, o0, o1, o2, k);
+    int cnt = __popc(first);
+    for (int t0 = 32; t0 < jn; t0 += 32)
+      cnt += __popc(cell_hits<MIXED, TOK>(a, R, pos, trec, L, jb, jn, tb, t0,
+                                          o0, o1, o2, k));
+    // places of the round's cells: exclusive prefix over the atom's lanes
+    int incl = cnt;
+#pragma unroll
+    for (int o = 1; o < LIST_LANES; o <<= 1) {
+      const int y = __shfl_up(incl, o, LIST_LANES);
+      if (s >= o) incl += y;
+    }
+    int m = run + incl - cnt;
+    run += __shfl(incl, LIST_LANES - 1, LIST_LANES);
+    const uint32_t ebase =
+        W16 ? ((uint32_t)k << IMDG_K16_BITS) | (uint32_t)(jb - cb[k])
+            : (uint32_t)jb | ((uint32_t)k << IMDG_IDX_BITS);
+    uint32_t hits = first;
+    for (int t0 = 0; t0 < jn; t0 += 32) {
+      if (t0 > 0)
+        hits = cell_hits<MIXED, TOK>(a, R, pos, trec, L, jb, jn, tb, t0, o0,
+                                     o1, o2, k);
+      while (hits) {
+        const int t = t0 + __builtin_ctz(hits);
+        hits &= hits - 1u;
+        if (m < L.kmax) list_at<W16>(L.lst, m, ebase + (uint32_t)t);
+        m++;
+      }
+    }
   }
-  if (!a.list_ends) return;
-  __shared__ int red[2 * IMDG_NWAVE], is_last;
-  if (threadIdx.x == 0) {
-    __threadfence();
-    unsigned d = atomicAdd(&a.ctl->done[DC_LIST], 1u);
-    is_last = (d == gridDim.x - 1);
-    if (is_last) a.ctl->done[DC_LIST] = 0;
+  if (run <= L.kmax) {
+    const uint32_t pad =
+        W16 ? ((uint32_t)IMDG_CODE_PAD << IMDG_K16_BITS) |
+                  (uint32_t)(L.i - cb[IMDG_CODE_PAD])
+            : (uint32_t)L.i | ((uint32_t)IMDG_CODE_PAD << IMDG_IDX_BITS);
+    const int mend =
+        ((run + IMDG_LIST_PAD - 1) / IMDG_LIST_PAD) * IMDG_LIST_PAD;
+    for (int m = run + s; m < mend; m += LIST_LANES)
+      list_at<W16>(L.lst, m, pad);
   }
-  __syncthreads();
-  if (!is_last) return;
-  __threadfence();
-  list_done(a.end, red);
+  return run;
+}
+
+// The list of systems whose blocks do not fill the chip (and of batches of
+// replicas, of which few rebuild in one step): a block per 64-slot chunk,
+// LIST_LANES lanes per atom.  k_list lasts as long as its longest lane's 370
+// candidates in a row, which bounds it while the chip is not full: 864 atoms
+// 60 us, here 32; of 64 replicas the few that rebuild in a step 78 us, here
+// 44 (a step of theirs 242 us, 201; LJ crystal of 4,000 atoms in FP64 20.4,
+// 17.2).  Eight lanes are no faster for those and slower from 100,000 atoms.
+// On a full chip the lanes' entry stores, 2 B each instead of 8, and the
+// drain of the masks cost more than the screens they save.
+template <bool MIXED>
+__global__ void __launch_bounds__(IMDG_CHUNK* LIST_LANES)
+    k_list_shared(BuildArgs a) {
+  extern __shared__ __align__(16) unsigned char list_lds[];
+  float3* trec = reinterpret_cast<float3*>(list_lds);
+  __shared__ Tile tile;
+  __shared__ float off[3 * IMDG_NCODES];
+  __shared__ int cbase[IMDG_META], wmax[LIST_LANES];
+  if (!a.ctl->any_rebuild || a.ctl->frozen || a.ctl->cell_over) return;
+  const int chunk = blockIdx.x;
+  const int r = a.blk_rep[chunk / (IMDG_BLOCK / IMDG_CHUNK)];
+  const RepDev& R = a.rep[r];
+  const bool flagged = a.rst[r].need_rebuild != 0;
+  const double4* pos = a.pos[a.ctl->pos_cur ^ 1];
+  const void* rec = build_records(a);
+  const int w = threadIdx.x / IMDG_WAVE, lane = threadIdx.x & (IMDG_WAVE - 1);
+  int seen = 0;
+  if (flagged) {
+    const int s0 = chunk * IMDG_CHUNK;
+    for (int k = threadIdx.x; k < 3 * IMDG_NCODES; k += blockDim.x)
+      off[k] = (float)((&R.offs[0][0])[k]);
+    if (w == 0)
+      build_tile(a, R, s0, IMDG_CHUNK, *reinterpret_cast<TileLds*>(list_lds),
+                 tile);
+    if (w == 1 && a.list16) {
+      const bool mine = s0 + lane - R.atom_off < R.natoms;
+      int cx = 0, cy = 0, cz = 0;
+      if (mine) cell_coords(R, a.acell[s0 + lane], cx, cy, cz);
+      (void)chunk_format(a, R, chunk, mine, cx, cy, cz, cbase);
+    }
+    __syncthreads();
+    const bool tok = tile.ok != 0;
+    if (tok) stage_tile<MIXED>(tile, rec, trec);
+    __syncthreads();
+    const bool w16 = a.list16 && cbase[IMDG_META_WIDE] == 0;
+    const int i = s0 + threadIdx.x / LIST_LANES, s = threadIdx.x % LIST_LANES;
+    if (i - R.atom_off < R.natoms) {  // all lanes of an atom
+      ListLane L;
+      L.i = i;
+      L.rec = rec;
+      L.ui = rec_xyz<MIXED>(rec, i);
+      const float cs = (float)R.cellsz;
+      L.lo = cs * (float)(1.0 - IMDG_SCREEN_BAND);
+      L.hi = cs * (float)(1.0 + IMDG_SCREEN_BAND);
+      L.cnt = 0;
+      L.kmax = a.kmax;
+      L.g0 = L.g1 = L.g2 = L.g3 = 0u;
+      cell_coords(R, a.acell[i], L.cx, L.cy, L.cz);
+      lds_float3* tr = (lds_float3*)trec;
+      if (w16) {
+        L.lst = const_cast<char*>(list16_of(a.nbr, i, a.kmax));
+        seen = tok ? list_shared<MIXED, true, true>(a, R, pos, tr, tile.run,
+                                                    tile.nrun, off, cbase, L,
+                                                    s)
+                   : list_shared<MIXED, false, true>(a, R, pos, tr, tile.run,
+                                                     tile.nrun, off, cbase, L,
+                                                     s);
+      } else {
+        L.lst = reinterpret_cast<char*>(
+            a.nbr + (((size_t)(i >> 6) * (a.kmax >> 2)) * IMDG_WAVE +
+                     (i & 63)) * IMDG_GROUP);
+        seen = tok ? list_shared<MIXED, true, false>(a, R, pos, tr, tile.run,
+                                                     tile.nrun, off, cbase, L,
+                                                     s)
+                   : list_shared<MIXED, false, false>(a, R, pos, tr, tile.run,
+                                                      tile.nrun, off, cbase, L,
+                                                      s);
+      }
+      if (s == 0) a.nnb[i] = min(seen, a.kmax);
+    }
+  }
+  list_block_end(a, chunk, seen, flagged && !tile.ok, wmax);
 }
 
 // The end of a rebuild as a launch of its own (one block), where no step
@@ -1013,7 +1254,15 @@ void launch_list(const BuildArgs& b, bool done, hipStream_t st) {
     hipLaunchKernelGGL(k_tile, dim3((b.nblk + 3) / 4), dim3(256), 0, st, b);
   const size_t tile_lds = std::max((size_t)(b.tile_cap + 4) * sizeof(float3),
                                    sizeof(TileLds));
-  if (b.mixed)
+  const dim3 sb(IMDG_CHUNK * LIST_LANES);
+  const int nchunk = b.nslots / IMDG_CHUNK;
+  if (b.list_shared && b.mixed)
+    hipLaunchKernelGGL((k_list_shared<true>), dim3(nchunk), sb, tile_lds, st,
+                       b);
+  else if (b.list_shared)
+    hipLaunchKernelGGL((k_list_shared<false>), dim3(nchunk), sb, tile_lds, st,
+                       b);
+  else if (b.mixed)
     hipLaunchKernelGGL((k_list<true>), dim3(b.nblk), dim3(IMDG_BLOCK),
                        tile_lds, st, b);
   else

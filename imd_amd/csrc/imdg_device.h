@@ -263,7 +263,7 @@ __device__ inline void list_done(const ListEnd& e, int* red) {
   int m = 0, fb = 0;
   if (!over)
     for (int b = threadIdx.x; b < e.nblk; b += blockDim.x)
-      if (e.rst[e.blk_rep[b]].need_rebuild) {
+      if (e.rst[e.blk_rep[b >> e.blk_shift]].need_rebuild) {
         const int v = e.blkmax[b];
         m = max(m, v & ~IMDG_BLK_FALLBACK);
         fb += v & IMDG_BLK_FALLBACK ? 1 : 0;

@@ -107,10 +107,6 @@
 // (about 1 us per 1024 cells and rebuild) and the scan's launch is left out
 // (1.7 us per step, one rebuild in 15 to 20 steps).
 #define IMDG_SCAN_FOLD 8192
-// Up to this many blocks the list's blocks build their own tiles (about 5 us
-// of latency in the list's launch); a larger system has a launch for them
-// (2,048,000 atoms, 16,000 blocks: list 694 us instead of 792).
-#define IMDG_TILE_FOLD 1024
 // Up to this many slots and cells (one replica) a step begins with a single
 // block that ends the step before and sorts, instead of three launches.
 #define IMDG_HEAD_SLOTS 7168
@@ -118,6 +114,12 @@
 // Pair-only systems of up to this many blocks end a rebuild in the list's
 // last block (a release fence in each); larger ones in a launch of its own.
 #define IMDG_LIST_ENDS 128
+// Up to this many blocks in the largest replica the list is built with four
+// lanes per atom, a block per chunk that builds its own tile: 256,000 atoms
+// (2,000 blocks) 73.9 us per step, 74.9 with one lane and the tiles from a
+// launch of their own; 500,000 atoms 116.3 and 115.0, 2,048,000 atoms 502 and
+// 484.
+#define IMDG_SHARE_BLOCKS 2560
 #define IMDG_BUCKET_MIN 32   // smallest bucket (atoms of a cell)
 
 // Flag bit of a block's list-length maximum (blkmax): its tile exceeded the
@@ -188,8 +190,10 @@ struct ListEnd {
   Ctl* ctl;
   RepState* rst;
   const int* blk_rep;
-  const int* blkmax;      // longest list of every block (k_list)
-  int nblk, nrep, kmax;
+  const int* blkmax;      // longest list of every block of the list
+  int nblk;               // those blocks; blk_shift: log2 of how many of them
+  int blk_shift;          // an IMDG_BLOCK-slot block (blk_rep) has
+  int nrep, kmax;
 };
 
 // Table of one interpolated function set on the device.
@@ -361,6 +365,7 @@ struct BuildArgs {
   void* rec_b;            // pair_only: the records of odd steps
   int pair_only;
   int list_ends;          // the last block of k_list ends the rebuild
+  int list_shared;        // several lanes per atom build its list
   int mixed;
   int* acell;             // cell of slot (new order)
   signed char* atype;     // type of slot (new order)
@@ -378,8 +383,7 @@ struct BuildArgs {
   int* nnb;
   int* blkmax;            // longest list of every block (k_list)
   ListEnd end;
-  Tile* tiles;            // tiles built by a launch of their own (NULL: by
-                          // the list's blocks)
+  Tile* tiles;            // without list_shared: the blocks' tiles
   int tile_cap;           // records a tile may hold (<= IMDG_TILE_CAP)
   int* cmeta;             // chunk metadata of the 16-bit list format
   int list16;             // build the 16-bit format where a chunk allows

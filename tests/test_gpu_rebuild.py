@@ -165,3 +165,36 @@ def test_pair_only_record_turns(nrep, cells, precision):
                         nbl_margin=0.15) as gpu:
         gpu.calc_forces()
         _check_static(gpu, orc, *TOL[precision], has_eam=False)
+
+
+def test_list_of_shared_lanes(monkeypatch):
+    """Several lanes per atom build the same list as one: cells of more than
+    32 atoms (screened again when they are written), tiles that do not fit,
+    open faces, in both entry formats; the pair sets are the oracle's and the
+    per-atom lists are in the same order (densities bit for bit)."""
+    eam = eam_tables()
+    dense = W.eam_crystal(n_cells=7, temp_k=0.0, seed=3, displace=0.08)
+    slab = W.fcc_system((8, 6, 5), 3.615, eam.masses, 0.0, 4,
+                        pbc=(1, 0, 0), vacuum_z=12.0, displace=0.05)
+    # a replica beyond the line: the batch takes one lane per atom
+    large = W.eam_crystal(n_cells=44, temp_k=0.0, seed=5, displace=0.02)
+    for s, margin in ((dense, 3.0), (dense, 0.4), (slab, 0.4)):
+        orc = oracle_eam(s, eam, nbl_margin=margin, timestep=W.FS)
+        orc.calc_forces()
+        want = canon_pairs_oracle(orc.pairs())
+        for list16 in ("1", "0"):
+            for limit in ("1536", "64"):
+                monkeypatch.setenv("IMDG_LIST16", list16)
+                monkeypatch.setenv("IMDG_TILE_LIMIT", limit)
+                got = []
+                for systems in ([s], [s, large]):
+                    with G.eam_context(eam, systems, precision=G.MIXED,
+                                       nbl_margin=margin) as gpu:
+                        gpu.set_tuning(1, 512, 1, 512)
+                        gpu.calc_forces()
+                        info = gpu.info()
+                        got.append(gpu.atoms()["rho"][:s.n])
+                        if len(systems) == 1:
+                            assert canon_pairs_gpu(gpu.pairs()) == want
+                        assert (info["tiles_fallback"] > 0) or limit != "64"
+                assert np.array_equal(got[0], got[1])
