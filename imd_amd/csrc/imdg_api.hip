@@ -117,6 +117,8 @@ struct imdg_ctx {
   int kmax = 0;
   // device memory
   std::vector<DevBuf> bufs;
+  char* arena = nullptr;      // current block of the small arrays
+  size_t arena_used = 0;
   RepDev* d_rep = nullptr;
   RepState* d_rst = nullptr;
   Ctl* d_ctl = nullptr;
@@ -256,6 +258,24 @@ int dalloc(imdg_ctx* c, void** p, size_t bytes) {
   return IMDG_OK;
 }
 
+// Device memory that lives as long as the atoms: small arrays share blocks
+// of ARENA bytes (a hipMalloc is some 10 us of a small system's set-up, which
+// has 40 of them).  Not for dfree.
+int dalloc_fixed(imdg_ctx* c, void** p, size_t bytes) {
+  const size_t ARENA = 4u << 20, ALIGN = 256;
+  bytes = (std::max<size_t>(bytes, 16) + ALIGN - 1) / ALIGN * ALIGN;
+  if (bytes > ARENA / 4) return dalloc(c, p, bytes);
+  if (!c->arena || c->arena_used + bytes > ARENA) {
+    c->arena = nullptr;
+    int rc = dalloc(c, (void**)&c->arena, ARENA);
+    if (rc) return rc;
+    c->arena_used = 0;
+  }
+  *p = c->arena + c->arena_used;
+  c->arena_used += bytes;
+  return IMDG_OK;
+}
+
 void dfree(imdg_ctx* c, void* p) {
   for (auto it = c->bufs.begin(); it != c->bufs.end(); ++it)
     if (it->p == p) {
@@ -268,6 +288,7 @@ void dfree(imdg_ctx* c, void* p) {
 void free_all(imdg_ctx* c) {
   for (auto& b : c->bufs) hipFree(b.p);
   c->bufs.clear();
+  c->arena = nullptr;
   c->d_nbr = nullptr;
   c->nbr_bytes = 0;
   c->d_stress = nullptr;
@@ -691,20 +712,20 @@ int upload_tables(imdg_ctx* c) {
         }
       }
     }
-    int rc64 = dalloc(c, &c->d_knots64, k64.size() * sizeof(double2));
+    int rc64 = dalloc_fixed(c, &c->d_knots64, k64.size() * sizeof(double2));
     if (rc64) return rc64;
     if (!k64.empty())
       HIPCHK(c, hipMemcpy(c->d_knots64, k64.data(),
                           k64.size() * sizeof(double2), hipMemcpyHostToDevice));
-    rc64 = dalloc(c, &c->d_tab64, sizeof t64);
+    rc64 = dalloc_fixed(c, &c->d_tab64, sizeof t64);
     if (rc64) return rc64;
     HIPCHK(c, hipMemcpy(c->d_tab64, t64, sizeof t64, hipMemcpyHostToDevice));
   }
-  int rc = dalloc(c, &c->d_knots, kn.size() * sizeof(R2));
+  int rc = dalloc_fixed(c, &c->d_knots, kn.size() * sizeof(R2));
   if (rc) return rc;
   HIPCHK(c, hipMemcpy(c->d_knots, kn.data(), kn.size() * sizeof(R2),
                       hipMemcpyHostToDevice));
-  rc = dalloc(c, &c->d_tabs, sizeof td);
+  rc = dalloc_fixed(c, &c->d_tabs, sizeof td);
   if (rc) return rc;
   HIPCHK(c, hipMemcpy(c->d_tabs, td, sizeof td, hipMemcpyHostToDevice));
   return IMDG_OK;
@@ -1730,7 +1751,7 @@ int imdg_set_atoms(imdg_ctx* c, int nrep, const imdg_replica* reps,
 
   int rc;
 #define ALLOC(ptr, bytes)                                        \
-  if ((rc = dalloc(c, (void**)&(ptr), (bytes)))) return rc
+  if ((rc = dalloc_fixed(c, (void**)&(ptr), (bytes)))) return rc
   size_t ns = c->nslots, rs = c->mixed ? sizeof(float) : sizeof(double);
   ALLOC(c->d_rep, sizeof(RepDev) * nrep);
   ALLOC(c->d_rst, sizeof(RepState) * nrep);
@@ -1751,7 +1772,9 @@ int imdg_set_atoms(imdg_ctx* c, int nrep, const imdg_replica* reps,
     if (R.nblk > IMDG_SHARE_BLOCKS) c->list_shared = false;
   c->d_tiles = nullptr;
   if (!c->list_shared) ALLOC(c->d_tiles, sizeof(Tile) * c->nblk);
-  ALLOC(c->d_bucket, sizeof(int) * c->bucket_cap * (size_t)c->ncells);
+  if ((rc = dalloc(c, (void**)&c->d_bucket,
+                   sizeof(int) * c->bucket_cap * (size_t)c->ncells)))
+    return rc;
   ALLOC(c->d_cell_cnt, sizeof(int) * c->ncells);
   ALLOC(c->d_cell_beg, sizeof(int) * c->ncells);
   ALLOC(c->d_cell_num, sizeof(int) * c->ncells);
