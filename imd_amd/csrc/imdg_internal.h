@@ -314,7 +314,10 @@ struct StepArgs {
                           // as three packed floats for the density loop;
                           // -1 if none
   int pairn;              // with frho: the pair halves of the jointn
-                          // records, 16 B apart (p len + k)
+                          // records, 16 B apart (p len + k), column
+                          // p = it * pairn_row + jt
+  int pairn_row;          // the number of types; 1: two types, phi_01 =
+                          // phi_10, columns 00, 01 and 11 only
   int cubic;              // tables hold cubic segments, two knots each
                           // (4-point or spline interpolation)
   int eeam;               // EEAM: second density P = sum rho^2, energy E(P)

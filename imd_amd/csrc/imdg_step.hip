@@ -1802,13 +1802,14 @@ __global__ void __launch_bounds__((ForceThreads<R, MODE>::value))
           const float2* FR =
               LT ? reinterpret_cast<const float2*>(K + (a.frho - klo))
                  : nullptr;
+          const int prow = LT ? a.pairn_row : nt;
           const TArg ta = targ(tp);
           if (a.type_bit)
             walk_either<L, NTL>(w16, a.nbr, i, a.kmax, gs, cs.nn,
                            [&](uint4 e4, auto pf, uint4& slot) {
                              force_group_sgn<true, LT>(
                                  e4, pf, slot, rec, atype, off, olo, ui,
-                                 0.5f * dFi, S, FR, it, it * nt, plen, ta,
+                                 0.5f * dFi, S, FR, it, it * prow, plen, ta,
                                  fx, fy, fz, ep, vir, vlo, r2min);
                            });
           else
@@ -1816,7 +1817,7 @@ __global__ void __launch_bounds__((ForceThreads<R, MODE>::value))
                            [&](uint4 e4, auto pf, uint4& slot) {
                              force_group_sgn<false, LT>(
                                  e4, pf, slot, rec, atype, off, olo, ui,
-                                 0.5f * dFi, S, FR, it, it * nt, plen, ta,
+                                 0.5f * dFi, S, FR, it, it * prow, plen, ta,
                                  fx, fy, fz, ep, vir, vlo, r2min);
                            });
           is_short |= (r2min < pb);

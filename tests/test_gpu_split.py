@@ -3,7 +3,10 @@ systems of a few chunks (four units a chunk with four lanes), at sizes where
 four or two units a chunk are chosen and where the chunks fill the chip,
 with the tables staged or read from L2, against the oracle at the bars of the launch shapes; one wavefront's chunk
 that is not full; replicas, whose partial sums are per unit, over several
-steps and lanes."""
+steps and lanes; the pair columns of two species, equal across the diagonal
+(three are stored) or not (all four)."""
+import copy
+
 import numpy as np
 import pytest
 
@@ -111,3 +114,30 @@ def test_replica_units(lanes):
         scale = np.abs(t1[:, 0, 1:6]).max(axis=0) + 1e-300
         scale[2] = np.abs(t1[:, 0, 1]).max()  # the virial's terms cancel
         assert np.all(np.abs(th[:, r, 1:6] - t1[:, 0, 1:6]) <= 1e-12 * scale)
+
+
+@pytest.mark.parametrize("last_knots_only", [True, False])
+def test_unequal_cross_columns_keep_four(last_knots_only, monkeypatch):
+    """phi_10 not phi_01, everywhere or in the last stored rows alone: no
+    column is shared, and the forces are the same bits as from the records of
+    all four columns (IMDG_RHO_BY_TYPE=0).  Equal columns are compared so in
+    test_gpu_branches.py."""
+    eam = copy.deepcopy(eam_tables(nspecies=2, rc=5.5))  # cached tables
+    v = np.array(eam.pair.values[2])
+    if last_knots_only:
+        v[-40:] += 1e-4     # the outermost 0.23 A^2 of r^2
+    else:
+        v *= 1.05
+    eam.pair.values[2] = v
+    s = W.fcc_system((7, 7, 5), 3.615, eam.masses, W.kT(700.0), 48,
+                     type_fractions=(0.7, 0.3), displace=0.04)
+    res = []
+    for by_type in ("1", "0"):
+        monkeypatch.setenv("IMDG_RHO_BY_TYPE", by_type)
+        ctx = G.eam_context(eam, [s], precision=G.MIXED)
+        monkeypatch.delenv("IMDG_RHO_BY_TYPE")
+        with ctx:
+            ctx.calc_forces()
+            res.append(ctx.atoms())
+    for k in ("f", "epot", "rho", "df"):
+        assert np.array_equal(res[0][k], res[1][k]), k
