@@ -820,8 +820,20 @@ int plan_steps(imdg_ctx* c) {
   // per CU, in a block of one wavefront (864 atoms 19.5 us per step, 21.3 in
   // full blocks).
   const bool tiny = no_lds && nt1 && c->nchunk * 16 <= c->ncu;
+  // From 24 chunks per CU on (393,000 atoms) the FP64 one-grid loops are
+  // faster with two lanes each, the density loop in blocks of 512 threads.
+  // At 2,048,000 atoms the density loop then issues 17 % fewer VALU
+  // instructions and misses the L2 42 % less often with half the wavefronts
+  // (357 -> 337 us); the force loop misses the L1 20 % less often (447 ->
+  // 425 us).  Step, four lanes and 1024 threads with one lane | two lanes
+  // and 512 threads with two: 256,000 atoms 112.5 | 112.7 us, 500,000 198 |
+  // 195, 864,000 383 | 367, 1,372,000 613 | 565, 2,048,000 854 | 804.
+  const bool large64 =
+      !fp32 && he && mode == 1 && !no_lds && c->nchunk >= 24L * c->ncu;
   if (c->thr_den <= 0) {
-    c->thr_den = tiny ? IMDG_WAVE : IMDG_STEP_THREADS;
+    c->thr_den = tiny                            ? IMDG_WAVE
+                 : large64 && c->lpa_den <= 0 ? 512
+                                              : IMDG_STEP_THREADS;
     c->thr_auto_den = true;
   }
   if (c->thr_frc <= 0) {
@@ -836,18 +848,18 @@ int plan_steps(imdg_ctx* c) {
   // lists need less padding (256,000 atoms 86.7 us, 88.0 with four; 864,000
   // atoms 215, 242).  The FP64 one-grid force loop on staged tables has two
   // wavefronts per SIMD and no latency to hide behind more lanes: one is
-  // fastest (256,000 atoms 124 us, 133 with four).  The other loops keep
-  // four (LJ crystal of 4,000 atoms in FP64: 39.3 us, 47.0 with one).
+  // fastest up to the sizes of large64 (256,000 atoms 124 us, 133 with
+  // four).  The other loops keep four (LJ crystal of 4,000 atoms in FP64: 39.3 us, 47.0 with one).
   const bool spread = (long)c->nchunk * 4 <= (long)c->ncu * IMDG_STEP_WAVES;
   if (c->lpa_den <= 0) {
     const bool onegrid = c->knots_dpoly >= 0 || c->knots_drho >= 0;
-    c->lpa_den = fp32 && onegrid && !spread ? 2 : 4;
+    c->lpa_den = (fp32 && onegrid && !spread) || large64 ? 2 : 4;
     c->lpa_auto_den = true;
   }
   if (c->lpa_frc <= 0) {
     c->lpa_frc = mode != 1 ? 4
                  : fp32    ? (spread ? 4 : 2)
-                           : (no_lds ? 4 : 1);
+                           : (no_lds ? 4 : large64 ? 2 : 1);
     c->lpa_auto_frc = true;
   }
   // density: the rho knots (the several-species segment records stay in

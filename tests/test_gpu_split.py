@@ -4,7 +4,8 @@ four or two units a chunk are chosen and where the chunks fill the chip,
 with the tables staged or read from L2, against the oracle at the bars of the launch shapes; one wavefront's chunk
 that is not full; replicas, whose partial sums are per unit, over several
 steps and lanes; the pair columns of two species, equal across the diagonal
-(three are stored) or not (all four)."""
+(three are stored) or not (all four); the FP64 default shapes on both sides
+of their line of size."""
 import copy
 
 import numpy as np
@@ -141,3 +142,27 @@ def test_unequal_cross_columns_keep_four(last_knots_only, monkeypatch):
             res.append(ctx.atoms())
     for k in ("f", "epot", "rho", "df"):
         assert np.array_equal(res[0][k], res[1][k]), k
+
+
+@pytest.mark.parametrize("cells", [(46, 46, 46), (47, 46, 47)])
+def test_large_fp64_default_shapes(cells):
+    """389,344 atoms (below 24 chunks per CU on 256 CUs) and 406,456 (above):
+    the default shape's densities and forces against the shape of the other
+    side.  Both sum the same ~60 terms per atom, each below 60 in magnitude,
+    in another order: 60 x 60 x 2^-53 x 2 < 1e-12."""
+    eam = eam_tables()
+    s = W.fcc_system(cells, 3.615, eam.masses, W.kT(600.0), 49, displace=0.03)
+    assert (s.x.shape[0] >= 24 * 256 * 64) == (cells[0] == 47)
+    below, above = (4, 1024, 1, 512), (2, 512, 2, 512)
+    res = []
+    with G.eam_context(eam, [s], precision=G.FP64) as gpu:
+        gpu.calc_forces()
+        t = gpu.tuning()
+        assert (t["density_lanes"], t["density_threads"], t["force_lanes"],
+                t["force_threads"]) == (above if cells[0] == 47 else below)
+        res.append(gpu.atoms())
+        gpu.set_tuning(*(below if cells[0] == 47 else above))
+        gpu.calc_forces()
+        res.append(gpu.atoms())
+    for k in ("f", "epot", "rho"):
+        assert np.abs(res[0][k] - res[1][k]).max() <= 1e-12, k
