@@ -989,11 +989,12 @@ __device__ __forceinline__ void density_group(
     p[u] = K[kk[u]];
     q[u] = K[kk[u] + 1];
   }
+  R body = 0;  // summed apart from the running sum: exacter, as add4
 #pragma unroll
   for (int u = 0; u < 4; u++) {
     bool in = r2[u] < ce[u];
     R v = tab_val<CUB, R>(p[u], q[u], chi[u]);
-    rho = fma(in ? (R)1 : (R)0, v, rho);
+    body = fma(in ? (R)1 : (R)0, v, body);
     // EEAM: P += rho^2 (src/imd_forces_nbl.c:591-593)
     if (EE) pee = fma(in ? v : (R)0, v, pee);
     if (NT1)
@@ -1001,6 +1002,21 @@ __device__ __forceinline__ void density_group(
     else
       is_short |= (in && r2[u] < cb[u]);
   }
+  rho += body;
+}
+
+// The four terms of a body into two running sums, two terms summed apart
+// into each: as many additions as term by term, half of them rounded at the
+// size of a term and half at half the slot's sum.  Two lanes per slot, whose
+// running sums are twice as long as those of four, lose no accuracy so
+// (256,000 atoms, relative RMS errors of rho and of the energy per atom:
+// four lanes term by term 7.22e-8 and 8.96e-8, two lanes 8.19e-8 and
+// 1.14e-7, two lanes with add4 7.02e-8 and 8.52e-8), and the loops take the
+// same time.  The force sums of the one-species loop are summed body by
+// body for the same reason.
+__device__ __forceinline__ void add4(const float* v, float& s0, float& s1) {
+  s0 += v[0] + v[1];
+  s1 += v[2] + v[3];
 }
 
 // FP32 single-species variant of density_group on the rho segment
@@ -1016,7 +1032,7 @@ template <typename PF>
 __device__ __forceinline__ void density_group_poly(
     uint4 e4, PF pf, uint4& slot, const float4* __restrict__ rec,
     const float4* off, const float4* olo, const float4& ui,
-    const float* __restrict__ DQ, const TArg& ta, float& rho,
+    const float* __restrict__ DQ, const TArg& ta, float& rho, float& rho2,
     float& r2min) {
   uint32_t en[4] = {e4.x, e4.y, e4.z, e4.w};
   float ux[4], uy[4], uz[4];
@@ -1053,11 +1069,13 @@ __device__ __forceinline__ void density_group_poly(
     q1[u] = DQ[3 * kk[u] + 1];
     q2[u] = DQ[3 * kk[u] + 2];
   }
+  float v[4];
 #pragma unroll
   for (int u = 0; u < 4; u++) {
-    rho += fmaf(chi[u], fmaf(chi[u], q2[u], q1[u]), q0[u]);
+    v[u] = fmaf(chi[u], fmaf(chi[u], q2[u], q1[u]), q0[u]);
     r2min = fminf(r2min, r2[u]);
   }
+  add4(v, rho, rho2);
 }
 
 // Four neighbours of the force loop (same phases as density_group).
@@ -1285,7 +1303,7 @@ __device__ __forceinline__ void force_group_sgf(
     uint4 e4, PF pf, uint4& slot, const float4* __restrict__ rec,
     const float4* off, const float4* olo, const float4& ui, float hFi,
     const float4* __restrict__ Q, const float2* __restrict__ Rr,
-    const TArg& ta, float& sx, float& sy, float& sz, float& ep, float& svir,
+    const TArg& ta, float& sx, float& sy, float& sz, float& ep, float& ep2, float& svir,
     float& svlo) {
   uint32_t en[4] = {e4.x, e4.y, e4.z, e4.w};
   float4 uj[4], o[4], ol[4];
@@ -1313,20 +1331,25 @@ __device__ __forceinline__ void force_group_sgf(
     q[u] = Q[kk[u]];
     rr[u] = Rr[kk[u]];
   }
+  float v[4], bx, by, bz, bv;
 #pragma unroll
   for (int u = 0; u < 4; u++) {
     float gp = fmaf(chi[u] + chi[u], q[u].z, q[u].y);
     float gr = fmaf(chi[u], rr[u].y, rr[u].x);
-    float vp = fmaf(chi[u], fmaf(chi[u], q[u].z, q[u].y), q[u].x);
+    v[u] = fmaf(chi[u], fmaf(chi[u], q[u].z, q[u].y), q[u].x);
     float h = fmaf(0.5f, uj[u].w, hFi);
     float g = fmaf(h, gr, gp);
-    ep += vp;
-    sx = fmaf(dx[u], g, sx);
-    sy = fmaf(dy[u], g, sy);
-    sz = fmaf(dz[u], g, sz);
-    svir = fmaf(r2[u], g, svir);
+    bx = u ? fmaf(dx[u], g, bx) : dx[u] * g;
+    by = u ? fmaf(dy[u], g, by) : dy[u] * g;
+    bz = u ? fmaf(dz[u], g, bz) : dz[u] * g;
+    bv = u ? fmaf(r2[u], g, bv) : r2[u] * g;
     svlo = fmaf(r2[u], q[u].w, svlo);
   }
+  add4(v, ep, ep2);
+  sx += bx;
+  sy += by;
+  sz += bz;
+  svir += bv;
 }
 
 // Several species on one grid (FP32): the record pair S[2 (p len + k)] of
@@ -1412,7 +1435,7 @@ __device__ __forceinline__ void density_group_polyn(
     uint4 e4, PF pf, uint4& slot, const float4* __restrict__ rec,
     const float4* off, const float4* olo, const float4& ui,
     const float4* __restrict__ DQ, int pbase, int len, const TArg& ta,
-    float& rho, float& r2min) {
+    float& rho, float& rho2, float& r2min) {
   uint32_t en[4] = {e4.x, e4.y, e4.z, e4.w};
   float4 uj[4], o[4], ol[4];
 #pragma unroll
@@ -1435,11 +1458,13 @@ __device__ __forceinline__ void density_group_polyn(
   float4 q[4];
 #pragma unroll
   for (int u = 0; u < 4; u++) q[u] = DQ[kk[u]];
+  float v[4];
 #pragma unroll
   for (int u = 0; u < 4; u++) {
-    rho += fmaf(chi[u], fmaf(chi[u], q[u].z, q[u].y), q[u].x);
+    v[u] = fmaf(chi[u], fmaf(chi[u], q[u].z, q[u].y), q[u].x);
     r2min = fminf(r2min, r2[u]);
   }
+  add4(v, rho, rho2);
 }
 
 // Several species on one grid, rho column it*nt + jt the same for every
@@ -1450,7 +1475,7 @@ template <typename PF>
 __device__ __forceinline__ void density_group_polyl(
     uint4 e4, PF pf, uint4& slot, const float4* __restrict__ rec,
     const float4* off, const float4* olo, const float4& ui, const float* DR,
-    int len, const TArg& ta, float& rho, float& r2min) {
+    int len, const TArg& ta, float& rho, float& rho2, float& r2min) {
   uint32_t en[4] = {e4.x, e4.y, e4.z, e4.w};
   float4 uj[4], o[4], ol[4];
 #pragma unroll
@@ -1477,11 +1502,13 @@ __device__ __forceinline__ void density_group_polyl(
     q1[u] = DR[kk[u] + 1];
     q2[u] = DR[kk[u] + 2];
   }
+  float v[4];
 #pragma unroll
   for (int u = 0; u < 4; u++) {
-    rho += fmaf(chi[u], fmaf(chi[u], q2[u], q1[u]), q0[u]);
+    v[u] = fmaf(chi[u], fmaf(chi[u], q2[u], q1[u]), q0[u]);
     r2min = fminf(r2min, r2[u]);
   }
+  add4(v, rho, rho2);
 }
 
 // ---------------------------------------------------------------------------
@@ -1548,7 +1575,7 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS)
     for (int p = un.p0; p < un.p1; p++) {
       const NextSlot<R> cs = next;
       const int i = cs.i;
-      R rho = (R)0, pee = (R)0;
+      R rho = (R)0, rho2 = (R)0, pee = (R)0;  // rho2: see add4
       if (p + 1 < un.p1) next.load(rec, a.nnb, i + IMDG_WAVE / L, cr);
       if (cs.mine) {
         const R4 ui = cs.u;
@@ -1562,7 +1589,7 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS)
           walk_either<L, NTL>(w16, a.nbr, i, a.kmax, gs, cs.nn,
                          [&](uint4 e4, auto pf, uint4& slot) {
                            density_group_poly(e4, pf, slot, rec, off, olo,
-                                              ui, DQ, ta, rho, r2min);
+                                              ui, DQ, ta, rho, rho2, r2min);
                          });
         } else {
           auto generic = [&]() {
@@ -1583,7 +1610,7 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS)
                              [&](uint4 e4, auto pf, uint4& slot) {
                                density_group_polyl(e4, pf, slot, rec, off,
                                                    olo, ui, DR, len0, ta, rho,
-                                                   r2min);
+                                                   rho2, r2min);
                              });
               is_short |= (r2min < b0);
             } else {
@@ -1599,7 +1626,7 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS)
                              [&](uint4 e4, auto pf, uint4& slot) {
                                density_group_polyn(e4, pf, slot, rec, off,
                                                    olo, ui, DQ, it * nt, len0,
-                                                   ta, rho, r2min);
+                                                   ta, rho, rho2, r2min);
                              });
               is_short |= (r2min < b0);
             } else {
@@ -1611,7 +1638,7 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS)
         }
         if (NT1) is_short |= (r2min < b0);
       }
-      rho = lane_group_sum<L>(rho);
+      rho = lane_group_sum<L>(rho + rho2);
       if (gs == p) rho_keep = rho;
       if (EE) {
         pee = lane_group_sum<L>(pee);
@@ -1785,7 +1812,7 @@ __global__ void __launch_bounds__((ForceThreads<R, MODE>::value))
     for (int p = un.p0; p < un.p1; p++) {
       const NextSlot<R> cs = next;
       const int i = cs.i;
-      R fx = 0, fy = 0, fz = 0, ep = 0, vir = 0, vlo = 0;
+      R fx = 0, fy = 0, fz = 0, ep = 0, ep2 = 0, vir = 0, vlo = 0;
       if (p + 1 < un.p1) next.load(rec, a.nnb, i + IMDG_WAVE / L, cr);
       if (cs.mine) {
         const R4 ui = cs.u;
@@ -1834,7 +1861,7 @@ __global__ void __launch_bounds__((ForceThreads<R, MODE>::value))
                            [&](uint4 e4, auto pf, uint4& slot) {
                              force_group_sgf(e4, pf, slot, rec, off, olo, ui,
                                              0.5f * dFi, Q, Rr, ta, fx, fy,
-                                             fz, ep, vir, vlo);
+                                             fz, ep, ep2, vir, vlo);
                            });
           } else {
             // LT: the launch stages the table values, the records stay
@@ -1869,7 +1896,7 @@ __global__ void __launch_bounds__((ForceThreads<R, MODE>::value))
       fx = lane_group_sum<L>(fx);
       fy = lane_group_sum<L>(fy);
       fz = lane_group_sum<L>(fz);
-      ep = lane_group_sum<L>(ep);
+      ep = lane_group_sum<L>(ep + ep2);
       vir = lane_group_sum<L>(vir);
       if (sizeof(R) == 4) vlo = lane_group_sum<L>(vlo);
       if (gs == p) {

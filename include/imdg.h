@@ -254,14 +254,15 @@ int  imdg_kernel_times(imdg_ctx *ctx, const char **names, double *ms,
    lanes of a wavefront, lane s taking entries s, s+lanes, ... (so every
    lane handles about K/lanes neighbours, and the records one gather reads
    for an atom are consecutive list entries); a block of `threads` threads
-   holds threads/lanes atoms at a time.  Results differ between shapes only
+   holds threads/lanes atoms at a time.  With four lanes, systems too small
+   to fill the chip are walked by 8 or 16.  Results differ between shapes only
    by the order of floating-point sums. */
 typedef struct {
   int    density_lanes;   /* 1, 2 or 4 */
-  int    density_threads; /* 256, 512 or 1024 */
+  int    density_threads; /* a multiple of 64 up to 1024 */
   int    force_lanes;     /* 1, 2 or 4 */
-  int    force_threads;   /* 256, 512, or up to the force loop's maximum
-                             (768 mixed, 512 FP64) */
+  int    force_threads;   /* a multiple of 64 up to the force loop's maximum
+                             (1024 mixed, 512 FP64) */
   double density_ms;      /* imdg_autotune: mean time of the chosen density
                              launch (0 otherwise) */
   double force_ms;        /* imdg_autotune: same for the force launch */

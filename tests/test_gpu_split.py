@@ -5,7 +5,7 @@ with the tables staged or read from L2, against the oracle at the bars of the la
 that is not full; replicas, whose partial sums are per unit, over several
 steps and lanes; the pair columns of two species, equal across the diagonal
 (three are stored) or not (all four); the FP64 default shapes on both sides
-of their line of size."""
+of their line of size; the accuracy of the mixed sums with two lanes."""
 import copy
 
 import numpy as np
@@ -166,3 +166,27 @@ def test_large_fp64_default_shapes(cells):
         res.append(gpu.atoms())
     for k in ("f", "epot", "rho"):
         assert np.abs(res[0][k] - res[1][k]).max() <= 1e-12, k
+
+
+@pytest.mark.parametrize("lanes", [None, 2, 4])
+def test_mixed_sums_keep_four_lane_accuracy(lanes):
+    """Two lanes per atom (the default beyond 65,000 atoms) sum twice as many
+    terms each as four.  Term by term that gives relative RMS errors of
+    8.2e-8 (rho) and 1.14e-7 (energy per atom) against FP64, four lanes
+    7.2e-8 and 9.0e-8: no shape may be worse than four lanes term by term,
+    plus 3 % for the sample."""
+    eam = eam_tables()
+    s = W.fcc_system((30, 30, 30), 3.615, eam.masses, W.kT(600.0), 50,
+                     displace=0.02)
+    with G.eam_context(eam, [s], precision=G.FP64) as gpu:
+        gpu.calc_forces()
+        ref = gpu.atoms()
+    with G.eam_context(eam, [s], precision=G.MIXED) as gpu:
+        if lanes:
+            gpu.set_tuning(lanes, 1024, lanes, 1024)
+        gpu.calc_forces()
+        got = gpu.atoms()
+    for k, bar in (("rho", 7.25e-8), ("epot", 9.0e-8)):
+        d = got[k].astype(np.float64) - ref[k]
+        err = np.sqrt(np.mean(d * d) / np.mean(ref[k] ** 2))
+        assert err <= 1.03 * bar, (k, err)
