@@ -1849,7 +1849,11 @@ int imdg_set_atoms(imdg_ctx* c, int nrep, const imdg_replica* reps,
   c->d_cmeta = nullptr;
   if (c->list16) ALLOC(c->d_cmeta, sizeof(int) * IMDG_META * c->nchunk);
   {
-    // room for any launch plan: at most 32 resident wavefronts per CU
+    // room for any launch plan: one partial per block or wavefront, at most
+    // 32 resident wavefronts per CU, or (part_chunk) one per unit: at most 4
+    // per chunk with up to four lanes; with 8 or 16 lanes the units are at
+    // most chunks x lanes, which pick_wide allows up to a quarter of the
+    // resident wavefronts
     c->units_cap = std::max(c->units_max, 32 * c->ncu);
     size_t units = std::max((size_t)c->nchunk * (c->part_chunk ? 4 : 1),
                             (size_t)c->units_cap);

@@ -922,7 +922,7 @@ __global__ void __launch_bounds__(IMDG_BLOCK) k_list(BuildArgs a) {
   int r = a.blk_rep[b];
   const RepDev& R = a.rep[r];
   bool flagged = a.rst[r].need_rebuild != 0;
-  // the permuted positions (k_list_done flips the buffers afterwards)
+  // the permuted positions (the end of the rebuild flips the buffers)
   const double4* pos = a.pos[a.ctl->pos_cur ^ 1];
   const void* rec = build_records(a);
   int kmax = a.kmax, seen = 0;

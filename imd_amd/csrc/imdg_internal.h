@@ -251,11 +251,13 @@ template <> struct V2<double> { typedef double2 T; };
 
 // Everything the per-step kernels need, passed by value.
 //
-// The per-step kernels are persistent: IMDG_STEP_THREADS-thread blocks, a
-// grid sized to the resident capacity, every wavefront walking its share of
-// the 64-slot chunks.  Reductions go to one partial per wavefront
-// (part_chunk = 0, a single replica) or one per chunk (part_chunk = 1,
-// several replicas); the last block to finish sums them in a fixed order.
+// The per-step kernels are persistent: blocks of up to IMDG_STEP_THREADS
+// threads, a grid of at most the resident capacity, every wavefront walking
+// its share of the units (a 64-slot chunk, or some of its passes).
+// Reductions go to one partial per block (part_chunk = 0, a single replica)
+// or one per unit (part_chunk = 1, several replicas); finalize_replica sums
+// them in a fixed order, in a launch of its own, in the next step's k_head
+// or (final_inline) in the last block of the force launch.
 template <typename R>
 struct StepArgs {
   typedef typename V4<R>::T R4;
@@ -285,7 +287,7 @@ struct StepArgs {
   Col0<R> col0[4];        // column 0 of pair, rho, embed, EEAM term
   Col0<double> col64[2];  // ... of the FP64 embedding and EEAM term
   int nchunk;             // 64-slot chunks of all replicas
-  int part_chunk;         // partials per chunk (1) or per wavefront (0)
+  int part_chunk;         // partials per unit (1) or per block (0)
   int unitsA;             // wavefront partials written by the density loop
   int unitsB;             // ... by the finalising force / move launch
   int store;              // write the per-atom outputs rho, epot, frc (the

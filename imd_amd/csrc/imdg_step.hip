@@ -1,14 +1,16 @@
 // imdg_step.hip -- CDNA4 (gfx950) per-step kernels of the neighbour-list
 // pair/EAM path: host density with embedding, pair + EAM forces fused with
 // the leapfrog step and the skin test, the unfused move, compensated FP64
-// reductions finished by the last block of each step.
+// reductions finished in a launch of their own, and for small systems the
+// one-block sort with the previous step's reduction (k_head).
 //
-// Execution model: persistent kernels.  A grid of IMDG_STEP_THREADS-thread
-// blocks sized to what the chip holds at once copies the knots of the
-// tables its neighbour loop reads into LDS (when they fit), then every
-// wavefront walks its share of the 64-slot chunks: lane = atom, neighbour
-// records gathered from HBM/L2 through the grouped full list (four entries
-// per lane and load, the next groups prefetched), table knots from LDS.
+// Execution model: persistent kernels.  A grid of blocks sized to what the
+// chip holds at once copies the knots of the tables its neighbour loop reads
+// into LDS (when they fit and the system is large enough to pay for it),
+// then every wavefront walks its share of the units (a 64-slot chunk or some
+// of its passes): 1 to 16 lanes per atom, neighbour records gathered from
+// HBM/L2 through the grouped full list (the next groups prefetched), table
+// knots from LDS.
 // There is no block barrier after the staging, so waves never wait for
 // each other.
 //
