@@ -917,11 +917,13 @@ __global__ void __launch_bounds__(IMDG_BLOCK) k_list(BuildArgs a) {
   __shared__ float off[3 * IMDG_NCODES];
   __shared__ int wmax[IMDG_NWAVE];
   __shared__ int cbase[IMDG_NWAVE][IMDG_META];
-  if (!a.ctl->any_rebuild || a.ctl->frozen || a.ctl->cell_over) return;
+  if (!a.ctl->any_rebuild || a.ctl->frozen) return;
   int b = blockIdx.x;
   int r = a.blk_rep[b];
   const RepDev& R = a.rep[r];
-  bool flagged = a.rst[r].need_rebuild != 0;
+  // a bucket that overflowed: no list, but the rebuild ends as always (its
+  // end freezes the state, and with list_ends only these blocks reach it)
+  const bool flagged = a.rst[r].need_rebuild != 0 && !a.ctl->cell_over;
   // the permuted positions (the end of the rebuild flips the buffers)
   const double4* pos = a.pos[a.ctl->pos_cur ^ 1];
   const void* rec = build_records(a);
@@ -1104,11 +1106,12 @@ __global__ void __launch_bounds__(IMDG_CHUNK* LIST_LANES)
   __shared__ Tile tile;
   __shared__ float off[3 * IMDG_NCODES];
   __shared__ int cbase[IMDG_META], wmax[LIST_LANES];
-  if (!a.ctl->any_rebuild || a.ctl->frozen || a.ctl->cell_over) return;
+  if (!a.ctl->any_rebuild || a.ctl->frozen) return;
   const int chunk = blockIdx.x;
   const int r = a.blk_rep[chunk / (IMDG_BLOCK / IMDG_CHUNK)];
   const RepDev& R = a.rep[r];
-  const bool flagged = a.rst[r].need_rebuild != 0;
+  // see k_list
+  const bool flagged = a.rst[r].need_rebuild != 0 && !a.ctl->cell_over;
   const double4* pos = a.pos[a.ctl->pos_cur ^ 1];
   const void* rec = build_records(a);
   const int w = threadIdx.x / IMDG_WAVE, lane = threadIdx.x & (IMDG_WAVE - 1);

@@ -1,0 +1,137 @@
+"""A cell that outgrows its bucket, in every way a rebuild can end: in the
+list's last block (pair-only systems of up to 128 blocks), in a launch of its
+own (larger ones), in the density loop's first block (EAM).  The host has to
+learn of it, enlarge the buckets and build again, both in the entry points
+and in the middle of fused steps."""
+import copy
+
+import numpy as np
+import pytest
+
+from imd_amd import imdg as G
+from imd_amd import workloads as W
+
+from helpers import (canon_pairs_gpu, canon_pairs_oracle, lj, oracle_lj)
+from test_gpu_tuning import TOL, _check_static
+
+pytestmark = pytest.mark.gpu
+
+PLACES = 32       # smallest bucket
+LJ_MARGIN = 0.9   # list radius 3.4 sigma: 42 atoms of the crystal in a cell
+LJ_CELL = 2.5 + LJ_MARGIN + 1e-6
+
+
+def _fullest(x, s, ncell):
+    """Atoms in the fullest cell of a periodic cube of ncell^3 cells."""
+    w = np.mod(x / np.diag(s.box), 1.0)
+    c = np.minimum((w * ncell).astype(int), ncell - 1)
+    return np.bincount((c[:, 0] * ncell + c[:, 1]) * ncell + c[:, 2]).max()
+
+
+def _in_box(s, ncell, cell, centre):
+    """The block s in an empty box of ncell^3 cells, centred at `centre`
+    (in cells)."""
+    s.x = s.x - s.x.mean(axis=0) + np.asarray(centre) * cell
+    s.box = np.diag([ncell * cell] * 3)
+    return s
+
+
+def _lj_cluster(cells, ncell, seed):
+    s = W.fcc_system((cells,) * 3, 1.5496, [1.0], 0.0, seed, displace=0.02)
+    return _in_box(s, ncell, LJ_CELL, (ncell // 2 + 0.5,) * 3)
+
+
+LJ_SYSTEMS = {
+    # 4,913 cells (no one-block sort), 2,048 atoms: the list's last block
+    "one": [(8, 17)],
+    "batch": [(8, 6), (7, 5)],
+    # 19,652 atoms, 154 blocks: a launch of its own
+    "large": [(17, 17)],
+}
+
+
+@pytest.mark.parametrize("precision", [G.FP64, G.MIXED])
+@pytest.mark.parametrize("which", sorted(LJ_SYSTEMS))
+def test_pair_only_overflow_static(which, precision):
+    systems = [_lj_cluster(c, n, 70 + k)
+               for k, (c, n) in enumerate(LJ_SYSTEMS[which])]
+    for s, (_, n) in zip(systems, LJ_SYSTEMS[which]):
+        assert _fullest(s.x, s, n) > PLACES
+    with G.pair_context(lj(), systems, precision=precision,
+                        nbl_margin=LJ_MARGIN) as gpu:
+        for first in (True, False):      # the buckets fit the second time
+            gpu.make_nblist() if not first else None
+            gpu.calc_forces()
+            pairs = gpu.pairs()
+            a = gpu.atoms()
+            at = 0
+            for r, s in enumerate(systems):
+                orc = oracle_lj(s, nbl_margin=LJ_MARGIN, timestep=0.002)
+                orc.calc_forces()
+                assert canon_pairs_gpu(pairs, r) == \
+                    canon_pairs_oracle(orc.pairs())
+                f = orc.atoms()["f"]
+                d = a["f"][at:at + s.n] - f
+                assert np.sqrt(np.mean(d * d) / np.mean(f * f)) <= \
+                    TOL[precision][0]
+                at += s.n
+
+
+STEPS = 48
+
+
+def _drifting(cells, ncell, cell, a, mass, dt, seed, gas=False):
+    """A small cube that starts where eight cells meet and moves into the
+    middle of one in 40 of the STEPS steps; gas: with one atom, out of reach of the
+    others, in each cell the cube stays away from."""
+    s = W.fcc_system((cells,) * 3, a, [mass], 0.0, seed, displace=0.02)
+    mid = ncell // 2
+    s = _in_box(s, ncell, cell, (mid,) * 3)
+    if gas:
+        g = np.stack(np.meshgrid(*[np.arange(ncell)] * 3, indexing="ij"),
+                     -1).reshape(-1, 3)
+        g = g[np.abs(g + 0.5 - mid).max(axis=1) > 2.0]
+        s.x = np.concatenate([s.x, (g + 0.25) * cell])
+        n = s.x.shape[0]
+        s.type, s.mass = np.zeros(n, np.int32), np.full(n, mass)
+        s.id = np.arange(n, dtype=np.int64)
+    s.p = np.full(s.x.shape, 0.5 * cell / (40 * dt) * mass)
+    return s
+
+
+def _same_run(make, systems, dense, ncell, lanes, precision):
+    """The run whose bucket overflows on the way has the trajectory of the
+    same systems beside a dense one, which sets larger buckets."""
+    got = []
+    for extra in ([], [dense]):
+        with make(systems + extra, precision) as gpu:
+            gpu.set_tuning(lanes, 512, lanes, 512)
+            gpu.run(STEPS)
+            th = gpu.thermo_history(0, STEPS)
+            got.append((gpu.atoms(), th[:, :len(systems), 0],
+                        th[:, :len(systems), 6]))
+    n = sum(s.n for s in systems)
+    s = systems[0]
+    assert _fullest(s.x, s, ncell) <= PLACES
+    assert _fullest(got[1][0]["x"][:s.n], s, ncell) > PLACES
+    for k in ("x", "p", "f", "epot", "rho"):
+        assert np.array_equal(got[0][0][k][:n], got[1][0][k][:n]), k
+    assert np.array_equal(got[0][1], got[1][1])
+    assert np.array_equal(got[0][2], got[1][2])
+    assert got[0][2][1:, 0].sum() > 0     # it rebuilt after the first step
+
+
+@pytest.mark.parametrize("precision", [G.FP64, G.MIXED])
+@pytest.mark.parametrize("which", ["one", "batch", "large"])
+def test_pair_only_overflow_in_run(which, precision):
+    ncell = {"one": 17, "batch": 6, "large": 27}[which]
+    systems = [_drifting(3, ncell, LJ_CELL, 1.5496, 1.0, 0.002, 80 + k,
+                         gas=which == "large")
+               for k in range(2 if which == "batch" else 1)]
+    dense = W.fcc_system((7, 7, 7), 1.5496, [1.0], 0.0, 90, displace=0.02)
+
+    def make(sys_, prec):
+        return G.pair_context(lj(), copy.deepcopy(sys_), precision=prec,
+                              nbl_margin=LJ_MARGIN)
+
+    _same_run(make, systems, dense, ncell, 2, precision)
