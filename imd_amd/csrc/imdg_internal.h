@@ -170,8 +170,10 @@ struct Ctl {
   int any_rebuild;        // some replica needs a list rebuild
   int frozen;             // list overflow: every kernel is a no-op until
                           // the host grows the list and re-runs the build
-                          // (set by list_done: a density block that began
-                          // before that only recomputes its outputs)
+                          // (set by list_done, in a step with EAM while the
+                          // density loop runs: its blocks read it once each,
+                          // and one that goes on computes outputs that the
+                          // step run again replaces)
   int overflow;
   int kmax_seen;
   int is_short;

@@ -1535,13 +1535,19 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS)
   __shared__ R4 wofs[IMDG_STEP_WAVES][2][IMDG_NCODES];
   __shared__ ColPar<R> cpr[IMDG_MAXCOLS];
   __shared__ int done_red[2 * IMDG_STEP_WAVES];
-  if (a.ctl->frozen) return;
+  __shared__ int stop;
   if (a.end_rebuild && blockIdx.x == 0) list_done(a.end, done_red);
+  // block 0 may freeze the state while the others run: one lane reads the
+  // flag for its block, or waves that see it late would go on with tables
+  // that the waves gone before did not stage
+  const int frozen = threadIdx.x == 0 ? a.ctl->frozen : 0;
   const Col0<R>& tr = a.col0[1];
   const int klo = LT ? a.lds_lo : 0;
   if (LT) stage_knots(a.knots, a.lds_lo, a.lds_n, (R2*)dyn_lds);
   if (!NT1) stage_colpar(tabs[1], klo, cpr);
+  if (threadIdx.x == 0) stop = frozen;
   __syncthreads();
+  if (stop) return;
   const R2* __restrict__ K = LT ? (const R2*)dyn_lds : a.knots;
   const R4* __restrict__ rec = a.rec_a;
   const int nt = a.ntypes;

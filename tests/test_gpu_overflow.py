@@ -11,7 +11,8 @@ import pytest
 from imd_amd import imdg as G
 from imd_amd import workloads as W
 
-from helpers import (canon_pairs_gpu, canon_pairs_oracle, lj, oracle_lj)
+from helpers import (canon_pairs_gpu, canon_pairs_oracle, eam_tables,
+                     emod_table, lj, oracle_lj)
 from test_gpu_tuning import TOL, _check_static
 
 pytestmark = pytest.mark.gpu
@@ -135,3 +136,29 @@ def test_pair_only_overflow_in_run(which, precision):
                               nbl_margin=LJ_MARGIN)
 
     _same_run(make, systems, dense, ncell, 2, precision)
+
+
+@pytest.mark.parametrize("variant", ["fp64", "mixed", "spline", "eeam"])
+def test_list_overflow_while_the_density_loop_runs(variant):
+    """With EAM the first block of the density loop freezes the state when
+    the list does not fit, while the other blocks start: the loops of several
+    species, which take their tables' layout from LDS, run through it and the
+    step is run again with the bits of a list that fits."""
+    eam = eam_tables(nspecies=2, rc=5.5)
+    s = W.alloy_slab((22, 21, 9), temp_k=900.0, seed=17)
+    kw = dict(precision=G.MIXED if variant in ("mixed", "eeam") else G.FP64)
+    if variant == "spline":
+        kw["interpolation"] = G.INTERP_SPLINE
+    if variant == "eeam":
+        kw["emod"] = emod_table(2)
+    got = []
+    for size in (0.3, 2.5):   # the vacuum halves the estimate from the mean
+        with G.eam_context(eam, [s], nbl_size=size, **kw) as gpu:
+            gpu.set_tuning(2, 512, 2, 512)
+            first = gpu.info()["kmax"]
+            gpu.run(12)
+            got.append((gpu.atoms(), gpu.thermo_history(0, 12)[..., :6]))
+            assert (gpu.info()["kmax"] > first) == (size == 0.3)
+    for k, v in got[0][0].items():
+        assert np.array_equal(v, got[1][0][k]), k
+    assert np.array_equal(got[0][1], got[1][1])
