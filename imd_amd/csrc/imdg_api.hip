@@ -2049,6 +2049,8 @@ int imdg_deallocate_nblist(imdg_ctx* c) {
   dfree(c, c->d_nbr);
   c->d_nbr = nullptr;
   c->nbr_bytes = 0;
+  // the list allocated next holds nothing until it is built
+  HIPCHK(c, hipMemsetAsync(c->d_nnb, 0, sizeof(int) * c->nslots, c->stream));
   return flag_all_for_rebuild(c);
 }
 

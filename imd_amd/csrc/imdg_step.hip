@@ -1540,7 +1540,10 @@ __global__ void __launch_bounds__(IMDG_STEP_THREADS)
   // block 0 may freeze the state while the others run: one lane reads the
   // flag for its block, or waves that see it late would go on with tables
   // that the waves gone before did not stage
-  const int frozen = threadIdx.x == 0 ? a.ctl->frozen : 0;
+  // (cell_over: the rebuild stopped before the list, which may not even hold
+  // an older one)
+  const int frozen =
+      threadIdx.x == 0 ? a.ctl->frozen | a.ctl->cell_over : 0;
   const Col0<R>& tr = a.col0[1];
   const int klo = LT ? a.lds_lo : 0;
   if (LT) stage_knots(a.knots, a.lds_lo, a.lds_n, (R2*)dyn_lds);

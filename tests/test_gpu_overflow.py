@@ -12,7 +12,7 @@ from imd_amd import imdg as G
 from imd_amd import workloads as W
 
 from helpers import (canon_pairs_gpu, canon_pairs_oracle, eam_tables,
-                     emod_table, lj, oracle_lj)
+                     emod_table, lj, oracle_eam, oracle_lj, rel_rms)
 from test_gpu_tuning import TOL, _check_static
 
 pytestmark = pytest.mark.gpu
@@ -162,3 +162,54 @@ def test_list_overflow_while_the_density_loop_runs(variant):
     for k, v in got[0][0].items():
         assert np.array_equal(v, got[1][0][k]), k
     assert np.array_equal(got[0][1], got[1][1])
+
+
+EAM_MARGIN = 4.0
+EAM_CELL = 5.0 + EAM_MARGIN + 1e-6
+
+
+@pytest.mark.parametrize("precision", [G.FP64, G.MIXED])
+def test_overflow_after_deallocate(precision):
+    """The list is given back and the next rebuild meets a cell that has
+    outgrown its bucket: nothing may read the new, empty list memory.  Then
+    calc_forces has the oracle's forces, and a fused run the bits of a context
+    that starts there with buckets large enough."""
+    eam = eam_tables()
+    ncell, kw = 6, dict(precision=precision, nbl_margin=EAM_MARGIN)
+    dense = W.eam_crystal(n_cells=8, temp_k=0.0, seed=91)
+    for what in ("calc_forces", "run"):
+        systems = [_drifting(3, ncell, EAM_CELL, 3.615, W.MASS_CU, W.FS,
+                             84 + r) for r in range(2)]
+        for s in systems:
+            s.p *= 40.0          # to the middle of the cell in one step
+            assert _fullest(s.x, s, ncell) <= PLACES
+        with G.eam_context(eam, systems, **kw) as gpu:
+            gpu.set_tuning(2, 512, 2, 512)
+            gpu.calc_forces()
+            gpu.move_atoms()
+            gpu.deallocate_nblist()
+            at = gpu.atoms()
+            n = systems[0].n
+            for r, s in enumerate(systems):
+                s.x, s.p = (at[k][r * n:(r + 1) * n].copy() for k in "xp")
+                assert _fullest(s.x, s, ncell) > PLACES
+            if what == "calc_forces":
+                gpu.calc_forces()
+                got = gpu.atoms()
+                for r, s in enumerate(systems):
+                    orc = oracle_eam(s, eam, nbl_margin=EAM_MARGIN,
+                                     timestep=W.FS)
+                    orc.calc_forces()
+                    assert canon_pairs_gpu(gpu.pairs(), r) == \
+                        canon_pairs_oracle(orc.pairs())
+                    assert rel_rms(got["f"][r * n:(r + 1) * n],
+                                   orc.atoms()["f"]) <= TOL[precision][0]
+                continue
+            gpu.run(2)
+            got = gpu.atoms()
+        with G.eam_context(eam, systems + [dense], **kw) as gpu:
+            gpu.set_tuning(2, 512, 2, 512)
+            gpu.run(2)
+            want = gpu.atoms()
+        for k, v in got.items():
+            assert np.array_equal(v, want[k][:2 * n]), k
