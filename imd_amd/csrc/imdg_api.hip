@@ -1343,6 +1343,9 @@ int fix_overflow(imdg_ctx* c, int* fixed) {
 
 int ensure_ready(imdg_ctx* c) {
   if (!c->atoms_set) return fail(c, IMDG_ERR_STATE, "no atoms set");
+  // the caller's thread may work with another device: allocations and
+  // launches belong on the context's
+  hipSetDevice(c->dev);
   if (!c->d_nbr) {
     size_t bytes = list_bytes(c, c->kmax);
     int rc = dalloc(c, (void**)&c->d_nbr, bytes);
@@ -2208,6 +2211,7 @@ int imdg_sync(imdg_ctx* c) {
 int imdg_get_atoms(imdg_ctx* c, double* x, double* p, double* f, double* epot,
                    double* rho, double* df) {
   if (!c || !c->atoms_set) return IMDG_ERR_ARG;
+  hipSetDevice(c->dev);
   // the wanted arrays one after the other in d_out
   const struct {
     double* host;
@@ -2497,6 +2501,7 @@ int imdg_set_tuning(imdg_ctx* c, const imdg_tuning* t) {
   c->lpa_frc = t->force_lanes;
   c->thr_frc = t->force_threads;
   if (!c->atoms_set) return IMDG_OK;
+  hipSetDevice(c->dev);  // the plan asks it what fits
   HIPCHK(c, hipStreamSynchronize(c->stream));
   if (plan(c) != IMDG_OK) {
     std::string why = c->err;

@@ -1,0 +1,76 @@
+"""The host side of libimdg.so on a HIP runtime without a GPU (hip_stub.c):
+which device its calls work on and what they allocate."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+from imd_amd import build as B
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+PRELUDE = """
+import ctypes as C, os, sys
+sys.path[:0] = [%r, %r]
+import numpy as np
+from imd_amd import imdg as G
+from imd_amd import workloads as W
+from helpers import eam_tables, lj
+stub = C.CDLL(os.environ["HIP_STUB"])
+for f in ("live", "peak"):
+    getattr(stub, "stub_" + f).restype = C.c_size_t
+stub.stub_limit.argtypes = [C.c_size_t]
+stub.stub_time.argtypes = [C.c_int, C.c_double]
+for f in ("wrong_device", "mallocs", "launches"):
+    getattr(stub, "stub_" + f).restype = C.c_long
+stub.stub_pinned_from.restype = C.c_void_p
+""" % (ROOT, os.path.join(ROOT, "tests"))
+
+
+@pytest.fixture(scope="module")
+def child(tmp_path_factory):
+    """Runs a Python text in a process whose HIP runtime is the stub."""
+    if not os.path.exists(B.LIB):
+        B.build_lib()
+    so = str(tmp_path_factory.mktemp("stub") / "libhip_stub.so")
+    subprocess.check_call(
+        ["gcc", "-std=gnu11", "-O1", "-shared", "-fPIC",
+         "-I/opt/rocm/include", "-o", so,
+         os.path.join(ROOT, "tests", "hip_stub.c")])
+    preload = ":".join(p for p in (so, os.environ.get("LD_PRELOAD")) if p)
+
+    def run(text, **env):
+        r = subprocess.run(
+            [sys.executable, "-c", PRELUDE + textwrap.dedent(text)],
+            env={**os.environ, "LD_PRELOAD": preload, "HIP_STUB": so, **env},
+            stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True,
+            timeout=120)
+        assert r.returncode == 0, r.stdout
+        return r.stdout
+    return run
+
+
+def test_every_call_selects_its_device(child):
+    """A context of device 1, called by a thread whose current device is 0:
+    allocations and launches are on device 1."""
+    child("""
+        s = W.eam_crystal(n_cells=6, temp_k=300.0, seed=1)
+        ctx = G.eam_context(eam_tables(), [s], device=1)
+        ctx.set_stress(True)
+        made = stub.stub_mallocs(0)
+        assert made == 0 and stub.stub_mallocs(1) > 0
+        calls = dict(
+            atoms=ctx.atoms, calc_forces=ctx.calc_forces,
+            move_atoms=ctx.move_atoms, check_nblist=ctx.check_nblist,
+            make_nblist=ctx.make_nblist,
+            deallocate_nblist=ctx.deallocate_nblist,
+            run=lambda: ctx.run(3, sync=False), stress=ctx.stress,
+            set_tuning=lambda: ctx.set_tuning(2, 512, 2, 512),
+            autotune=lambda: ctx.autotune(1))
+        for name, call in calls.items():
+            stub.hipSetDevice(0)
+            call()
+            assert stub.stub_wrong_device() == 0, name
+            assert stub.stub_mallocs(0) == 0, name
+    """)
