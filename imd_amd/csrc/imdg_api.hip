@@ -1448,36 +1448,54 @@ int plan(imdg_ctx* c) {
   return c->mixed ? plan_steps<float>(c) : plan_steps<double>(c);
 }
 
-// Try every lanes-per-slot x block-size variant of the density loop, then
-// of the force loop, on the current state; keep the fastest of each.
+// Try the shape in use and every lanes-per-slot x block-size variant of the
+// density loop, then of the force loop, on the current state; keep the
+// fastest of each.  The shape in use comes first: the default of the smallest
+// systems is none of the others.  A default that stays the fastest stays a
+// default, chosen anew for the next system.
+struct Shape {
+  int lanes, threads;
+};
+std::vector<Shape> shapes_to_time(Shape in_use, std::initializer_list<int> thr,
+                                  int thr_max) {
+  std::vector<Shape> s = {in_use};
+  for (int l : {1, 2, 4})
+    for (int t : thr)
+      if (t <= thr_max && (l != in_use.lanes || t != in_use.threads))
+        s.push_back({l, t});
+  return s;
+}
+
 template <typename R>
 int autotune_t(imdg_ctx* c, int reps, imdg_tuning* out) {
-  static const int lanes[3] = {1, 2, 4};
-  const int fmax = force_threads<R>(c->force_mode);
-  const int thr_d[3] = {256, 512, 1024};
-  const int thr_f[4] = {256, 512, 768, 1024};
   int rc;
   double best_d = 0.0, best_f = 0.0;
+  const bool auto_den[2] = {c->lpa_auto_den, c->thr_auto_den};
+  const bool auto_frc[2] = {c->lpa_auto_frc, c->thr_auto_frc};
   c->lpa_auto_den = c->lpa_auto_frc = false;
   c->thr_auto_den = c->thr_auto_frc = false;
   if (c->tab[1].present) {
-    int bl = c->lpa_den, bt = c->thr_den;
+    const Shape in_use = {c->lpa_den, c->thr_den};
+    Shape best = in_use;
     best_d = 1e300;
-    for (int li = 0; li < 3; li++)
-      for (int ti = 0; ti < 3; ti++) {
-        c->lpa_den = lanes[li];
-        c->thr_den = thr_d[ti];
-        if (plan(c) != IMDG_OK) continue;  // not launchable this way
-        double ms;
-        if ((rc = time_loop<R>(c, true, reps, &ms))) return rc;
-        if (ms < best_d) {
-          best_d = ms;
-          bl = lanes[li];
-          bt = thr_d[ti];
-        }
+    for (const Shape& s :
+         shapes_to_time(in_use, {256, 512, 1024}, IMDG_STEP_THREADS)) {
+      c->lpa_den = s.lanes;
+      c->thr_den = s.threads;
+      if (plan(c) != IMDG_OK) continue;  // not launchable this way
+      double ms;
+      if ((rc = time_loop<R>(c, true, reps, &ms))) return rc;
+      if (ms < best_d) {
+        best_d = ms;
+        best = s;
       }
-    c->lpa_den = bl;
-    c->thr_den = bt;
+    }
+    c->lpa_den = best.lanes;
+    c->thr_den = best.threads;
+    if (best.lanes == in_use.lanes && best.threads == in_use.threads) {
+      c->lpa_auto_den = auto_den[0];
+      c->thr_auto_den = auto_den[1];
+    }
     if ((rc = plan(c))) return rc;
     double ms;
     if ((rc = time_loop<R>(c, true, 0, &ms))) return rc;  // records for B
@@ -1509,22 +1527,23 @@ int autotune_t(imdg_ctx* c, int reps, imdg_tuning* out) {
       HIPCHK(c, hipMemcpyAsync(sr, c->d_reca, rb, hipMemcpyDeviceToDevice,
                                c->stream));
     }
-    int bl = c->lpa_frc, bt = c->thr_frc;
+    const Shape in_use = {c->lpa_frc, c->thr_frc};
+    Shape best = in_use;
     best_f = 1e300;
-    for (int li = 0; li < 3 && rc == IMDG_OK; li++)
-      for (int ti = 0; ti < 4; ti++) {
-        if (thr_f[ti] > fmax) continue;
-        c->lpa_frc = lanes[li];
-        c->thr_frc = thr_f[ti];
-        if (plan(c) != IMDG_OK) continue;
-        double ms;
-        if ((rc = time_loop<R>(c, false, reps, &ms, integ))) break;
-        if (ms < best_f) {
-          best_f = ms;
-          bl = lanes[li];
-          bt = thr_f[ti];
-        }
+    rc = IMDG_OK;
+    for (const Shape& s :
+         shapes_to_time(in_use, {256, 512, 768, 1024},
+                        force_threads<R>(c->force_mode))) {
+      c->lpa_frc = s.lanes;
+      c->thr_frc = s.threads;
+      if (plan(c) != IMDG_OK) continue;
+      double ms;
+      if ((rc = time_loop<R>(c, false, reps, &ms, integ))) break;
+      if (ms < best_f) {
+        best_f = ms;
+        best = s;
       }
+    }
     if (integ) {
       hipMemcpyAsync(c->d_pos[pc], sp, 32 * ns, hipMemcpyDeviceToDevice,
                      c->stream);
@@ -1537,8 +1556,12 @@ int autotune_t(imdg_ctx* c, int reps, imdg_tuning* out) {
       hipFree(sr);
     }
     if (rc) return rc;
-    c->lpa_frc = bl;
-    c->thr_frc = bt;
+    c->lpa_frc = best.lanes;
+    c->thr_frc = best.threads;
+    if (best.lanes == in_use.lanes && best.threads == in_use.threads) {
+      c->lpa_auto_frc = auto_frc[0];
+      c->thr_auto_frc = auto_frc[1];
+    }
   }
   if ((rc = plan(c))) return rc;
   c->err.clear();

@@ -274,8 +274,8 @@ int  imdg_get_tuning(imdg_ctx *ctx, imdg_tuning *out);
 /* Takes effect for the next launch; IMDG_ERR_ARG (and no change) for a
    shape the loops cannot be launched with. */
 int  imdg_set_tuning(imdg_ctx *ctx, const imdg_tuning *t);
-/* Times every lanes x threads shape of the density loop and then of the
-   force loop on the current state (reps launches each, the list is built
+/* Times the shape in use and every lanes x threads shape of the density loop
+   and then of the force loop on the current state (reps launches each, the list is built
    first if needed) and keeps the fastest of each.  The state does not
    advance; forces and energies are left as imdg_calc_forces leaves them.
    *chosen (may be NULL) receives the result. */

@@ -74,3 +74,37 @@ def test_every_call_selects_its_device(child):
             assert stub.stub_wrong_device() == 0, name
             assert stub.stub_mallocs(0) == 0, name
     """)
+
+
+def test_autotune_times_the_shape_in_use(child):
+    """The default shape of the smallest systems (blocks of one wavefront) is
+    among those timed: kept, and still a default, where it is the fastest;
+    replaced where another one is."""
+    child("""
+        small = W.eam_crystal(n_cells=6, temp_k=300.0, seed=1)
+        large = W.eam_crystal(n_cells=20, temp_k=300.0, seed=2)
+        for prec in (G.FP64, G.MIXED):
+            with G.eam_context(eam_tables(), [small], precision=prec) as ctx:
+                default = ctx.tuning()
+                assert default["density_threads"] == 64
+                assert default["force_threads"] == 64
+                stub.stub_time(64, 0.25)
+                got = ctx.autotune(2)
+                stub.stub_time(64, 0.0)
+                assert abs(got["density_ms"] - 0.25) < 1e-6
+                assert abs(got["force_ms"] - 0.25) < 1e-6
+                assert [got[k] for k in default][:4] == \\
+                    [default[k] for k in default][:4]
+                ctx.set_systems([large])
+                assert ctx.tuning()["density_threads"] == 1024
+                ctx.set_systems([small])
+                stub.stub_time(256, 0.125)
+                got = ctx.autotune(2)
+                stub.stub_time(256, 0.0)
+                assert got["density_threads"] == got["force_threads"] == 256
+                ctx.set_systems([large])          # a chosen shape stays
+                assert ctx.tuning()["density_threads"] == 256
+        with G.pair_context(lj(), [W.lj_crystal(6)]) as ctx:
+            stub.stub_time(64, 0.25)
+            assert ctx.autotune(2)["force_threads"] == 64
+    """)
