@@ -127,7 +127,8 @@ struct imdg_ctx {
   int* d_aid[2] = {nullptr, nullptr};
   double4* d_xnbl = nullptr;
   int *d_acell = nullptr, *d_bucket = nullptr;
-  int bucket_cap = 0;
+  int bucket_cap = 0;        // places per cell; 0: no buckets
+  long bucket_bytes = -1;    // most they may take; -1: by the system
   bool list_shared = false;  // several lanes per atom build its list
   Tile* d_tiles = nullptr;   // (then without tiles in memory)
   signed char* d_atype = nullptr;
@@ -295,6 +296,7 @@ void free_all(imdg_ctx* c) {
   c->d_stress = nullptr;
   c->d_spart = nullptr;
   c->stress_valid = false;
+  c->d_bucket = nullptr;
   c->d_out = nullptr;
   c->out_len = 0;
 }
@@ -1299,6 +1301,27 @@ size_t list_bytes(imdg_ctx* c, int kmax) {
   return (size_t)(c->nslots / IMDG_WAVE) * kmax * IMDG_WAVE * 4;
 }
 
+// Memory of the cell sort: buckets of at least `places` atoms per cell, or
+// 12 B per slot where they would take too much (IMDG_BUCKET_BYTES).
+int alloc_bucket(imdg_ctx* c, int places) {
+  dfree(c, c->d_bucket);
+  c->d_bucket = nullptr;
+  const size_t cap = ((size_t)std::max(IMDG_BUCKET_MIN, places) + 7) / 8 * 8;
+  const size_t most =
+      c->bucket_bytes >= 0
+          ? (size_t)c->bucket_bytes
+          : std::max((size_t)IMDG_BUCKET_BYTES,
+                     (size_t)IMDG_BUCKET_SLOT * c->nslots);
+  if (cap <= most / sizeof(int) / c->ncells) {
+    c->bucket_cap = (int)cap;
+    if (!dalloc(c, (void**)&c->d_bucket, sizeof(int) * cap * c->ncells))
+      return IMDG_OK;
+    c->err.clear();  // the memory is not there: without buckets then
+  }
+  c->bucket_cap = 0;
+  return dalloc(c, (void**)&c->d_bucket, sizeof(int) * 3 * (size_t)c->nslots);
+}
+
 // Grow the list (or the cells' buckets) after an overflow and rebuild;
 // *fixed = 1 if it had to.
 int fix_overflow(imdg_ctx* c, int* fixed) {
@@ -1311,12 +1334,7 @@ int fix_overflow(imdg_ctx* c, int* fixed) {
   if (h.cell_over) {
     // more atoms in a cell than its bucket has places: larger buckets, and
     // the counters that the cell sort would have cleared
-    c->bucket_cap = (h.cell_over + h.cell_over / 4 + 15) / 8 * 8;
-    dfree(c, c->d_bucket);
-    c->d_bucket = nullptr;
-    if ((rc = dalloc(c, (void**)&c->d_bucket,
-                     sizeof(int) * c->bucket_cap * (size_t)c->ncells)))
-      return rc;
+    if ((rc = alloc_bucket(c, h.cell_over + h.cell_over / 4 + 8))) return rc;
     HIPCHK(c, hipMemsetAsync(c->d_cell_cnt, 0, sizeof(int) * c->ncells,
                              c->stream));
     int zero = 0;
@@ -1628,6 +1646,8 @@ int imdg_ctx_create(const imdg_config* cfg, imdg_ctx** out) {
   if (const char* e = getenv("IMDG_SPLIT_MOVE")) c->split_move = atoi(e) != 0;
   if (const char* e = getenv("IMDG_TILE_LIMIT"))
     c->tile_cap = std::max(0, std::min(atoi(e), IMDG_TILE_CAP));
+  if (const char* e = getenv("IMDG_BUCKET_LIMIT"))
+    c->bucket_bytes = std::max(0l, atol(e));
   if (const char* e = getenv("IMDG_LIST_NT")) c->list_nt = atoi(e) != 0;
   if (const char* e = getenv("IMDG_FINAL_KERNEL"))
     c->final_inline = atoi(e) == 0;
@@ -1797,8 +1817,6 @@ int imdg_set_atoms(imdg_ctx* c, int nrep, const imdg_replica* reps,
   c->nstile = stile;
   c->kmax = std::max(16, (int)ceil(kest * c->cfg.nbl_size * 1.25));
   c->kmax = (c->kmax + IMDG_LIST_PAD - 1) / IMDG_LIST_PAD * IMDG_LIST_PAD;
-  // places of a cell's bucket: twice the mean (an overflow enlarges it)
-  c->bucket_cap = std::max(IMDG_BUCKET_MIN, (int)ceil(2 * percell) + 7) / 8 * 8;
 
   int rc;
 #define ALLOC(ptr, bytes)                                        \
@@ -1823,9 +1841,8 @@ int imdg_set_atoms(imdg_ctx* c, int nrep, const imdg_replica* reps,
     if (R.nblk > IMDG_SHARE_BLOCKS) c->list_shared = false;
   c->d_tiles = nullptr;
   if (!c->list_shared) ALLOC(c->d_tiles, sizeof(Tile) * c->nblk);
-  if ((rc = dalloc(c, (void**)&c->d_bucket,
-                   sizeof(int) * c->bucket_cap * (size_t)c->ncells)))
-    return rc;
+  // places of a cell: twice the mean (an overflow enlarges them)
+  if ((rc = alloc_bucket(c, (int)ceil(2 * percell)))) return rc;
   ALLOC(c->d_cell_cnt, sizeof(int) * c->ncells);
   ALLOC(c->d_cell_beg, sizeof(int) * c->ncells);
   ALLOC(c->d_cell_num, sizeof(int) * c->ncells);

@@ -40,7 +40,8 @@ __device__ __forceinline__ int block_replica(const int* blk_rep) {
 // goes there in the cell's bucket (bucket_cap places; the order inside a
 // cell is fixed by k_sort).  A cell with more atoms than places is noted in
 // the control block: the chain then stops and the host enlarges the
-// buckets.
+// buckets.  Without buckets (bucket_cap 0) cell and place are kept per slot
+// and k_place puts the slot index where the cell's atoms start.
 #define BIN_HASH 256
 
 // Exclusive scan of the cell counts of every rebuilt replica by one block,
@@ -126,10 +127,14 @@ __global__ void __launch_bounds__(IMDG_BLOCK) k_bin(BuildArgs a) {
   __syncthreads();
   if (active) {
     const int m = hbase[h] + rank;
-    if (m < a.bucket_cap)
+    if (a.bucket_cap == 0) {
+      a.bucket[i] = cell;
+      a.bucket[a.nslots + i] = m;
+    } else if (m < a.bucket_cap) {
       a.bucket[(size_t)cell * a.bucket_cap + m] = i;
-    else
+    } else {
       atomicMax(&a.ctl->cell_over, m + 1);
+    }
   }
   if (!a.scan_in_bin) return;
   // the last block to finish scans the cell counts
@@ -225,6 +230,20 @@ __device__ __forceinline__ int cell_first_slot(const BuildArgs& a,
   return a.tile_off[R.stile_off + lc / IMDG_SCAN_TILE] + a.cell_loc[cell];
 }
 
+// The slots in cell order, where there are no buckets (more cells than atoms
+// and gigabytes of them): an idle launch of 1.7 us per step that the others
+// do without.
+__global__ void __launch_bounds__(IMDG_BLOCK) k_place(BuildArgs a) {
+  if (!a.ctl->any_rebuild || a.ctl->frozen) return;
+  const int r = block_replica(a.blk_rep);
+  if (!a.rst[r].need_rebuild) return;
+  const RepDev& R = a.rep[r];
+  const int i = blockIdx.x * IMDG_BLOCK + threadIdx.x;
+  if (i - R.atom_off >= R.natoms) return;
+  const int first = cell_first_slot(a, R, a.bucket[i]);
+  a.bucket[2 * a.nslots + first + a.bucket[a.nslots + i]] = i;
+}
+
 // Per cell: first slot and count, counter reset, and the atoms of the cell
 // moved to their new slots in the other buffers, ordered by input index
 // (deterministic list order), with the cell-relative records.  32 lanes per
@@ -254,7 +273,8 @@ __global__ void __launch_bounds__(256) k_sort(BuildArgs a) {
       continue;
     }
     const int b = cell_first_slot(a, R, c), n = a.cell_cnt[c];
-    const int* p = a.bucket + (size_t)c * a.bucket_cap;
+    const int* p = a.bucket_cap ? a.bucket + (size_t)c * a.bucket_cap
+                                : a.bucket + 2 * a.nslots + b;
     if (n <= SORT_LANES) {
       int v = l < n ? p[l] : 0;
       int key = l < n ? aid[v] : 0x7fffffff;
@@ -1247,6 +1267,8 @@ void launch_sort(const BuildArgs& b, int grid, hipStream_t st) {
   hipLaunchKernelGGL(k_bin, dim3(b.nblk), dim3(IMDG_BLOCK), 0, st, b);
   if (!b.scan_in_bin)
     hipLaunchKernelGGL(k_scan, dim3(b.nstile), dim3(IMDG_SCAN_TILE), 0, st, b);
+  if (b.bucket_cap == 0)
+    hipLaunchKernelGGL(k_place, dim3(b.nblk), dim3(IMDG_BLOCK), 0, st, b);
   hipLaunchKernelGGL(k_sort, dim3(grid), dim3(256), 0, st, b);
 }
 

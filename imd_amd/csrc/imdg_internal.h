@@ -121,6 +121,13 @@
 // 484.
 #define IMDG_SHARE_BLOCKS 2560
 #define IMDG_BUCKET_MIN 32   // smallest bucket (atoms of a cell)
+// The buckets take memory by the cell, and one full cell enlarges them all.
+// Beyond this many bytes, and 128 B per slot (as much as positions and
+// momenta), the sort keeps 12 B per slot instead and has one launch more.
+// (A crystal's buckets take 10 B per atom; a particle of 200,000 atoms in a
+// box of 10^8 cells would have 12.8 GB of them.)
+#define IMDG_BUCKET_BYTES (1l << 30)
+#define IMDG_BUCKET_SLOT 128
 
 // Flag bit of a block's list-length maximum (blkmax): its tile exceeded the
 // tile cap and the list build read its candidates from HBM/L2.
@@ -377,7 +384,9 @@ struct BuildArgs {
   int* acell;             // cell of slot (new order)
   signed char* atype;     // type of slot (new order)
   int* bucket;            // slots (old order) of each cell's atoms,
-  int bucket_cap;         // bucket_cap places per cell
+  int bucket_cap;         // bucket_cap places per cell; 0: per slot its cell
+                          // (nslots), its place there (nslots), then the
+                          // slots (old order) in the order of the cells
   int scan_in_bin;        // the last block of k_bin scans the cell counts
   int* cell_cnt;          // atomic counters (zero outside a rebuild)
   int* cell_loc;          // first slot of a cell relative to its scan tile

@@ -213,3 +213,64 @@ def test_overflow_after_deallocate(precision):
             want = gpu.atoms()
         for k, v in got.items():
             assert np.array_equal(v, want[k][:2 * n]), k
+
+
+SORTS = {
+    # EAM, scan of the cells in the binning's last block and in its own launch
+    "crystal": lambda: [W.eam_crystal(n_cells=14, temp_k=1200.0, seed=61)],
+    "large": lambda: [W.eam_crystal(n_cells=42, temp_k=1200.0, seed=62)],
+    "batch": lambda: [W.eam_crystal(n_cells=n, temp_k=t, seed=63 + n)
+                      for n, t in ((5, 1.0), (8, 1500.0), (6, 900.0))],
+    # 2,048 atoms in 13^3 cells: most of them empty, some beyond 32 atoms
+    "cluster": lambda: [_in_box(W.eam_crystal(n_cells=8, temp_k=900.0,
+                                              seed=64, displace=0.02),
+                                13, EAM_CELL, (6.5, 6.5, 6.5))],
+}
+
+
+@pytest.mark.parametrize("graph", ["0", "1"])
+@pytest.mark.parametrize("precision", [G.FP64, G.MIXED])
+@pytest.mark.parametrize("which", sorted(SORTS))
+def test_sort_without_buckets(which, precision, graph, monkeypatch):
+    """Cells too many for buckets: the sort by place gives the bits of the
+    sort through buckets, over fused steps with rebuilds and from captured
+    ones."""
+    margin = EAM_MARGIN if which == "cluster" else 0.4
+    monkeypatch.setenv("IMDG_GRAPH", graph)
+    got = []
+    for limit in (None, "0"):
+        if limit:
+            monkeypatch.setenv("IMDG_BUCKET_LIMIT", limit)
+        with G.eam_context(eam_tables(), SORTS[which](), precision=precision,
+                           nbl_margin=margin) as gpu:
+            gpu.run(40)
+            th = gpu.thermo_history(0, 40)
+            gpu.make_nblist()
+            got.append((gpu.atoms(), th, gpu.pairs(), gpu.cells()))
+    for k, v in got[0][0].items():
+        assert np.array_equal(v, got[1][0][k]), k
+    for a, b in zip(got[0][1:], got[1][1:]):
+        assert np.array_equal(a, b)
+    assert got[0][1][1:, :, 6].sum() > 0 or which == "cluster"
+
+
+@pytest.mark.parametrize("precision", [G.FP64, G.MIXED])
+@pytest.mark.parametrize("which", sorted(LJ_SYSTEMS))
+def test_pair_only_sort_without_buckets(which, precision, monkeypatch):
+    """The same for the pair-only systems whose buckets overflow, against
+    runs whose buckets have grown."""
+    systems = [_lj_cluster(c, n, 70 + k)
+               for k, (c, n) in enumerate(LJ_SYSTEMS[which])]
+    for s in systems:
+        s.p = W.maxwell_momenta(np.random.default_rng(7), s.mass, 0.4)
+    got = []
+    for limit in (None, "0"):
+        if limit:
+            monkeypatch.setenv("IMDG_BUCKET_LIMIT", limit)
+        with G.pair_context(lj(), systems, precision=precision,
+                            nbl_margin=LJ_MARGIN) as gpu:
+            gpu.run(60)
+            got.append((gpu.atoms(), gpu.thermo_history(0, 60)))
+    for k, v in got[0][0].items():
+        assert np.array_equal(v, got[1][0][k]), k
+    assert np.array_equal(got[0][1], got[1][1])

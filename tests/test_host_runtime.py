@@ -108,3 +108,52 @@ def test_autotune_times_the_shape_in_use(child):
             stub.stub_time(64, 0.25)
             assert ctx.autotune(2)["force_threads"] == 64
     """)
+
+
+@pytest.fixture(scope="module")
+def ctl_offsets(tmp_path_factory):
+    """Where the control block keeps what the tests set in the kernels'
+    place."""
+    d = tmp_path_factory.mktemp("ctl")
+    (d / "o.cpp").write_text(
+        '#include <cstddef>\n#include <cstdio>\n#include "%s"\n'
+        "int main() {\n"
+        '  printf("%%zu %%zu %%zu", offsetof(Ctl, frozen),\n'
+        "         offsetof(Ctl, cell_over), offsetof(Ctl, export_bad)); }\n"
+        % os.path.join(ROOT, "imd_amd", "csrc", "imdg_internal.h"))
+    subprocess.check_call(
+        ["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+         "-o", str(d / "o"), str(d / "o.cpp")])
+    return subprocess.check_output([str(d / "o")], text=True).split()
+
+
+def test_empty_cells_take_little_memory(child, ctl_offsets):
+    """2,048 atoms in 43 million cells take the 20 B per cell of the cell
+    arrays and no buckets; in a million cells there are buckets (128 B each),
+    until one full cell would make gigabytes of them."""
+    child("""
+        frozen, over, _ = %s
+        def cluster(ncell):
+            s = W.lj_crystal(8)
+            s.box = np.diag([2.8001 * ncell] * 3)
+            return s
+        with G.pair_context(lj(), [cluster(350)]) as ctx:
+            assert ctx.grid() == (350, 350, 350)
+            assert stub.stub_peak() < 20 * 350 ** 3 + (32 << 20)
+        stub.stub_reset_peak()
+        with G.pair_context(lj(), [cluster(100)]) as ctx:
+            assert stub.stub_live() > 148 * 10 ** 6
+            ctx.calc_forces()
+            ctl = stub.stub_pinned_from()
+            for n, least, most in ((40, 276, 300), (1200, 20, 60)):
+                C.c_int.from_address(ctl + over).value = n
+                C.c_int.from_address(ctl + frozen).value = 1
+                ctx.calc_forces()
+                assert C.c_int.from_address(ctl + over).value == 0
+                assert least * 10 ** 6 < stub.stub_live() < most * 10 ** 6, n
+            assert stub.stub_peak() < 500 * 10 ** 6
+        # no room for the buckets: the sort does without
+        stub.stub_limit(60 * 10 ** 6)
+        with G.pair_context(lj(), [cluster(100)]) as ctx:
+            ctx.calc_forces()
+    """ % ("(%s)" % ", ".join(ctl_offsets)))
