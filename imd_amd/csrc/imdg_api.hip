@@ -1418,8 +1418,12 @@ int export_check(imdg_ctx* c) {
   Ctl h;
   int rc = read_ctl(c, &h);
   if (rc) return rc;
-  if (h.export_bad) return fail(c, IMDG_ERR_STATE, "a slot has no atom");
-  return IMDG_OK;
+  if (!h.export_bad) return IMDG_OK;
+  const int zero = 0;  // the next export is judged by its own slots
+  HIPCHK(c, hipMemcpyAsync(&c->d_ctl->export_bad, &zero, sizeof(int),
+                           hipMemcpyHostToDevice, c->stream));
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  return fail(c, IMDG_ERR_STATE, "a slot has no atom");
 }
 
 // Mean time of `reps` launches of one neighbour loop (the density loop, or

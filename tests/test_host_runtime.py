@@ -157,3 +157,22 @@ def test_empty_cells_take_little_memory(child, ctl_offsets):
         with G.pair_context(lj(), [cluster(100)]) as ctx:
             ctx.calc_forces()
     """ % ("(%s)" % ", ".join(ctl_offsets)))
+
+
+def test_a_bad_export_is_reported_once(child, ctl_offsets):
+    """A slot without an atom, met by one export, is that call's error and
+    not the next one's."""
+    child("""
+        bad = %s
+        s = W.eam_crystal(n_cells=6, temp_k=300.0, seed=1)
+        ctx = G.eam_context(eam_tables(), [s])
+        ctx.atoms()
+        C.c_int.from_address(stub.stub_pinned_from() + bad).value = 1
+        try:
+            ctx.atoms()
+        except G.ImdgError as e:
+            assert "no atom" in str(e)
+        else:
+            raise AssertionError("not reported")
+        ctx.atoms()
+    """ % ctl_offsets[2])
