@@ -253,9 +253,11 @@ int dalloc(imdg_ctx* c, void** p, size_t bytes) {
   *p = nullptr;
   if (bytes == 0) bytes = 16;
   hipError_t e = hipMalloc(p, bytes);
-  if (e != hipSuccess)
+  if (e != hipSuccess) {
+    (void)hipGetLastError();  // or the next launch would be told of it
     return fail(c, IMDG_ERR_NOMEM, "hipMalloc(%zu): %s", bytes,
                 hipGetErrorString(e));
+  }
   c->bufs.push_back({*p, bytes});
   return IMDG_OK;
 }

@@ -12,6 +12,7 @@
 #define MAXTHR 2048
 
 static __thread int current = 0;
+static __thread hipError_t last_error = hipSuccess;   /* until it is read */
 
 /* --- what the tests read and set ------------------------------------------ */
 static size_t live = 0, peak = 0, limit = (size_t)1 << 46;
@@ -50,14 +51,17 @@ hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t attr, int dev) {
 const char *hipGetErrorString(hipError_t e) {
   return e == hipErrorOutOfMemory ? "out of memory" : "stub";
 }
-hipError_t hipGetLastError(void) { return hipSuccess; }
+hipError_t hipGetLastError(void) {
+  const hipError_t e = last_error;
+  last_error = hipSuccess;
+  return e;
+}
 
 /* --- memory: 64 bytes in front of each block hold its size ------------------ */
 hipError_t hipMalloc(void **p, size_t n) {
   *p = NULL;
-  if (n > limit || live > limit - n) return hipErrorOutOfMemory;
-  char *b = calloc(1, n + 64);
-  if (!b) return hipErrorOutOfMemory;
+  char *b = n > limit || live > limit - n ? NULL : calloc(1, n + 64);
+  if (!b) return last_error = hipErrorOutOfMemory;
   *(size_t *)b = n;
   live += n;
   if (live > peak) peak = live;
