@@ -41,10 +41,11 @@ template <typename R>
 hipError_t launch_stress(const StepArgs<R>&, const TabDev<R>*, double*,
                          double*, int, hipStream_t);
 template <typename R>
-hipError_t launch_export(const StepArgs<R>&, int* const[2], long,
+hipError_t launch_export(const StepArgs<R>&, int* const[2], long, long, long,
                          const ExportDst&, int, hipStream_t);
 hipError_t launch_unsort(const RepDev*, Ctl*, const int*, int* const[2], long,
-                         const double*, int, double*, int, hipStream_t);
+                         long, long, const double*, int, double*, int,
+                         hipStream_t);
 template <typename R>
 bool head_fits(int);
 template <typename R>
@@ -1403,15 +1404,24 @@ int read_slots(imdg_ctx* c, SlotView& v) {
   return IMDG_OK;
 }
 
-// Room for len doubles of results in input order.
-int reserve_out(imdg_ctx* c, size_t len) {
-  if (c->d_out && len <= c->out_len) return IMDG_OK;
+// Room for results of `per` doubles per atom in input order: *window atoms at
+// a time, all n of them up to IMDG_OUT_BYTES, fewer where the memory is short.
+int reserve_out(imdg_ctx* c, size_t per, size_t n, size_t* window) {
+  const size_t most = IMDG_OUT_BYTES / sizeof(double) / std::max<size_t>(per, 1);
+  size_t m = std::min(n, most);
+  *window = m;
+  if (c->d_out && m * per <= c->out_len) return IMDG_OK;
   dfree(c, c->d_out);
   c->d_out = nullptr;
   c->out_len = 0;
-  int rc = dalloc(c, (void**)&c->d_out, sizeof(double) * len);
-  if (rc) return rc;
-  c->out_len = len;
+  for (;; m = (m + 1) / 2) {
+    int rc = dalloc(c, (void**)&c->d_out, sizeof(double) * m * per);
+    if (!rc) break;
+    if (m <= IMDG_OUT_MIN) return rc;
+    c->err.clear();
+  }
+  c->out_len = m * per;
+  *window = m;
   return IMDG_OK;
 }
 
@@ -2219,13 +2229,17 @@ int imdg_get_stress(imdg_ctx* c, double* per_atom, double* total) {
   }
   if (per_atom) {
     const size_t n = c->natoms_tot;
-    if ((rc = reserve_out(c, 6 * n))) return rc;
-    HIPCHK(c, launch_unsort(c->d_rep, c->d_ctl, c->d_blk_rep, c->d_aid, n,
-                            c->d_stress, 6, c->d_out, c->nblk, c->stream));
-    if ((rc = export_check(c))) return rc;
-    if (n)
-      HIPCHK(c, hipMemcpy(per_atom, c->d_out, sizeof(double) * 6 * n,
-                          hipMemcpyDeviceToHost));
+    size_t window;
+    if ((rc = reserve_out(c, 6, n, &window))) return rc;
+    for (size_t in0 = 0; in0 < n; in0 += window) {
+      const size_t m = std::min(window, n - in0);
+      HIPCHK(c, launch_unsort(c->d_rep, c->d_ctl, c->d_blk_rep, c->d_aid, n,
+                              in0, m, c->d_stress, 6, c->d_out, c->nblk,
+                              c->stream));
+      if ((rc = export_check(c))) return rc;
+      HIPCHK(c, hipMemcpy(per_atom + 6 * in0, c->d_out,
+                          sizeof(double) * 6 * m, hipMemcpyDeviceToHost));
+    }
   }
   return IMDG_OK;
 }
@@ -2258,36 +2272,40 @@ int imdg_get_atoms(imdg_ctx* c, double* x, double* p, double* f, double* epot,
                    double* rho, double* df) {
   if (!c || !c->atoms_set) return IMDG_ERR_ARG;
   hipSetDevice(c->dev);
-  // the wanted arrays one after the other in d_out
+  // a window of the wanted arrays, one after the other in d_out
   const struct {
     double* host;
     size_t comp;
   } want[6] = {{x, 3}, {p, 3}, {f, 3}, {epot, 1}, {rho, 1}, {df, 1}};
   const size_t n = c->natoms_tot;
-  size_t len = 0;
+  size_t per = 0, window;
   for (auto& w : want)
-    if (w.host) len += w.comp * n;
-  int rc = reserve_out(c, len);
+    if (w.host) per += w.comp;
+  int rc = reserve_out(c, per, n, &window);
   if (rc) return rc;
-  double* dev[6];
-  size_t at = 0;
-  for (int k = 0; k < 6; k++) {
-    dev[k] = want[k].host ? c->d_out + at : nullptr;
-    if (want[k].host) at += want[k].comp * n;
+  window = std::max<size_t>(window, 1);
+  for (size_t in0 = 0; in0 == 0 || in0 < n; in0 += window) {
+    const size_t m = std::min(window, n - in0);
+    double* dev[6];
+    size_t at = 0;
+    for (int k = 0; k < 6; k++) {
+      dev[k] = want[k].host ? c->d_out + at : nullptr;
+      if (want[k].host) at += want[k].comp * m;
+    }
+    const ExportDst d = {dev[0], dev[1], dev[2], dev[3], dev[4], dev[5]};
+    if (c->mixed)
+      HIPCHK(c, launch_export<float>(step_args<float>(c), c->d_aid, n, in0, m,
+                                     d, c->nblk, c->stream));
+    else
+      HIPCHK(c, launch_export<double>(step_args<double>(c), c->d_aid, n, in0,
+                                      m, d, c->nblk, c->stream));
+    if ((rc = export_check(c))) return rc;
+    for (int k = 0; k < 6; k++)
+      if (dev[k] && m)
+        HIPCHK(c, hipMemcpy(want[k].host + want[k].comp * in0, dev[k],
+                            sizeof(double) * want[k].comp * m,
+                            hipMemcpyDeviceToHost));
   }
-  const ExportDst d = {dev[0], dev[1], dev[2], dev[3], dev[4], dev[5]};
-  if (c->mixed)
-    HIPCHK(c, launch_export<float>(step_args<float>(c), c->d_aid, n, d,
-                                   c->nblk, c->stream));
-  else
-    HIPCHK(c, launch_export<double>(step_args<double>(c), c->d_aid, n, d,
-                                    c->nblk, c->stream));
-  if ((rc = export_check(c))) return rc;
-  for (int k = 0; k < 6; k++)
-    if (dev[k] && n)
-      HIPCHK(c, hipMemcpy(want[k].host, dev[k],
-                          sizeof(double) * want[k].comp * n,
-                          hipMemcpyDeviceToHost));
   return IMDG_OK;
 }
 

@@ -120,6 +120,10 @@
 // launch of their own; 500,000 atoms 116.3 and 115.0, 2,048,000 atoms 502 and
 // 484.
 #define IMDG_SHARE_BLOCKS 2560
+// Device memory that a context keeps for its downloads: larger ones go out
+// in windows of this size (2.8 million atoms with every array).
+#define IMDG_OUT_BYTES (256l << 20)
+#define IMDG_OUT_MIN 4096    // fewest atoms of a window, when memory is short
 #define IMDG_BUCKET_MIN 32   // smallest bucket (atoms of a cell)
 // The buckets take memory by the cell, and one full cell enlarges them all.
 // Beyond this many bytes, and 128 B per slot (as much as positions and
@@ -350,8 +354,8 @@ struct StepArgs {
   int thr_den, thr_frc;   // threads per block of the density / force loops
 };
 
-// Destination of the export kernel: the caller's arrays on the device, in
-// input order (NULL: not wanted).
+// Destination of the export kernel: a window of the caller's arrays on the
+// device, in input order (NULL: not wanted).
 struct ExportDst {
   double *x, *p, *f, *epot, *rho, *df;
 };

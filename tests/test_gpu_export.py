@@ -77,3 +77,31 @@ def test_stress_in_input_order(precision):
     want = np.stack([s.p[:, a] * s.p[:, b] / s.mass for a, b in
                      ((0, 0), (1, 1), (2, 2), (1, 2), (2, 0), (0, 1))], 1)
     assert np.array_equal(per, want)
+
+
+def test_windows_of_a_large_download():
+    """5.8 million atoms: all arrays together go out in three windows, the
+    stress tensor in two, an array alone in one; the bytes are the same, and
+    free particles have p p^T / m."""
+    s = W.fcc_system((113, 113, 113), 3.615, [W.MASS_CU], W.kT(300.0), 9)
+    assert s.n * 12 * 8 > 2 * (256 << 20) and s.n * 6 * 8 > 256 << 20
+    flat = W.table_from_functions([lambda r: 0.0 * r + 1.0], 1.0, 25.0, 500)
+    ctx = G.Context(precision=G.MIXED, ntypes=1, timestep=W.FS,
+                    nbl_margin=0.4)
+    with ctx:
+        ctx.set_tables(G.TableArrays.from_format2(flat))
+        ctx.set_systems([s])
+        ctx.set_stress(True)
+        ctx.run(1)
+        full = ctx.atoms()
+        assert np.array_equal(full["p"], s.p)
+        for q, k in enumerate(("x", "p", "f", "epot", "rho", "df")):
+            one = np.full_like(full[k], 7.0)
+            ptr = [None] * 6
+            ptr[q] = one.ctypes.data_as(C.POINTER(C.c_double))
+            assert G.lib().imdg_get_atoms(ctx._h, *ptr) == G.OK
+            assert np.array_equal(one, full[k]), k
+        per, _ = ctx.stress()
+    want = np.stack([s.p[:, a] * s.p[:, b] / s.mass for a, b in
+                     ((0, 0), (1, 1), (2, 2), (1, 2), (2, 0), (0, 1))], 1)
+    assert np.array_equal(per, want)

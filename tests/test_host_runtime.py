@@ -176,3 +176,34 @@ def test_a_bad_export_is_reported_once(child, ctl_offsets):
             raise AssertionError("not reported")
         ctx.atoms()
     """ % ctl_offsets[2])
+
+
+def test_downloads_in_bounded_memory(child):
+    """What a context keeps for its downloads is bounded (256 MiB), and a
+    download needs no more than the memory that is left."""
+    child("""
+        s = W.eam_crystal(n_cells=92, temp_k=0.0, seed=1)   # 3.1 million
+        ctx = G.eam_context(eam_tables(), [s])
+        ctx.set_stress(True)
+        ctx.run(1, sync=False)
+        before = stub.stub_live()
+        ctx.atoms()
+        assert before < stub.stub_live() <= before + (256 << 20)
+        ctx.stress()
+        assert stub.stub_live() <= before + (256 << 20)
+        ctx.deallocate_nblist()
+        ctx.set_systems([s])
+        ctx.run(1, sync=False)                   # the stress arrays
+        before = stub.stub_live()
+        stub.stub_limit(before + (3 << 20))
+        ctx.atoms()
+        ctx.stress()
+        assert stub.stub_live() > before + (1 << 20)
+        stub.stub_limit(before)
+        try:
+            ctx.atoms()
+        except G.ImdgError as e:
+            assert "(%d)" % G.ERR_NOMEM in str(e)
+        else:
+            raise AssertionError("no memory at all")
+    """)
