@@ -107,6 +107,12 @@
 // (about 1 us per 1024 cells and rebuild) and the scan's launch is left out
 // (1.7 us per step, one rebuild in 15 to 20 steps).
 #define IMDG_SCAN_FOLD 8192
+// ... of up to this many replicas: it takes them one after the other (about
+// 3 us each when all rebuild, and a read each when none does), the launch side
+// by side.  500-atom replicas at 1200 K, folded and not: 8 of them 37.2 us per
+// step and 40.3, 16 51.2 and 52.1, 24 61.8 and 61.0, 64 90.2 and 76.9, 300
+// 213.9 and 124.0; make_nblist of 300 1,145 us and 203.
+#define IMDG_SCAN_FOLD_REPS 20
 // Up to this many slots and cells (one replica) a step begins with a single
 // block that ends the step before and sorts, instead of three launches.
 #define IMDG_HEAD_SLOTS 7168

@@ -1,0 +1,51 @@
+"""Batches of replicas on both sides of the lines by which the rebuild chain
+is chosen: the scan of the cell counts in the binning's last block or in its
+own launch, by the number of replicas."""
+import numpy as np
+import pytest
+
+from imd_amd import imdg as G
+from imd_amd import workloads as W
+
+from helpers import (canon_pairs_gpu, canon_pairs_oracle, eam_tables,
+                     oracle_eam, rel_rms)
+from test_gpu_tuning import TOL
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nrep", [20, 21])
+def test_scan_by_number_of_replicas(nrep):
+    """Small replicas of different sizes (27 to 80 cells): the pairs and
+    forces of three of them are the oracle's, and a run of the batch rebuilds
+    them as each does alone."""
+    eam = eam_tables()
+    systems = [W.fcc_system((5 + r % 3, 5 + r % 2, 5), 3.615, eam.masses,
+                            W.kT(300.0 + 60.0 * r), 30 + r, displace=0.03)
+               for r in range(nrep)]
+    with G.eam_context(eam, systems, precision=G.FP64) as gpu:
+        gpu.calc_forces()
+        pairs, a = gpu.pairs(), gpu.atoms()
+        at = 0
+        for r, s in enumerate(systems):
+            if r in (0, nrep // 2, nrep - 1):
+                orc = oracle_eam(s, eam, nbl_margin=0.4, timestep=W.FS)
+                orc.calc_forces()
+                assert canon_pairs_gpu(pairs, r) == \
+                    canon_pairs_oracle(orc.pairs())
+                assert rel_rms(a["f"][at:at + s.n],
+                               orc.atoms()["f"]) <= TOL[G.FP64][0]
+            at += s.n
+    with G.eam_context(eam, systems, precision=G.MIXED) as gpu:
+        gpu.set_tuning(2, 512, 2, 512)
+        gpu.run(60)
+        both, th = gpu.atoms(), gpu.thermo_history(0, 60)
+    at = sum(s.n for s in systems[:-1])
+    with G.eam_context(eam, systems[-1:], precision=G.MIXED) as one:
+        one.set_tuning(2, 512, 2, 512)
+        one.run(60)
+        alone, t1 = one.atoms(), one.thermo_history(0, 60)
+    for k, v in alone.items():
+        assert np.array_equal(both[k][at:], v), k
+    assert np.array_equal(th[:, -1, 6], t1[:, 0, 6])
+    assert t1[1:, 0, 6].sum() > 0

@@ -207,3 +207,18 @@ def test_downloads_in_bounded_memory(child):
         else:
             raise AssertionError("no memory at all")
     """)
+
+
+def test_batches_scan_their_cells_side_by_side(child):
+    """The one launch of 1,024 threads in a step of small blocks is the scan
+    of the cells: left out for a few small replicas, there for many."""
+    child("""
+        s = W.eam_crystal(n_cells=5, temp_k=300.0, seed=1)   # 27 cells each
+        for nrep, per_step in ((2, 0), (20, 0), (21, 1), (64, 1)):
+            with G.eam_context(eam_tables(), [s] * nrep) as ctx:
+                ctx.set_tuning(4, 512, 4, 512)
+                ctx.run(1, sync=False)
+                stub.stub_reset_launches()
+                ctx.run(10, sync=False)
+                assert stub.stub_launches(1024) == 10 * per_step
+    """)
