@@ -7,9 +7,9 @@
 // the host.  Each such idle launch costs the device about 1.7 us and the
 // host 2.7 us, which is what a small system's step consists of, so the chain
 // has as few as its data dependences allow: bin (with the scan of the cell
-// counts, for up to IMDG_SCAN_FOLD cells of a few replicas), sort, list (with
-// its blocks' tiles, up to IMDG_SHARE_WORK); what ends it (list_done) runs in
-// the step's next kernel.
+// counts, for up to IMDG_SCAN_FOLD cells), sort, list (with its blocks' tiles,
+// for up to IMDG_SHARE_BLOCKS blocks); what ends it
+// (list_done) runs in the step's next kernel.
 //
 // Reference semantics (paths relative to the reference root):
 //   binning / wrap     src/imd_fix_cells_3d.c:36-201, src/imd_main_3d.c:1972-2065,
@@ -1109,18 +1109,15 @@ __device__ __forceinline__ int list_shared(
   return run;
 }
 
-// The list of systems whose blocks do not fill the chip (IMDG_SHARE_WORK; and
-// of batches of replicas, of which few rebuild in one step): a block per
-// 64-slot chunk, LIST_LANES lanes per atom.  k_list lasts as long as its
-// longest lane's 370 candidates in a row, which bounds it while the chip is
-// not full: 864 atoms 60 us, here 32; of 64 replicas the few that rebuild in a
-// step 78 us, here 44 (a step of theirs 242 us, 201; LJ crystal of 4,000 atoms
-// in FP64 20.4, 17.2).  Eight lanes are no faster for those and slower from
-// 100,000 atoms.  On a full chip the lanes' entry stores, 2 B each instead of
-// 8, and the drain of the masks cost more than the screens they save: LJ of
-// 219,000 atoms 148 us as a crystal, where the wavefront's 16 atoms write the
-// same places of their lists, and 256 as a liquid, where every entry is a
-// request of its own; k_list 147 and 153.
+// The list of systems whose blocks do not fill the chip (and of batches of
+// replicas, of which few rebuild in one step): a block per 64-slot chunk,
+// LIST_LANES lanes per atom.  k_list lasts as long as its longest lane's 370
+// candidates in a row, which bounds it while the chip is not full: 864 atoms
+// 60 us, here 32; of 64 replicas the few that rebuild in a step 78 us, here
+// 44 (a step of theirs 242 us, 201; LJ crystal of 4,000 atoms in FP64 20.4,
+// 17.2).  Eight lanes are no faster for those and slower from 100,000 atoms.
+// On a full chip the lanes' entry stores, 2 B each instead of 8, and the
+// drain of the masks cost more than the screens they save.
 template <bool MIXED>
 __global__ void __launch_bounds__(IMDG_CHUNK* LIST_LANES)
     k_list_shared(BuildArgs a) {
@@ -1278,7 +1275,7 @@ void launch_sort(const BuildArgs& b, int grid, hipStream_t st) {
 // The list, after the sort.  done: end the rebuild here (otherwise the
 // density loop of the step does).
 void launch_list(const BuildArgs& b, bool done, hipStream_t st) {
-  if (!b.list_shared)
+  if (b.tiles)
     hipLaunchKernelGGL(k_tile, dim3((b.nblk + 3) / 4), dim3(256), 0, st, b);
   const size_t tile_lds = std::max((size_t)(b.tile_cap + 4) * sizeof(float3),
                                    sizeof(TileLds));

@@ -120,26 +120,12 @@
 // Pair-only systems of up to this many blocks end a rebuild in the list's
 // last block (a release fence in each); larger ones in a launch of its own.
 #define IMDG_LIST_ENDS 128
-// Up to this many blocks x atoms per cell (which is what the candidates to
-// screen go with) the list is built with four lanes per atom, a block per
-// chunk that builds its own tile; beyond it with one and the tiles from a
-// launch of their own.  Four lanes are faster while the chip is not full; on
-// a full one the entries' stores, 2 B each, cost more than the lanes save, in
-// a liquid above all, where no two atoms' lists fill alike.  us per step,
-// four lanes and one: EAM crystal of 256,000 atoms (2,000 blocks, 15 a cell)
-// 73.9 and 74.9, hot and of 318,000 (2,485) 100.4 and 101.6, of 500,000 116.3
-// and 115.0; LJ liquid (24 a cell) of 108,000 atoms (844 blocks) 44.1 and
-// 47.5, of 219,000 (1,715) 67.1 and 63.1, of 318,000 97.0 and 89.8.
-#define IMDG_SHARE_WORK 37000
-// The line is each replica's own (of several, few rebuild in one step) but
-// when all of a batch rebuild at once, which the host knows in make_nblist
-// and for the first list: then one lane beyond it in all, in mixed precision
-// or with cells of at least this many atoms.  make_nblist, four lanes and
-// one: mixed EAM 30 x 32,000 atoms 607 us and 561, 4 x 318,000 771 and 666,
-// LJ liquids 300 x 2,048 835 and 516; FP64 EAM 100 x 4,000 (19 a cell) 307
-// and 427, LJ liquids 300 x 2,916 (46 a cell) 3,472 and 1,481, LJ crystals 30
-// x 32,000 (24 a cell) 766 and 895, their liquids 1,211 and 987.
-#define IMDG_SHARE_DENSE 20
+// Up to this many blocks in the largest replica the list is built with four
+// lanes per atom, a block per chunk that builds its own tile: 256,000 atoms
+// (2,000 blocks) 73.9 us per step, 74.9 with one lane and the tiles from a
+// launch of their own; 500,000 atoms 116.3 and 115.0, 2,048,000 atoms 502 and
+// 484.
+#define IMDG_SHARE_BLOCKS 2560
 // Device memory that a context keeps for its downloads: larger ones go out
 // in windows of this size (2.8 million atoms with every array).
 #define IMDG_OUT_BYTES (256l << 20)

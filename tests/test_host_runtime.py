@@ -222,37 +222,3 @@ def test_batches_scan_their_cells_side_by_side(child):
                 ctx.run(10, sync=False)
                 assert stub.stub_launches(1024) == 10 * per_step
     """)
-
-
-def test_list_kernel_of_full_rebuilds(child):
-    """Lanes per atom of the list build, told by its blocks (128 threads with
-    one lane, as the binning's, 256 with four): by blocks x atoms per cell of
-    the largest replica, and of all of them where all rebuild at once."""
-    child("""
-        eam = eam_tables()
-        def crystal(n):
-            return W.eam_crystal(n_cells=n, temp_k=0.0, seed=1)
-        def liquid(n):
-            return W.fcc_system((n, n, n), 1.5496, [1.0], 0.0, 1)
-        cases = [  # systems, pair only, precision; lanes: all rebuild, some do
-            ([crystal(42)], 0, G.MIXED, 4, 4),
-            ([crystal(44)], 0, G.MIXED, 1, 1),
-            ([crystal(20)] * 8, 0, G.MIXED, 4, 4),    # 250 x 14.5 each
-            ([crystal(20)] * 11, 0, G.MIXED, 1, 4),
-            ([crystal(20)] * 11, 0, G.FP64, 4, 4),    # fewer than 20 a cell
-            ([liquid(10)] * 34, 1, G.FP64, 4, 4),     # 32 x 32 each
-            ([liquid(10)] * 39, 1, G.FP64, 1, 4),
-        ]
-        for systems, lj_only, prec, lanes_all, lanes_step in cases:
-            ctx = G.pair_context(lj(), systems, precision=prec) if lj_only \\
-                else G.eam_context(eam, systems, precision=prec)
-            with ctx:
-                ctx.set_tuning(2, 512, 2, 512)
-                for call, lanes in ((ctx.make_nblist, lanes_all),
-                                    (lambda: ctx.run(1, sync=False),
-                                     lanes_step)):
-                    stub.stub_reset_launches()
-                    call()
-                    got = 1 if stub.stub_launches(128) == 2 else 4
-                    assert got == lanes, (len(systems), systems[0].n, prec)
-    """)
