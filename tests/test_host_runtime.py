@@ -112,19 +112,29 @@ def test_autotune_times_the_shape_in_use(child):
 
 @pytest.fixture(scope="module")
 def ctl_offsets(tmp_path_factory):
-    """Where the control block keeps what the tests set in the kernels'
-    place."""
+    """Where the control block keeps what the tests look for or set in the
+    kernels' place."""
     d = tmp_path_factory.mktemp("ctl")
+    names = ("frozen", "cell_over", "export_bad", "exact_pairs", "steps_done",
+             "done")
     (d / "o.cpp").write_text(
         '#include <cstddef>\n#include <cstdio>\n#include "%s"\n'
-        "int main() {\n"
-        '  printf("%%zu %%zu %%zu", offsetof(Ctl, frozen),\n'
-        "         offsetof(Ctl, cell_over), offsetof(Ctl, export_bad)); }\n"
-        % os.path.join(ROOT, "imd_amd", "csrc", "imdg_internal.h"))
+        "int main() {\n%s\n}\n"
+        % (os.path.join(ROOT, "imd_amd", "csrc", "imdg_internal.h"),
+           "\n".join('  printf("%%zu ", offsetof(Ctl, %s));' % n
+                     for n in names)))
     subprocess.check_call(
         ["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
          "-o", str(d / "o"), str(d / "o.cpp")])
-    return subprocess.check_output([str(d / "o")], text=True).split()
+    out = subprocess.check_output([str(d / "o")], text=True).split()
+    return dict(zip(names, map(int, out)))
+
+
+def test_contended_counter_has_its_own_line(ctl_offsets):
+    """The counter that the whole list build adds to shares no 128 B line
+    with what its blocks read."""
+    line = {k: v // 128 for k, v in ctl_offsets.items()}
+    assert list(line.values()).count(line["exact_pairs"]) == 1
 
 
 def test_empty_cells_take_little_memory(child, ctl_offsets):
@@ -132,7 +142,7 @@ def test_empty_cells_take_little_memory(child, ctl_offsets):
     arrays and no buckets; in a million cells there are buckets (128 B each),
     until one full cell would make gigabytes of them."""
     child("""
-        frozen, over, _ = %s
+        frozen, over = %s
         def cluster(ncell):
             s = W.lj_crystal(8)
             s.box = np.diag([2.8001 * ncell] * 3)
@@ -156,7 +166,7 @@ def test_empty_cells_take_little_memory(child, ctl_offsets):
         stub.stub_limit(60 * 10 ** 6)
         with G.pair_context(lj(), [cluster(100)]) as ctx:
             ctx.calc_forces()
-    """ % ("(%s)" % ", ".join(ctl_offsets)))
+    """ % str((ctl_offsets["frozen"], ctl_offsets["cell_over"])))
 
 
 def test_a_bad_export_is_reported_once(child, ctl_offsets):
@@ -175,7 +185,7 @@ def test_a_bad_export_is_reported_once(child, ctl_offsets):
         else:
             raise AssertionError("not reported")
         ctx.atoms()
-    """ % ctl_offsets[2])
+    """ % ctl_offsets["export_bad"])
 
 
 def test_downloads_in_bounded_memory(child):
