@@ -54,8 +54,7 @@ void launch_sort(const BuildArgs&, int, hipStream_t);
 void launch_list(const BuildArgs&, bool, hipStream_t);
 const char* noalloc_message();
 void launch_check(const RepDev*, RepState*, Ctl*, const int*, const double4*,
-                  const double4*, const double4*, double*, int, int, int*,
-                  hipStream_t);
+                  const double4*, const double4*, int, int, int*, hipStream_t);
 }  // namespace imdg
 
 using namespace imdg;
@@ -143,7 +142,7 @@ struct imdg_ctx {
   void *d_reca = nullptr, *d_recb = nullptr;
   void *d_rho = nullptr, *d_epot = nullptr, *d_frc = nullptr;
   void *d_eeP = nullptr, *d_eedm = nullptr;  // EEAM: P and 2E'(P) per slot
-  double *d_partA = nullptr, *d_partB = nullptr, *d_maxd = nullptr;
+  double *d_partA = nullptr, *d_partB = nullptr;
   ThermoRec* d_ring = nullptr;
   void* d_tabs = nullptr;        // TabDev<R>[4]
   void* d_knots = nullptr;       // knots of all tables
@@ -1880,7 +1879,6 @@ int imdg_set_atoms(imdg_ctx* c, int nrep, const imdg_replica* reps,
     ALLOC(c->d_eedm, rs * ns);
   }
   ALLOC(c->d_frc, rs * 4 * ns);
-  ALLOC(c->d_maxd, sizeof(double) * c->nblk);
   ALLOC(c->d_ring, sizeof(ThermoRec) * IMDG_RING * nrep);
   if ((rc = c->mixed ? upload_tables<float>(c) : upload_tables<double>(c)))
     return rc;
@@ -2066,7 +2064,7 @@ int imdg_check_nblist(imdg_ctx* c, int* invalid) {
   int rc = ensure_ready(c);
   if (rc) return rc;
   launch_check(c->d_rep, c->d_rst, c->d_ctl, c->d_blk_rep, c->d_pos[0],
-               c->d_pos[1], c->d_xnbl, c->d_maxd, c->nrep, c->nblk,
+               c->d_pos[1], c->d_xnbl, c->nrep, c->nblk,
                &c->h_pin->invalid, c->stream);
   HIPCHK(c, hipGetLastError());
   HIPCHK(c, hipStreamSynchronize(c->stream));

@@ -1200,57 +1200,45 @@ __global__ void __launch_bounds__(1024) k_list_done(ListEnd e) {
   list_done(e, red);
 }
 
-// check_nblist alone: max displacement^2 per block of IMDG_BLOCK slots; the
-// last block to finish takes each replica's maximum, marks the replicas
-// beyond half the skin and tells the host (*invalid, host memory) whether
-// any replica is marked.
+// check_nblist alone: the largest displacement^2 of each block of IMDG_BLOCK
+// slots, and its replica marked where that is beyond half the skin (every
+// such block stores the same value).
 __global__ void __launch_bounds__(IMDG_BLOCK)
-    k_check(const RepDev* rep, RepState* rst, Ctl* ctl, const int* blk_rep,
-            const double4* pos0, const double4* pos1, const double4* xnbl,
-            double* maxd, int nrep, int* invalid) {
+    k_check(const RepDev* rep, RepState* rst, const Ctl* ctl,
+            const int* blk_rep, const double4* pos0, const double4* pos1,
+            const double4* xnbl) {
   __shared__ double red[IMDG_NWAVE];
-  __shared__ int is_last, any;
+  if (ctl->frozen) return;
   int lb = blockIdx.x;
-  if (!ctl->frozen) {
-    int r = blk_rep[lb];
-    const RepDev& Rp = rep[r];
-    int i = lb * IMDG_BLOCK + threadIdx.x;
-    const double4* pos = ctl->pos_cur ? pos1 : pos0;
-    double v = 0.0;
-    if ((i - Rp.atom_off) < Rp.natoms) v = disp2(pos[i], xnbl[i]);
-    v = wave_max(v);
-    if ((threadIdx.x % IMDG_WAVE) == 0) red[threadIdx.x / IMDG_WAVE] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      double m = red[0];
-      for (int k = 1; k < IMDG_NWAVE; k++) m = fmax(m, red[k]);
-      maxd[lb] = m;
-    }
-  }
-  if (threadIdx.x == 0) {
-    __threadfence();
-    unsigned d = atomicAdd(&ctl->done[DC_CHECK], 1u);
-    is_last = (d == gridDim.x - 1);
-    if (is_last) ctl->done[DC_CHECK] = 0;
-    any = 0;
-  }
+  int r = blk_rep[lb];
+  const RepDev& Rp = rep[r];
+  int i = lb * IMDG_BLOCK + threadIdx.x;
+  const double4* pos = ctl->pos_cur ? pos1 : pos0;
+  double v = 0.0;
+  if ((i - Rp.atom_off) < Rp.natoms) v = disp2(pos[i], xnbl[i]);
+  v = wave_max(v);
+  if ((threadIdx.x % IMDG_WAVE) == 0) red[threadIdx.x / IMDG_WAVE] = v;
   __syncthreads();
-  if (!is_last) return;
-  __threadfence();
-  // one wavefront per replica
-  const int lane = threadIdx.x % IMDG_WAVE;
-  for (int r = threadIdx.x / IMDG_WAVE; r < nrep; r += IMDG_NWAVE) {
-    const RepDev& Rp = rep[r];
-    double m = 0.0;
-    for (int b = lane; b < Rp.nblk; b += IMDG_WAVE)
-      m = fmax(m, __hip_atomic_load(&maxd[Rp.blk_off + b], __ATOMIC_RELAXED,
-                                    __HIP_MEMORY_SCOPE_AGENT));
-    m = wave_max(m);
-    if (lane == 0) {
-      if (m > Rp.skin2) rst[r].need_rebuild = 1;
-      if (rst[r].need_rebuild) atomicOr(&any, 1);
-    }
+  if (threadIdx.x == 0) {
+    double m = red[0];
+    for (int k = 1; k < IMDG_NWAVE; k++) m = fmax(m, red[k]);
+    if (m > Rp.skin2) rst[r].need_rebuild = 1;
   }
+}
+
+// Whether any replica is marked, also for the host (*invalid, host memory).
+// A launch of its own, one block: ended by k_check's last block the call took
+// 15 to 20 us up to 256 blocks, 61 at 2,000 and 518 at 16,000 (a fence and a
+// count in every block); so 15, 15 and 32.
+__global__ void __launch_bounds__(1024)
+    k_check_end(const RepState* rst, Ctl* ctl, int nrep, int* invalid) {
+  __shared__ int any;
+  if (threadIdx.x == 0) any = 0;
+  __syncthreads();
+  int mine = 0;
+  for (int r = threadIdx.x; r < nrep; r += blockDim.x)
+    mine |= rst[r].need_rebuild;
+  if (mine) atomicOr(&any, 1);
   __syncthreads();
   if (threadIdx.x == 0) {
     ctl->any_rebuild = any;
@@ -1299,10 +1287,12 @@ void launch_list(const BuildArgs& b, bool done, hipStream_t st) {
 
 void launch_check(const RepDev* rep, RepState* rst, Ctl* ctl,
                   const int* blk_rep, const double4* pos0,
-                  const double4* pos1, const double4* xnbl, double* maxd,
-                  int nrep, int nblk, int* invalid, hipStream_t st) {
+                  const double4* pos1, const double4* xnbl, int nrep, int nblk,
+                  int* invalid, hipStream_t st) {
   hipLaunchKernelGGL(k_check, dim3(nblk), dim3(IMDG_BLOCK), 0, st, rep, rst,
-                     ctl, blk_rep, pos0, pos1, xnbl, maxd, nrep, invalid);
+                     ctl, blk_rep, pos0, pos1, xnbl);
+  hipLaunchKernelGGL(k_check_end, dim3(1), dim3(1024), 0, st, rst, ctl, nrep,
+                     invalid);
 }
 
 }  // namespace imdg

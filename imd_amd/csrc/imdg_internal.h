@@ -99,8 +99,7 @@
 #define DC_SCAN 1
 #define DC_FINBLK 2   // finalising blocks of a step done (several replicas)
 #define DC_LIST 3
-#define DC_CHECK 4
-#define DC_N 5
+#define DC_N 4
 
 #define IMDG_SCAN_TILE 1024  // cells per block of the cell-count scan
 // Up to this many cells the last block of the binning scans their counts

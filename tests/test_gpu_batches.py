@@ -49,3 +49,34 @@ def test_scan_by_number_of_replicas(nrep):
         assert np.array_equal(both[k][at:], v), k
     assert np.array_equal(th[:, -1, 6], t1[:, 0, 6])
     assert t1[1:, 0, 6].sum() > 0
+
+
+@pytest.mark.parametrize("cells,nrep", [(22, 1), (14, 4), (5, 70),
+                                        (5, 1100)])
+def test_skin_test_of_many_blocks(cells, nrep):
+    """imdg_check_nblist of large replicas and of many: the loop of the three
+    entry points rebuilds in the steps in which the fused run does, with the
+    same bits, and the call's answer is the record's decision."""
+    eam = eam_tables()
+    systems = [W.eam_crystal(n_cells=cells, temp_k=200.0 + 1300.0 * r / nrep,
+                             seed=70 + r) for r in range(1, nrep + 1)]
+    got = []
+    for fused in (True, False):
+        with G.eam_context(eam, systems, precision=G.FP64) as gpu:
+            assert gpu.info()["nslots"] > 256 * 128
+            gpu.set_tuning(2, 512, 2, 512)
+            answers = []
+            if fused:
+                gpu.run(40)
+            else:
+                for _ in range(40):
+                    gpu.calc_forces()
+                    gpu.move_atoms()
+                    answers.append(gpu.check_nblist())
+            got.append((gpu.atoms(), gpu.thermo_history(0, 40)))
+    skin2 = (0.5 * 0.4) ** 2
+    assert answers == (got[1][1][:, :, 5] > skin2).any(axis=1).tolist()
+    assert any(answers)
+    assert np.array_equal(got[0][1][..., 5:], got[1][1][..., 5:])
+    for k in ("x", "p"):
+        assert np.array_equal(got[0][0][k], got[1][0][k]), k

@@ -232,3 +232,18 @@ def test_batches_scan_their_cells_side_by_side(child):
                 ctx.run(10, sync=False)
                 assert stub.stub_launches(1024) == 10 * per_step
     """)
+
+
+def test_check_ends_in_its_own_launch(child):
+    """The skin test of imdg_check_nblist is two launches, the second one
+    block of 1,024 threads: no fence and no count in the blocks of the
+    first."""
+    child("""
+        for cells, nrep in ((6, 1), (21, 1), (5, 65)):
+            s = W.eam_crystal(n_cells=cells, temp_k=0.0, seed=1)
+            with G.eam_context(eam_tables(), [s] * nrep) as ctx:
+                stub.stub_reset_launches()
+                ctx.check_nblist()
+                assert stub.stub_launches(128) == 1
+                assert stub.stub_launches(1024) == 1, (cells, nrep)
+    """)
