@@ -1084,8 +1084,9 @@ BuildArgs build_args(imdg_ctx* c) {
   b.atype = c->d_atype;
   b.bucket = c->d_bucket;
   b.bucket_cap = c->bucket_cap;
-  b.scan_in_bin =
-      c->ncells <= IMDG_SCAN_FOLD && c->nrep <= IMDG_SCAN_FOLD_REPS ? 1 : 0;
+  b.scan_in_bin = c->ncells <= IMDG_SCAN_FOLD &&
+                  c->nrep <= IMDG_SCAN_FOLD_REPS &&
+                  c->nblk <= IMDG_SCAN_FOLD_BLOCKS;
   b.cell_cnt = c->d_cell_cnt;
   b.cell_beg = c->d_cell_beg;
   b.cell_num = c->d_cell_num;

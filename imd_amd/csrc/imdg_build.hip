@@ -7,9 +7,9 @@
 // the host.  Each such idle launch costs the device about 1.7 us and the
 // host 2.7 us, which is what a small system's step consists of, so the chain
 // has as few as its data dependences allow: bin (with the scan of the cell
-// counts, for up to IMDG_SCAN_FOLD cells), sort, list (with its blocks' tiles,
-// for up to IMDG_SHARE_BLOCKS blocks); what ends it
-// (list_done) runs in the step's next kernel.
+// counts, for up to IMDG_SCAN_FOLD cells, a few replicas and blocks), sort,
+// list (with its blocks' tiles, for up to IMDG_SHARE_BLOCKS blocks); what ends
+// it (list_done) runs in the step's next kernel.
 //
 // Reference semantics (paths relative to the reference root):
 //   binning / wrap     src/imd_fix_cells_3d.c:36-201, src/imd_main_3d.c:1972-2065,

@@ -112,6 +112,14 @@
 // step and 40.3, 16 51.2 and 52.1, 24 61.8 and 61.0, 64 90.2 and 76.9, 300
 // 213.9 and 124.0; make_nblist of 300 1,145 us and 203.
 #define IMDG_SCAN_FOLD_REPS 20
+// ... and of up to this many blocks: their fences and counts take 45 ns a
+// block one after the other, 50 us of a rebuild's binning at 1,080 (20 LJ
+// replicas of 6,900 atoms 91.0 us per step folded and 79.4 not, their
+// make_nblist 313 and 199; 16 EAM replicas of 6,900 79.8 and 70.4, 214 and
+// 142; an LJ liquid of 187,000 atoms, 1,458 blocks, 61.9 us and 56.1; EAM of
+// 108,000, 844 blocks, 51.4 and 50.2; two LJ replicas of 32,000, 500 blocks,
+// 39.7 and 41.0).
+#define IMDG_SCAN_FOLD_BLOCKS 704
 // Up to this many slots and cells (one replica) a step begins with a single
 // block that ends the step before and sorts, instead of three launches.
 #define IMDG_HEAD_SLOTS 7168

@@ -80,3 +80,31 @@ def test_skin_test_of_many_blocks(cells, nrep):
     assert np.array_equal(got[0][1][..., 5:], got[1][1][..., 5:])
     for k in ("x", "p"):
         assert np.array_equal(got[0][0][k], got[1][0][k]), k
+
+
+# 686 and 763 blocks, at most 8,192 cells: the scan folded and not
+@pytest.mark.parametrize("cells,nrep", [(28, 1), (29, 1), (20, 2), (20, 3)])
+def test_scan_by_number_of_blocks(cells, nrep, monkeypatch):
+    """The sort is the same whichever launch scans the cells: one that takes
+    no buckets and one that does give the bits of each other through
+    rebuilds, and a static evaluation the oracle's pairs."""
+    eam = eam_tables()
+    systems = [W.eam_crystal(n_cells=cells, temp_k=1400.0, seed=40 + r)
+               for r in range(nrep)]
+    got = []
+    for limit in (None, "0"):
+        if limit:
+            monkeypatch.setenv("IMDG_BUCKET_LIMIT", limit)
+        with G.eam_context(eam, systems, precision=G.MIXED) as gpu:
+            gpu.run(40)
+            got.append((gpu.atoms(), gpu.thermo_history(0, 40)))
+    for k, v in got[0][0].items():
+        assert np.array_equal(v, got[1][0][k]), k
+    assert np.array_equal(got[0][1], got[1][1])
+    assert got[0][1][1:, 0, 6].sum() > 0
+    with G.eam_context(eam, systems, precision=G.FP64) as gpu:
+        gpu.make_nblist()
+        pairs = gpu.pairs()
+    orc = oracle_eam(systems[-1], eam, nbl_margin=0.4, timestep=W.FS)
+    orc.calc_forces()
+    assert canon_pairs_gpu(pairs, nrep - 1) == canon_pairs_oracle(orc.pairs())

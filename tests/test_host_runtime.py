@@ -219,12 +219,15 @@ def test_downloads_in_bounded_memory(child):
     """)
 
 
-def test_batches_scan_their_cells_side_by_side(child):
+def test_scan_of_the_cells_in_its_own_launch(child):
     """The one launch of 1,024 threads in a step of small blocks is the scan
-    of the cells: left out for a few small replicas, there for many."""
+    of the cells: left out for a few small replicas, there for many and for
+    large ones."""
     child("""
-        s = W.eam_crystal(n_cells=5, temp_k=300.0, seed=1)   # 27 cells each
-        for nrep, per_step in ((2, 0), (20, 0), (21, 1), (64, 1)):
+        for cells, nrep, per_step in ((5, 2, 0), (5, 20, 0), (5, 21, 1),
+                                      (5, 64, 1), (28, 1, 0), (29, 1, 1),
+                                      (20, 2, 0), (20, 3, 1)):
+            s = W.eam_crystal(n_cells=cells, temp_k=300.0, seed=1)
             with G.eam_context(eam_tables(), [s] * nrep) as ctx:
                 ctx.set_tuning(4, 512, 4, 512)
                 ctx.run(1, sync=False)
