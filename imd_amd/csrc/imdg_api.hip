@@ -129,8 +129,11 @@ struct imdg_ctx {
   int *d_acell = nullptr, *d_bucket = nullptr;
   int bucket_cap = 0;        // places per cell; 0: no buckets
   long bucket_bytes = -1;    // most they may take; -1: by the system
-  bool list_shared = false;  // several lanes per atom build its list
-  Tile* d_tiles = nullptr;   // (then without tiles in memory)
+  bool list_shared = false;  // several lanes per atom build its list,
+  bool one_for_all = false;  // but one where all replicas rebuild at once
+  bool all_flagged = false;  // the next rebuild is one of all replicas
+  bool shared_now = false;   // what the last rebuild enqueued does
+  Tile* d_tiles = nullptr;   // tiles of the blocks (one lane per atom)
   signed char* d_atype = nullptr;
   int *d_cell_cnt = nullptr, *d_cell_beg = nullptr, *d_cell_num = nullptr;
   int *d_cell_loc = nullptr, *d_tile_sum = nullptr, *d_tile_off = nullptr,
@@ -1056,7 +1059,7 @@ StepArgs<R> step_args(imdg_ctx* c) {
 }
 
 ListEnd list_end(imdg_ctx* c) {
-  const int sh = c->list_shared ? 1 : 0;  // a block per chunk: two per block
+  const int sh = c->shared_now ? 1 : 0;  // a block per chunk: two per block
   return {c->d_ctl, c->d_rst, c->d_blk_rep, c->d_blkmax, c->nblk << sh,
           sh,       c->nrep,  c->kmax};
 }
@@ -1096,7 +1099,7 @@ BuildArgs build_args(imdg_ctx* c) {
   b.tile_rep = c->d_tile_rep;
   b.blkmax = c->d_blkmax;
   b.end = list_end(c);
-  b.list_shared = c->list_shared ? 1 : 0;
+  b.list_shared = c->shared_now ? 1 : 0;
   b.tiles = c->d_tiles;
   b.nbr = c->d_nbr;
   b.nnb = c->d_nnb;
@@ -1170,6 +1173,8 @@ int grid_build(imdg_ctx* c) {
 // (small systems).
 int enqueue_build(imdg_ctx* c, bool done, bool fin) {
   ProfScope ps(c, KC_BUILD);
+  c->shared_now = c->list_shared && !(c->all_flagged && c->one_for_all);
+  c->all_flagged = false;
   const BuildArgs b = build_args(c);
   if (c->head) {
     // the partials of the step before are those of its integrating force
@@ -1856,8 +1861,11 @@ int imdg_set_atoms(imdg_ctx* c, int nrep, const imdg_replica* reps,
   c->list_shared = true;
   for (const RepDev& R : c->rep)
     if (R.nblk > IMDG_SHARE_BLOCKS) c->list_shared = false;
+  c->one_for_all = nrep > 1 && c->nblk > IMDG_SHARE_ALL &&
+                   (c->mixed || percell >= IMDG_SHARE_DENSE);
   c->d_tiles = nullptr;
-  if (!c->list_shared) ALLOC(c->d_tiles, sizeof(Tile) * c->nblk);
+  if (!c->list_shared || c->one_for_all)
+    ALLOC(c->d_tiles, sizeof(Tile) * c->nblk);
   // places of a cell: twice the mean (an overflow enlarges them)
   if ((rc = alloc_bucket(c, (int)ceil(2 * percell)))) return rc;
   ALLOC(c->d_cell_cnt, sizeof(int) * c->ncells);
@@ -2008,6 +2016,7 @@ int imdg_set_atoms(imdg_ctx* c, int nrep, const imdg_replica* reps,
                            st));
   HIPCHK(c, hipStreamSynchronize(st));
   c->atoms_set = true;
+  c->all_flagged = true;
   c->target_steps = 0;
   return ensure_ready(c);
 }
@@ -2079,6 +2088,7 @@ static int flag_all_for_rebuild(imdg_ctx* c) {
                            hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   for (auto& s : st) s.need_rebuild = 1;
+  c->all_flagged = true;
   int one = 1;
   HIPCHK(c, hipMemcpyAsync(c->d_rst, st.data(), sizeof(RepState) * c->nrep,
                            hipMemcpyHostToDevice, c->stream));
@@ -2117,6 +2127,7 @@ int imdg_deallocate_nblist(imdg_ctx* c) {
 // operations (nothing in the step clears memory with a memset).
 static int capture_step(imdg_ctx* c) {
   hipGraph_t g = nullptr;
+  c->all_flagged = false;  // the captured rebuild is that of any step
   HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
   int rc = enqueue_build(c, false, false);
   if (!rc) rc = enqueue_forces(c, !c->split_move, true, true, true);

@@ -1263,7 +1263,7 @@ void launch_sort(const BuildArgs& b, int grid, hipStream_t st) {
 // The list, after the sort.  done: end the rebuild here (otherwise the
 // density loop of the step does).
 void launch_list(const BuildArgs& b, bool done, hipStream_t st) {
-  if (b.tiles)
+  if (!b.list_shared)
     hipLaunchKernelGGL(k_tile, dim3((b.nblk + 3) / 4), dim3(256), 0, st, b);
   const size_t tile_lds = std::max((size_t)(b.tile_cap + 4) * sizeof(float3),
                                    sizeof(TileLds));

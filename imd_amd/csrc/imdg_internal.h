@@ -133,6 +133,16 @@
 // launch of their own; 500,000 atoms 116.3 and 115.0, 2,048,000 atoms 502 and
 // 484.
 #define IMDG_SHARE_BLOCKS 2560
+// When all replicas of a batch rebuild at once, which the host knows in
+// make_nblist and for the first list, one lane from this many blocks of all of
+// them on, in mixed precision or with cells of at least so many atoms (whose
+// tiles do not fit).  make_nblist, four lanes and one: mixed EAM 100 x 4,000
+// atoms (3,200 blocks) 326 us and 343, 2 x 318,000 (4,970) 442 and 395, 30 x
+// 32,000 608 and 553, 4 x 318,000 781 and 665, LJ 300 x 2,048 556 and 445;
+// FP64 EAM 100 x 4,000 309 and 427, LJ 300 x 2,916 (46 a cell) 3,465 and
+// 1,481.
+#define IMDG_SHARE_ALL 4096
+#define IMDG_SHARE_DENSE 40
 // Device memory that a context keeps for its downloads: larger ones go out
 // in windows of this size (2.8 million atoms with every array).
 #define IMDG_OUT_BYTES (256l << 20)

@@ -1,13 +1,15 @@
 """Batches of replicas on both sides of the lines by which the rebuild chain
 is chosen: the scan of the cell counts in the binning's last block or in its
-own launch, by the number of replicas."""
+own launch, by the number of replicas and of blocks; the lanes per atom of the
+list build where all replicas rebuild at once.  The skin test of the entry
+points."""
 import numpy as np
 import pytest
 
 from imd_amd import imdg as G
 from imd_amd import workloads as W
 
-from helpers import (canon_pairs_gpu, canon_pairs_oracle, eam_tables,
+from helpers import (canon_pairs_gpu, canon_pairs_oracle, eam_tables, lj,
                      oracle_eam, rel_rms)
 from test_gpu_tuning import TOL
 
@@ -108,3 +110,43 @@ def test_scan_by_number_of_blocks(cells, nrep, monkeypatch):
     orc = oracle_eam(systems[-1], eam, nbl_margin=0.4, timestep=W.FS)
     orc.calc_forces()
     assert canon_pairs_gpu(pairs, nrep - 1) == canon_pairs_oracle(orc.pairs())
+
+
+@pytest.mark.parametrize("graph", ["0", "1"])
+@pytest.mark.parametrize("case", ["eam-mixed", "lj-fp64"])
+def test_first_list_of_a_full_chip(case, graph, monkeypatch):
+    """A batch beyond the line: its first list and make_nblist take one lane
+    per atom, the rebuilds of its steps four.  The replicas follow the
+    trajectories they have alone (four lanes throughout), bit for bit, before
+    and after a make_nblist between their steps."""
+    monkeypatch.setenv("IMDG_GRAPH", graph)
+    eam = eam_tables()
+    if case == "eam-mixed":
+        systems = [W.eam_crystal(n_cells=20, temp_k=1200.0, seed=5 + r)
+                   for r in range(17)]
+
+        def make(s):
+            return G.eam_context(eam, s, precision=G.MIXED)
+    else:
+        systems = [W.fcc_system((9, 9, 9), 1.5496, [1.0], 0.7, 5 + r)
+                   for r in range(179)]
+
+        def make(s):
+            return G.pair_context(lj(), s, precision=G.FP64, nbl_margin=0.3)
+
+    def run(s):
+        with make(s) as gpu:
+            gpu.set_tuning(2, 512, 2, 512)
+            gpu.run(30)
+            gpu.make_nblist()
+            gpu.run(30)
+            return gpu.atoms(), gpu.thermo_history(0, 60)[:, :, 6]
+
+    both, rebuilt = run(systems)
+    for r in (0, len(systems) - 1):
+        alone, t1 = run([systems[r]])
+        at = sum(s.n for s in systems[:r])
+        for k, v in alone.items():
+            assert np.array_equal(both[k][at:at + systems[r].n], v), (r, k)
+        assert np.array_equal(rebuilt[:, r], t1[:, 0])
+        assert t1[1:, 0].sum() > 1

@@ -250,3 +250,37 @@ def test_check_ends_in_its_own_launch(child):
                 assert stub.stub_launches(128) == 1
                 assert stub.stub_launches(1024) == 1, (cells, nrep)
     """)
+
+
+def test_list_kernel_of_full_rebuilds(child):
+    """Lanes per atom of the list build, told by its blocks (128 threads with
+    one lane, as the binning's, 256 with four): by the blocks of the largest
+    replica, and of all where all rebuild at once."""
+    child("""
+        eam = eam_tables()
+        def crystal(n):
+            return W.eam_crystal(n_cells=n, temp_k=0.0, seed=1)
+        def dense(n):
+            return W.fcc_system((n, n, n), 1.5496, [1.0], 0.0, 1)
+        cases = [  # systems, pair only, precision; lanes: all rebuild, some do
+            ([crystal(43)], 0, G.MIXED, 4, 4),
+            ([crystal(44)], 0, G.MIXED, 1, 1),
+            ([crystal(20)] * 16, 0, G.MIXED, 4, 4),   # 250 blocks each
+            ([crystal(20)] * 17, 0, G.MIXED, 1, 4),
+            ([crystal(20)] * 17, 0, G.FP64, 4, 4),    # 15 atoms a cell
+            ([dense(9)] * 179, 1, G.FP64, 1, 4),      # 46, 23 blocks each
+            ([dense(10)] * 129, 1, G.FP64, 4, 4),      # 32, 32 blocks each
+        ]
+        for systems, lj_only, prec, lanes_all, lanes_step in cases:
+            ctx = G.pair_context(lj(), systems, precision=prec) if lj_only \\
+                else G.eam_context(eam, systems, precision=prec)
+            with ctx:
+                ctx.set_tuning(2, 512, 2, 512)
+                for call, lanes in ((ctx.make_nblist, lanes_all),
+                                    (lambda: ctx.run(1, sync=False),
+                                     lanes_step)):
+                    stub.stub_reset_launches()
+                    call()
+                    got = 1 if stub.stub_launches(128) == 2 else 4
+                    assert got == lanes, (len(systems), systems[0].n, prec)
+    """)
