@@ -782,8 +782,9 @@ int pick_wide(int nchunk, int waves, int lanes) {
   return w;
 }
 
-// Blocks of a loop of `units` units: no more than there are units (a block beyond that would only stage tables and add
-// a partial), a multiple of the 8 XCDs.
+// Blocks of a loop of `units` units: no more than there are units (a block
+// beyond that would only stage tables and add a partial), a multiple of the 8
+// XCDs.
 int pick_grid(int resident, long units) {
   if (units >= resident) return resident;
   return std::min<long>(resident, (units + 7) / 8 * 8);
@@ -856,7 +857,8 @@ int plan_steps(imdg_ctx* c) {
   // atoms 215, 242).  The FP64 one-grid force loop on staged tables has two
   // wavefronts per SIMD and no latency to hide behind more lanes: one is
   // fastest up to the sizes of large64 (256,000 atoms 124 us, 133 with
-  // four).  The other loops keep four (LJ crystal of 4,000 atoms in FP64: 39.3 us, 47.0 with one).
+  // four).  The other loops keep four (LJ crystal of 4,000 atoms in FP64: 39.3
+  // us, 47.0 with one).
   const bool spread = (long)c->nchunk * 4 <= (long)c->ncu * IMDG_STEP_WAVES;
   if (c->lpa_den <= 0) {
     const bool onegrid = c->knots_dpoly >= 0 || c->knots_drho >= 0;

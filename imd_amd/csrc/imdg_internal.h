@@ -328,8 +328,8 @@ struct StepArgs {
   Col0<double> col64[2];  // ... of the FP64 embedding and EEAM term
   int nchunk;             // 64-slot chunks of all replicas
   int part_chunk;         // partials per unit (1) or per block (0)
-  int unitsA;             // wavefront partials written by the density loop
-  int unitsB;             // ... by the finalising force / move launch
+  int unitsA;             // partials (one per block) of the density loop
+  int unitsB;             // ... of the finalising force / move launch
   int store;              // write the per-atom outputs rho, epot, frc (the
                           // fused steps of a run skip them but on the last)
   int final_inline;       // the last block of that launch ends the step

@@ -280,7 +280,7 @@ __device__ __forceinline__ void stage_colpar(const TabDev<R>& t, int klo,
 }
 
 // ---------------------------------------------------------------------------
-// finalisation (last block of a step kernel)
+// finalisation (the end of a step)
 // ---------------------------------------------------------------------------
 
 // Per-replica end of a step from the replica's summed partials (tot[PB_N]
