@@ -2115,6 +2115,7 @@ int imdg_make_nblist(imdg_ctx* c) {
 int imdg_deallocate_nblist(imdg_ctx* c) {
   if (!c) return IMDG_ERR_ARG;
   if (!c->atoms_set) return IMDG_OK;
+  hipSetDevice(c->dev);
   HIPCHK(c, hipStreamSynchronize(c->stream));
   drop_graph(c);
   dfree(c, c->d_nbr);

@@ -94,7 +94,7 @@ hipError_t hipMemcpyAsync(void *d, const void *s, size_t n,
   return hipMemcpy(d, s, n, kind);
 }
 hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t st) {
-  (void)st;
+  if (st && *(int *)st != current) wrong_device++;   /* a fill is a launch */
   memset(d, v, n);
   return hipSuccess;
 }
